@@ -113,7 +113,7 @@ static void free_all(fsim_ctx* ctx) {
     gfx_free(ctx);
     void* ptrs[] = {ctx->P.base, ctx->Palt.base, ctx->key, ctx->rank, ctx->perm, ctx->removed, ctx->u, ctx->v, ctx->w,
                     ctx->u2, ctx->v2, ctx->w2, ctx->label, ctx->valid, ctx->density, ctx->cell_count, ctx->cell_start,
-                    ctx->scan_tmp, ctx->nbinfo, ctx->chunk_flags, ctx->b, ctx->r, ctx->z, ctx->s, ctx->q, ctx->y, ctx->P32, ctx->P64,
+                    ctx->scan_tmp, ctx->nbinfo, ctx->b, ctx->r, ctx->z, ctx->s, ctx->q, ctx->P32, ctx->P64,
                     ctx->x, ctx->partials, ctx->scal, ctx->obs_dev, ctx->ybnd, ctx->zbnd, ctx->s2, ctx->red_count,
                     ctx->wave_ticket, ctx->wave_err, ctx->sor64, ctx->colw};
     for (void* p : ptrs)
@@ -171,6 +171,8 @@ int fsim_create(const fsim_grid_desc* grid, const fsim_params* params, fsim_ctx*
     g.ny = grid->ny;
     g.nz = grid->nz;
     g.nc = (int64_t)g.nx * g.ny * g.nz;
+    g.nxp = rot_planes(g.nx);
+    g.ncr = (int64_t)g.nxp * g.ny * g.nz;
     g.cd = grid->cell_d;
     g.cdinv = 1.0 / grid->cell_d;
     g.two_d = grid->two_d ? 1 : 0;
@@ -181,24 +183,22 @@ int fsim_create(const fsim_grid_desc* grid, const fsim_params* params, fsim_ctx*
     g.dims[2] = g.nz * g.cdz;
     g.pr = grid->particle_r;
     ctx->prm = *params;
-    const int64_t nc = g.nc;
+    const int64_t nc = g.nc, ncr = g.ncr;
     int rc = FSIM_OK;
     if ((rc = dalloc(ctx, &ctx->u, nc)) || (rc = dalloc(ctx, &ctx->v, nc)) || (rc = dalloc(ctx, &ctx->w, nc)) ||
         (rc = dalloc(ctx, &ctx->u2, nc)) || (rc = dalloc(ctx, &ctx->v2, nc)) || (rc = dalloc(ctx, &ctx->w2, nc)) ||
         (rc = dalloc(ctx, &ctx->label, nc)) || (rc = dalloc(ctx, &ctx->valid, nc)) ||
         (rc = dalloc(ctx, &ctx->density, nc)) || (rc = dalloc(ctx, &ctx->cell_count, nc + 1)) ||
-        (rc = dalloc(ctx, &ctx->cell_start, nc + 2)) || (rc = dalloc(ctx, &ctx->nbinfo, nc)) ||
-        (rc = dalloc(ctx, &ctx->chunk_flags, nc / 64 + 1)) ||
-        (rc = dalloc(ctx, &ctx->b, nc)) || (rc = dalloc(ctx, &ctx->r, nc)) || (rc = dalloc(ctx, &ctx->z, nc)) ||
-        (rc = dalloc(ctx, &ctx->s, nc)) || (rc = dalloc(ctx, &ctx->s2, nc)) || (rc = dalloc(ctx, &ctx->q, nc)) ||
-        (rc = dalloc(ctx, &ctx->y, nc)) || (rc = dalloc(ctx, &ctx->red_count, 1)) ||
-        (rc = dalloc(ctx, &ctx->P32, nc)) || (rc = dalloc(ctx, &ctx->P64, nc)) || (rc = dalloc(ctx, &ctx->x, nc)) ||
+        (rc = dalloc(ctx, &ctx->cell_start, nc + 2)) || (rc = dalloc(ctx, &ctx->nbinfo, ncr)) ||
+        (rc = dalloc(ctx, &ctx->b, ncr)) || (rc = dalloc(ctx, &ctx->r, ncr)) || (rc = dalloc(ctx, &ctx->z, ncr)) ||
+        (rc = dalloc(ctx, &ctx->s, ncr)) || (rc = dalloc(ctx, &ctx->s2, ncr)) || (rc = dalloc(ctx, &ctx->q, ncr)) ||
+        (rc = dalloc(ctx, &ctx->red_count, 1)) ||
+        (rc = dalloc(ctx, &ctx->P32, ncr)) || (rc = dalloc(ctx, &ctx->P64, ncr)) || (rc = dalloc(ctx, &ctx->x, ncr)) ||
         (rc = dalloc(ctx, &ctx->scal, 1)) || (rc = dalloc(ctx, &ctx->obs_dev, kMaxObstacles)))
         return fail(rc);
     ctx->scan_tmp_cap = (nc + 2) / 4096 + 2;
     if ((rc = dalloc(ctx, &ctx->scan_tmp, ctx->scan_tmp_cap))) return fail(rc);
-    ctx->partials_cap = 2 * (int)nblocks(nc) + 16;
-    if ((rc = dalloc(ctx, &ctx->partials, ctx->partials_cap))) return fail(rc);
+    if ((rc = dalloc(ctx, &ctx->partials, 2 * kMaxParts))) return fail(rc);   // 2 per block of a reduction
     if (hipHostMalloc(reinterpret_cast<void**>(&ctx->scal_host), sizeof(SolveScalars), hipHostMallocDefault) != hipSuccess)
         return fail(FSIM_ERR_OOM);
     for (auto& e : ctx->ev)
@@ -208,14 +208,16 @@ int fsim_create(const fsim_grid_desc* grid, const fsim_params* params, fsim_ctx*
         hipEventCreateWithFlags(&ctx->x_ev, hipEventDisableTiming) != hipSuccess)
         return fail(FSIM_ERR_HIP);
     // initial grid state: zero faces, AIR labels (MacGrid ctor, macGrid.cpp:9-17)
-    float* f32s[] = {ctx->u, ctx->v, ctx->w, ctx->u2, ctx->v2, ctx->w2, ctx->density, ctx->b, ctx->r, ctx->z, ctx->s, ctx->s2,
-                     ctx->q, ctx->y, ctx->P32};
+    float* f32s[] = {ctx->u, ctx->v, ctx->w, ctx->u2, ctx->v2, ctx->w2, ctx->density};
     for (float* p : f32s)
         if (fill_f32(ctx, p, 0.0f, nc)) return fail(FSIM_ERR_HIP);
-    if (fill_u8(ctx, ctx->label, FSIM_AIR, nc) || fill_f64(ctx, ctx->x, 0.0, nc) || fill_f64(ctx, ctx->P64, 0.0, nc) ||
+    float* solver[] = {ctx->b, ctx->r, ctx->z, ctx->s, ctx->s2, ctx->q, ctx->P32};
+    for (float* p : solver)
+        if (fill_f32(ctx, p, 0.0f, ncr)) return fail(FSIM_ERR_HIP);
+    if (fill_u8(ctx, ctx->label, FSIM_AIR, nc) || fill_f64(ctx, ctx->x, 0.0, ncr) || fill_f64(ctx, ctx->P64, 0.0, ncr) ||
         fill_i32(ctx, ctx->cell_count, 0, nc + 1) || fill_i32(ctx, ctx->cell_start, 0, nc + 2))
         return fail(FSIM_ERR_HIP);
-    if (hipMemsetAsync(ctx->nbinfo, 0, sizeof(uint16_t) * nc, ctx->stream) != hipSuccess ||
+    if (hipMemsetAsync(ctx->nbinfo, 0, sizeof(uint16_t) * ncr, ctx->stream) != hipSuccess ||
         hipMemsetAsync(ctx->red_count, 0, sizeof(unsigned), ctx->stream) != hipSuccess ||
         hipStreamSynchronize(ctx->stream) != hipSuccess)
         return fail(FSIM_ERR_HIP);
@@ -479,15 +481,15 @@ int fsim_get_grid(fsim_ctx* ctx, int field, void* dst, size_t bytes) {
     }
     // solver vectors are stored in the rotated layout: gather into flat order
     const size_t elem = need / nc;
-    std::vector<unsigned char> tmp(need);
-    FSIM_HIP(ctx, hipMemcpy(tmp.data(), src, need, hipMemcpyDeviceToHost));
+    std::vector<unsigned char> tmp(elem * ctx->g.ncr);
+    FSIM_HIP(ctx, hipMemcpy(tmp.data(), src, tmp.size(), hipMemcpyDeviceToHost));
     unsigned char* out = static_cast<unsigned char*>(dst);
     const GridDims& g = ctx->g;
     for (int x = 0; x < g.nx; x++)
         for (int y = 0; y < g.ny; y++)
             for (int z = 0; z < g.nz; z++) {
                 const int64_t i = ((int64_t)x * g.ny + y) * g.nz + z;
-                std::memcpy(out + i * elem, tmp.data() + ridx(x, y, z, g.nx, g.ny, g.nz) * elem, elem);
+                std::memcpy(out + i * elem, tmp.data() + ridx(x, y, z, g.nxp, g.ny, g.nz) * elem, elem);
             }
     return FSIM_OK;
 }

@@ -7,9 +7,9 @@
 //     conditions, the reference's Face::v) and u2,v2,w2 (Face::v2);
 //   * labels are uint8 fsim_cell_type; nbinfo (uint16) caches, per WATER cell,
 //     which of the 6 neighbours are WATER and how many are not SOLID;
-//   * pressure-solve vectors are dense FP32 (b, r, z, s, q, y) with FP64
+//   * pressure-solve vectors are dense FP32 (b, r, z, s, q) with FP64
 //     pressure x and FP64 MIC(0) diagonal; entries outside WATER cells are 0;
-//     they, nbinfo and the packed W use the rotated layout of ridx() below;
+//     they and nbinfo use the rotated layout of ridx() below;
 //   * particles are FP32 SoA (pos, vel, APIC C) plus the int32 particle id
 //     (its index in the reference's particle vector), kept sorted by cell
 //     after every BIN stage.
@@ -27,6 +27,7 @@ namespace fsim {
 
 constexpr int kMaxObstacles = 64;
 constexpr int kBlock = 256;
+constexpr unsigned kMaxParts = 2048;   // reduction grids have at most this many blocks
 
 // nbinfo bit layout
 constexpr uint16_t NB_FLUID = 1u << 0;      // the cell itself is an interior WATER cell
@@ -43,89 +44,161 @@ constexpr int NB_UP_SHIFT = 10;
 
 // Persistent wavefront kernels (MIC(0) factor and triangular sweeps): a tile
 // of WF_TY x WF_TZ (y, z) columns per workgroup, WF_NW compute waves of WF_R
-// rows each plus two communication waves.
+// rows each plus three communication waves.
 #ifndef FSIM_WF_R
 #define FSIM_WF_R 2
 #endif
 #ifndef FSIM_WF_NW
-#define FSIM_WF_NW 4
+#define FSIM_WF_NW 3
 #endif
 constexpr int WF_R = FSIM_WF_R;
 constexpr int WF_NW = FSIM_WF_NW;
 constexpr int WF_TY = WF_R * WF_NW;
 constexpr int WF_TZ = 64;
-constexpr int WF_THREADS = (WF_NW + 4) * WF_TZ;   // compute waves, 2 receiving and 2 sending edge waves
-#ifndef FSIM_WF_PREFETCH
-#define FSIM_WF_PREFETCH 8
-#endif
-constexpr int WF_PREFETCH = FSIM_WF_PREFETCH;   // steps of per-cell inputs loaded ahead (and the loop unroll)
-// Steps of one tile: all rows of compute wave w are at x-index t - w - tz at
-// step t, so the last cell (wave WF_NW-1, lane 63, x-index nxi-1) is at step
-// nxi + WF_NW + WF_TZ - 3; rounded up to whole blocks of WF_PREFETCH steps
-// (the extra steps are inactive everywhere) so that no path through the step
-// loop skips a prefetch.
-__host__ __device__ inline int wave_steps(int nxi) {
-    return (nxi + WF_NW + WF_TZ - 2 + WF_PREFETCH - 1) / WF_PREFETCH * WF_PREFETCH;
-}
-// the wavefront kernels address cells with 32-bit byte offsets into arrays
-// of up to 8-byte words; larger grids use the plane-by-plane kernels
+constexpr int WF_G = 4;                           // planes per storage group (and steps per handshake)
+constexpr int WF_THREADS = (WF_NW + 3) * WF_TZ;   // compute waves, 2 receiving and a sending edge wave
+// the wavefront kernels address cells with 32-bit byte offsets into arrays of
+// 4-byte words, whose padded length is at most twice the cells (nx = 4 is
+// stored as 8 planes); larger grids use the plane-by-plane kernels
 constexpr int64_t kWaveMaxCells = ((int64_t(1) << 31) - 1) / 8;
 
-// Solver-vector layout ("rotated"): cell (x, y, z) of the pressure solve is
-// stored at plane (x + ((z - 1) mod 64)) mod nx of a dense nx*ny*nz array,
-// row y, column z.  The map is a bijection on every (y, z) column, and the
-// 64 cells of a z-tile [1 + 64k, 64 + 64k] that one wavefront step visits
-// (x = c - ((z - 1) mod 64)) share one plane, so a step reads and writes 64
-// contiguous words.  Stencil neighbours stay contiguous chunks too.
+// Solver-vector layout ("rotated, in groups of four planes").  Cell (x, y, z)
+// of the pressure solve belongs to plane p = (x + ((z - 1) mod 64)) mod nxp,
+// so that the 64 cells of a z-tile [1 + 64k, 64 + 64k] that one wavefront
+// step visits (x = c - ((z - 1) mod 64)) share one plane.  Four consecutive
+// planes are stored interleaved, the plane fastest: a lane that owns a (y, z)
+// column moves the values of four steps with one 16-byte access, and a wave
+// 1 KB of contiguous memory (a vector-memory instruction costs a compute unit
+// about 16 cycles whether its lanes move 4 or 16 bytes).  The map is a
+// bijection of every (y, z) column onto nxp planes, nxp = nx + 1 rounded up to
+// whole groups: the planes beyond nx hold no cell (zeros), and no group holds
+// both the first and the last interior cells of a column.
+__host__ __device__ inline int rot_planes(int nx) { return (nx + WF_G) / WF_G * WF_G; }
 __host__ __device__ inline int rot_of(int z) { return (z - 1) & (WF_TZ - 1); }
-__host__ __device__ inline int rot_plane(int x, int z, int nx) {
+__host__ __device__ inline int rot_plane(int x, int z, int nxp) {
     const int p = x + rot_of(z);
-    return p < nx ? p : p % nx;
+    return p < nxp ? p : p % nxp;
 }
-__host__ __device__ inline int unrot_x(int p, int z, int nx) {
+// x of plane p's cell in column z: nx .. nxp - 1 on a padding plane
+__host__ __device__ inline int unrot_x(int p, int z, int nxp) {
     const int x = p - rot_of(z);
-    return x >= 0 ? x : (x % nx + nx) % nx;
+    return x >= 0 ? x : (x % nxp + nxp) % nxp;
 }
-__host__ __device__ inline int64_t ridx(int x, int y, int z, int nx, int ny, int nz) {
-    return ((int64_t)rot_plane(x, z, nx) * ny + y) * nz + z;
+// storage index of plane p, row y, column z
+__host__ __device__ inline int64_t pidx(int p, int y, int z, int ny, int nz) {
+    return ((((int64_t)(p / WF_G) * ny + y) * nz + z) * WF_G) + (p & (WF_G - 1));
+}
+__host__ __device__ inline int64_t ridx(int x, int y, int z, int nxp, int ny, int nz) {
+    return pidx(rot_plane(x, z, nxp), y, z, ny, nz);
 }
 
 // Dimensions and scale of a pressure solve; stencil neighbours in the rotated layout.
 struct SolveArgs {
     int nx, ny, nz;
-    int off63;          // 63 mod nx: the plane shift of a z step across a 64-wide z-tile edge
-    int64_t nc;
+    int nxp;            // planes of the rotated layout
+    int off63;          // 63 mod nxp: the plane shift of a z step across a 64-wide z-tile edge
+    int64_t nc;         // cells (flat fields)
+    int64_t ncr;        // values of a solver vector: nxp * ny * nz
     float scale_f;      // dt / (rho dx^2)
     double scale;
 };
 
 // flat index of the grid fields (labels, velocities, density)
 __device__ inline int64_t sidx(const SolveArgs& S, int x, int y, int z) { return ((int64_t)x * S.ny + y) * S.nz + z; }
-// index of the solver vectors, nbinfo and W (rotated layout)
-__device__ inline int64_t rsidx(const SolveArgs& S, int x, int y, int z) { return ridx(x, y, z, S.nx, S.ny, S.nz); }
-// Rotated indices of the six neighbours of the interior cell stored at
-// plane p, row y, column z (rotated index i): +-y are +-nz; +-x are the
-// next/previous plane; +-z move one column and one plane, except across a
-// 64-wide z-tile edge where rot(z) wraps 63 <-> 0 and the plane moves by 63.
+// index of the solver vectors, nbinfo and the factor (rotated layout)
+__device__ inline int64_t rsidx(const SolveArgs& S, int x, int y, int z) { return ridx(x, y, z, S.nxp, S.ny, S.nz); }
+// Rotated indices of the six neighbours of the interior cell at plane p, row
+// y, column z: +-y stay in the plane; +-x are the next/previous plane; +-z
+// move one column and one plane, except across a 64-wide z-tile edge where
+// rot(z) wraps 63 <-> 0 and the plane moves by 63.
 struct RNeighbours {
     int64_t px, mx, py, my, pz, mz;
 };
-__device__ inline RNeighbours rneighbours(const SolveArgs& S, int64_t i, int p, int y, int z) {
-    const int64_t plane = (int64_t)S.ny * S.nz;
-    const int64_t yz = (int64_t)y * S.nz + z;
+__device__ inline RNeighbours rneighbours(const SolveArgs& S, int p, int y, int z) {
     const int rz = rot_of(z);
-    const int pn = p + 1 == S.nx ? 0 : p + 1;
-    const int pp = p == 0 ? S.nx - 1 : p - 1;
-    RNeighbours n;
-    n.px = pn * plane + yz;
-    n.mx = pp * plane + yz;
-    n.py = i + S.nz;
-    n.my = i - S.nz;
+    const int pn = p + 1 == S.nxp ? 0 : p + 1;
+    const int pp = p == 0 ? S.nxp - 1 : p - 1;
     const int o = S.off63;
-    n.pz = (rz == WF_TZ - 1 ? (p >= o ? p - o : p - o + S.nx) : pn) * plane + yz + 1;
-    n.mz = (rz == 0 ? (p + o >= S.nx ? p + o - S.nx : p + o) : pp) * plane + yz - 1;
+    RNeighbours n;
+    n.px = pidx(pn, y, z, S.ny, S.nz);
+    n.mx = pidx(pp, y, z, S.ny, S.nz);
+    n.py = pidx(p, y + 1, z, S.ny, S.nz);
+    n.my = pidx(p, y - 1, z, S.ny, S.nz);
+    n.pz = pidx(rz == WF_TZ - 1 ? (p >= o ? p - o : p - o + S.nxp) : pn, y, z + 1, S.ny, S.nz);
+    n.mz = pidx(rz == 0 ? (p + o >= S.nxp ? p + o - S.nxp : p + o) : pp, y, z - 1, S.ny, S.nz);
     return n;
 }
+// Indices around the four cells that one lane owns: planes 4g .. 4g + 3 of
+// column (y, z).  +-y are the same planes of the next rows; the +-x
+// neighbours of three of the four are the lane's own, the fourth's are element
+// 0 of the next group and element 3 of the previous one; +-z move one column
+// and one plane: elements 1, 2, 3 of group gp and 0 of the group after it (+z),
+// element 3 of the group before gm and 0, 1, 2 of gm (-z), with gp = gm = g
+// except across a z-tile edge, where the plane moves 63 = 4 * 16 - 1 back or
+// ahead.  All are in range for an interior column.
+struct ColumnNeighbours {
+    int64_t own, yp, ym, zp, zm;      // 16-byte accesses
+    int64_t xp3, xm0, zp3, zm0;       // single values: +x and +z of element 3, -x and -z of element 0
+};
+__device__ inline ColumnNeighbours column_neighbours(int ny, int nz, int ng, int g, int y, int z) {
+    const int64_t gs = (int64_t)ny * nz * WF_G;
+    const int64_t col = ((int64_t)y * nz + z) * WF_G;
+    const int rz = rot_of(z);
+    const int far = ng > 16 ? 16 : 16 % ng;
+    const int gp = rz == WF_TZ - 1 ? (g >= far ? g - far : g - far + ng) : g;
+    const int gm = rz == 0 ? (g + far >= ng ? g + far - ng : g + far) : g;
+    ColumnNeighbours n;
+    n.own = g * gs + col;
+    n.yp = n.own + (int64_t)nz * WF_G;
+    n.ym = n.own - (int64_t)nz * WF_G;
+    n.zp = gp * gs + col + WF_G;
+    n.zm = gm * gs + col - WF_G;
+    n.xp3 = (g + 1 == ng ? 0 : g + 1) * gs + col;
+    n.xm0 = (g == 0 ? ng - 1 : g - 1) * gs + col + 3;
+    n.zp3 = (gp + 1 == ng ? 0 : gp + 1) * gs + col + WF_G;
+    n.zm0 = (gm == 0 ? ng - 1 : gm - 1) * gs + col - WF_G + 3;
+    return n;
+}
+// Work split of the stencil kernels over the columns: a block of kRowWaves
+// waves takes kRowWaves consecutive interior rows of one plane group and one
+// z-tile at a time (wave: row, lane l: column z0 + l, whose rotation is l).
+// Workgroups are dispatched round-robin over the 8 XCDs (blockIdx mod 8), so
+// the block items are cut into 8 contiguous ranges, one per XCD: the +-x/+-y
+// neighbours a block reads were loaded by blocks of the same XCD (its L2).
+constexpr int kRowWaves = 4;
+struct RowItems {
+    int ntile, nrow;
+    int end;           // end of this XCD's item range (items fit in 32 bits: at most a 64th of the values)
+    int first, step;   // this block's first item and stride
+};
+__host__ __device__ inline int row_item_count(int ny, int nz, int nxp) {
+    return nxp / WF_G * ((ny - 2 + kRowWaves - 1) / kRowWaves) * ((nz - 2 + WF_TZ - 1) / WF_TZ);
+}
+__device__ inline RowItems row_items(int ny, int nz, int nxp) {
+    RowItems it;
+    it.ntile = (nz - 2 + WF_TZ - 1) / WF_TZ;
+    it.nrow = (ny - 2 + kRowWaves - 1) / kRowWaves;
+    const int total = row_item_count(ny, nz, nxp);
+    const int per_xcd = (total + 7) / 8;
+    const int begin = (int)(blockIdx.x & 7) * per_xcd;
+    it.end = min(total, begin + per_xcd);
+    it.first = begin + (int)(blockIdx.x >> 3);
+    it.step = (int)(gridDim.x >> 3);
+    return it;
+}
+// plane group, row and column of this thread for item k; false past the grid's rows or columns
+__device__ inline bool item_column(const RowItems& it, int k, int ny, int nz, int& g, int& y, int& z) {
+    const int c = k % it.ntile;
+    const int rest = k / it.ntile;
+    y = 1 + rest % it.nrow * kRowWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    g = rest / it.nrow;
+    z = 1 + c * WF_TZ + (threadIdx.x & 63);
+    return y <= ny - 2 && z <= nz - 2;
+}
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+
 // rotated indices of the +a and -a neighbours of interior cell (x, y, z)
 __device__ inline int64_t rnb_plus(const SolveArgs& S, int x, int y, int z, int a) {
     return rsidx(S, x + (a == 0), y + (a == 1), z + (a == 2));
@@ -135,9 +208,9 @@ __device__ inline int64_t rnb_minus(const SolveArgs& S, int x, int y, int z, int
 }
 
 struct WaveArgs {
-    int nx, ny, nz;
+    int nx, ny, nz, nxp;
     int TJ, TK;                   // tiles along y and z
-    int SP;                       // boundary-packet rows (steps) per tile
+    int SG;                       // boundary-packet rows (groups of WF_G steps) per tile
     const uint16_t* nbinfo;
     const float* in;
     float* out;
@@ -145,19 +218,21 @@ struct WaveArgs {
     double scale;                 // dt / (rho dx^2)
     double* P64;
     float* P32;
-    uint64_t* ybnd;               // packets across y tile edges: [tile J*TK+K][step][64][words]
-    uint64_t* zbnd;               // packets across z tile edges: [tile J*TK+K][step][WF_TY][words]
+    uint4* ybnd;                  // packets across y tile edges: [tile J*TK+K][group][1 or 2][64]
+    uint4* zbnd;                  // packets across z tile edges: [tile J*TK+K][group][1 or 2][WF_TY]
     unsigned long long* ticket;
     unsigned long long ticket_base;
-    uint32_t epoch;
     int* err;
     const uint8_t* colw;          // [y * nz + z]: 1 if the (y, z) column holds a WATER cell
-    int send_delay;               // test option: s_sleep(127) periods of the sending waves per step
+    const int* xrange;            // {least x, greatest x} of the WATER cells
+    int send_delay;               // test option: s_sleep(127) periods of the sending waves per group
 };
 
 struct GridDims {
     int nx, ny, nz;
     int64_t nc;
+    int nxp;              // planes of the solver vectors' rotated layout
+    int64_t ncr;          // values of a solver vector
     double cd, cdinv;     // cellD.x == cellD.y
     double cdz, cdzinv;   // cellD.z (cd except in 2D)
     double dims[3];
@@ -168,6 +243,7 @@ struct GridDims {
 // Device-resident scalars of the pressure solve (one cache line each group).
 struct SolveScalars {
     double sigma, alpha, beta, sq;   // PCG scalars
+    double alpha_prev;               // alpha of the direction step before
     double rr, rmax, bb;             // recursive residual ||r||^2, max|r|, ||b||^2
     double tr_ss, tr_max;            // true residual ||b-Ax||^2, max|b-Ax|
     double zr;                       // z.r
@@ -231,11 +307,13 @@ struct fsim_ctx {
     int32_t* cell_start = nullptr;   // Nc + 2
     int32_t* scan_tmp = nullptr;
     uint16_t* nbinfo = nullptr;
-    uint8_t* colw = nullptr;          // WATER columns (y, z) of the current labels, for the wavefront kernels
-    uint32_t* chunk_flags = nullptr;  // solver-vector chunks (64 or 256 cells) holding a WATER cell, per solve
+    uint8_t* colw = nullptr;          // WATER columns (y, z) of the current labels, for the wavefront kernels,
+                                      // and behind them the x range of the WATER cells (WaveArgs::xrange)
+                                      // and the chunk flags
+    uint32_t* chunk_flags = nullptr;  // solver-vector chunks (256 values) holding a WATER cell, per solve
 
     // pressure solve
-    float *b = nullptr, *r = nullptr, *z = nullptr, *s = nullptr, *q = nullptr, *y = nullptr;
+    float *b = nullptr, *r = nullptr, *z = nullptr, *s = nullptr, *q = nullptr;
     float* s2 = nullptr;              // second search-direction buffer (swapped with s)
     float* P32 = nullptr;
     double* P64 = nullptr;
@@ -258,17 +336,16 @@ struct fsim_ctx {
     int wave_send_delay = 0;              // test option: sending-wave pause per step (s_sleep 127 units)
     int learned_gen = 0;                  // bumped when the network's per-size buffers are reallocated
     bool mg_harvesting = false;           // a solve run by fsim_learned_harvest
-    int partials_cap = 0;
     fsim::SolveScalars* scal = nullptr;   // device
     fsim::SolveScalars* scal_host = nullptr;  // pinned host mirror
     double last_dt = 0.0;
     // wavefront sweeps
     fsim::WaveArgs wave{};
-    uint64_t* ybnd = nullptr;
-    uint64_t* zbnd = nullptr;
+    uint4* ybnd = nullptr;
+    uint4* zbnd = nullptr;
     unsigned long long* wave_ticket = nullptr;   // 3 counters: factor, fwd, bwd
     unsigned long long wave_ticket_base[3] = {0, 0, 0};
-    uint32_t wave_epoch = 0;
+    int64_t wave_packets[2] = {0, 0};            // 16-byte packets of ybnd, zbnd
     int* wave_err = nullptr;
     int sweep_mode = 0;                          // 0 wavefront, 1 one launch per plane
     int learned_smoothing = 2;                   // red-black sweeps after the network on the coarsest level

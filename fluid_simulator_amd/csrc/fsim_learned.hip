@@ -442,13 +442,14 @@ __global__ void k_upcat(const __bf16* __restrict__ coarse, const __bf16* __restr
 // the solver's r and nbinfo (rotated layout: the 7-point operator of the
 // WATER cells, couplings 1 towards WATER neighbours) ...
 __global__ void k_net_input(const float* __restrict__ r, const uint16_t* __restrict__ nbinfo,
-                            const float* __restrict__ scale, __bf16* __restrict__ x0, Dims nd, int nx, int ny, int nz) {
+                            const float* __restrict__ scale, __bf16* __restrict__ x0, Dims nd, int nx, int ny, int nz,
+                            int nxp) {
     const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= nd.V()) return;
     const int z = (int)(v % nd.W), y = (int)((v / nd.W) % nd.H), x = (int)(v / ((int64_t)nd.W * nd.H));
     float val = 0.f, fl = 0.f, dg = 0.f, cx = 0.f, cy = 0.f, cz = 0.f;
     if (x < nx && y < ny && z < nz) {
-        const int64_t i = ridx(x, y, z, nx, ny, nz);
+        const int64_t i = ridx(x, y, z, nxp, ny, nz);
         const uint16_t f = nbinfo[i];
         if (f & NB_FLUID) {
             fl = 1.f;
@@ -520,13 +521,13 @@ __global__ void k_conv1_fwd(const __bf16* __restrict__ d0, const float* __restri
 // z (solver layout) = WATER ? out * s * mult : 0
 __global__ void k_net_output(const float* __restrict__ out, const uint16_t* __restrict__ nbinfo,
                              const float* __restrict__ scale, float mult, float* __restrict__ z, Dims nd, int nx, int ny,
-                             int nz) {
+                             int nz, int nxp) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int64_t nc = (int64_t)nx * ny * nz;
     if (i >= nc) return;
     // i is a flat cell index; write its rotated slot
     const int zc = (int)(i % nz), yc = (int)((i / nz) % ny), xc = (int)(i / ((int64_t)nz * ny));
-    const int64_t ri = ridx(xc, yc, zc, nx, ny, nz);
+    const int64_t ri = ridx(xc, yc, zc, nxp, ny, nz);
     const int64_t v = ((int64_t)xc * nd.H + yc) * nd.W + zc;
     if (nbinfo[ri] & NB_FLUID) z[ri] = out[v] * *scale * mult;
 }
@@ -1073,15 +1074,15 @@ int learned_apply_level0(fsim_ctx* ctx, const float* r, float* z, float binv) {
     hipStream_t st = ctx->stream;
     const int64_t nc = ctx->g.nc;
     FSIM_TRY(fill_i32(ctx, reinterpret_cast<int32_t*>(N->scale_bits), 0, 1));   // a kernel: graph-capturable
-    hipLaunchKernelGGL(k_absmax, dim3(std::min<unsigned>(gb(nc), 2048u)), dim3(256), 0, st, r, ctx->nbinfo, nc,
-                       N->scale_bits);
+    hipLaunchKernelGGL(k_absmax, dim3(std::min<unsigned>(gb(ctx->g.ncr), 2048u)), dim3(256), 0, st, r, ctx->nbinfo,
+                       ctx->g.ncr, N->scale_bits);
     static_assert(sizeof(unsigned) == sizeof(float), "scale bits");
     const float* sc = reinterpret_cast<const float*>(N->scale_bits);
     hipLaunchKernelGGL(k_net_input, dim3(gb(N->lv[0].V())), dim3(256), 0, st, r, ctx->nbinfo, sc, N->x0, N->lv[0],
-                       ctx->g.nx, ctx->g.ny, ctx->g.nz);
+                       ctx->g.nx, ctx->g.ny, ctx->g.nz, ctx->g.nxp);
     FSIM_TRY(net_forward(ctx, false));
     hipLaunchKernelGGL(k_net_output, dim3(gb(nc)), dim3(256), 0, st, N->out, ctx->nbinfo, sc, binv, z, N->lv[0], ctx->g.nx,
-                       ctx->g.ny, ctx->g.nz);
+                       ctx->g.ny, ctx->g.nz, ctx->g.nxp);
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;
 }

@@ -30,6 +30,7 @@
 #include <algorithm>
 #include <cmath>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "fsim_internal.hpp"
@@ -54,24 +55,12 @@ __device__ inline void unlin(int64_t i, int ny, int nz, int& x, int& y, int& z) 
 }
 
 struct Mg0 {               // level 0: the solve's operator in the rotated layout
-    int nx, ny, nz, off63;
-    int64_t nc;
+    int nx, ny, nz, nxp;
     const uint16_t* nbinfo;
     const float* b;        // r of the PCG iteration
     float* x;              // z
     float binv;            // 1 / s: level 0 solves L0 x = r / s
 };
-__device__ inline SolveArgs mg0_args(const Mg0& A) {
-    SolveArgs S;
-    S.nx = A.nx;
-    S.ny = A.ny;
-    S.nz = A.nz;
-    S.off63 = A.off63;
-    S.nc = A.nc;
-    S.scale_f = 0.f;
-    S.scale = 0.0;
-    return S;
-}
 __device__ inline int nb_nonsolid(uint16_t nb) { return (nb >> NB_NONSOLID_SHIFT) & 7; }
 
 // ---- coarsening ---------------------------------------------------------------------
@@ -90,7 +79,7 @@ __global__ void __launch_bounds__(kBlock) k_mg_coarsen0(Mg0 F, int cx, int cy, i
         const int a = k >> 2, b = (k >> 1) & 1, e = k & 1;
         const int x = 2 * X + a, y = 2 * Y + b, z = 2 * Z + e;
         if (x >= F.nx || y >= F.ny || z >= F.nz) continue;
-        const uint16_t nb = F.nbinfo[ridx(x, y, z, F.nx, F.ny, F.nz)];
+        const uint16_t nb = F.nbinfo[ridx(x, y, z, F.nxp, F.ny, F.nz)];
         if (!(nb & NB_FLUID)) continue;
         d += (float)nb_nonsolid(nb);
         const bool up[3] = {(nb & NB_PX) != 0, (nb & NB_PY) != 0, (nb & NB_PZ) != 0};
@@ -140,12 +129,9 @@ __global__ void __launch_bounds__(kBlock) k_mg_coarsen(MgGrid F, int cx, int cy,
 }
 
 // ---- smoothing: one red-black half-sweep --------------------------------------------
-// Launch shape of the per-cell kernels: a block is kMgBy rows (y) x kMgBz
-// columns (z) of one plane (level 0: rotated plane p; coarse levels: x), the
-// grid (z chunks, y chunks, planes), so no thread divides its index.  In the
-// rotated layout x + z is constant along each 64-column z-tile of a plane
-// row (x = p - ((z - 1) mod 64) up to the wrap by nx), so for even nx a row
-// has one colour and a half-sweep's other-colour rows leave at once.
+// Launch shape of the coarse levels' per-cell kernels: a block is kMgBy rows
+// (y) x kMgBz columns (z) of one plane x, the grid (z chunks, y chunks,
+// planes), so no thread divides its index.
 constexpr int kMgBz = 64, kMgBy = 4;
 struct MgLaunch {
     dim3 grid, block;
@@ -158,39 +144,81 @@ static MgLaunch mg_launch(int nx, int ny, int nz) {
                     dim3((unsigned)bz, (unsigned)by)};
 }
 
+// Level 0: a lane owns the four cells of a column of a plane group
+// (ColumnNeighbours).  x + z = p + 1 (mod 2) on plane p, since (z - 1) mod 64
+// has the parity of z - 1 and the wrap adds nxp, a multiple of 4: the cells of
+// one colour in row y are the elements c with (c + 1 + y) mod 2 equal to it,
+// two of a lane's four.  A wave has one row, so the choice is uniform.
+struct Column4 {
+    f32x4 own, yp, ym, zp, zm;
+    float xe, ze;   // the neighbours of the colour's outer element from the next or previous group
+};
+// odd: elements 1 and 3 (whose outer neighbours are ahead), else 0 and 2 (behind)
+__device__ inline Column4 load_column(const float* x, const ColumnNeighbours& n, bool odd) {
+    Column4 v;
+    v.own = *reinterpret_cast<const f32x4*>(x + n.own);
+    v.yp = *reinterpret_cast<const f32x4*>(x + n.yp);
+    v.ym = *reinterpret_cast<const f32x4*>(x + n.ym);
+    v.zp = *reinterpret_cast<const f32x4*>(x + n.zp);
+    v.zm = *reinterpret_cast<const f32x4*>(x + n.zm);
+    v.xe = x[odd ? n.xp3 : n.xm0];
+    v.ze = x[odd ? n.zp3 : n.zm0];
+    return v;
+}
+// the neighbours of element c in the order -x, +x, -y, +y, -z, +z
+template <int C>
+__device__ inline void column_terms(const Column4& v, float (&t)[6]) {
+    t[0] = C > 0 ? v.own[(C + 3) & 3] : v.xe;
+    t[1] = C < 3 ? v.own[(C + 1) & 3] : v.xe;
+    t[2] = v.ym[C];
+    t[3] = v.yp[C];
+    t[4] = C > 0 ? v.zm[(C + 3) & 3] : v.ze;
+    t[5] = C < 3 ? v.zp[(C + 1) & 3] : v.ze;
+}
+constexpr uint16_t kMgNb[6] = {NB_MX, NB_PX, NB_MY, NB_PY, NB_MZ, NB_PZ};
+
 // FIRST: the first half-sweep from x = 0 (no neighbour terms; the other colour
-// is set to 0 on the level's unknowns).  ROWS (even nx, not FIRST): the grid
-// covers only the rows of colour PAR: x + z = p + 1 (mod 2) on every rotated
-// row, since (z - 1) mod 64 has the parity of z - 1 and the wrap adds nx.
-template <int PAR, bool FIRST, bool ROWS = false>
-__global__ void __launch_bounds__(kMgBz * kMgBy) k_mg_rbgs0(Mg0 A) {
-    static_assert(!(FIRST && ROWS), "the first half-sweep also clears the other colour");
-    const int z = blockIdx.x * blockDim.x + threadIdx.x;
-    const int p = blockIdx.z;
-    const int yr = blockIdx.y * blockDim.y + threadIdx.y;
-    const int y = ROWS ? 2 * yr + ((PAR + p + 1) & 1) : yr;
-    if (z >= A.nz || y >= A.ny) return;
-    const int x = unrot_x(p, z, A.nx);
-    const bool mine = ROWS || ((x + y + z) & 1) == PAR;
-    if (!FIRST && !mine) return;
-    const int64_t i = ((int64_t)p * A.ny + y) * A.nz + z;
-    const uint16_t nb = A.nbinfo[i];
-    if (!(nb & NB_FLUID)) return;
-    if (!mine) {
-        A.x[i] = 0.f;   // FIRST only
-        return;
+// is set to 0).
+template <int PAR, bool FIRST>
+__global__ void __launch_bounds__(kBlock) k_mg_rbgs0(Mg0 A) {
+    const RowItems it = row_items(A.ny, A.nz, A.nxp);
+    for (int k = it.first; k < it.end; k += it.step) {
+        int g, y, z;
+        if (!item_column(it, k, A.ny, A.nz, g, y, z)) continue;
+        const ColumnNeighbours n = column_neighbours(A.ny, A.nz, A.nxp / WF_G, g, y, z);
+        const u16x4 nb = *reinterpret_cast<const u16x4*>(A.nbinfo + n.own);
+        if (((nb[0] | nb[1] | nb[2] | nb[3]) & NB_FLUID) == 0) continue;
+        const f32x4 b = *reinterpret_cast<const f32x4*>(A.b + n.own);
+        const bool odd = ((PAR + 1 + y) & 1) != 0;
+        if constexpr (FIRST) {
+            f32x4 out = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < 4; c++)
+                if ((c & 1) == (int)odd && (nb[c] & NB_FLUID)) out[c] = b[c] * A.binv / (float)nb_nonsolid(nb[c]);
+            *reinterpret_cast<f32x4*>(A.x + n.own) = out;
+        } else {
+            const Column4 v = load_column(A.x, n, odd);
+            f32x4 out = v.own;
+            auto cell = [&](auto cc) {
+                constexpr int c = decltype(cc)::value;
+                if (!(nb[c] & NB_FLUID)) return;
+                float t[6];
+                column_terms<c>(v, t);
+                float s = b[c] * A.binv;
+#pragma unroll
+                for (int j = 0; j < 6; j++) s = (nb[c] & kMgNb[j]) ? s + t[j] : s;
+                out[c] = s / (float)nb_nonsolid(nb[c]);
+            };
+            if (odd) {
+                cell(std::integral_constant<int, 1>{});
+                cell(std::integral_constant<int, 3>{});
+            } else {
+                cell(std::integral_constant<int, 0>{});
+                cell(std::integral_constant<int, 2>{});
+            }
+            *reinterpret_cast<f32x4*>(A.x + n.own) = out;
+        }
     }
-    float s = A.b[i] * A.binv;
-    if (!FIRST) {
-        const RNeighbours n = rneighbours(mg0_args(A), i, p, y, z);
-        if (nb & NB_MX) s += A.x[n.mx];
-        if (nb & NB_PX) s += A.x[n.px];
-        if (nb & NB_MY) s += A.x[n.my];
-        if (nb & NB_PY) s += A.x[n.py];
-        if (nb & NB_MZ) s += A.x[n.mz];
-        if (nb & NB_PZ) s += A.x[n.pz];
-    }
-    A.x[i] = s / (float)nb_nonsolid(nb);
 }
 
 template <int PAR, bool FIRST>
@@ -224,75 +252,59 @@ __global__ void __launch_bounds__(kMgBz * kMgBy) k_mg_rbgs(MgGrid G) {
 
 // ---- residual + restriction -----------------------------------------------------------
 // b_{l+1}[I] = sum over the fluid children i of (b_i - (L x)_i).
-// Level 0 takes two passes.  The children of a coarse cell lie in different
-// rotated planes (x + ((z - 1) mod 64) differs between them), so a thread per
-// coarse cell gathering them reads every word from another plane.  Instead,
-// k_mg_resid0 writes the level-0 residual in the rotated layout (0 off the
-// unknowns), a block-coalesced pass like the smoothing; then each block of
-// k_mg_restrict_rot reads the rotated rows that hold a 64 (x) x 2 (y) x 64 (z)
-// fine box, each row a contiguous run along z, into LDS, and sums every
+// Level 0: the children of a coarse cell lie in different rotated planes (x +
+// ((z - 1) mod 64) differs between them), so a thread per coarse cell
+// gathering them would read every value from another plane.  Instead a block
+// computes the residual of a 64 (x) x 2 (y) x 64 (z) fine box by columns of
+// plane groups, each wave contiguous memory, puts it into LDS, and sums every
 // coarse cell's 8 children there in a fixed order.
 // The residual follows the last pre-smoothing half-sweep, which solved the
-// rows of colour 0 exactly: their residual is 0 (up to rounding) and ROWS
-// (even nx, whose rotated rows each have one colour) computes only the rows
-// of colour 1; the buffer's colour-0 rows keep the zeros of its allocation.
-template <bool ROWS>
-__global__ void __launch_bounds__(kMgBz * kMgBy) k_mg_resid0(Mg0 A, float* __restrict__ res) {
-    const int z = blockIdx.x * blockDim.x + threadIdx.x;
-    const int p = blockIdx.z;
-    const int yr = blockIdx.y * blockDim.y + threadIdx.y;
-    const int y = ROWS ? 2 * yr + (p & 1) : yr;   // colour 1: p + 1 + y odd
-    if (z >= A.nz || y >= A.ny) return;
-    const int64_t i = ((int64_t)p * A.ny + y) * A.nz + z;
-    const uint16_t nb = A.nbinfo[i];
-    float r = 0.f;
-    if (nb & NB_FLUID) {
-        const RNeighbours n = rneighbours(mg0_args(A), i, p, y, z);
-        float ax = (float)nb_nonsolid(nb) * A.x[i];
-        if (nb & NB_MX) ax -= A.x[n.mx];
-        if (nb & NB_PX) ax -= A.x[n.px];
-        if (nb & NB_MY) ax -= A.x[n.my];
-        if (nb & NB_PY) ax -= A.x[n.py];
-        if (nb & NB_MZ) ax -= A.x[n.mz];
-        if (nb & NB_PZ) ax -= A.x[n.pz];
-        r = A.b[i] * A.binv - ax;
-    }
-    res[i] = r;
-}
-
+// cells of colour 0 exactly: their residual is 0 (up to rounding) and only the
+// cells of colour 1 are computed.
 constexpr int kRtC = 32;   // coarse cells per block along x and along z (a 64 x 2 x 64 fine box)
-constexpr int kRtBatch = 8;   // rotated rows a wave loads before storing them
-__global__ void __launch_bounds__(256) k_mg_restrict_rot(Mg0 A, const float* __restrict__ res, MgGrid C) {
-    // fine box [yy][x - fx0][z - fz0]; a row of 64 words: the lanes of one rotated
-    // row store with a stride of -63 words, a different bank each
+__global__ void __launch_bounds__(256) k_mg_resid_restrict0(Mg0 A, MgGrid C) {
+    // fine box [yy][x - fx0][z - fz0]; a row of 64 words: the lanes of a wave store into a different
+    // bank each
     __shared__ float F[2][2 * kRtC][2 * kRtC];
     const int X0 = blockIdx.x * kRtC, Y = blockIdx.y, Z0 = blockIdx.z * kRtC;
     const int fx0 = 2 * X0, fz0 = 2 * Z0;
     for (int k = threadIdx.x; k < 2 * 2 * kRtC * 2 * kRtC; k += blockDim.x) (&F[0][0][0])[k] = 0.f;
     __syncthreads();
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwaves = blockDim.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nwaves = blockDim.x >> 6;
     const int z = fz0 + lane;
     const int rz = rot_of(z);
-    // the cells x in [fx0, fx0 + 64) of column z are in the rotated rows fx0 + rz .. fx0 + rz + 63:
-    // rows fx0 .. fx0 + 126 cover the box; each wave loads kRtBatch rows, then stores them
-    constexpr int kRows = 2 * kRtC + 63;
-    for (int k0 = wave * kRtBatch; k0 < 2 * kRows; k0 += nwaves * kRtBatch) {
-        float v[kRtBatch];
-        int dst[kRtBatch];
+    const int ng = A.nxp / WF_G;
+    // the cells x in [fx0, fx0 + 64) of column z are on the planes fx0 + rz .. fx0 + rz + 63
+    constexpr int kGroups = (2 * kRtC + 63) / WF_G + 1;
+    for (int k = wave; k < 2 * kGroups; k += nwaves) {
+        const int yy = k / kGroups, gu = fx0 / WF_G + k % kGroups;   // unwrapped group
+        const int y = 2 * Y + yy;
+        const int x0 = WF_G * gu - rz;                               // x of element 0
+        if (y < 1 || y > A.ny - 2 || z < 1 || z > A.nz - 2 || x0 + 3 < fx0 || x0 >= fx0 + 2 * kRtC) continue;
+        const ColumnNeighbours n = column_neighbours(A.ny, A.nz, ng, gu % ng, y, z);
+        const u16x4 nb = *reinterpret_cast<const u16x4*>(A.nbinfo + n.own);
+        if (((nb[0] | nb[1] | nb[2] | nb[3]) & NB_FLUID) == 0) continue;
+        const bool odd = (y & 1) != 0;   // colour 1: (c + 1 + y) odd
+        const Column4 v = load_column(A.x, n, odd);
+        const f32x4 b = *reinterpret_cast<const f32x4*>(A.b + n.own);
+        auto cell = [&](auto cc) {
+            constexpr int c = decltype(cc)::value;
+            const int x = x0 + c;
+            if (!(nb[c] & NB_FLUID) || x < fx0 || x >= fx0 + 2 * kRtC || x >= A.nx) return;
+            float t[6];
+            column_terms<c>(v, t);
+            float ax = (float)nb_nonsolid(nb[c]) * v.own[c];
 #pragma unroll
-        for (int j = 0; j < kRtBatch; j++) {
-            const int k = k0 + j;
-            const int yy = k / kRows, pr = fx0 + k % kRows;
-            const int y = 2 * Y + yy;
-            const int x = pr - rz;
-            const bool ok = k < 2 * kRows && y < A.ny && z < A.nz && x >= fx0 && x < fx0 + 2 * kRtC && x < A.nx;
-            const int prow = pr < A.nx ? pr : pr % A.nx;   // rot_plane(x, z)
-            v[j] = ok ? res[((int64_t)prow * A.ny + y) * A.nz + z] : 0.f;
-            dst[j] = ok ? (yy * 2 * kRtC + (x - fx0)) * 2 * kRtC + lane : -1;
+            for (int j = 0; j < 6; j++) ax = (nb[c] & kMgNb[j]) ? ax - t[j] : ax;
+            F[yy][x - fx0][lane] = b[c] * A.binv - ax;
+        };
+        if (odd) {
+            cell(std::integral_constant<int, 1>{});
+            cell(std::integral_constant<int, 3>{});
+        } else {
+            cell(std::integral_constant<int, 0>{});
+            cell(std::integral_constant<int, 2>{});
         }
-#pragma unroll
-        for (int j = 0; j < kRtBatch; j++)
-            if (dst[j] >= 0) (&F[0][0][0])[dst[j]] = v[j];
     }
     __syncthreads();
     for (int k = threadIdx.x; k < kRtC * kRtC; k += blockDim.x) {
@@ -340,15 +352,22 @@ __global__ void __launch_bounds__(kBlock) k_mg_restrict(MgGrid F, MgGrid C) {
 }
 
 // ---- prolongation: x_i += 1.6 x_{l+1}[parent(i)] on the level's unknowns ----------------
-__global__ void __launch_bounds__(kMgBz * kMgBy) k_mg_prolong0(Mg0 A, MgGrid C) {
-    const int z = blockIdx.x * blockDim.x + threadIdx.x;
-    const int y = blockIdx.y * blockDim.y + threadIdx.y;
-    const int p = blockIdx.z;
-    if (z >= A.nz || y >= A.ny) return;
-    const int64_t i = ((int64_t)p * A.ny + y) * A.nz + z;
-    if (!(A.nbinfo[i] & NB_FLUID)) return;
-    const int x = unrot_x(p, z, A.nx);
-    A.x[i] += kMgOverCorrect * C.x[lin(C.nx, C.ny, C.nz, x >> 1, y >> 1, z >> 1)];
+__global__ void __launch_bounds__(kBlock) k_mg_prolong0(Mg0 A, MgGrid C) {
+    const RowItems it = row_items(A.ny, A.nz, A.nxp);
+    for (int k = it.first; k < it.end; k += it.step) {
+        int g, y, z;
+        if (!item_column(it, k, A.ny, A.nz, g, y, z)) continue;
+        const int64_t i = pidx(g * WF_G, y, z, A.ny, A.nz);
+        const u16x4 nb = *reinterpret_cast<const u16x4*>(A.nbinfo + i);
+        if (((nb[0] | nb[1] | nb[2] | nb[3]) & NB_FLUID) == 0) continue;
+        f32x4 x = *reinterpret_cast<const f32x4*>(A.x + i);
+#pragma unroll
+        for (int c = 0; c < 4; c++)
+            if (nb[c] & NB_FLUID)
+                x[c] += kMgOverCorrect *
+                        C.x[lin(C.nx, C.ny, C.nz, unrot_x(g * WF_G + c, z, A.nxp) >> 1, y >> 1, z >> 1)];
+        *reinterpret_cast<f32x4*>(A.x + i) = x;
+    }
 }
 
 __global__ void __launch_bounds__(kMgBz * kMgBy) k_mg_prolong(MgGrid F, MgGrid C) {
@@ -370,7 +389,6 @@ struct MgLevelBuf {
 struct MgState {
     int nlev = 0;   // levels 0 .. nlev-1; nlev-1 is the coarse (network) level
     MgLevelBuf lv[kMgMaxLevels];
-    float* res0 = nullptr;   // level-0 residual, rotated layout
     std::vector<void*> allocs;
     // harvest: up to cap coarse (b, x) pairs of the running solve
     int harvest_cap = 0, harvest_n = 0;
@@ -426,12 +444,6 @@ static int mg_alloc(fsim_ctx* ctx) {
     M->lv[0].ny = ctx->g.ny;
     M->lv[0].nz = ctx->g.nz;
     M->lv[0].nc = ctx->g.nc;
-    if (M->nlev > 1) {
-        if (hipMalloc(reinterpret_cast<void**>(&M->res0), sizeof(float) * (size_t)ctx->g.nc) != hipSuccess)
-            return set_err(ctx, FSIM_ERR_OOM, "multigrid residual allocation failed");
-        M->allocs.push_back(M->res0);
-        FSIM_TRY(fill_f32(ctx, M->res0, 0.0f, ctx->g.nc));   // the colour-0 rows stay 0 (k_mg_resid0)
-    }
     for (int l = 1; l < M->nlev; l++) {
         MgLevelBuf& L = M->lv[l];
         L.nx = (M->lv[l - 1].nx + 1) / 2;
@@ -454,8 +466,7 @@ static Mg0 mg0(fsim_ctx* ctx, const float* r, float* z, double scale) {
     A.nx = ctx->g.nx;
     A.ny = ctx->g.ny;
     A.nz = ctx->g.nz;
-    A.off63 = 63 % ctx->g.nx;
-    A.nc = ctx->g.nc;
+    A.nxp = ctx->g.nxp;
     A.nbinfo = ctx->nbinfo;
     A.b = r;
     A.x = z;
@@ -487,18 +498,17 @@ int mg_setup(fsim_ctx* ctx) {
     return FSIM_OK;
 }
 
+// blocks of the level-0 column kernels: one per item
+static dim3 mg0_blocks(const Mg0& A) {
+    return dim3((unsigned)(row_item_count(A.ny, A.nz, A.nxp) + 7) / 8 * 8);
+}
+
 static void smooth0(fsim_ctx* ctx, const Mg0& A, int sweeps, bool first) {
-    const MgLaunch L = mg_launch(A.nx, A.ny, A.nz);
-    const dim3 g = L.grid, b = L.block;
-    // even nx: the non-first half-sweeps launch the rows of their colour only
-    const MgLaunch H = mg_launch(A.nx, (A.ny + 1) / 2, A.nz);
-    const bool rows = (A.nx & 1) == 0;
+    const dim3 g = mg0_blocks(A), b(kBlock);
     for (int k = 0; k < sweeps; k++) {
         if (first && k == 0) hipLaunchKernelGGL((k_mg_rbgs0<1, true>), g, b, 0, ctx->stream, A);
-        else if (rows) hipLaunchKernelGGL((k_mg_rbgs0<1, false, true>), H.grid, H.block, 0, ctx->stream, A);
         else hipLaunchKernelGGL((k_mg_rbgs0<1, false>), g, b, 0, ctx->stream, A);
-        if (rows) hipLaunchKernelGGL((k_mg_rbgs0<0, false, true>), H.grid, H.block, 0, ctx->stream, A);
-        else hipLaunchKernelGGL((k_mg_rbgs0<0, false>), g, b, 0, ctx->stream, A);
+        hipLaunchKernelGGL((k_mg_rbgs0<0, false>), g, b, 0, ctx->stream, A);
     }
 }
 static void smooth(fsim_ctx* ctx, const MgLevelBuf& L, int sweeps, bool first) {
@@ -555,16 +565,9 @@ static int vcycle(fsim_ctx* ctx, const float* r, float* z, double scale) {
     // down: level 0, then 1 .. c-1
     smooth0(ctx, A, kMgPreSweeps, true);
     {
-        if ((A.nx & 1) == 0) {
-            const MgLaunch R = mg_launch(A.nx, (A.ny + 1) / 2, A.nz);
-            hipLaunchKernelGGL(k_mg_resid0<true>, R.grid, R.block, 0, ctx->stream, A, M->res0);
-        } else {
-            const MgLaunch R = mg_launch(A.nx, A.ny, A.nz);
-            hipLaunchKernelGGL(k_mg_resid0<false>, R.grid, R.block, 0, ctx->stream, A, M->res0);
-        }
         const MgLevelBuf& L1 = M->lv[1];
         const dim3 g((unsigned)((L1.nx + kRtC - 1) / kRtC), (unsigned)L1.ny, (unsigned)((L1.nz + kRtC - 1) / kRtC));
-        hipLaunchKernelGGL(k_mg_restrict_rot, g, dim3(256), 0, ctx->stream, A, M->res0, grid_of(L1));
+        hipLaunchKernelGGL(k_mg_resid_restrict0, g, dim3(256), 0, ctx->stream, A, grid_of(L1));
     }
     for (int l = 1; l < c; l++) {
         smooth(ctx, M->lv[l], kMgPreSweeps, true);
@@ -578,8 +581,7 @@ static int vcycle(fsim_ctx* ctx, const float* r, float* z, double scale) {
         hipLaunchKernelGGL(k_mg_prolong, P.grid, P.block, 0, ctx->stream, grid_of(M->lv[l]), grid_of(M->lv[l + 1]));
         smooth(ctx, M->lv[l], kMgPostSweeps, false);
     }
-    const MgLaunch P0 = mg_launch(A.nx, A.ny, A.nz);
-    hipLaunchKernelGGL(k_mg_prolong0, P0.grid, P0.block, 0, ctx->stream, A, grid_of(M->lv[1]));
+    hipLaunchKernelGGL(k_mg_prolong0, mg0_blocks(A), dim3(kBlock), 0, ctx->stream, A, grid_of(M->lv[1]));
     smooth0(ctx, A, kMgPostSweeps, false);
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;

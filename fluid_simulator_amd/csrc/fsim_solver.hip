@@ -47,7 +47,6 @@ __device__ inline double wave_max(double v) {
 // counter.  The sum's order does not depend on which block is last, so the
 // result is deterministic, and no separate finalize launch is needed.
 constexpr int AUX_NONE = 0, AUX_MAX = 1, AUX_SUM = 2;
-constexpr unsigned kMaxParts = 2048;   // reduction grids have at most this many blocks, a multiple of 8
 enum FinOp {
     FIN_NONE = -1, FIN_BB = 0, FIN_SIGMA0 = 1, FIN_ALPHA = 2, FIN_RES = 3, FIN_BETA = 4, FIN_TRUE = 5, FIN_ZQ = 6,
     FIN_FBETA = 7
@@ -69,6 +68,7 @@ __device__ inline void apply_fin(int op, double s, double m, SolveScalars* sc) {
         sc->sigma = sc->zr;
         sc->sq = s;
         const double alpha = sc->sigma / s;
+        sc->alpha_prev = sc->alpha;
         sc->alpha = alpha;
         if (alpha != alpha) sc->nan_flag |= 1;
         break;
@@ -173,6 +173,8 @@ __device__ void block_finish(double sum, double aux, const Reduce& R) {
     }
 }
 
+constexpr int kChunk = 256;   // values of a solver vector per chunk flag (the streaming kernels)
+
 // ---- RHS and neighbour masks (calculateRHS :79-89, calculateAMatrix :40-77) ------
 struct RhsArgs {
     SolveArgs S;
@@ -181,9 +183,10 @@ struct RhsArgs {
     const float* v2;
     const float* w2;
     const float* density;
-    uint16_t* nbinfo;
+    uint16_t* info_flat;   // masks and b in flat order (k_rotate moves them to the solver's layout)
+    float* b_flat;
     uint8_t* colw;   // set to 1 for the (y, z) column of each WATER cell (cleared before)
-    float* b;
+    uint8_t* xw;     // the same for the x rows
     double inv_dx;
     double avg_p, pk;
     int pressure_enabled;
@@ -192,6 +195,40 @@ struct RhsArgs {
 
 __device__ inline bool is_fluid(const SolveArgs& S, const uint8_t* label, int x, int y, int z) {
     return x > 0 && y > 0 && z > 0 && x < S.nx - 1 && y < S.ny - 1 && z < S.nz - 1 && label[sidx(S, x, y, z)] == FSIM_WATER;
+}
+
+// Neighbour mask of interior cell (x, y, z), 0 unless it is WATER.
+__device__ inline uint16_t neighbour_mask(const SolveArgs& S, const uint8_t* label, int x, int y, int z) {
+    if (!is_fluid(S, label, x, y, z)) return 0;
+    const int64_t st[3] = {(int64_t)S.ny * S.nz, S.nz, 1};
+    const int64_t i = sidx(S, x, y, z);
+    uint16_t info = NB_FLUID;
+    int nonsolid = 0;
+    const int p[3] = {x, y, z};
+    for (int a = 0; a < 3; a++) {
+        int qp[3] = {p[0], p[1], p[2]}, qm[3] = {p[0], p[1], p[2]};
+        qp[a] += 1;
+        qm[a] -= 1;
+        uint8_t lp = label[i + st[a]], lm = label[i - st[a]];
+        if (lp != FSIM_SOLID) nonsolid++;
+        if (lm != FSIM_SOLID) nonsolid++;
+        if (is_fluid(S, label, qp[0], qp[1], qp[2])) info |= (uint16_t)(NB_PX << a);
+        if (is_fluid(S, label, qm[0], qm[1], qm[2])) info |= (uint16_t)(NB_MX << a);
+    }
+    info |= (uint16_t)(nonsolid << NB_NONSOLID_SHIFT);
+    // for each -a neighbour that is WATER: are its +(a+1)%3 and
+    // +(a+2)%3 neighbours WATER (the MIC(0) "other" off-diagonals)
+    for (int a = 0; a < 3; a++) {
+        if (!(info & (NB_MX << a))) continue;
+        for (int k = 0; k < 2; k++) {
+            const int b = (a + 1 + k) % 3;
+            int q[3] = {p[0], p[1], p[2]};
+            q[a] -= 1;
+            q[b] += 1;
+            if (is_fluid(S, label, q[0], q[1], q[2])) info |= (uint16_t)(1u << (NB_UP_SHIFT + 2 * a + k));
+        }
+    }
+    return info;
 }
 
 __global__ void __launch_bounds__(kBlock) k_nbinfo_rhs(RhsArgs A, int with_rhs) {
@@ -204,52 +241,103 @@ __global__ void __launch_bounds__(kBlock) k_nbinfo_rhs(RhsArgs A, int with_rhs) 
     for (int z = threadIdx.x; z < S.nz; z += blockDim.x) {
         const int x = row / S.ny, y = row - x * S.ny;
         const int64_t i = (int64_t)row * S.nz + z;
-        uint16_t info = 0;
+        const uint16_t info = neighbour_mask(S, A.label, x, y, z);
         float bv = 0.f;
-        if (is_fluid(S, A.label, x, y, z)) {
-            const int64_t st[3] = {(int64_t)S.ny * S.nz, S.nz, 1};
-            info = NB_FLUID;
+        if (info) {
             nfl += 1.0;
             A.colw[y * S.nz + z] = 1;
-            int nonsolid = 0;
-            const int p[3] = {x, y, z};
-            for (int a = 0; a < 3; a++) {
-                int qp[3] = {p[0], p[1], p[2]}, qm[3] = {p[0], p[1], p[2]};
-                qp[a] += 1;
-                qm[a] -= 1;
-                uint8_t lp = A.label[i + st[a]], lm = A.label[i - st[a]];
-                if (lp != FSIM_SOLID) nonsolid++;
-                if (lm != FSIM_SOLID) nonsolid++;
-                if (is_fluid(S, A.label, qp[0], qp[1], qp[2])) info |= (uint16_t)(NB_PX << a);
-                if (is_fluid(S, A.label, qm[0], qm[1], qm[2])) info |= (uint16_t)(NB_MX << a);
-            }
-            info |= (uint16_t)(nonsolid << NB_NONSOLID_SHIFT);
-            // for each -a neighbour that is WATER: are its +(a+1)%3 and
-            // +(a+2)%3 neighbours WATER (the MIC(0) "other" off-diagonals)
-            for (int a = 0; a < 3; a++) {
-                if (!(info & (NB_MX << a))) continue;
-                for (int k = 0; k < 2; k++) {
-                    const int b = (a + 1 + k) % 3;
-                    int q[3] = {p[0], p[1], p[2]};
-                    q[a] -= 1;
-                    q[b] += 1;
-                    if (is_fluid(S, A.label, q[0], q[1], q[2])) info |= (uint16_t)(1u << (NB_UP_SHIFT + 2 * a + k));
-                }
-            }
+            A.xw[x] = 1;
             if (with_rhs) {
-                double dv = (double)A.u2[i] + (double)A.v2[i] + (double)A.w2[i] - (double)A.u2[i - st[0]] -
-                            (double)A.v2[i - st[1]] - (double)A.w2[i - st[2]];
+                double dv = (double)A.u2[i] + (double)A.v2[i] + (double)A.w2[i] - (double)A.u2[i - (int64_t)S.ny * S.nz] -
+                            (double)A.v2[i - S.nz] - (double)A.w2[i - 1];
                 double bd = -A.inv_dx * dv +
                             (A.pressure_enabled ? ((double)A.density[i] - A.avg_p) * A.pk : 0.0);
                 bsq += bd * bd;
                 bv = (float)bd;
             }
         }
-        const int64_t ri = rsidx(S, x, y, z);
-        A.nbinfo[ri] = info;
-        if (with_rhs) A.b[ri] = bv;
+        A.info_flat[i] = info;
+        if (with_rhs) A.b_flat[i] = bv;
     }
     if (with_rhs) block_finish<AUX_SUM>(bsq, nfl, A.red);
+}
+
+// Masks and b from flat order into the solver's layout, with the chunk flags.
+// A block item: W planes of one row y and one z-tile.  The cells of a rotated
+// plane lie in 64 different x rows, so the block reads flat rows (lanes along
+// z), puts them into LDS by plane, and writes each column's groups of four
+// planes with 8- and 16-byte stores; every interior column's value moves once.
+// The right-hand-side kernel used to scatter 2- and 4-byte values over 64
+// planes itself: 0.57 ms at 256^3, 0.27 ms for the two kernels.
+template <int W>
+__global__ void __launch_bounds__(kBlock) k_rotate(SolveArgs S, const uint16_t* __restrict__ info_flat,
+                                                   const float* __restrict__ b_flat, uint16_t* __restrict__ nbinfo,
+                                                   float* __restrict__ b, uint32_t* __restrict__ flags,
+                                                   const uint8_t* __restrict__ xw, int* __restrict__ xrange) {
+    __shared__ uint16_t info_lds[W][WF_TZ];
+    __shared__ float b_lds[W][WF_TZ];
+    constexpr int nwaves = kBlock / 64, kRows = (W + WF_TZ - 1 + nwaves - 1) / nwaves;   // rows per wave
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int ntile = (S.nz - 2 + WF_TZ - 1) / WF_TZ;
+    const int k = blockIdx.x;
+    const int z0 = 1 + k % ntile * WF_TZ, y = 1 + k / ntile % (S.ny - 2), p0 = k / (ntile * (S.ny - 2)) * W;
+    const int np = min(W, S.nxp - p0), cols = min(WF_TZ, S.nz - 1 - z0);
+    const int z = z0 + lane;
+    // row t (x = t mod nxp) holds the cells of planes t + lane; loads in batches of 8 rows
+    for (int k0 = 0; k0 < kRows; k0 += 8) {
+        uint16_t n[8];
+        float v[8];
+        int slot[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int t = p0 - (cols - 1) + (k0 + j) * nwaves + wave;
+            const int p = t + lane;
+            const int x = t >= 0 ? (t < S.nxp ? t : 0) : (t % S.nxp + S.nxp) % S.nxp;
+            const bool on = k0 + j < kRows && lane < cols && p >= p0 && p < p0 + np;
+            const bool cell = on && x < S.nx;
+            const int64_t i = cell ? sidx(S, x, y, z) : 0;
+            slot[j] = on ? (p - p0) * WF_TZ + lane : -1;
+            n[j] = cell ? info_flat[i] : (uint16_t)0;
+            v[j] = cell && b_flat ? b_flat[i] : 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (slot[j] >= 0) {
+                (&info_lds[0][0])[slot[j]] = n[j];
+                (&b_lds[0][0])[slot[j]] = v[j];
+            }
+    }
+    if (k == 0 && wave == 0) {   // the x range with WATER, for the wavefront kernels
+        int xlo = S.nx, xhi = -1;
+        for (int x = lane; x < S.nx; x += 64)
+            if (xw[x]) {
+                xlo = min(xlo, x);
+                xhi = x;
+            }
+        for (int d = 32; d >= 1; d >>= 1) {
+            xlo = min(xlo, __shfl_down(xlo, d, 64));
+            xhi = max(xhi, __shfl_down(xhi, d, 64));
+        }
+        if (lane == 0) {
+            xrange[0] = xlo;
+            xrange[1] = xhi;
+        }
+    }
+    __syncthreads();
+    if (lane >= cols) return;
+    for (int g = wave; g < np / WF_G; g += nwaves) {
+        const int64_t i = pidx(p0 + g * WF_G, y, z, S.ny, S.nz);
+        u16x4 n;
+        f32x4 v;
+#pragma unroll
+        for (int c = 0; c < WF_G; c++) {
+            n[c] = info_lds[g * WF_G + c][lane];
+            v[c] = b_lds[g * WF_G + c][lane];
+        }
+        *reinterpret_cast<u16x4*>(nbinfo + i) = n;
+        if (b_flat) *reinterpret_cast<f32x4*>(b + i) = v;
+        if ((n[0] | n[1] | n[2] | n[3]) & NB_FLUID) flags[i / kChunk] = 1u;
+    }
 }
 
 // ---- MIC(0) factor, one i+j+k plane per launch (FP64) -----------------------------
@@ -343,47 +431,16 @@ __global__ void __launch_bounds__(kBlock) k_bwd_plane(PlaneArgs A, const float* 
 // ---- SpMV (applyAMatrix :165-198) with the s.q dot ---------------------------------
 constexpr int SPMV_PLAIN = 0, SPMV_COPY = 1, SPMV_XPAY = 2;
 
-// Work split of the stencil kernels: one work item is a 256-cell chunk of an
-// interior rotated row (plane p, row y in 1..ny-2, z in 1..nz-2), handled by
-// one wave with 4 cells per lane (z = z0 + lane + 64k, coalesced for each k).
-// Workgroups are dispatched round-robin over the 8 XCDs (blockIdx mod 8), so
-// the items are cut into 8 contiguous ranges, one per XCD: the +-x/+-y
-// neighbour rows a wave reads were loaded by waves of the same XCD (its L2).
-constexpr int kRowCells = 4 * 64;
-struct RowItems {
-    int nchunk, ny2;
-    int end;           // end of this XCD's item range (items fit in 32 bits: nc < 2^31)
-    int first, step;   // this wave's first item and stride
-};
-__device__ inline RowItems row_items(const SolveArgs& S) {
-    RowItems it;
-    it.nchunk = (S.nz - 2 + kRowCells - 1) / kRowCells;
-    it.ny2 = S.ny - 2;
-    const int total = S.nx * it.ny2 * it.nchunk;
-    const int per_xcd = (total + 7) / 8;
-    const int xcd = blockIdx.x & 7;
-    const int begin = xcd * per_xcd;
-    it.end = min(total, begin + per_xcd);
-    const int waves_per_block = blockDim.x / 64;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    it.first = begin + (int)(blockIdx.x >> 3) * waves_per_block + wave;
-    it.step = (int)(gridDim.x >> 3) * waves_per_block;
-    return it;
-}
-// (plane, row, first z) of item k
-__device__ inline void item_cells(const RowItems& it, int k, int& p, int& y, int& z0) {
-    const int c = k % it.nchunk;
-    const int rest = k / it.nchunk;
-    y = 1 + rest % it.ny2;
-    p = rest / it.ny2;
-    z0 = 1 + c * kRowCells;
-}
-
 // SPMV_PLAIN: q = A s.  SPMV_COPY: s' = z, q = A s'.  SPMV_XPAY: s' = s * beta + z
 // (multSelfAndAdd :229-242), q = A s'.  The new search direction s' goes to a
 // second buffer and is recomputed for the neighbours from z and the old s, so
-// no block reads a value another block has already replaced.  Only WATER
-// cells are written: q is zeroed before a solve and never read elsewhere.
+// no block reads a value another block has already replaced.  A lane owns the
+// four cells of one column of a plane group and stores them whole, zero off
+// WATER (q and s are zeroed before a solve, so the columns without WATER that
+// it leaves out hold zeros as well).  Per 64 x 4 cells it issues 10 16-byte and 8
+// 4-byte vector loads where one cell per lane took 56 4-byte ones; 75 us at
+// 256^3 (80 us before), bound by memory.
+static_assert(kBlock == 64 * kRowWaves, "a wave per row of an item");
 template <int MODE>
 __global__ void __launch_bounds__(kBlock) k_spmv(SolveArgs S, const uint16_t* __restrict__ nbinfo,
                                                  const float* __restrict__ z, const float* __restrict__ s,
@@ -396,84 +453,63 @@ __global__ void __launch_bounds__(kBlock) k_spmv(SolveArgs S, const uint16_t* __
         else if constexpr (MODE == SPMV_COPY) return z[j];
         else return s[j] * beta + z[j];
     };
-    const RowItems it = row_items(S);
-    const int lane = threadIdx.x & 63;
-    // the nbinfo words of the next item are loaded while this item's gathers are in flight
-    auto load_info = [&](int k, uint16_t (&inf)[4]) {
-        if (k >= it.end) return;
-        int p, y, z0;
-        item_cells(it, k, p, y, z0);
-        const int64_t rowbase = ((int64_t)p * S.ny + y) * S.nz;
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const int zc = z0 + lane + 64 * c;
-            inf[c] = zc < S.nz - 1 ? nbinfo[rowbase + zc] : (uint16_t)0;
-        }
+    auto dir4 = [&](int64_t j) {
+        if constexpr (MODE == SPMV_PLAIN) return *reinterpret_cast<const f32x4*>(s + j);
+        else if constexpr (MODE == SPMV_COPY) return *reinterpret_cast<const f32x4*>(z + j);
+        else return *reinterpret_cast<const f32x4*>(s + j) * beta + *reinterpret_cast<const f32x4*>(z + j);
     };
-    uint16_t info_next[4] = {0, 0, 0, 0};
-    load_info(it.first, info_next);
+    const RowItems it = row_items(S.ny, S.nz, S.nxp);
+    const int ng = S.nxp / WF_G;
+    // the nbinfo words of the next item are loaded while this item's gathers are in flight
+    auto load_info = [&](int k) {
+        int g, y, z;
+        if (k >= it.end || !item_column(it, k, S.ny, S.nz, g, y, z)) return u16x4{0, 0, 0, 0};
+        return *reinterpret_cast<const u16x4*>(nbinfo + pidx(g * WF_G, y, z, S.ny, S.nz));
+    };
+    u16x4 info_next = load_info(it.first);
     for (int k = it.first; k < it.end; k += it.step) {
-        int p, y, z0;
-        item_cells(it, k, p, y, z0);
-        const int64_t rowbase = ((int64_t)p * S.ny + y) * S.nz;
-        uint16_t info[4];
-        int zc[4];
-        bool any = false;
+        const u16x4 info = info_next;
+        info_next = load_info(k + it.step);
+        if (((info[0] | info[1] | info[2] | info[3]) & NB_FLUID) == 0) continue;   // no WATER in the lane's cells
+        int g, y, zc;
+        item_column(it, k, S.ny, S.nz, g, y, zc);
+        // all gathers first, then the sums with the reference's term order, by mask
+        const ColumnNeighbours n = column_neighbours(S.ny, S.nz, ng, g, y, zc);
+        const f32x4 own = dir4(n.own), yp = dir4(n.yp), ym = dir4(n.ym), zp = dir4(n.zp), zm = dir4(n.zm);
+        const float xp3 = dir(n.xp3), xm0 = dir(n.xm0), zp3 = dir(n.zp3), zm0 = dir(n.zm0);
+        f32x4 out, snew;
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            info[c] = info_next[c];
-            zc[c] = min(z0 + lane + 64 * c, S.nz - 2);   // lanes past the row gather an interior cell, unused
-            any |= (info[c] & NB_FLUID) != 0;
-        }
-        load_info(k + it.step, info_next);
-        if (__builtin_amdgcn_ballot_w64(any) == 0) continue;   // no WATER cell in the wave's chunk
-        // all gathers of the 4 cells first (interior cells: every neighbour index is in range),
-        // then the sums with the reference's term order, by mask
-        float v[4][7];
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const int64_t i = rowbase + zc[c];
-            const RNeighbours n = rneighbours(S, i, p, y, zc[c]);
-            v[c][0] = dir(i);
-            v[c][1] = dir(n.px);
-            v[c][2] = dir(n.py);
-            v[c][3] = dir(n.pz);
-            v[c][4] = dir(n.mx);
-            v[c][5] = dir(n.my);
-            v[c][6] = dir(n.mz);
-        }
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const uint16_t f = info[c];
-            if (!(f & NB_FLUID)) continue;
-            const int64_t i = rowbase + zc[c];
+            const uint32_t f = info[c];
             const int cnt = (f >> NB_NONSOLID_SHIFT) & 7;
-            const float si = v[c][0];
+            const float si = own[c];
             float val = (S.scale_f * (float)cnt) * si;
-            val = (f & NB_PX) ? val + ms * v[c][1] : val;
-            val = (f & NB_PY) ? val + ms * v[c][2] : val;
-            val = (f & NB_PZ) ? val + ms * v[c][3] : val;
-            val = (f & NB_MX) ? val + ms * v[c][4] : val;
-            val = (f & NB_MY) ? val + ms * v[c][5] : val;
-            val = (f & NB_MZ) ? val + ms * v[c][6] : val;
-            d += (double)si * (double)val;
-            q[i] = val;
-            if (MODE != SPMV_PLAIN) s_new[i] = si;
+            val = (f & NB_PX) ? val + ms * (c < 3 ? own[(c + 1) & 3] : xp3) : val;
+            val = (f & NB_PY) ? val + ms * yp[c] : val;
+            val = (f & NB_PZ) ? val + ms * (c < 3 ? zp[(c + 1) & 3] : zp3) : val;
+            val = (f & NB_MX) ? val + ms * (c > 0 ? own[(c + 3) & 3] : xm0) : val;
+            val = (f & NB_MY) ? val + ms * ym[c] : val;
+            val = (f & NB_MZ) ? val + ms * (c > 0 ? zm[(c + 3) & 3] : zm0) : val;
+            const bool fl = (f & NB_FLUID) != 0;
+            out[c] = fl ? val : 0.f;
+            snew[c] = fl ? si : 0.f;
+            d += (double)snew[c] * (double)out[c];
         }
+        *reinterpret_cast<f32x4*>(q + n.own) = out;
+        if (MODE != SPMV_PLAIN) *reinterpret_cast<f32x4*>(s_new + n.own) = snew;
     }
     block_finish<AUX_NONE>(d, 0.0, red);
 }
 
 // Streaming kernels without per-cell masks: the solver vectors r, q and z
-// are exactly zero off WATER (zeroed at the start of a solve, written on
-// WATER cells only), so the extra terms are exact zeros.  The vectors are cut
-// into chunks of CH cells (256 with float4 accesses when nc is a multiple of
-// 4, else 64); a chunk without WATER is skipped.  Its flag is one 32-bit word
-// (built with nbinfo for every solve), so a wave reads it with a scalar load;
-// a wave takes kUnits chunks per trip (grid stride) and issues all their
-// loads before using any, so several memory round trips are in flight.
+// are exactly zero off WATER (zeroed at the start of a solve, written with
+// zeros there), so the extra terms are exact zeros.  The vectors are cut
+// into chunks of 256 values (16 bytes per lane); a chunk without WATER is
+// skipped.  Its flag is one 32-bit word (built with nbinfo for every solve),
+// so a wave reads it with a scalar load; a wave takes kUnits chunks per trip
+// (grid stride) and issues all their loads before using any, so several
+// memory round trips are in flight.
 constexpr int kUnits = 4;
-__host__ __device__ constexpr int stream_chunk(bool vec4) { return vec4 ? 256 : 64; }
 // 1024 measured fastest at 256^3 (the dot: 38 us per launch with 2048 blocks, 29 us with 1024;
 // 512 is slower again)
 #ifndef FSIM_STREAM_BLOCKS
@@ -481,35 +517,15 @@ __host__ __device__ constexpr int stream_chunk(bool vec4) { return vec4 ? 256 : 
 #endif
 static_assert(FSIM_STREAM_BLOCKS % 8 == 0 && FSIM_STREAM_BLOCKS <= (int)kMaxParts, "stream grid within the reduction");
 // blocks of the flagged-chunk kernels (at most kMaxParts, a multiple of 8)
-static unsigned stream_blocks(int64_t nc) {
-    const unsigned need = (unsigned)((nc / stream_chunk(true) + kUnits * 4 - 1) / (kUnits * 4));
+static unsigned stream_blocks(int64_t n) {
+    const unsigned need = (unsigned)((n / kChunk + kUnits * 4 - 1) / (kUnits * 4));
     return std::max(8u, std::min<unsigned>((need + 7) / 8 * 8, FSIM_STREAM_BLOCKS));
 }
 
-template <int CH>
-__global__ void __launch_bounds__(kBlock) k_chunk_flags(int64_t nc, const uint16_t* __restrict__ nbinfo,
-                                                        uint32_t* __restrict__ flags) {
+template <int NV, class Load, class Use>
+__device__ inline void for_flagged_chunks(int64_t n, const uint32_t* __restrict__ flags, Load&& load, Use&& use) {
     const int lane = threadIdx.x & 63;
-    const int nchunks = (int)((nc + CH - 1) / CH);
-    const int nwaves = (int)(gridDim.x * (blockDim.x / 64));
-    for (int u = (int)(blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6)); u < nchunks; u += nwaves) {
-        bool any = false;
-#pragma unroll
-        for (int k = 0; k < CH / 64; k++) {
-            const int64_t i = (int64_t)u * CH + k * 64 + lane;
-            any = any || (i < nc && (nbinfo[i] & NB_FLUID));
-        }
-        any = __builtin_amdgcn_ballot_w64(any) != 0;
-        if (lane == 0) flags[u] = any ? 1u : 0u;
-    }
-}
-
-template <bool VEC4, int NV, class Load, class Use>
-__device__ inline void for_flagged_chunks(int64_t nc, const uint32_t* __restrict__ flags, Load&& load, Use&& use) {
-    constexpr int CH = stream_chunk(VEC4);
-    using V = typename std::conditional<VEC4, float4, float>::type;
-    const int lane = threadIdx.x & 63;
-    const int nchunks = (int)((nc + CH - 1) / CH);
+    const int nchunks = (int)((n + kChunk - 1) / kChunk);
     const int nwaves = (int)(gridDim.x * (blockDim.x / 64));
     const int w0 = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6)));
     for (int u0 = w0; u0 < nchunks; u0 += kUnits * nwaves) {
@@ -521,13 +537,13 @@ __device__ inline void for_flagged_chunks(int64_t nc, const uint32_t* __restrict
         }
         // loads without branches (a skipped lane reads cell 0 and uses nothing), so that all
         // kUnits x NV loads are issued before the first wait
-        V v[kUnits][NV];
+        float4 v[kUnits][NV];
         bool on[kUnits];
         int64_t at[kUnits];
 #pragma unroll
         for (int k = 0; k < kUnits; k++) {
-            const int64_t i = (int64_t)(u0 + k * nwaves) * CH + (VEC4 ? 4 : 1) * lane;
-            on[k] = f[k] != 0u && i < nc;
+            const int64_t i = (int64_t)(u0 + k * nwaves) * kChunk + 4 * lane;
+            on[k] = f[k] != 0u && i < n;
             at[k] = on[k] ? i : 0;
             load(at[k], v[k]);
         }
@@ -538,10 +554,8 @@ __device__ inline void for_flagged_chunks(int64_t nc, const uint32_t* __restrict
 }
 
 // r -= alpha q, with ||r||^2 and max|r|
-template <bool VEC4>
-__global__ void __launch_bounds__(kBlock) k_update_r(int64_t nc, const uint32_t* __restrict__ flags,
+__global__ void __launch_bounds__(kBlock) k_update_r(int64_t n, const uint32_t* __restrict__ flags,
                                                      const float* __restrict__ q, float* __restrict__ r, Reduce red) {
-    using V = typename std::conditional<VEC4, float4, float>::type;
     double ss = 0.0, mx = 0.0;
     const float malpha = (float)(-red.sc->alpha);
     auto cell = [&](float qv, float& rv) {
@@ -549,64 +563,72 @@ __global__ void __launch_bounds__(kBlock) k_update_r(int64_t nc, const uint32_t*
         ss += (double)rv * (double)rv;
         mx = fmax(mx, fabs((double)rv));
     };
-    for_flagged_chunks<VEC4, 2>(
-        nc, flags,
-        [&](int64_t i, V(&v)[2]) {
-            v[0] = *reinterpret_cast<const V*>(q + i);
-            v[1] = *reinterpret_cast<const V*>(r + i);
+    for_flagged_chunks<2>(
+        n, flags,
+        [&](int64_t i, float4(&v)[2]) {
+            v[0] = *reinterpret_cast<const float4*>(q + i);
+            v[1] = *reinterpret_cast<const float4*>(r + i);
         },
-        [&](int64_t i, V(&v)[2]) {
-            if constexpr (VEC4) {
-                cell(v[0].x, v[1].x);
-                cell(v[0].y, v[1].y);
-                cell(v[0].z, v[1].z);
-                cell(v[0].w, v[1].w);
-            } else {
-                cell(v[0], v[1]);
-            }
-            *reinterpret_cast<V*>(r + i) = v[1];
+        [&](int64_t i, float4(&v)[2]) {
+            cell(v[0].x, v[1].x);
+            cell(v[0].y, v[1].y);
+            cell(v[0].z, v[1].z);
+            cell(v[0].w, v[1].w);
+            *reinterpret_cast<float4*>(r + i) = v[1];
         });
     block_finish<AUX_MAX>(ss, mx, red);
 }
 
 // a . b (FP64 products of the FP32 values)
-template <bool VEC4>
-__global__ void __launch_bounds__(kBlock) k_dot(int64_t nc, const uint32_t* __restrict__ flags,
+__global__ void __launch_bounds__(kBlock) k_dot(int64_t n, const uint32_t* __restrict__ flags,
                                                 const float* __restrict__ a, const float* __restrict__ b, Reduce red) {
-    using V = typename std::conditional<VEC4, float4, float>::type;
     double d = 0.0;
-    for_flagged_chunks<VEC4, 2>(
-        nc, flags,
-        [&](int64_t i, V(&v)[2]) {
-            v[0] = *reinterpret_cast<const V*>(a + i);
-            v[1] = *reinterpret_cast<const V*>(b + i);
+    for_flagged_chunks<2>(
+        n, flags,
+        [&](int64_t i, float4(&v)[2]) {
+            v[0] = *reinterpret_cast<const float4*>(a + i);
+            v[1] = *reinterpret_cast<const float4*>(b + i);
         },
-        [&](int64_t i, V(&v)[2]) {
-            if constexpr (VEC4) {
-                d += (double)v[0].x * (double)v[1].x;
-                d += (double)v[0].y * (double)v[1].y;
-                d += (double)v[0].z * (double)v[1].z;
-                d += (double)v[0].w * (double)v[1].w;
-            } else {
-                d += (double)v[0] * (double)v[1];
-            }
+        [&](int64_t i, float4(&v)[2]) {
+            d += (double)v[0].x * (double)v[1].x;
+            d += (double)v[0].y * (double)v[1].y;
+            d += (double)v[0].z * (double)v[1].z;
+            d += (double)v[0].w * (double)v[1].w;
         });
     block_finish<AUX_NONE>(d, 0.0, red);
 }
 
-// x += alpha s (FP64) for WATER cells.  One cell per thread: it runs on a
-// second stream beside the r update, and a lighter HBM load there costs the
-// r update less than a vectorised kernel does (measured at 256^3).  A NaN
+// x += alpha s (FP64) for WATER cells, of the last direction step (STEPS 1) or
+// of the last two in their order (STEPS 2: s_prev and the alpha before).  A NaN
 // alpha leaves x as it is: the reference breaks before multAdd
 // (bridsonSolverGrid.cpp:270-272) and applies the last pressure.
-__global__ void __launch_bounds__(kBlock) k_update_x(int64_t n, const uint16_t* __restrict__ nbinfo,
-                                                     const float* __restrict__ s, double* __restrict__ x,
-                                                     const SolveScalars* __restrict__ sc) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || !(nbinfo[i] & NB_FLUID) || (sc->nan_flag & 1)) return;
-    x[i] += (double)s[i] * sc->alpha;
+template <int STEPS>
+__global__ void __launch_bounds__(kBlock) k_update_x(int64_t n, const uint32_t* __restrict__ flags,
+                                                     const uint16_t* __restrict__ nbinfo, const float* __restrict__ s_prev, const float* __restrict__ s,
+                                                     double* __restrict__ x, const SolveScalars* __restrict__ sc) {
+    const int lane = threadIdx.x & 63;
+    const int nchunks = (int)((n + kChunk - 1) / kChunk);
+    const int nwaves = (int)(gridDim.x * (blockDim.x / 64));
+    const double alpha_prev = sc->alpha_prev, alpha = sc->alpha;
+    const bool last = !(sc->nan_flag & 1);
+    for (int u = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6))); u < nchunks;
+         u += nwaves) {
+        const int64_t i = (int64_t)u * kChunk + 4 * lane;
+        if (flags[u] == 0u || i >= n) continue;
+        const u16x4 nb = *reinterpret_cast<const u16x4*>(nbinfo + i);
+        f64x4 v = *reinterpret_cast<const f64x4*>(x + i);
+        f32x4 a = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (STEPS == 2) a = *reinterpret_cast<const f32x4*>(s_prev + i);
+        const f32x4 b = *reinterpret_cast<const f32x4*>(s + i);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            if (!(nb[c] & NB_FLUID)) continue;
+            if constexpr (STEPS == 2) v[c] += (double)a[c] * alpha_prev;
+            if (last) v[c] += (double)b[c] * alpha;
+        }
+        *reinterpret_cast<f64x4*>(x + i) = v;
+    }
 }
-
 
 // FP64 true residual t = b - A x; optionally r = (float)t.
 __global__ void __launch_bounds__(kBlock) k_true_residual(SolveArgs S, const uint16_t* __restrict__ nbinfo,
@@ -614,24 +636,17 @@ __global__ void __launch_bounds__(kBlock) k_true_residual(SolveArgs S, const uin
                                                           float* __restrict__ r, int replace, Reduce red) {
 #pragma clang fp contract(off)
     double ss = 0.0, mx = 0.0;
-    const RowItems it = row_items(S);
-    const int lane = threadIdx.x & 63;
+    const RowItems it = row_items(S.ny, S.nz, S.nxp);
     for (int k = it.first; k < it.end; k += it.step) {
-        int p, y, z0;
-        item_cells(it, k, p, y, z0);
-        const int64_t rowbase = ((int64_t)p * S.ny + y) * S.nz;
-        uint16_t info[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const int zc = z0 + lane + 64 * c;
-            info[c] = zc < S.nz - 1 ? nbinfo[rowbase + zc] : (uint16_t)0;
-        }
+        int g, y, zc;
+        if (!item_column(it, k, S.ny, S.nz, g, y, zc)) continue;
+        const u16x4 info = *reinterpret_cast<const u16x4*>(nbinfo + pidx(g * WF_G, y, zc, S.ny, S.nz));
 #pragma unroll
         for (int c = 0; c < 4; c++) {
             if (!(info[c] & NB_FLUID)) continue;
-            const int zc = z0 + lane + 64 * c;
-            const int64_t i = rowbase + zc;
-            const RNeighbours n = rneighbours(S, i, p, y, zc);
+            const int p = g * WF_G + c;
+            const int64_t i = pidx(p, y, zc, S.ny, S.nz);
+            const RNeighbours n = rneighbours(S, p, y, zc);
             // all 7 loads first (a WATER cell is interior: every neighbour index is in range), then the
             // reference's terms in order, each kept by its flag
             const double xi = x[i], xpx = x[n.px], xpy = x[n.py], xpz = x[n.pz], xmx = x[n.mx], xmy = x[n.my],
@@ -694,10 +709,18 @@ static SolveArgs solve_args(const fsim_ctx* ctx, double dt) {
     S.ny = ctx->g.ny;
     S.nz = ctx->g.nz;
     S.nc = ctx->g.nc;
-    S.off63 = (WF_TZ - 1) % S.nx;
+    S.nxp = ctx->g.nxp;
+    S.ncr = ctx->g.ncr;
+    S.off63 = (WF_TZ - 1) % S.nxp;
     S.scale = dt / (ctx->prm.fluid_density * ctx->g.cd * ctx->g.cd);
     S.scale_f = (float)S.scale;
     return S;
+}
+
+// No boundary packet is on its way (the wavefront kernels leave the rows so): every word empty
+static int clear_packets(fsim_ctx* ctx) {
+    FSIM_TRY(fill_i32(ctx, reinterpret_cast<int32_t*>(ctx->ybnd), -1, 4 * ctx->wave_packets[0]));
+    return fill_i32(ctx, reinterpret_cast<int32_t*>(ctx->zbnd), -1, 4 * ctx->wave_packets[1]);
 }
 
 // A wavefront kernel whose boundary poll ran out of spins sets wave_err; its
@@ -709,6 +732,7 @@ static int check_wave_err(fsim_ctx* ctx) {
     FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (err) {
         FSIM_HIP(ctx, hipMemsetAsync(ctx->wave_err, 0, sizeof(int), ctx->stream));
+        FSIM_TRY(clear_packets(ctx));   // what the launch sent and nobody received
         return set_err(ctx, FSIM_ERR_TIMEOUT, "wavefront sweep boundary wait timed out");
     }
     return FSIM_OK;
@@ -723,7 +747,11 @@ static unsigned red_blocks(int64_t n) { return std::min<unsigned>((nblocks(n) + 
 #define FSIM_SPMV_BLOCKS 2048
 #endif
 static_assert(FSIM_SPMV_BLOCKS % 8 == 0 && FSIM_SPMV_BLOCKS <= (int)kMaxParts, "SpMV grid within the reduction");
-static unsigned spmv_blocks(int64_t n) { return std::min<unsigned>(red_blocks(n), FSIM_SPMV_BLOCKS); }
+// blocks of the column kernels: one per item, up to FSIM_SPMV_BLOCKS
+static unsigned spmv_blocks(const SolveArgs& S) {
+    const unsigned items = (unsigned)row_item_count(S.ny, S.nz, S.nxp);
+    return std::max(8u, std::min<unsigned>((items + 7) / 8 * 8, FSIM_SPMV_BLOCKS));
+}
 
 static Reduce reduce_to(fsim_ctx* ctx, int op) { return Reduce{ctx->partials, ctx->red_count, ctx->scal, op}; }
 // the same, with the finished scalars also written to the pinned host copy (read after an event)
@@ -737,6 +765,14 @@ static int read_scalars(fsim_ctx* ctx) {
     return FSIM_OK;
 }
 
+// colw: one byte per (y, z) column; behind it, each from a multiple of 4 bytes,
+// the two words of xrange, a byte per x row, and the chunk flags, cleared with it
+static int64_t colw_columns(int ny, int nz) { return ((int64_t)ny * nz + 3) / 4 * 4; }
+static int64_t colw_bytes(const SolveArgs& S) {
+    return colw_columns(S.ny, S.nz) + 8 + (S.nx + 3) / 4 * 4 + 4 * (S.ncr / kChunk + 1);
+}
+static int* xrange_of(uint8_t* colw, int ny, int nz) { return reinterpret_cast<int*>(colw + colw_columns(ny, nz)); }
+
 static int build_nbinfo(fsim_ctx* ctx, const SolveArgs& S, bool with_rhs) {
     FSIM_PROF(ctx, KID_RHS);
     RhsArgs A{};
@@ -746,22 +782,30 @@ static int build_nbinfo(fsim_ctx* ctx, const SolveArgs& S, bool with_rhs) {
     A.v2 = ctx->v2;
     A.w2 = ctx->w2;
     A.density = ctx->density;
-    A.nbinfo = ctx->nbinfo;
+    // the search directions are free between solves
+    A.info_flat = reinterpret_cast<uint16_t*>(ctx->s);
+    A.b_flat = ctx->s2;
     A.colw = ctx->colw;
-    A.b = ctx->b;
+    A.xw = reinterpret_cast<uint8_t*>(xrange_of(ctx->colw, S.ny, S.nz) + 2);
     A.inv_dx = 1.0 / ctx->g.cd;
     A.avg_p = ctx->prm.average_pressure;
     A.pk = ctx->prm.pressure_k;
     A.pressure_enabled = ctx->prm.pressure_enabled;
     A.red = reduce_to(ctx, FIN_BB);
-    FSIM_TRY(fill_u8(ctx, ctx->colw, 0, (int64_t)S.ny * S.nz));
+    FSIM_TRY(fill_u8(ctx, ctx->colw, 0, colw_bytes(S)));   // and xrange and the chunk flags behind it
     hipLaunchKernelGGL(k_nbinfo_rhs, dim3(red_blocks(S.nc)), dim3(kBlock), 0, ctx->stream, A, with_rhs ? 1 : 0);
-    if (S.nc % 4 == 0)
-        hipLaunchKernelGGL(k_chunk_flags<stream_chunk(true)>, dim3(nblocks(S.nc / 4)), dim3(kBlock), 0, ctx->stream, S.nc,
-                           ctx->nbinfo, ctx->chunk_flags);
+    // wide windows leave fewer lanes idle, narrow ones give small grids more and shorter blocks
+    auto items = [&](int w) {
+        return (unsigned)((S.nxp + w - 1) / w * (S.ny - 2) * ((S.nz - 2 + WF_TZ - 1) / WF_TZ));
+    };
+    const float* b_flat = with_rhs ? A.b_flat : nullptr;
+    int* xrange = xrange_of(ctx->colw, S.ny, S.nz);
+    if (items(64) >= 2 * 256)
+        hipLaunchKernelGGL(k_rotate<64>, dim3(items(64)), dim3(kBlock), 0, ctx->stream, S, A.info_flat, b_flat, ctx->nbinfo,
+                           ctx->b, ctx->chunk_flags, A.xw, xrange);
     else
-        hipLaunchKernelGGL(k_chunk_flags<stream_chunk(false)>, dim3(nblocks(S.nc)), dim3(kBlock), 0, ctx->stream, S.nc,
-                           ctx->nbinfo, ctx->chunk_flags);
+        hipLaunchKernelGGL(k_rotate<16>, dim3(items(16)), dim3(kBlock), 0, ctx->stream, S, A.info_flat, b_flat, ctx->nbinfo,
+                           ctx->b, ctx->chunk_flags, A.xw, xrange);
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;
 }
@@ -770,8 +814,8 @@ static int nplane_threads(const SolveArgs& S) { return (S.nx - 2) * (S.ny - 2); 
 
 static int mic_factor(fsim_ctx* ctx, const SolveArgs& S) {
     FSIM_PROF(ctx, KID_MIC_FACTOR);
-    FSIM_TRY(fill_f64(ctx, ctx->P64, 0.0, S.nc));
-    FSIM_TRY(fill_f32(ctx, ctx->P32, 0.0f, S.nc));
+    FSIM_TRY(fill_f64(ctx, ctx->P64, 0.0, S.ncr));
+    FSIM_TRY(fill_f32(ctx, ctx->P32, 0.0f, S.ncr));
     if (ctx->sweep_mode == 0) return wave_launch(ctx, 0, nullptr, nullptr, S.scale);
     PlaneArgs A{S, ctx->nbinfo, 0};
     const int nt = nplane_threads(S);
@@ -784,7 +828,7 @@ static int mic_factor(fsim_ctx* ctx, const SolveArgs& S) {
     return FSIM_OK;
 }
 
-// z = M^-1 r (q is scratch)
+// z = M^-1 r (q is scratch; the backward sweep may run in place, q == z)
 static int mic_apply(fsim_ctx* ctx, const SolveArgs& S, const float* r, float* q, float* z) {
     if (ctx->sweep_mode == 0) {
         {
@@ -811,7 +855,7 @@ static int mic_apply(fsim_ctx* ctx, const SolveArgs& S, const float* r, float* q
 
 static int true_residual(fsim_ctx* ctx, const SolveArgs& S, bool replace) {
     FSIM_PROF(ctx, KID_TRUE_RES);
-    hipLaunchKernelGGL(k_true_residual, dim3(red_blocks(S.nc)), dim3(kBlock), 0, ctx->stream, S, ctx->nbinfo, ctx->b, ctx->x,
+    hipLaunchKernelGGL(k_true_residual, dim3(spmv_blocks(S)), dim3(kBlock), 0, ctx->stream, S, ctx->nbinfo, ctx->b, ctx->x,
                        ctx->r, replace ? 1 : 0, reduce_to(ctx, FIN_TRUE));
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;
@@ -819,13 +863,9 @@ static int true_residual(fsim_ctx* ctx, const SolveArgs& S, bool replace) {
 
 static int dot_with(fsim_ctx* ctx, const float* a, const float* b, int op) {
     FSIM_PROF(ctx, KID_DOT);
-    const int64_t nc = ctx->g.nc;
-    if (nc % 4 == 0)
-        hipLaunchKernelGGL(k_dot<true>, dim3(stream_blocks(nc)), dim3(kBlock), 0, ctx->stream, nc, ctx->chunk_flags, a, b,
-                           reduce_to(ctx, op));
-    else
-        hipLaunchKernelGGL(k_dot<false>, dim3(stream_blocks(nc)), dim3(kBlock), 0, ctx->stream, nc, ctx->chunk_flags, a, b,
-                           reduce_to(ctx, op));
+    const int64_t n = ctx->g.ncr;
+    hipLaunchKernelGGL(k_dot, dim3(stream_blocks(n)), dim3(kBlock), 0, ctx->stream, n, ctx->chunk_flags, a, b,
+                       reduce_to(ctx, op));
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;
 }
@@ -836,7 +876,7 @@ static int dot_zr(fsim_ctx* ctx, int op) { return dot_with(ctx, ctx->z, ctx->r, 
 static int direction_step(fsim_ctx* ctx, const SolveArgs& S, bool copy) {
     {
         FSIM_PROF(ctx, KID_SPMV);
-        const dim3 grid(spmv_blocks(S.nc)), block(kBlock);
+        const dim3 grid(spmv_blocks(S)), block(kBlock);
         const Reduce red = reduce_to(ctx, FIN_ALPHA);
         if (copy)
             hipLaunchKernelGGL(k_spmv<SPMV_COPY>, grid, block, 0, ctx->stream, S, ctx->nbinfo, ctx->z, ctx->s, ctx->s2,
@@ -850,18 +890,25 @@ static int direction_step(fsim_ctx* ctx, const SolveArgs& S, bool copy) {
     return FSIM_OK;
 }
 
-// x += alpha s of the direction step just queued, on the second stream: it
-// runs beside the r update instead of inside the next direction step
-// (measured at 256^3: started after the r update instead, it slows the
-// latency-bound forward sweep by more than it slows the r update here).  The
-// next direction step replaces alpha and, one step later, this s buffer, so
-// the main stream waits for it (join_x) before the next direction step and
-// before anything else reads x.
-static int update_x_beside(fsim_ctx* ctx) {
+// x += alpha s of the last `steps` (1 or 2) direction steps, on the second
+// stream beside what the main stream runs next.  The next direction step
+// replaces alpha and the older of the two s buffers, so the main stream waits
+// for it (join_x) before the next direction step and before anything else
+// reads x.
+#ifndef FSIM_X_BLOCKS
+#define FSIM_X_BLOCKS 2048
+#endif
+static int update_x_beside(fsim_ctx* ctx, int steps) {
     FSIM_HIP(ctx, hipEventRecord(ctx->dir_ev, ctx->stream));
     FSIM_HIP(ctx, hipStreamWaitEvent(ctx->xstream, ctx->dir_ev, 0));
-    hipLaunchKernelGGL(k_update_x, dim3(nblocks(ctx->g.nc)), dim3(kBlock), 0, ctx->xstream, ctx->g.nc, ctx->nbinfo,
-                       ctx->s, ctx->x, ctx->scal);
+    const int64_t n = ctx->g.ncr;
+    const dim3 grid(std::max(1u, std::min(nblocks(n / 4), (unsigned)FSIM_X_BLOCKS))), block(kBlock);
+    if (steps == 2)
+        hipLaunchKernelGGL(k_update_x<2>, grid, block, 0, ctx->xstream, n, ctx->chunk_flags, ctx->nbinfo, ctx->s2, ctx->s,
+                           ctx->x, ctx->scal);
+    else
+        hipLaunchKernelGGL(k_update_x<1>, grid, block, 0, ctx->xstream, n, ctx->chunk_flags, ctx->nbinfo, ctx->s2, ctx->s,
+                           ctx->x, ctx->scal);
     FSIM_HIP(ctx, hipGetLastError());
     FSIM_HIP(ctx, hipEventRecord(ctx->x_ev, ctx->xstream));
     return FSIM_OK;
@@ -886,7 +933,7 @@ static bool stop_met(const fsim_ctx* ctx, double ss, double mx, double bnorm) {
 // learned multigrid V-cycle (fsim_mg.hip), whose coarsest level the network
 // solves.
 static int precondition(fsim_ctx* ctx, const SolveArgs& S, bool flexible) {
-    if (!flexible) return mic_apply(ctx, S, ctx->r, ctx->y, ctx->z);
+    if (!flexible) return mic_apply(ctx, S, ctx->r, ctx->z, ctx->z);
     return mg_apply(ctx, ctx->r, ctx->z, S.scale);
 }
 
@@ -916,18 +963,18 @@ struct PcgResult {
 // One host round trip per iteration: the iteration's scalars are copied after
 // the r update, and the next preconditioner application and its dots run
 // while the host waits for them.  If the solve stops or restarts, those
-// results are discarded.  x += alpha s runs on the second stream
-// (update_x_beside) and is joined before the next direction step.
+// results are discarded.  x += alpha s runs on the second stream beside the
+// preconditioner and is joined before the next direction step.
 static int pcg_run(fsim_ctx* ctx, const SolveArgs& S, double bnorm, bool flexible, int max_it, PcgResult* res) {
     const JoinXOnExit join_on_exit{ctx};
-    const int64_t nc = S.nc;
+    const int64_t n = S.ncr;
     fsim_step_stats& st = ctx->stats;
-    FSIM_TRY(fill_f64(ctx, ctx->x, 0.0, nc));
-    hipLaunchKernelGGL(k_copy_f32, dim3(nblocks(nc)), dim3(kBlock), 0, ctx->stream, nc, ctx->b, ctx->r);
-    FSIM_TRY(fill_f32(ctx, ctx->q, 0.0f, nc));
-    FSIM_TRY(fill_f32(ctx, ctx->z, 0.0f, nc));
-    FSIM_TRY(fill_f32(ctx, ctx->s, 0.0f, nc));
-    FSIM_TRY(fill_f32(ctx, ctx->s2, 0.0f, nc));
+    FSIM_TRY(fill_f64(ctx, ctx->x, 0.0, n));
+    hipLaunchKernelGGL(k_copy_f32, dim3(nblocks(n)), dim3(kBlock), 0, ctx->stream, n, ctx->b, ctx->r);
+    FSIM_TRY(fill_f32(ctx, ctx->q, 0.0f, n));
+    FSIM_TRY(fill_f32(ctx, ctx->z, 0.0f, n));
+    FSIM_TRY(fill_f32(ctx, ctx->s, 0.0f, n));
+    FSIM_TRY(fill_f32(ctx, ctx->s2, 0.0f, n));
     FSIM_TRY(precondition(ctx, S, flexible));
     FSIM_TRY(dot_zr(ctx, FIN_SIGMA0));
     const int max_reliable = 64;
@@ -935,20 +982,22 @@ static int pcg_run(fsim_ctx* ctx, const SolveArgs& S, double bnorm, bool flexibl
     double last_true = bnorm;
     bool copy = true;
     int it = 0;
+    int behind = 0;   // direction steps that x does not hold yet (0 or 1 between iterations)
     res->converged = false;
     res->nan = false;
     for (; it < max_it; it++) {
         FSIM_TRY(join_x(ctx));
         FSIM_TRY(direction_step(ctx, S, copy));
-        FSIM_TRY(update_x_beside(ctx));
+        // x takes two steps at a time: it is read and written half as often (both s buffers still hold
+        // their step)
+        if (++behind == 2) {
+            FSIM_TRY(update_x_beside(ctx, 2));
+            behind = 0;
+        }
         {
             FSIM_PROF(ctx, KID_UPDATE);
-            if (nc % 4 == 0)
-                hipLaunchKernelGGL(k_update_r<true>, dim3(stream_blocks(nc)), dim3(kBlock), 0, ctx->stream, nc,
-                                   ctx->chunk_flags, ctx->q, ctx->r, reduce_to_host(ctx, FIN_RES));
-            else
-                hipLaunchKernelGGL(k_update_r<false>, dim3(stream_blocks(nc)), dim3(kBlock), 0, ctx->stream, nc,
-                                   ctx->chunk_flags, ctx->q, ctx->r, reduce_to_host(ctx, FIN_RES));
+            hipLaunchKernelGGL(k_update_r, dim3(stream_blocks(n)), dim3(kBlock), 0, ctx->stream, n, ctx->chunk_flags, ctx->q,
+                               ctx->r, reduce_to_host(ctx, FIN_RES));
         }
         FSIM_HIP(ctx, hipGetLastError());
         // the r update's finishing block wrote rr, rmax and nan_flag into scal_host; the event orders the read
@@ -969,6 +1018,8 @@ static int pcg_run(fsim_ctx* ctx, const SolveArgs& S, double bnorm, bool flexibl
         }
         bool restart = false;
         if (stop_met(ctx, h.rr, h.rmax, bnorm) || std::sqrt(h.rr) < kDelta * last_true) {
+            if (behind) FSIM_TRY(update_x_beside(ctx, 1));
+            behind = 0;
             FSIM_TRY(join_x(ctx));
             const bool replace = st.reliable_updates < max_reliable;
             FSIM_TRY(true_residual(ctx, S, replace));
@@ -991,6 +1042,7 @@ static int pcg_run(fsim_ctx* ctx, const SolveArgs& S, double bnorm, bool flexibl
         }
         copy = restart;
     }
+    if (behind) FSIM_TRY(update_x_beside(ctx, 1));
     FSIM_TRY(join_x(ctx));
     res->iterations = it;
     return FSIM_OK;
@@ -1068,7 +1120,7 @@ static int stage_basic_sor(fsim_ctx* ctx, const SolveArgs& S) {
         }
     }
     FSIM_HIP(ctx, hipMemsetAsync(ctx->scal, 0, sizeof(SolveScalars), ctx->stream));
-    FSIM_TRY(fill_f64(ctx, ctx->x, 0.0, nc));   // no pressure field
+    FSIM_TRY(fill_f64(ctx, ctx->x, 0.0, S.ncr));   // no pressure field
     FSIM_TRY(build_nbinfo(ctx, S, true));
     FSIM_TRY(read_scalars(ctx));
     const double b0 = std::sqrt(ctx->scal_host->bb);
@@ -1202,23 +1254,24 @@ int wave_init(fsim_ctx* ctx) {
     A.nx = ctx->g.nx;
     A.ny = ctx->g.ny;
     A.nz = ctx->g.nz;
+    A.nxp = ctx->g.nxp;
     A.TJ = (A.ny - 2 + WF_TY - 1) / WF_TY;
     A.TK = (A.nz - 2 + WF_TZ - 1) / WF_TZ;
-    // packet rows: one per step of a tile; two words per value (the factor's
-    // FP64), the sweeps use one
-    A.SP = wave_steps(A.nx - 2);
-    const int64_t ny_pk = 2 * (int64_t)A.TJ * A.TK * A.SP * WF_TZ;   // per tile (J, K)
-    const int64_t nz_pk = 2 * (int64_t)A.TJ * A.TK * A.SP * WF_TY;
+    // packet rows: one per plane group that a tile's march can reach (planes x + rot(z)); two words per
+    // value (the factor's FP64), the sweeps use one
+    A.SG = (A.nx - 2 + WF_TZ - 1) / WF_G + 1;
+    ctx->wave_packets[0] = 2 * (int64_t)A.TJ * A.TK * A.SG * WF_TZ;
+    ctx->wave_packets[1] = 2 * (int64_t)A.TJ * A.TK * A.SG * WF_TY;
     if (ctx->g.nc > kWaveMaxCells) ctx->sweep_mode = 1;
-    if (hipMalloc(&ctx->ybnd, sizeof(uint64_t) * ny_pk) != hipSuccess ||
-        hipMalloc(&ctx->zbnd, sizeof(uint64_t) * nz_pk) != hipSuccess ||
+    if (hipMalloc(&ctx->ybnd, sizeof(uint4) * ctx->wave_packets[0]) != hipSuccess ||
+        hipMalloc(&ctx->zbnd, sizeof(uint4) * ctx->wave_packets[1]) != hipSuccess ||
         hipMalloc(&ctx->wave_ticket, sizeof(unsigned long long) * 3) != hipSuccess ||
         hipMalloc(&ctx->wave_err, sizeof(int)) != hipSuccess ||
-        hipMalloc(&ctx->colw, (size_t)A.ny * A.nz) != hipSuccess)
+        hipMalloc(&ctx->colw, (size_t)colw_bytes(solve_args(ctx, 1.0))) != hipSuccess)
         return set_err(ctx, FSIM_ERR_OOM, "wavefront buffer allocation failed");
-    FSIM_TRY(fill_u8(ctx, ctx->colw, 0, (int64_t)A.ny * A.nz));
-    FSIM_HIP(ctx, hipMemsetAsync(ctx->ybnd, 0, sizeof(uint64_t) * ny_pk, ctx->stream));
-    FSIM_HIP(ctx, hipMemsetAsync(ctx->zbnd, 0, sizeof(uint64_t) * nz_pk, ctx->stream));
+    FSIM_TRY(fill_u8(ctx, ctx->colw, 0, colw_bytes(solve_args(ctx, 1.0))));
+    ctx->chunk_flags = reinterpret_cast<uint32_t*>(xrange_of(ctx->colw, A.ny, A.nz) + 2 + (A.nx + 3) / 4);
+    FSIM_TRY(clear_packets(ctx));
     FSIM_HIP(ctx, hipMemsetAsync(ctx->wave_ticket, 0, sizeof(unsigned long long) * 3, ctx->stream));
     FSIM_HIP(ctx, hipMemsetAsync(ctx->wave_err, 0, sizeof(int), ctx->stream));
     A.nbinfo = ctx->nbinfo;
@@ -1228,50 +1281,50 @@ int wave_init(fsim_ctx* ctx) {
     A.zbnd = ctx->zbnd;
     A.err = ctx->wave_err;
     A.colw = ctx->colw;
+    A.xrange = xrange_of(ctx->colw, A.ny, A.nz);
     return FSIM_OK;
 }
 
 int solver_apply(fsim_ctx* ctx, int op, double dt, const double* in, double* out) {
     const SolveArgs S = solve_args(ctx, dt);
-    const int64_t nc = S.nc;
+    const int64_t nc = S.nc, n = S.ncr;
     FSIM_TRY(build_nbinfo(ctx, S, false));
     // host vectors are in flat order, device solver vectors in the rotated one
     std::vector<int64_t> rmap(nc);
     for (int x = 0; x < S.nx; x++)
         for (int y = 0; y < S.ny; y++)
-            for (int z = 0; z < S.nz; z++) rmap[((int64_t)x * S.ny + y) * S.nz + z] = ridx(x, y, z, S.nx, S.ny, S.nz);
-    std::vector<float> hin(nc), hout(nc);
+            for (int z = 0; z < S.nz; z++) rmap[((int64_t)x * S.ny + y) * S.nz + z] = ridx(x, y, z, S.nxp, S.ny, S.nz);
+    std::vector<float> hin(n), hout(n);   // padding values 0
     if (op == FSIM_OP_FACTOR_MIC0) {
         FSIM_TRY(mic_factor(ctx, S));
         FSIM_TRY(check_wave_err(ctx));
-        std::vector<double> hp(nc);
-        FSIM_HIP(ctx, hipMemcpyAsync(hp.data(), ctx->P64, sizeof(double) * nc, hipMemcpyDeviceToHost, ctx->stream));
+        std::vector<double> hp(n);
+        FSIM_HIP(ctx, hipMemcpyAsync(hp.data(), ctx->P64, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
         FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
         for (int64_t i = 0; i < nc; i++) out[i] = hp[rmap[i]];
         return FSIM_OK;
     }
     for (int64_t i = 0; i < nc; i++) hin[rmap[i]] = (float)in[i];
-    FSIM_HIP(ctx, hipMemcpyAsync(ctx->r, hin.data(), sizeof(float) * nc, hipMemcpyHostToDevice, ctx->stream));
+    FSIM_HIP(ctx, hipMemcpyAsync(ctx->r, hin.data(), sizeof(float) * n, hipMemcpyHostToDevice, ctx->stream));
     if (op == FSIM_OP_APPLY_A) {
-        FSIM_TRY(fill_f32(ctx, ctx->q, 0.0f, nc));   // the SpMV writes WATER cells only
-        hipLaunchKernelGGL(k_spmv<SPMV_PLAIN>, dim3(red_blocks(nc)), dim3(kBlock), 0, ctx->stream, S, ctx->nbinfo, nullptr,
+        FSIM_TRY(fill_f32(ctx, ctx->q, 0.0f, n));   // the SpMV skips columns without WATER
+        hipLaunchKernelGGL(k_spmv<SPMV_PLAIN>, dim3(spmv_blocks(S)), dim3(kBlock), 0, ctx->stream, S, ctx->nbinfo, nullptr,
                            ctx->r, nullptr, ctx->q, reduce_to(ctx, FIN_NONE));
         FSIM_HIP(ctx, hipGetLastError());
-        FSIM_HIP(ctx, hipMemcpyAsync(hout.data(), ctx->q, sizeof(float) * nc, hipMemcpyDeviceToHost, ctx->stream));
+        FSIM_HIP(ctx, hipMemcpyAsync(hout.data(), ctx->q, sizeof(float) * n, hipMemcpyDeviceToHost, ctx->stream));
     } else if (op == FSIM_OP_APPLY_MIC0) {
         FSIM_TRY(mic_factor(ctx, S));
-        FSIM_TRY(fill_f32(ctx, ctx->y, 0.0f, nc));
-        FSIM_TRY(fill_f32(ctx, ctx->z, 0.0f, nc));
-        FSIM_TRY(mic_apply(ctx, S, ctx->r, ctx->y, ctx->z));
+        FSIM_TRY(fill_f32(ctx, ctx->z, 0.0f, n));
+        FSIM_TRY(mic_apply(ctx, S, ctx->r, ctx->z, ctx->z));
         FSIM_TRY(check_wave_err(ctx));
-        FSIM_HIP(ctx, hipMemcpyAsync(hout.data(), ctx->z, sizeof(float) * nc, hipMemcpyDeviceToHost, ctx->stream));
+        FSIM_HIP(ctx, hipMemcpyAsync(hout.data(), ctx->z, sizeof(float) * n, hipMemcpyDeviceToHost, ctx->stream));
     } else if (op == FSIM_OP_APPLY_MG) {
         if (ctx->mg_coarse == FSIM_MG_COARSE_NETWORK && !learned_ready(ctx))
             return set_err(ctx, FSIM_ERR_INVALID, "the multigrid's coarse network has no parameters");
         FSIM_TRY(mg_setup(ctx));
-        FSIM_TRY(fill_f32(ctx, ctx->z, 0.0f, nc));
+        FSIM_TRY(fill_f32(ctx, ctx->z, 0.0f, n));
         FSIM_TRY(mg_apply(ctx, ctx->r, ctx->z, S.scale));
-        FSIM_HIP(ctx, hipMemcpyAsync(hout.data(), ctx->z, sizeof(float) * nc, hipMemcpyDeviceToHost, ctx->stream));
+        FSIM_HIP(ctx, hipMemcpyAsync(hout.data(), ctx->z, sizeof(float) * n, hipMemcpyDeviceToHost, ctx->stream));
     } else {
         return set_err(ctx, FSIM_ERR_INVALID, "unknown solver op");
     }

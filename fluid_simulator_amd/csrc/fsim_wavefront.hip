@@ -7,44 +7,60 @@
 // cell performs the same operations in the same order as the serial loop, so
 // the result is bit-identical to it whatever the schedule.
 //
-// Decomposition.  One workgroup owns a tile of WF_TY x 64 interior (y, z)
-// columns and marches along x.  Lane tz of tile row ty processes
-// x = t - ty - tz at step t, so its three upstream values were produced at
-// step t-1: the -x value by the lane itself, the -z value by lane tz-1 of the
-// same row (DPP wave shift) and the -y value by row ty-1: a register when the
-// two rows belong to the same wave (WF_R rows per wave), otherwise the LDS
-// ring below.  The backward sweep mirrors y, and z inside each 64-wide
-// z-tile, so that its upstream is also ty-1, tz-1, x-1 in local terms.
+// Decomposition.  One workgroup owns a tile of WF_TY x 64 (y, z) columns and
+// marches along x, one rotated plane (ridx) per step: lane tz of every row
+// works on x = p - rot(z) at plane p, so its -z value was produced by lane
+// tz - 1 one step earlier (DPP wave shift), its -x value by itself one step
+// earlier, and its -y value by the row above at the same step.  A compute wave
+// holds WF_R rows, whose -y values pass in registers; between waves they pass
+// through LDS rings.  The backward sweep mirrors y, z inside a z-tile, and the
+// planes, so that its upstream is also the row above, lane tz - 1 and the
+// previous step.
 //
-// Memory.  The solver vectors use the rotated layout (ridx): the 64 cells a
-// row visits at one step share one rotated plane, so every load and store
-// of a step covers 64 contiguous words.  Each row keeps its plane offset in
-// a scalar register (advanced and wrapped per step) and each lane a constant
-// in-plane offset, so addressing costs no vector instructions; lanes outside
-// the grid carry an out-of-range buffer offset (loads read 0, stores drop).
+// Groups.  Everything outside the arithmetic happens once per group of WF_G =
+// 4 steps.  The solver vectors interleave four planes, so a lane loads and
+// stores the four steps of one row with one 16-byte access each; a wave hands
+// its last row's four values per lane on with one 16-byte LDS write, and one
+// readiness test covers the group.  A sweep is a chain of about
+// nx + nz + 4 * ny / WF_R dependent steps, and a step's cost is its instruction
+// count (a wave issues one per 4.7 cycles, measured; an LDS read returns after
+// 50, a branch on a vector comparison takes 35), so what is spent per step
+// decides.  One handshake, one tag test and six 4-byte memory accesses per
+// step measured 0.30 us a step, 209 and 202 us a sweep at 256^3 (water in 0.6
+// of the height) and 98 us at 128^3; groups take 0.07 us a step, 132 and 126
+// us at 256^3 and 46 us at 128^3, the same bits.  At 256^3 the tiles' memory
+// traffic counts: a compute unit moves 24 KB per group of an 8-row tile, and
+// without the result's stores the sweep takes 113 us.  Three compute waves of
+// two rows measured best (2 x 4: 142 us forward, 2 x 8: 190 us, 1 x 4: 164 us,
+// 4 x 2: 154 us); storing waves that take the results over LDS, so that the
+// in-order memory counter does not hold loads behind stores, did not pay
+// (166 us), nor did stores past the caches.
 //
-// Inside a workgroup the compute waves form a pipeline along y.  The last
-// row of each wave is written into an LDS ring as 64-bit words
-// (step << 32 | value bits); the next wave reads the word it needs and
-// accepts it when the step tag matches, so a step costs one LDS round trip
-// and needs no counters, fences or drains (an aligned 64-bit LDS access is
-// never seen half-written).  Ring reuse is checked every kBpEvery steps
-// against the downstream wave's own tags.
+// Memory.  Buffer resources: a wave's group offset lives in a scalar register
+// and each lane has a constant in-plane offset per row, replaced by an
+// out-of-range one (loads read 0, stores drop) while none of the lane's cells
+// of the group is in the marched x range, or the lane is off the grid.  A
+// group never holds the first and the last cells of a column at once
+// (rot_planes), so the values around the range inside a group belong to cells
+// without WATER: their factor is 0 and so is every value derived from it.
+// Storing such zeros needs no mask.  The march covers the x range that holds
+// WATER (xrange), which the first pass over the labels found.
 //
-// Across workgroups, values at the tile edges travel through boundary
-// buffers in HBM as 64-bit packets (launch epoch << 32 | value bits) written
-// with device-scope stores, one packet row per step of the consuming tile
-// (ybnd[tile][s][64], zbnd[tile][s][WF_TY] of the producing tile), so a
-// step's packets are contiguous.
-// Four communication waves per workgroup keep all of this traffic out of
-// the compute waves: two read the upstream tiles' packets, a few steps at a
-// time, and republish them into LDS rings tagged with the step; two take this
-// tile's edge values from LDS out-rings (the last compute wave's row, lane 63
-// of every row) and store them as packets.  On gfx9 the memory counter
-// completes in order, so a global read whose result is needed "now", or a
-// slowly acknowledged device-scope store, would stall the compute waves'
-// prefetch stream (per-cell inputs are loaded kPrefetch steps ahead, each
-// prefetch slot in a fixed register).
+// Hand-over inside a workgroup: a ring slot per group and a counter of groups
+// published.  LDS executes one wave's accesses in order, so a reader that sees
+// the counter sees the slot, and a reader issues counter and slot reads
+// together, one group ahead; only if the counter was too low are they read
+// again.  The consumers' counters bound the reuse of the slots.
+//
+// Across workgroups, values at the tile edges travel through boundary buffers
+// in HBM as packets of four values per lane, written with device-scope stores
+// (see "boundary packets").  The last compute wave stores the +y edge itself;
+// three communication waves per workgroup do the rest: two poll the upstream
+// tiles' packets and republish them into LDS rings, one takes the +z edge
+// values from LDS and stores them.  On gfx9 the memory counter completes in
+// order, so a global read whose result is needed "now" would stall the compute
+// waves' prefetch stream (kPrefetch groups ahead, each prefetch slot in fixed
+// registers).
 //
 // Every wait is bounded: past kSpinLimit polls, or as soon as any wave in the
 // grid has given up, a wave raises the error flag and carries on, so the
@@ -53,7 +69,6 @@
 // workgroups already running.
 #include <hip/hip_runtime.h>
 
-#include <climits>
 #include <type_traits>
 
 #include "fsim_internal.hpp"
@@ -61,29 +76,32 @@
 namespace fsim {
 
 constexpr int kSpinLimit = 1 << 21;
-constexpr int kBusyPolls = 32;   // polls before a waiting wave starts to sleep
-constexpr int kPrefetch = WF_PREFETCH;   // compute-wave register prefetch (steps)
-constexpr int kRingV = kPrefetch;   // LDS ring of row values between compute waves (steps)
-constexpr int kBpEvery = 4;      // ring-reuse check period (steps); allowed lag kRingV - kBpEvery
-constexpr int kRingO = 32;       // LDS rings of this tile's +y / +z edge values (steps), a power of two
+constexpr int kBusyPolls = 64;   // polls before a waiting wave starts to sleep
+constexpr int kRing = 8;         // ring slots (groups) between waves, and the unroll of the group loop
+#ifndef FSIM_WF_PREFETCH
+#define FSIM_WF_PREFETCH 6
+#endif
+constexpr int kPrefetch = FSIM_WF_PREFETCH;   // groups of per-cell inputs loaded ahead
+static_assert(kPrefetch >= 1 && kPrefetch <= kRing, "a prefetch slot per unrolled group");
+constexpr int kRingZ = 32;   // +z out-ring slots (groups): the z edge runs 16 groups behind its tile
+constexpr int kAll = 0x3fffffff;              // counter value "everything": no upstream, or no consumer
 constexpr uint32_t kOob = 0x80000000u;        // buffer offset beyond every array: reads 0, drops stores
+constexpr uint32_t kEmpty = 0xffffffffu;      // boundary-packet word that has not been sent
 constexpr int kRawBufferFlags = 0x00020000;   // buffer resource word 3 (raw 32-bit access, gfx9)
+constexpr int kDeviceScope = 16;              // sc1 of a buffer access: past the L1, through the L2
+constexpr int kVolatile = (int)0x80000000;    // a buffer load that is neither merged nor moved
 
 template <int KIND>
 struct Kind {   // 1 = forward sweep, 2 = backward sweep (FP32)
     using T = float;
     static constexpr bool FWD = KIND == 1;
-    static constexpr int NP = 1;       // 32-bit words per value
-    static constexpr int BATCH = 4;    // comm-wave poll batch (steps): short polls keep hop latency low
-    static constexpr int RINGP = 64;   // LDS ring of boundary packets (steps)
+    static constexpr int NP = 1;     // 32-bit words per value
 };
 template <>
 struct Kind<0> {   // MIC(0) factor (FP64)
     using T = double;
     static constexpr bool FWD = true;
     static constexpr int NP = 2;
-    static constexpr int BATCH = 4;
-    static constexpr int RINGP = 32;
 };
 
 // f(integral_constant<int, 0>), ..., f(integral_constant<int, N-1>) in order
@@ -94,58 +112,63 @@ __device__ __forceinline__ void unroll(F&& f) {
         unroll<N, I + 1>(f);
     }
 }
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 
-__device__ inline uint64_t pack(uint32_t bits, uint32_t tag) { return ((uint64_t)tag << 32) | bits; }
-__device__ inline int tag_of(uint64_t v) { return (int)(uint32_t)(v >> 32); }
-__device__ inline uint64_t gpeek(const uint64_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-__device__ inline void lput(uint64_t* p, uint64_t v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
-__device__ inline uint64_t lpeek(const uint64_t* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
-__device__ inline void lput32(int* p, int v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
-__device__ inline int lpeek32(const int* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
 __device__ inline bool gave_up(const int* err) { return __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0; }
 
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
-// 16-byte LDS accesses (ds_read_b128 / ds_write_b128) through an explicit LDS pointer
-typedef __attribute__((address_space(3))) volatile u64x2 lds_u64x2;
-__device__ inline u64x2 lpeek2(const uint64_t* p) { return *(lds_u64x2*)(p); }
-__device__ inline void lput2(uint64_t* p, u64x2 v) { *(lds_u64x2*)(p) = v; }
+// LDS accesses that keep their order among each other (volatile, explicit LDS pointers)
+typedef __attribute__((address_space(3))) volatile u32x4 lds_u32x4;
+typedef __attribute__((address_space(3))) volatile uint32_t lds_u32;
+typedef __attribute__((address_space(3))) volatile int lds_i32;
+typedef __attribute__((address_space(3))) volatile i32x4 lds_i32x4;
+__device__ inline int lget(const int* p) { return *(lds_i32*)p; }
+__device__ inline i32x4 lget4(const int* p) { return *(lds_i32x4*)p; }
+__device__ inline void lput(int* p, int v) { *(lds_i32*)p = v; }
+__device__ inline uint32_t lget(const uint32_t* p) { return *(lds_u32*)p; }
+__device__ inline u32x4 lget4(const uint32_t* p) { return *(lds_u32x4*)p; }
+__device__ inline void lput4(uint32_t* p, u32x4 v) { *(lds_u32x4*)p = v; }
+
 __device__ inline __amdgpu_buffer_rsrc_t rsrc(const void* p, int64_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, (int)bytes, kRawBufferFlags);
 }
-__device__ inline uint64_t bload64(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-    return __builtin_bit_cast(uint64_t, __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0));
-}
-__device__ inline float bload32f(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, soff, 0));
-}
-__device__ inline uint32_t bload16(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-    return (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(r, voff, soff, 0);
-}
-template <int AUX = 0>
-__device__ inline void bstore64(uint64_t v, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, voff, soff, AUX);
-}
-__device__ inline void bstore32(uint32_t v, __amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff) {
-    __builtin_amdgcn_raw_buffer_store_b32(v, r, voff, soff, 0);
+
+// lane i receives lane i-1's value, lane 0 receives `first` (DPP wave_shr:1)
+__device__ inline uint32_t shr1_bits(uint32_t first, uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)first, (int)v, 0x138, 0xf, 0xf, false);
 }
 
-// lane i receives lane i-1's value, lane 0 receives 0 (DPP wave_shr:1)
-__device__ inline float shr1(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, false));
-}
-__device__ inline double shr1(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)__double2loint(v), 0x138, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)__double2hiint(v), 0x138, 0xf, 0xf, false);
-    return __hiloint2double(hi, lo);
-}
-
-__device__ inline uint32_t word(float v, int) { return __float_as_uint(v); }
-__device__ inline uint32_t word(double v, int k) { return k ? (uint32_t)__double2hiint(v) : (uint32_t)__double2loint(v); }
-__device__ inline void from_words(float& v, const uint64_t* w) { v = __uint_as_float((uint32_t)w[0]); }
-__device__ inline void from_words(double& v, const uint64_t* w) {
-    v = __hiloint2double((int)(uint32_t)w[1], (int)(uint32_t)w[0]);
-}
+// the four values of a lane's group as 32-bit words: value j, word k at [j * NP + k]
+template <class T>
+struct Group;
+template <>
+struct Group<float> {
+    u32x4 q[1];
+    __device__ float get(int j) const { return __uint_as_float(q[0][j]); }
+    __device__ void set(int j, float v) { q[0][j] = __float_as_uint(v); }
+    // lane i - 1's value, +0 on lane 0 (a DPP operand of the instruction that uses it)
+    __device__ static float shr1(float v) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x138, 0xf, 0xf, true));
+    }
+};
+template <>
+struct Group<double> {
+    u32x4 q[2];
+    __device__ double get(int j) const {
+        return __hiloint2double((int)q[j >> 1][2 * (j & 1) + 1], (int)q[j >> 1][2 * (j & 1)]);
+    }
+    __device__ void set(int j, double v) {
+        q[j >> 1][2 * (j & 1)] = (uint32_t)__double2loint(v);
+        q[j >> 1][2 * (j & 1) + 1] = (uint32_t)__double2hiint(v);
+    }
+    __device__ static double shr1(double first, double v) {
+        const uint32_t lo = shr1_bits((uint32_t)__double2loint(first), (uint32_t)__double2loint(v));
+        const uint32_t hi = shr1_bits((uint32_t)__double2hiint(first), (uint32_t)__double2hiint(v));
+        return __hiloint2double((int)hi, (int)lo);
+    }
+};
 
 // Ticket in [0, TJ*TK), or -1 (with *err raised) if the counter is out of
 // step with the launch (only after a failed launch); the caller then exits.
@@ -179,75 +202,142 @@ __device__ inline int col_water(const WaveArgs& A, int J, int K, int ty, int tz)
     return A.colw[y_of<FWD>(A, J, ty) * A.nz + z];
 }
 
+// The march of a tile's z column K: groups of planes, counted from 0 in the
+// order of the march.  All tiles of one K share it.
+struct March {
+    int xa, xb;   // x range with WATER
+    int g0;       // plane group of march group 0 (unwrapped planes: x + rot)
+    int ng;       // groups
+};
+template <bool FWD>
+__device__ inline March march_of(const WaveArgs& A, int K, int xa, int xb) {
+    const int kz = FWD ? K : A.TK - 1 - K;
+    const int cols = min(WF_TZ, A.nz - 2 - kz * WF_TZ);
+    const int first = xa / WF_G, last = (xb + cols - 1) / WF_G;
+    return March{xa, xb, FWD ? first : last, last - first + 1};
+}
+// The element (step) of the upstream z tile's march that holds the -z value of
+// element e of tile K's march is e + z_shift: the upstream lane 63 is 63 planes
+// away from lane 0 (forward: ahead, backward: behind), and the two marches may
+// start at different groups.
+template <bool FWD>
+__device__ inline int z_shift(const March& up, const March& me) {
+    return WF_TZ - 1 - (FWD ? 0 : WF_G * (me.g0 - up.g0));
+}
+// march groups in which lane 0 of tile K is inside the x range, counted from 0
+template <bool FWD>
+__device__ inline int z_groups(const March& me) {
+    return FWD ? me.xb / WF_G - me.g0 + 1 : me.g0 - (me.xa + WF_TZ - 1) / WF_G + 1;
+}
+
+// What the waves of a workgroup share.  Counters: a compute wave reads one
+// record a group.  in: groups of its -y values published (by the wave above, or
+// the receiving wave); zin: groups of the -z edge published; out: groups it may
+// have written to its ring (those its reader is done with, plus the ring's
+// slots); zout: the same for zo.
+struct Counters {
+    int in, zin, out, zout;
+};
 template <int KIND>
 struct WaveLds {
-    static constexpr int NP = Kind<KIND>::NP, RINGP = Kind<KIND>::RINGP;
-    // tagged last-row values of compute waves 0 .. WF_NW-2 (the last wave's go to yo)
-    uint64_t v[WF_NW - 1][kRingV][NP][WF_TZ];
-    uint64_t yp[RINGP][NP][WF_TZ];          // tagged -y packets for row 0
-    alignas(16) uint64_t zp[RINGP][NP][WF_TY];   // tagged -z packets for lane 0 of each row
-    int prog[WF_NW];                        // a step whose packets the compute wave has consumed
-    uint64_t yo[kRingO][NP][WF_TZ];         // tagged last row of the last compute wave: the +y edge
-    alignas(16) uint64_t zo[kRingO][NP][WF_TY];   // tagged lane-63 value of every row: the +z edge
-    // sweeps: +z writes of lanes 0..62, never read
-    alignas(16) uint64_t zsink[KIND == 0 ? 1 : WF_NW][WF_TZ - 1][NP * WF_TY];
-    int sprog[2];                           // compute step up to which the +y / +z edge has been sent
+    static constexpr int NP = Kind<KIND>::NP;
+    // ring 0: the -y edge; ring w + 1: the last row of compute wave w
+    alignas(16) uint32_t ring[WF_NW][kRing][NP][WF_TZ][4];
+    // -z edge: lane 0's upstream value of every row; the other lanes read zeros from beside it
+    alignas(16) uint32_t zi[2][kRing][WF_TY][NP][4];
+    alignas(16) uint32_t zo[WF_TY][kRingZ * WF_G * NP];           // +z edge: lane 63's values of every row
+    // of compute wave w at [w + 1]; what the first wave hands up and the last one down goes to the
+    // outer records.  cnt[w + 2].in is what compute wave w has finished
+    alignas(16) Counters cnt[WF_NW + 2];
 };
 
-// ---- communication wave: upstream tile edge -> LDS packet ring ------------
-// The -y edge carries 64 values per step (row 0, lane l), the -z edge WF_TY
-// (lane 0 of row l).  The upstream tile writes every packet of a step at
-// once, so the wave forwards whole steps: step s once all its packets carry
-// this launch's epoch and the ring slot s mod RINGP is free.
+struct Tile {
+    int J, K;
+    March m;
+    bool yup, zup;   // an upstream tile along y / z that holds WATER
+    bool ydn, zdn;   // a downstream one
+};
+
+// ---- boundary packets -----------------------------------------------------------
+// One row of 16-byte packets per group and edge: NL lanes x NP packets, a
+// lane's four values.  A word that has not been sent holds kEmpty, a NaN that
+// no value takes (may_send); of an FP64 value the high word tells.  The
+// receiver puts kEmpty back, so a row is empty again when the kernel ends: a
+// tile sends exactly the groups that its downstream tile receives.
+template <int NP>
+__device__ inline u32x4 may_send(u32x4 v) {
+    if constexpr (NP == 1) {
+        for (int k = 0; k < 4; k++) v[k] = min(v[k], kEmpty - 1);
+    } else {
+        v[1] = min(v[1], kEmpty - 1);
+        v[3] = min(v[3], kEmpty - 1);
+    }
+    return v;
+}
+template <int NP>
+__device__ inline bool is_sent(u32x4 v) {
+    if constexpr (NP == 1) return max(max(v[0], v[1]), max(v[2], v[3])) != kEmpty;
+    else return max(v[1], v[3]) != kEmpty;
+}
+
+// ---- receiving wave: upstream tile edge -> LDS ring ---------------------------
+// The -y edge carries 64 lanes, the -z edge WF_TY rows; the wave forwards whole
+// groups, once all packets of a group are there and its ring slot is free.
 template <int KIND, bool YEDGE>
-__device__ void comm_wave(const WaveArgs& A, WaveLds<KIND>& S, int J, int K, bool yup, bool zup) {
-    using KD = Kind<KIND>;
-    constexpr int NP = KD::NP, B = KD::BATCH, RINGP = KD::RINGP;
-    constexpr int NL = YEDGE ? WF_TZ : WF_TY;    // values per step
-    if (YEDGE ? !yup : !zup) return;   // no upstream tile, or one without WATER (its edge is all zeros)
+__device__ void recv_wave(const WaveArgs& A, WaveLds<KIND>& S, const Tile& T) {
+    constexpr int NP = Kind<KIND>::NP;
+    constexpr int B = 4;   // groups polled at once: a poll takes as long as two to three groups
+    constexpr int NL = YEDGE ? WF_TZ : WF_TY;
+    constexpr uint32_t kRow = NL * NP * 16;   // bytes per group
+    if (YEDGE ? !T.yup : !T.zup) return;      // no upstream tile, or one without WATER (its edge is all zeros)
     const int l = threadIdx.x % 64;
     const bool on = l < NL;
     const int li = on ? l : 0;
-    const int nxi = A.nx - 2;
-    // steps 0 .. end-1 are consumed: row 0 lane l at l .. l+nxi-1 (-y edge),
-    // lane 0 of the rows of wave w at w .. w+nxi-1 (-z edge)
-    const int end = (YEDGE ? WF_TZ - 1 : WF_NW - 1) + nxi;
-    // packets written by the upstream tile (J-1, K) or (J, K-1)
-    const int64_t up = YEDGE ? (int64_t)(J - 1) * A.TK + K : (int64_t)J * A.TK + K - 1;
-    const uint64_t* base = YEDGE ? A.ybnd + up * A.SP * WF_TZ * NP : A.zbnd + up * A.SP * WF_TY * NP;
+    const int end = YEDGE ? T.m.ng : z_groups<Kind<KIND>::FWD>(T.m);
+    const int64_t up = YEDGE ? (int64_t)(T.J - 1) * A.TK + T.K : (int64_t)T.J * A.TK + T.K - 1;
+    const __amdgpu_buffer_rsrc_t buf = rsrc((YEDGE ? A.ybnd : A.zbnd) + up * A.SG * (kRow / 16), (int64_t)A.SG * kRow);
     // the consumer of lane l: wave 0 for the -y edge, the wave holding row l for the -z edge
-    const int* cprog = &S.prog[YEDGE ? 0 : li / WF_R];
-    int s0 = 0, idle = 0;
-    while (s0 < end) {
-        uint64_t buf[B][NP];
+    const int* used = &S.cnt[(YEDGE ? 0 : li / WF_R) + 2].in;
+    auto publish = [&](int g) {
+        if (YEDGE) {
+            if (l == 0) lput(&S.cnt[1].in, g);
+        } else if (l < WF_NW) {
+            lput(&S.cnt[l + 1].zin, g);
+        }
+    };
+    int g0 = 0, idle = 0;
+    while (g0 < end) {
+        u32x4 v[B][NP];
 #pragma unroll
         for (int b = 0; b < B; b++) {
-            const int sb = min(s0 + b, end - 1);
-            const uint64_t* p = base + ((int64_t)sb * NL + li) * NP;
+            const uint32_t row = (uint32_t)min(g0 + b, end - 1) * kRow;
 #pragma unroll
-            for (int k = 0; k < NP; k++) buf[b][k] = gpeek(p + k);
+            for (int c = 0; c < NP; c++)
+                v[b][c] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                    buf, (uint32_t)(c * NL + li) * 16u, row, kDeviceScope | kVolatile));
         }
-        const int limit = lpeek32(cprog) + RINGP;   // slot of step sb is free if sb - RINGP was consumed
-        int published = 0;
+        const int limit = lget(used) + kRing;   // groups below it have a free slot
+        int n = 0;
         bool stop = false;
 #pragma unroll
         for (int b = 0; b < B; b++) {
-            const int sb = s0 + b;
-            bool ok = !on || sb <= limit;
+            bool ok = g0 + b < limit;
 #pragma unroll
-            for (int k = 0; k < NP; k++) ok = ok && (!on || (uint32_t)(buf[b][k] >> 32) == A.epoch);
-            stop = stop || sb >= end || !__all(ok);
+            for (int c = 0; c < NP; c++) ok = ok && is_sent<NP>(v[b][c]);
+            stop = stop || g0 + b >= end || !__all(!on || ok);
             if (!stop) {
+                const int slot = (g0 + b) % kRing;
                 if (on) {
-                    uint64_t* slot = YEDGE ? &S.yp[sb % RINGP][0][li] : &S.zp[sb % RINGP][0][li];
 #pragma unroll
-                    for (int k = 0; k < NP; k++) lput(slot + k * NL, pack((uint32_t)buf[b][k], (uint32_t)sb));
+                    for (int c = 0; c < NP; c++)
+                        lput4(YEDGE ? &S.ring[0][slot][c][li][0] : &S.zi[0][slot][li][c][0], v[b][c]);
                 }
-                published++;
+                n++;
+                publish(g0 + n);
             }
         }
-        s0 += published;
-        if (published > 0) {
+        g0 += n;
+        if (n > 0) {
             idle = 0;
         } else {
             if (++idle > kSpinLimit / 64) {
@@ -255,388 +345,241 @@ __device__ void comm_wave(const WaveArgs& A, WaveLds<KIND>& S, int J, int K, boo
                 break;
             }
             if ((idle & 15) == 0 && gave_up(A.err)) break;
-            __builtin_amdgcn_s_sleep(2);
         }
     }
+    publish(kAll);
+    // empty the rows again, after the last poll: the memory counter orders a poll behind older stores
+    if (on)
+        for (int g = 0; g < end; g++)
+#pragma unroll
+            for (int c = 0; c < NP; c++)
+                __builtin_amdgcn_raw_buffer_store_b128(u32x4{kEmpty, kEmpty, kEmpty, kEmpty}, buf,
+                                                       (uint32_t)(c * NL + li) * 16u, (uint32_t)g * kRow, 0);
 }
 
-// ---- sending wave: this tile's edge (LDS out-ring) -> HBM packets ----------
-// The packet of downstream step s is the value the compute waves produced at
-// step s + lag (lag NW-1 for the +y edge: the last row of wave NW-1; 63 for
-// the +z edge: lane 63 of every row).  The wave waits until every value of
-// that step carries its step tag, stores the step's packets with
-// device-scope stores and reports its progress every 4 steps, which the
-// compute waves check before reusing an out-ring slot.  The device-scope
-// stores stay out of the compute waves, whose memory counter also orders
-// their prefetch loads.
-template <int KIND, bool YEDGE>
-__device__ void send_wave(const WaveArgs& A, WaveLds<KIND>& S, int J, int K) {
+// ---- sending wave: this tile's +z edge (LDS) -> packets ---------------------------
+// Element e of the downstream march is element e + z_shift of this tile's lane
+// 63 (zero outside this march).
+template <int KIND>
+__device__ void send_wave(const WaveArgs& A, WaveLds<KIND>& S, const Tile& T) {
+    constexpr bool FWD = Kind<KIND>::FWD;
     constexpr int NP = Kind<KIND>::NP;
-    constexpr int NL = YEDGE ? WF_TZ : WF_TY;
-    int* prog = &S.sprog[YEDGE ? 0 : 1];
+    constexpr int NL = WF_TY;
+    constexpr uint32_t kRow = NL * NP * 16;
+    constexpr int kMask = kRingZ * WF_G - 1;
+    if (!T.zdn) return;   // nobody downstream: counters preset to kAll
     const int l = threadIdx.x % 64;
-    if (YEDGE ? J == A.TJ - 1 : K == A.TK - 1) return;   // no downstream tile: progress preset to "all sent"
     const bool on = l < NL;
     const int li = on ? l : 0;
-    const int lag = YEDGE ? WF_NW - 1 : WF_TZ - 1;
-    const int end = (YEDGE ? WF_TZ - 1 : WF_NW - 1) + (A.nx - 2);   // downstream steps consumed
-    const int64_t tile = (int64_t)J * A.TK + K;
-    uint64_t* out = YEDGE ? A.ybnd + tile * A.SP * WF_TZ * NP : A.zbnd + tile * A.SP * WF_TY * NP;
-    for (int s = 0; s < end; s++) {
-        const int t = s + lag;
-        const uint64_t* src = YEDGE ? &S.yo[t & (kRingO - 1)][0][li] : &S.zo[t & (kRingO - 1)][0][li];
-        uint64_t v[NP];
-        int spins = 0;
-        for (;;) {
-            bool ok = true;
-#pragma unroll
-            for (int k = 0; k < NP; k++) {
-                v[k] = lpeek(src + k * NL);
-                ok = ok && (!on || tag_of(v[k]) == t);
-            }
-            if (__all(ok)) break;
+    const int64_t tile = (int64_t)T.J * A.TK + T.K;
+    const __amdgpu_buffer_rsrc_t buf = rsrc(A.zbnd + tile * A.SG * (kRow / 16), (int64_t)A.SG * kRow);
+    const March dn = march_of<FWD>(A, T.K + 1, T.m.xa, T.m.xb);
+    const int end = z_groups<FWD>(dn), shift = z_shift<FWD>(T.m, dn);
+    const int* ready = &S.cnt[li / WF_R + 2].in;
+    auto release = [&](int g) {   // zo slots below g have been sent
+        if (l < WF_NW) lput(&S.cnt[l + 1].zout, g + kRingZ);
+    };
+    for (int g = 0; g < end; g++) {
+        const int e0 = WF_G * g + shift;   // first element of this march that the group needs
+        const int need = min((e0 + 2 * WF_G - 1) / WF_G, T.m.ng);
+        for (int spins = 0; !__all(!on || lget(ready) >= need);) {
             if (++spins > kSpinLimit || ((spins & 1023) == 0 && gave_up(A.err))) {
-                if (l == 0) {
-                    atomicOr(A.err, 1);
-                    lput32(prog, INT_MAX);   // never block the compute waves
-                }
+                if (l == 0) atomicOr(A.err, 1);
+                release(kAll);   // never block the compute waves
                 return;
             }
             if (spins > kBusyPolls) __builtin_amdgcn_s_sleep(1);
         }
         if (on) {
+            u32x4 v[NP];
 #pragma unroll
-            for (int k = 0; k < NP; k++)
-                __hip_atomic_store(out + ((int64_t)s * NL + li) * NP + k, pack((uint32_t)v[k], A.epoch), __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
+            for (int k = 0; k < WF_G * NP; k++) {
+                const int e = e0 + k / NP;
+                const uint32_t u = lget(&S.zo[li][(e & kMask) * NP + k % NP]);
+                v[k / 4][k % 4] = e < 0 || e >= WF_G * T.m.ng ? 0u : u;
+            }
+#pragma unroll
+            for (int c = 0; c < NP; c++)
+                __builtin_amdgcn_raw_buffer_store_b128(may_send<NP>(v[c]), buf, (uint32_t)(c * NL + li) * 16u,
+                                                       (uint32_t)g * kRow, kDeviceScope);
         }
-        if ((s & 3) == 3 && l == 0) lput32(prog, t);
+        release(max(0, (e0 + WF_G) / WF_G));   // groups whose elements all lie below the next one needed
         for (int i = 0; i < A.send_delay; i++) __builtin_amdgcn_s_sleep(127);
     }
-    if (l == 0) lput32(prog, INT_MAX);
+    release(kAll);
 }
 
 // ---- compute waves -------------------------------------------------------------
 // Factor (KIND 0, FP64):   e = diag - sum_a (A_a p_a)^2 - tau sum_a A_a (o1 + o2) p_a^2,
-//                          guarded by sigma, p = 1/sqrt(e)  (calculatePreconditioner)
-// forward sweep (KIND 1):  q = (r - sum_{-a fluid} A_a q_a p_a) * p, wave value q*p
-// backward sweep (KIND 2): z = (q - p * sum_{+a fluid} A_a z_a) * p, wave value z
+//                          guarded by sigma, p = 1/sqrt(e)  (calculatePreconditioner); passes p on
+// forward sweep (KIND 1):  q = (r - sum_{-a fluid} A_a q_a p_a) * p; passes m = A_a q p on
+// backward sweep (KIND 2): z = (q - p * sum_{+a fluid} A_a z_a) * p; passes m = A_a z on
 // with A_a = -scale, products and sums in the reference's order (x, y, z).
-// In the sweeps a neighbour that is not WATER carries exactly +0, whose term
-// -scale * (+0) = -0 leaves any partial sum unchanged, so they sum all three.
-template <int KIND>
-__device__ void compute_wave(const WaveArgs& A, WaveLds<KIND>& S, int J, int K, bool yup, bool zup) {
+// A sweep's neighbour term A_a * value is the same for the three cells that use
+// it, so the cell computes it once (same rounding).  A neighbour that is not
+// WATER carries +0 (the fused multiply-add with +0 turns -0 into it), which
+// leaves any partial sum unchanged, so the sweeps sum all three.
+// LAST: the tile's last wave, whose last row is the +y edge: it stores the packets itself, which
+// spares the edge a round trip through LDS and another wave.
+template <int KIND, bool LAST>
+__device__ __forceinline__ void compute_wave(const WaveArgs& A, WaveLds<KIND>& S, const Tile& T) {
 #pragma clang fp contract(off)
     using KD = Kind<KIND>;
-    using T = typename KD::T;
+    using V = typename KD::T;
     constexpr bool FWD = KD::FWD;
-    constexpr int NP = KD::NP, RINGP = KD::RINGP, R = WF_R, NW = WF_NW, TY = WF_TY;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    constexpr int NP = KD::NP, R = WF_R;
+    const int w = LAST ? WF_NW - 1 : __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const int tz = threadIdx.x % 64;
-    const int nx = A.nx, nxi = A.nx - 2;
-    const int nsteps = wave_steps(nxi);
-    const uint32_t plane = (uint32_t)(A.ny * A.nz);
-    const uint32_t nc = (uint32_t)nx * plane;   // below 2^28 (kWaveMaxCells)
-    // Plane offsets are byte offsets for the widest element a kernel addresses: 8-byte (the
-    // factor's P64) or 4-byte (the sweeps), so the sweeps use them without a shift.
-    constexpr uint32_t kUnit = KIND == 0 ? 8u : 4u;
-    const uint32_t plane8 = plane * kUnit, nc8 = nc * kUnit;
-    auto off4 = [](uint32_t o) { return KIND == 0 ? o >> 1 : o; };   // 4-byte elements
-    // buffer resources.  factor: rA nbinfo, rC P64, rD P32;  sweeps: rA P32, rB in, rC out.
-    // The sweeps read P32 alone: it is 0 for every non-WATER cell (cleared before each factor,
-    // which writes WATER cells only), so P != 0 is the WATER test and the neighbour flags are
-    // not needed (non-WATER values are 0 on the upstream side).
-    __amdgpu_buffer_rsrc_t rA, rB, rC, rD;
+    const uint32_t cells = (uint32_t)(A.ny * A.nz);   // of one plane
+    const uint32_t ngroups = (uint32_t)(A.nxp / WF_G);
+    // byte offsets are counted for the float vectors: 16 per (y, z) column and group
+    const uint32_t gstride = cells * 16u, total = gstride * ngroups;
+    // buffer resources.  sweeps: rA P32, rB in, rC out; factor: rA nbinfo (offsets halved), rC P32
+    __amdgpu_buffer_rsrc_t rA, rB, rC;
     if constexpr (KIND == 0) {
-        rA = rsrc(A.nbinfo, (int64_t)nc * 2);
+        rA = rsrc(A.nbinfo, (int64_t)total / 2);
+        rC = rsrc(A.P32, (int64_t)total);
         rB = rA;
-        rC = rsrc(A.P64, (int64_t)nc * 8);
-        rD = rsrc(A.P32, (int64_t)nc * 4);
     } else {
         // ranges one and two words longer than the arrays (never addressed): distinct descriptor
         // words keep the compiler from rebuilding one descriptor from another at every access
-        rA = rsrc(A.P32, (int64_t)nc * 4 + 8);
-        rB = rsrc(A.in, (int64_t)nc * 4);
-        rC = rsrc(A.out, (int64_t)nc * 4 + 4);
+        rA = rsrc(A.P32, (int64_t)total + 8);
+        rB = rsrc(A.in, (int64_t)total);
+        rC = rsrc(A.out, (int64_t)total + 4);
         // opaque to the compiler from here on, so that it keeps each descriptor whole in
         // four SGPRs instead of sharing equal words and reassembling them at every access
         asm volatile("" : "+s"(rA), "+s"(rB), "+s"(rC));
-        rD = rC;
     }
     const float ms = A.ms;
     const double scale = A.scale;
-
-    // All R rows of wave w process x-index xl = t - w - tz at step t (row r
-    // uses row r-1's value of the same step), so the lane enters the grid
-    // along x at step w + tz, and the wave's cells of one step lie in one
-    // rotated plane: FWD x + rot(z) = 1 + t - w;  BWD x + rot(z) = nx + 61 + w - t.
-    // Per row: the lane's in-plane byte offsets for 8-, 4- and 2-byte
-    // elements (kOob, shifted, stays out of range for every array).  Per
-    // wave: the byte offsets (8-byte elements) of the rotated plane of the
-    // current step and of the prefetch step, in scalar registers.
-    uint32_t lo8[R], lo4[R], lo2[R];
-    bool colr[R], colz[R];
-    const int z = z_of<FWD>(A, K, tz);
-    const int base = w + tz;
-    uint32_t oc = (uint32_t)(FWD ? ((1 - w) % nx + nx) % nx : (61 + w) % nx) * plane8;
-    uint32_t op = oc;
+    const int z = z_of<FWD>(A, T.K, tz);
+    const int rho = FWD ? tz : WF_TZ - 1 - tz;   // rot(z)
+    uint32_t off[R];                             // the lane's byte offset per row, kOob off the grid
     unroll<R>([&](auto rc) {
         constexpr int r = decltype(rc)::value;
         const int ty = w * R + r;
-        const int y = y_of<FWD>(A, J, ty);
-        const bool rowin = J * TY + ty < A.ny - 2;
-        colr[r] = rowin && z <= A.nz - 2;
-        lo8[r] = colr[r] ? (uint32_t)(y * A.nz + z) * 8u : kOob;
-        lo4[r] = lo8[r] >> 1;
-        lo2[r] = lo8[r] >> 2;
-        // lane 0 of the row reads -z packets when there is an upstream z tile
-        colz[r] = zup && rowin;
+        const int y = y_of<FWD>(A, T.J, ty);
+        const bool in = T.J * WF_TY + ty < A.ny - 2 && z <= A.nz - 2;
+        off[r] = in ? (uint32_t)(y * A.nz + z) * 16u : kOob;
     });
-    // the rotated plane of the next step; readfirstlane keeps the offset in a
-    // scalar register (a per-lane copy turns each buffer access into a loop)
+    // the lane has cells of the x range in the march groups first .. first + span
+    const int glo = (T.m.xa + rho) / WF_G, ghi = (T.m.xb + rho) / WF_G;
+    const int first = FWD ? glo - T.m.g0 : T.m.g0 - ghi;
+    const uint32_t span = (uint32_t)(ghi - glo);
+    // ORed onto the offsets of group g: 0 inside, kOob outside (opaque, so that it stays a select)
+    auto outside = [&](int g) {
+        uint32_t o = (uint32_t)(g - first) <= span ? 0u : kOob;
+        asm volatile("" : "+v"(o));
+        return o;
+    };
     auto advance = [&](uint32_t& o) {
         if (FWD) {
-            o += plane8;
-            if (o >= nc8) o -= nc8;
+            o += gstride;
+            if (o >= total) o -= total;
         } else {
-            // o - plane8 wraps above every offset when o < plane8: the smaller of the two is the
-            // wrapped-around plane (scalar subtract, add and min, as in the forward direction)
-            const uint32_t below = o - plane8, wrapped = o + (nc8 - plane8);
+            // o - gstride wraps above every offset when o < gstride: the smaller of the two is the
+            // wrapped-around group
+            const uint32_t below = o - gstride, wrapped = o + (total - gstride);
             o = below < wrapped ? below : wrapped;
         }
-        o = __builtin_amdgcn_readfirstlane(o);
+        o = __builtin_amdgcn_readfirstlane(o);   // a per-lane copy turns each buffer access into a loop
     };
-    // prefetch ring: per-cell inputs of the next kPrefetch steps
-    uint32_t wring[kPrefetch][R];   // factor: nbinfo; sweeps: P32 bits
-    float iring[kPrefetch][R];
-    auto fetch = [&](int d, int r) {
-        if constexpr (KIND == 0) {
-            wring[d][r] = bload16(rA, lo2[r], op >> 2);
-            iring[d][r] = 0.f;
-        } else {
-            wring[d][r] = __float_as_uint(bload32f(rA, lo4[r], off4(op)));
-            iring[d][r] = bload32f(rB, lo4[r], off4(op));
-        }
-    };
-    // issue order pinned, and each prologue step issues as many memory
-    // operations as the loop steps do (the stores of a step, here dropped as
-    // out of range, then the loads): the wait for slot d then allows the same
-    // number of younger operations on entry as at every later step
-    constexpr int kStores = (KIND == 0 ? 2 : 1) * R;
-    unroll<kPrefetch>([&](auto dc) {
+    uint32_t op = __builtin_amdgcn_readfirstlane((uint32_t)T.m.g0 % ngroups * gstride);   // prefetched group's offset
+    // inputs of the next kPrefetch groups, with the offsets they were loaded from: the result of a
+    // group goes to the same place of another vector.  factor: nbinfo; sweeps: P32 and the input vector
+    f32x4 pq[kRing][R], iq[kRing][R];
+    u32x2 nq[kRing][R];
+    uint32_t lo[kRing][R], go[kRing];
+    auto fetch = [&](auto dc, int g) {
         constexpr int d = decltype(dc)::value;
-        unroll<kStores>([&](auto) { bstore32(0u, rC, kOob, 0); });
-        unroll<R>([&](auto rc) { fetch(d, decltype(rc)::value); });
+        const uint32_t out = outside(g);
+        go[d] = op;
+        unroll<R>([&](auto rc) {
+            constexpr int r = decltype(rc)::value;
+            const uint32_t o = off[r] | out;
+            lo[d][r] = o;
+            if constexpr (KIND == 0) {
+                nq[d][r] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rA, o >> 1, op >> 1, 0));
+            } else {
+                pq[d][r] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rA, o, op, 0));
+                iq[d][r] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rB, o, op, 0));
+            }
+        });
         advance(op);
+    };
+    // issue order pinned, and each prologue group issues as many memory operations as the loop's
+    // groups do (the stores, here dropped as out of range, then the loads): the wait for slot d then
+    // allows the same number of younger operations on entry as at every later group
+    constexpr int kStores = (KIND == 0 ? 3 : 1) * R + (LAST ? NP : 0);
+    unroll<kPrefetch>([&](auto dc) {
+        unroll<kStores>([&](auto kc) {
+            __builtin_amdgcn_raw_buffer_store_b128(u32x4{}, rC, kOob + 16u * decltype(kc)::value, 0, 0);
+        });
+        fetch(dc, decltype(dc)::value);
         __builtin_amdgcn_sched_barrier(0);
     });
-    // Value rings: wave w < NW-1 writes its last row into v[w] (slot t mod kRingV), the last wave
-    // into the +y out-ring yo (slot t mod kRingO), which the sending wave forwards and wave NW-2's
-    // reuse check reads.  Both have kSlotV words per slot, so a step's slot is a constant offset
-    // from the block's base.
-    constexpr int kSlotV = NP * WF_TZ;   // words per ring slot
-    const uint64_t* up_base = &S.v[w > 0 ? w - 1 : 0][0][0][tz];
-    const uint64_t* dn_base = &S.v[w < NW - 2 ? w + 1 : 0][0][0][tz];
-    const bool dn_yo = w == NW - 2;   // the downstream wave's ring is yo
-    // +z out-ring: lane 63 writes its rows into zo[slot][k][w R + r]; the other lanes write the same
-    // pattern into a sink of their own, so the store needs no lane mask (slot stride 0 there)
-    const bool zl = tz == WF_TZ - 1;
-    uint64_t* const zo_lane = zl ? &S.zo[0][0][w * R] : &S.zsink[w][tz][0];
-    const uint32_t zo_stride = zl ? NP * TY : 0;   // words per ring slot
-    const uint64_t* yp_base = &S.yp[0][0][tz];
-    const uint64_t* zp_base = &S.zp[0][0][w * R];
-    const bool cy = w == 0 && yup;
-    // Sweeps: the readiness test as 64-bit lane masks.  Each tag test is one
-    // compare whose ballot is ANDed with a mask of the lanes that need it:
-    // the uniform conditions select a whole mask in scalar code, the lane
-    // conditions (row in the grid, x in the grid) are ballots of single
-    // compares, so no boolean is turned into a lane value and back.
-    // Row 0's value is needed by every lane for w > 0 (at t = 0 the ring's
-    // initial tag -1 matches t - 1), and for wave 0 by the lanes of its first
-    // row that are in the grid, when there is an upstream y tile.
-    // Row 0's value is needed by every lane for w > 0 (at t = 0 the ring's
-    // initial tag -1 matches t - 1), and for wave 0 by the lanes of its first
-    // row that are in the grid, when there is an upstream y tile.  The -z
-    // packets are needed by the rows with an upstream z tile while the row's
-    // lane 0 is in the grid.
-    const bool cy_u = __builtin_amdgcn_readfirstlane(cy ? 1 : 0) != 0;
-    const uint64_t ma_all = w > 0 ? ~0ull : 0ull;
-    const uint64_t ma_row = cy_u ? __builtin_amdgcn_ballot_w64(colr[0]) : 0ull;
-    uint64_t colz_m[R];
-    unroll<R>([&](auto rc) {
-        constexpr int r = decltype(rc)::value;
-        colz_m[r] = __builtin_amdgcn_ballot_w64(colz[r]);
-    });
-    T prev[R];
-    unroll<R>([&](auto rc) { prev[decltype(rc)::value] = 0; });
-    // Upstream values of one step: the previous wave's last row (ring slot),
-    // the -y and -z packets and, every kBpEvery steps, the next wave's ring
-    // slot (reuse check).  The reads of step t+1 are issued right after step
-    // t's ring write, so their latency overlaps the rest of step t; the tag
-    // test at the top of step t+1 re-reads only if a value was not there yet.
-    // Sweeps: row 0's -y value comes from one ring, the previous wave's
-    // (w > 0, tagged t - 1) or, for wave 0, the -y packets (tagged t; a first
-    // y tile's ring holds zeros), so one read, one tag test and no select.
-    uint64_t a[NP], c[NP], zq[R][NP], bp = 0;
-    const uint64_t* a0_base = (KIND != 0 && w == 0) ? yp_base : up_base;
-    int spy = 0, spz = 0;   // progress of the sending waves (read on reuse-check steps)
-    // ring slots of the current block of kPrefetch steps: step t0 + d uses slot pz0 + d of the
-    // packet rings and so0 + d of the out-rings (no wrap inside a block), so the slot offsets of
-    // the unrolled steps are constants
-    static_assert(RINGP % kPrefetch == 0 && kRingO % kPrefetch == 0, "blocks do not wrap the rings");
-    int pz0 = 0, so0 = 0;
-    // sweeps: the block's base for row 0's -y value, so that step t0 + d2 (d2 = 1 .. kPrefetch-1)
-    // reads at a constant offset (d2 - 1 slots): the upstream wave's ring (slot d2 - 1) or, for
-    // wave 0, the packet ring (slot pz0 + d2)
-    const uint64_t* a_blk = up_base;
-    auto rd_at = [&](auto dc2, int tt) {
-        constexpr int d2 = decltype(dc2)::value;   // tt mod kPrefetch (= tt mod kRingV)
-        constexpr int s_up = (d2 + kRingV - 1) % kRingV, s_bp = (d2 + kBpEvery) % kRingV;
-        // tt = t0 + d2 inside the block (d2 > 0), or the first step of the next block
-        const int ps = d2 != 0 ? pz0 + d2 : tt % RINGP;
-        if constexpr (KIND != 0) {
-            static_assert(NP == 1, "one word per sweep value");
-            if constexpr (d2 != 0) {
-                a[0] = lpeek(a_blk + (d2 - 1) * kSlotV);
-            } else {   // tt = t0 + kPrefetch, or tt = t0 (re-read) / 0 (first read)
-                const int aoff = w > 0 ? s_up * kSlotV : ps * NP * WF_TZ;
-                a[0] = lpeek(a0_base + aoff);
-            }
-        } else {
+    constexpr int kSlot = NP * WF_TZ * 4, kSlotZ = WF_TY * NP * 4;   // words per ring slot
+    const uint32_t* const in_ring = &S.ring[w][0][0][tz][0];
+    uint32_t* const out_ring = &S.ring[LAST ? 0 : w + 1][0][0][tz][0];   // LAST: not used
+    const uint32_t* const z_ring = &S.zi[tz == 0 ? 0 : 1][0][w * R][0][0];
+    const int* const my_cnt = &S.cnt[w + 1].in;
+    int* const in_below = &S.cnt[w + 2].in;
+    int* const out_above = &S.cnt[w].out;
+    // ends with the march's groups, or is empty if nobody is downstream: what is sent is received
+    const __amdgpu_buffer_rsrc_t ybuf = rsrc(A.ybnd + ((int64_t)T.J * A.TK + T.K) * A.SG * (WF_TZ * NP),
+                                             LAST && T.ydn ? (int64_t)T.m.ng * WF_TZ * NP * 16 : 0);
+    // upstream values of a group: its ring slots, read once the counters vouch for them
+    Group<V> up, zp[R];
+    auto read_slots = [&](auto dc) {
+        constexpr int d = decltype(dc)::value % kRing;
 #pragma unroll
-            for (int k = 0; k < NP; k++) {
-                a[k] = lpeek(up_base + s_up * kSlotV + k * WF_TZ);
-                c[k] = lpeek(yp_base + ps * NP * WF_TZ + k * WF_TZ);
-            }
-        }
-        if constexpr (KIND != 0 && R == 2) {
-            // both rows' words in one 16-byte LDS read (each word carries its own tag)
-            const u64x2 q = lpeek2(zp_base + ps * TY);
-            zq[0][0] = q.x;
-            zq[1][0] = q.y;
-        } else {
-            unroll<R>([&](auto rc) {
-                constexpr int r = decltype(rc)::value;
+        for (int c = 0; c < NP; c++) up.q[c] = lget4(in_ring + d * kSlot + c * WF_TZ * 4);
+        unroll<R>([&](auto rc) {
+            constexpr int r = decltype(rc)::value;
 #pragma unroll
-                for (int k = 0; k < NP; k++) zq[r][k] = lpeek(zp_base + ps * NP * TY + k * TY + r);
-            });
-        }
-        if constexpr (d2 % kBpEvery == 0) {
-            // the downstream wave's slot of step tt - (kRingV - kBpEvery)
-            const int so_bp = ((d2 != 0 ? so0 + d2 : tt) - (kRingV - kBpEvery)) & (kRingO - 1);
-            bp = lpeek(dn_yo ? &S.yo[so_bp][0][tz] : dn_base + s_bp * kSlotV);
-            spy = lpeek32(&S.sprog[0]);
-            spz = lpeek32(&S.sprog[1]);
+            for (int c = 0; c < NP; c++) zp[r].q[c] = lget4(z_ring + d * kSlotZ + (r * NP + c) * 4);
+        });
+    };
+    // waits until group g can run: its upstream values are there, and the slots it writes are free
+    auto wait_for = [&](i32x4 cnt, int g, auto dc) {
+        auto behind = [&]() {
+            return __builtin_amdgcn_ballot_w64(min(min(cnt[0], cnt[1]), min(cnt[2], cnt[3])) <= g) != 0;
+        };
+        if (__builtin_expect(behind(), 0)) {
+            int spins = 0;
+            do {
+                if (spins > kBusyPolls) __builtin_amdgcn_s_sleep(1);
+                cnt = lget4(my_cnt);
+                read_slots(dc);
+                if ((++spins & 1023) == 0 && (spins >= kSpinLimit || gave_up(A.err))) {
+                    if (tz == 0) atomicOr(A.err, 1);
+                    cnt = i32x4{kAll, kAll, kAll, kAll};   // carry on with whatever is there
+                }
+            } while (behind());
         }
     };
-    static_assert(kRingV == kPrefetch, "ring slots are indexed by the unrolled step");
-    rd_at(std::integral_constant<int, 0>{}, 0);
-    for (int t0 = 0; t0 < nsteps; t0 += kPrefetch) {
-        pz0 = t0 % RINGP;
-        so0 = t0 & (kRingO - 1);
-        uint64_t* const my_blk = w == NW - 1 ? &S.yo[so0][0][tz] : &S.v[w][0][0][tz];
-        a_blk = w > 0 ? up_base : yp_base + (pz0 + 1) * NP * WF_TZ;
-        uint64_t* const zblk = zo_lane + (uint32_t)so0 * zo_stride;
-        // compile-time step index, so each prefetch slot stays in one register
-        // and the value-ring slots are constants
-        unroll<kPrefetch>([&](auto dc) {
-            constexpr int d = decltype(dc)::value;
-            constexpr bool bp_step = d % kBpEvery == 0;
-            const int t = t0 + d;
-            // the tail of the previous step (prefetch, plane advance) stays ahead of the
-            // tag checks, so the latency of the values read ahead is overlapped
-            __builtin_amdgcn_sched_barrier(0);
-            // ---- receive: tag checks of the values read ahead (re-read while not ready)
-            const bool need_up = w > 0 && t > 0;
-            const bool need_bp = bp_step && w < NW - 1 && t >= kRingV - kBpEvery;
-            const int t_bp = t - (kRingV - kBpEvery);
-            // out-ring slots of steps t .. t + kBpEvery - 1 are free once the sending waves passed
-            // step t + kBpEvery - 1 - kRingO (the last wave feeds the +y ring, every wave the +z ring)
-            const int t_bo = t + kBpEvery - 1 - kRingO;
-            // the lane's x-index is in the grid (same for all rows of the wave),
-            // and the same test for lane 0 (the -z packet consumer)
-            const bool xin = (unsigned)(t - base) < (unsigned)nxi;
-            const bool xin0 = (unsigned)(t - w) < (unsigned)nxi;
-            bool act[R], need_z[R];
+    V prev[R];
+    unroll<R>([&](auto rc) { prev[decltype(rc)::value] = 0; });
+    wait_for(i32x4{0, 0, 0, 0}, 0, std::integral_constant<int, 0>{});
+    auto group = [&](auto dc, int g, uint32_t* zo) {
+        constexpr int d = decltype(dc)::value;
+        __builtin_amdgcn_sched_barrier(0);
+        // ---- the group's 4 steps of R rows
+        Group<V> mine[R];    // what the rows pass on
+        f32x4 res[R];        // sweeps: the result; factor: the FP32 copy
+        unroll<WF_G>([&](auto jc) {
+            constexpr int j = decltype(jc)::value;
+            constexpr int e = FWD ? j : WF_G - 1 - j;   // the step's plane inside the storage group
+            V above = up.get(j);
             unroll<R>([&](auto rc) {
                 constexpr int r = decltype(rc)::value;
-                act[r] = colr[r] && xin;
-                need_z[r] = colz[r] && xin0;
-            });
-            const bool need_y = cy && act[0];
-            // branch-free: per-lane masks, one ballot (the -z packet slots are
-            // read by every lane from one address, so their test is uniform).
-            // The out-ring test reads the sending waves' progress as last read,
-            // so each re-read of the spin loop below can pass it.
-            auto ready = [&]() {
-                const bool bo_ok = !bp_step || (spz >= t_bo && (w != NW - 1 || spy >= t_bo));
-                if constexpr (KIND != 0) {
-                    const int ta = w > 0 ? t - 1 : t;
-                    const uint64_t m_a = ma_all | (ma_row & __builtin_amdgcn_ballot_w64(xin));
-                    const bool xin0_u = (unsigned)(t - w) < (unsigned)nxi;
-                    uint64_t bad = __builtin_amdgcn_ballot_w64(tag_of(a[0]) != ta) & m_a;
-                    if constexpr (bp_step) {
-                        if (w < NW - 1 && t >= kRingV - kBpEvery) bad |= __builtin_amdgcn_ballot_w64(tag_of(bp) < t_bp);
-                    }
-                    unroll<R>([&](auto rc) {
-                        constexpr int r = decltype(rc)::value;
-                        bad |= __builtin_amdgcn_ballot_w64(tag_of(zq[r][0]) != t) & (xin0_u ? colz_m[r] : 0ull);
-                    });
-                    return bo_ok && bad == 0;
-                }
-                unsigned lane = (unsigned)(tag_of(bp) >= t_bp) | (unsigned)!need_bp;
-#pragma unroll
-                for (int k = 0; k < NP; k++) {
-                    lane &= ((unsigned)(tag_of(a[k]) == t - 1) | (unsigned)!need_up) &
-                            ((unsigned)(tag_of(c[k]) == t) | (unsigned)!need_y);
-                    unroll<R>([&](auto rc) {
-                        constexpr int r = decltype(rc)::value;
-                        lane &= (unsigned)(tag_of(zq[r][k]) == t) | (unsigned)!need_z[r];
-                    });
-                }
-                return bo_ok && __builtin_amdgcn_ballot_w64(lane == 0u) == 0;
-            };
-            if (__builtin_expect(!ready(), 0)) {   // the spin path out of line: the ready step falls through
-                int spins = 0;
-                do {
-                    if (++spins > kSpinLimit) {
-                        if (tz == 0) atomicOr(A.err, 1);
-                        break;
-                    }
-                    if ((spins & 1023) == 0 && gave_up(A.err)) break;
-                    if (spins > kBusyPolls) __builtin_amdgcn_s_sleep(1);
-                    rd_at(dc, t);
-                } while (!ready());
-            }
-            // ---- compute the R rows (all upstream values are from step t-1)
-            T vnew[R];
-            unroll<R>([&](auto rc) {
-                constexpr int r = decltype(rc)::value;
-                T vy = 0, vz, vin;
-                if constexpr (KIND != 0) {
-                    // -z: lane tz - 1's previous value; lane 0 keeps the -z packet (DPP "old" operand;
-                    // zeros on a first z tile).  Lane 0 is active exactly when its packet is needed.
-                    vz = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp((int)(uint32_t)zq[r][0],
-                                                                               __builtin_bit_cast(int, prev[r]),
-                                                                               0x138, 0xf, 0xf, false));
-                    if constexpr (r > 0) vy = vnew[r - 1];   // the row above, same step (same x)
-                    else from_words(vin, a), vy = vin;
-                } else {
-                    vz = shr1(prev[r]);
-                    if constexpr (r > 0) {
-                        vy = vnew[r - 1];
-                    } else {
-                        if (w > 0) from_words(vin, a), vy = vin;
-                        else if (need_y) from_words(vin, c), vy = vin;
-                    }
-                    if (tz == 0 && need_z[r]) from_words(vin, zq[r]), vz = vin;
-                }
                 if constexpr (KIND == 0) {
-                    const uint32_t info = act[r] ? (uint32_t)wring[d][r] : 0u;
+                    const V vz = Group<V>::shr1(zp[r].get(j), prev[r]);
+                    const uint32_t info = (nq[d][r][e >> 1] >> (16 * (e & 1))) & 0xffffu;
                     double v = 0;
                     if (info & NB_FLUID) {
                         const double tau = 0.97, sigma = 0.25;
-                        const double upv[3] = {prev[r], vy, vz};
+                        const double upv[3] = {prev[r], above, vz};
                         double eneg = 0, eneg_tau = 0;
 #pragma unroll
                         for (int ax = 0; ax < 3; ax++) {
@@ -648,120 +591,146 @@ __device__ void compute_wave(const WaveArgs& A, WaveLds<KIND>& S, int J, int K, 
                             eneg += ap * ap;
                             eneg_tau += ap * (o1 + o2) * pj;
                         }
-                        const int cnt = (info >> NB_NONSOLID_SHIFT) & 7;
+                        const int cnt6 = (info >> NB_NONSOLID_SHIFT) & 7;
                         double diag = 0;
-                        for (int k = 0; k < cnt; k++) diag += scale;
-                        double e = diag - eneg - eneg_tau * tau;
-                        if (e < sigma * diag) e = diag < 1e-6 ? 1.0 : diag;
-                        v = 1.0 / sqrt(e);
+                        for (int k = 0; k < cnt6; k++) diag += scale;
+                        double ee = diag - eneg - eneg_tau * tau;
+                        if (ee < sigma * diag) ee = diag < 1e-6 ? 1.0 : diag;
+                        v = 1.0 / sqrt(ee);
                     }
-                    const bool fl = (info & NB_FLUID) != 0;
-                    const float p32 = (float)v;
-                    vnew[r] = v;
-                    // P64/P32 for WATER cells (both were cleared before the factor)
-                    bstore64(__builtin_bit_cast(uint64_t, v), rC, fl ? lo8[r] : kOob, oc);
-                    bstore32(__float_as_uint(p32), rD, fl ? lo4[r] : kOob, off4(oc));
+                    res[r][e] = (float)v;
+                    prev[r] = v;
                 } else {
-                    const float p = __uint_as_float(wring[d][r]);
-                    // stores of WATER cells only: storing every interior cell doubles the stores, and
-                    // the in-order memory counter then delays the prefetch waits (measured: slower)
-                    const bool fl = act[r] && wring[d][r] != 0u;
-                    // 0 + ms * prev in one rounding: fma(ms, prev, +0) equals the product, and +0 for -0
-                    float acc = __builtin_fmaf(ms, prev[r], 0.f);
-                    acc += ms * vy;
-                    acc += ms * vz;
+                    const float p = pq[d][r][e];
+                    // -z: the packet's value on lane 0 (+0 on the others), lane tz - 1's on the others (+0 on
+                    // lane 0): their sum is the one that counts
+                    const float vz = zp[r].get(j) + Group<V>::shr1(prev[r]);
+                    float acc = prev[r] + above;
+                    acc += vz;
                     float outv, v;
                     if (FWD) {
-                        outv = (iring[d][r] - acc) * p;
+                        outv = (iq[d][r][e] - acc) * p;
                         v = outv * p;
                     } else {
-                        outv = (iring[d][r] - acc * p) * p;
+                        outv = (iq[d][r][e] - acc * p) * p;
                         v = outv;
                     }
-                    vnew[r] = fl ? v : 0.f;
-                    bstore32(__float_as_uint(outv), rC, fl ? lo4[r] : kOob, off4(oc));
+                    res[r][e] = outv;
+                    prev[r] = __builtin_fmaf(ms, v, 0.f);
                 }
+                mine[r].set(j, prev[r]);
+                above = prev[r];
             });
-            // ---- publish: the last row for wave w+1 (the last wave's into the +y out-ring), lane 63 of
-            // every row into the +z out-ring (both sent by the sending waves), then read ahead,
-            // advance and prefetch step t + kPrefetch
+        });
+        // ---- publish first (the next wave waits for it) and ask for the next group's counters; store
+        // while they come; then the next group's slots, whose latency the prefetch covers
+        int next = g + 1;
+        asm volatile("" : "+s"(next));   // stays a scalar beside the lane branch below
 #pragma unroll
-            for (int k = 0; k < NP; k++) lput(my_blk + d * kSlotV + k * WF_TZ, pack(word(vnew[R - 1], k), (uint32_t)t));
-            // (the factor's FP64 values would make the sink writes of all lanes cost more LDS
-            // bandwidth than the lane mask costs instructions: it keeps the mask)
-            if (KIND != 0 || zl) {
-                uint64_t* zdst = zblk + (uint32_t)d * zo_stride;
-                if constexpr (KIND != 0 && R == 2) {
-                    // both rows in one 16-byte LDS write (the sending wave reads them word by word)
-                    u64x2 q;
-                    q.x = pack(word(vnew[0], 0), (uint32_t)t);
-                    q.y = pack(word(vnew[1], 0), (uint32_t)t);
-                    lput2(zdst, q);
-                } else {
-                    unroll<R>([&](auto rc) {
-                        constexpr int r = decltype(rc)::value;
-#pragma unroll
-                        for (int k = 0; k < NP; k++) lput(zdst + k * TY + r, pack(word(vnew[r], k), (uint32_t)t));
-                    });
-                }
-            }
-            rd_at(std::integral_constant<int, (d + 1) % kPrefetch>{}, t + 1);
-            // the packet reads of steps <= t have completed (their values were used above)
-            if (d == kPrefetch - 1 && tz == 0) lput32(&S.prog[w], t);
+        for (int c = 0; c < NP; c++) {
+            if constexpr (LAST)
+                __builtin_amdgcn_raw_buffer_store_b128(may_send<NP>(mine[R - 1].q[c]), ybuf,
+                                                       (uint32_t)(c * WF_TZ + tz) * 16u, (uint32_t)g * (WF_TZ * NP * 16),
+                                                       kDeviceScope);
+            else lput4(out_ring + d * kSlot + c * WF_TZ * 4, mine[R - 1].q[c]);
+        }
+        if (tz == WF_TZ - 1) {
             unroll<R>([&](auto rc) {
                 constexpr int r = decltype(rc)::value;
-                prev[r] = vnew[r];
-                fetch(d, r);
+#pragma unroll
+                for (int c = 0; c < NP; c++)
+                    lput4(zo + (r * kRingZ + d) * WF_G * NP + c * 4, mine[r].q[c]);
             });
-            advance(oc);
-            advance(op);
+            lput(in_below, next);   // also tells the sending wave that zo is there
+            lput(out_above, next + kRing);
+        }
+        const i32x4 cnt = lget4(my_cnt);
+        read_slots(std::integral_constant<int, d + 1>{});
+        unroll<R>([&](auto rc) {
+            constexpr int r = decltype(rc)::value;
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, res[r]), rC, lo[d][r], go[d], 0);
+            if constexpr (KIND == 0) {
+                // FP64: 32 bytes per column and group, beyond 32-bit offsets on the largest grids
+                if (lo[d][r] < kOob) {
+                    f64x2* p64 = reinterpret_cast<f64x2*>(reinterpret_cast<char*>(A.P64) + 2 * ((int64_t)go[d] + lo[d][r]));
+                    p64[0] = f64x2{mine[r].get(0), mine[r].get(1)};
+                    p64[1] = f64x2{mine[r].get(2), mine[r].get(3)};
+                }
+            }
         });
+        fetch(std::integral_constant<int, (d + kPrefetch) % kRing>{}, g + kPrefetch);
+        __builtin_amdgcn_sched_barrier(0);
+        wait_for(cnt, next, std::integral_constant<int, d + 1>{});
+    };
+    // whole blocks of kRing groups: the groups past the march have no cells (their waits are met at
+    // once, their packets fall outside ybuf), and without exits inside a block every prefetch slot has
+    // the same number of younger memory operations whenever it is waited for
+    for (int g0 = 0; g0 < T.m.ng; g0 += kRing) {
+        uint32_t* const zo = &S.zo[w * R][(g0 & (kRingZ - 1)) * WF_G * NP];
+        unroll<kRing>([&](auto dc) { group(dc, g0 + decltype(dc)::value, zo); });
     }
-    if (tz == 0) lput32(&S.prog[w], nsteps);
+    // nobody waits for this wave any more (the last group has waited for one more than there is)
+    if (tz == 0) {
+        lput(in_below, kAll);
+        lput(out_above, kAll);
+    }
 }
 
 template <int KIND>
 __global__ void __launch_bounds__(WF_THREADS) k_wave(WaveArgs A) {
     using KD = Kind<KIND>;
-    constexpr int NP = KD::NP, RINGP = KD::RINGP;
+    constexpr int NP = KD::NP;
     __shared__ WaveLds<KIND> S;
     const int tile = take_tile(A);
     if (tile < 0) return;
-    const int J = tile / A.TK, K = tile % A.TK;
+    Tile T;
+    T.J = __builtin_amdgcn_readfirstlane(tile / A.TK);
+    T.K = __builtin_amdgcn_readfirstlane(tile % A.TK);
     // A tile none of whose (y, z) columns holds WATER has nothing to compute
-    // (its cells' values are 0, and only WATER cells are stored): it leaves at
-    // once.  Its downstream tiles take its edge values as the zeros they are,
-    // exactly as on a first tile, instead of waiting for packets.
-    int mine = 0, upy = 0, upz = 0;
+    // (its cells' values are 0 from before the solve): it leaves at once.  Its
+    // downstream tiles take its edge values as the zeros they are, exactly as
+    // on a first tile, instead of waiting for packets, and its upstream tiles
+    // send it none.
+    int mine = 0, near[4] = {0, 0, 0, 0};
     for (int c = threadIdx.x; c < WF_TY * WF_TZ; c += WF_THREADS) {
         const int ty = c / WF_TZ, tz = c % WF_TZ;
-        mine |= col_water<KD::FWD>(A, J, K, ty, tz);
-        if (J > 0) upy |= col_water<KD::FWD>(A, J - 1, K, ty, tz);
-        if (K > 0) upz |= col_water<KD::FWD>(A, J, K - 1, ty, tz);
+        mine |= col_water<KD::FWD>(A, T.J, T.K, ty, tz);
+        if (T.J > 0) near[0] |= col_water<KD::FWD>(A, T.J - 1, T.K, ty, tz);
+        if (T.K > 0) near[1] |= col_water<KD::FWD>(A, T.J, T.K - 1, ty, tz);
+        if (T.J < A.TJ - 1) near[2] |= col_water<KD::FWD>(A, T.J + 1, T.K, ty, tz);
+        if (T.K < A.TK - 1) near[3] |= col_water<KD::FWD>(A, T.J, T.K + 1, ty, tz);
     }
     if (!__syncthreads_or(mine)) return;
-    const bool yup = __syncthreads_or(upy) != 0, zup = __syncthreads_or(upz) != 0;
-    for (int i = threadIdx.x; i < (WF_NW - 1) * kRingV * NP * WF_TZ; i += WF_THREADS) (&S.v[0][0][0][0])[i] = ~0ull;
-    // sweeps on a first y / z tile, or below / beside a tile without WATER, read their -y / -z
-    // values from a ring of zeros (never refilled)
-    const uint64_t yp_init = KIND != 0 && !yup ? 0ull : ~0ull, zp_init = KIND != 0 && !zup ? 0ull : ~0ull;
-    for (int i = threadIdx.x; i < RINGP * NP * WF_TZ; i += WF_THREADS) (&S.yp[0][0][0])[i] = yp_init;
-    for (int i = threadIdx.x; i < RINGP * NP * WF_TY; i += WF_THREADS) (&S.zp[0][0][0])[i] = zp_init;
-    for (int i = threadIdx.x; i < kRingO * NP * WF_TZ; i += WF_THREADS) (&S.yo[0][0][0])[i] = ~0ull;
-    for (int i = threadIdx.x; i < kRingO * NP * WF_TY; i += WF_THREADS) (&S.zo[0][0][0])[i] = ~0ull;
-    if (threadIdx.x < WF_NW) S.prog[threadIdx.x] = -1;
-    // steps below a sending wave's lag are never sent; without a downstream tile nothing is
-    if (threadIdx.x == 0) {
-        S.sprog[0] = J == A.TJ - 1 ? INT_MAX : WF_NW - 2;
-        S.sprog[1] = K == A.TK - 1 ? INT_MAX : WF_TZ - 2;
+    // readfirstlane: scalars for the compiler, as everything below depends on them uniformly
+    auto any = [](int v) { return __builtin_amdgcn_readfirstlane(__syncthreads_or(v)) != 0; };
+    T.yup = any(near[0]);
+    T.zup = any(near[1]);
+    T.ydn = any(near[2]);
+    T.zdn = any(near[3]);
+    const int xa = __builtin_amdgcn_readfirstlane(A.xrange[0]);
+    const int xb = __builtin_amdgcn_readfirstlane(A.xrange[1]);
+    T.m = march_of<KD::FWD>(A, T.K, xa, xb);
+    // without an upstream tile (or below / beside one without WATER) the -y / -z rings hold zeros
+    for (int i = threadIdx.x; i < kRing * NP * WF_TZ * 4; i += WF_THREADS) (&S.ring[0][0][0][0][0])[i] = 0;
+    for (int i = threadIdx.x; i < 2 * kRing * WF_TY * NP * 4; i += WF_THREADS) (&S.zi[0][0][0][0][0])[i] = 0;
+    if (threadIdx.x < WF_NW + 2) {
+        const int w = (int)threadIdx.x - 1;
+        Counters c;
+        c.in = w == 0 && !T.yup ? kAll : 0;
+        c.zin = T.zup ? 0 : kAll;
+        c.out = w == WF_NW - 1 ? kAll : kRing;   // the last row's packets have a row per group
+        // zo: leading groups that no packet needs are free at once
+        c.zout = kAll;
+        if (T.zdn) c.zout = kRingZ + max(0, z_shift<KD::FWD>(T.m, march_of<KD::FWD>(A, T.K + 1, xa, xb)) / WF_G);
+        S.cnt[threadIdx.x] = c;
     }
     __syncthreads();
     const int wave = threadIdx.x / 64;
-    if (wave < WF_NW) compute_wave<KIND>(A, S, J, K, yup, zup);
-    else if (wave == WF_NW) comm_wave<KIND, true>(A, S, J, K, yup, zup);
-    else if (wave == WF_NW + 1) comm_wave<KIND, false>(A, S, J, K, yup, zup);
-    else if (wave == WF_NW + 2) send_wave<KIND, true>(A, S, J, K);
-    else send_wave<KIND, false>(A, S, J, K);
+    if (wave < WF_NW - 1) compute_wave<KIND, false>(A, S, T);
+    else if (wave == WF_NW - 1) compute_wave<KIND, true>(A, S, T);
+    else if (wave == WF_NW) recv_wave<KIND, true>(A, S, T);
+    else if (wave == WF_NW + 1) recv_wave<KIND, false>(A, S, T);
+    else send_wave<KIND>(A, S, T);
 }
 
 int wave_launch(fsim_ctx* ctx, int kind, const float* in, float* out, double scale) {
@@ -774,7 +743,6 @@ int wave_launch(fsim_ctx* ctx, int kind, const float* in, float* out, double sca
     A.ticket = ctx->wave_ticket + kind;
     A.ticket_base = ctx->wave_ticket_base[kind];
     ctx->wave_ticket_base[kind] += ntiles;
-    A.epoch = ++ctx->wave_epoch;
     A.send_delay = ctx->wave_send_delay;
     if (kind == 0) hipLaunchKernelGGL(k_wave<0>, dim3(ntiles), dim3(WF_THREADS), 0, ctx->stream, A);
     else if (kind == 1) hipLaunchKernelGGL(k_wave<1>, dim3(ntiles), dim3(WF_THREADS), 0, ctx->stream, A);

@@ -324,9 +324,9 @@ typedef enum fsim_option {
      * give the same bits. */
     FSIM_OPT_P2G_KERNEL = 10,
     /* test option: the sending waves of the wavefront kernels pause about
-     * value x 3.4 us after each step they send (0 .. 64, default 0), so the
-     * compute waves run into the out-ring limit and wait for them.  The
-     * results are the same bits; only the time changes. */
+     * value x 3.4 us after each group of four steps they send (0 .. 64,
+     * default 0), so the compute waves run into the out-ring limit and wait
+     * for them.  The results are the same bits; only the time changes. */
     FSIM_OPT_WAVE_SEND_DELAY = 11
 } fsim_option;
 int fsim_set_option(fsim_ctx* ctx, int option, int value);

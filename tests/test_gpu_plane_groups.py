@@ -1,0 +1,101 @@
+"""The solver's storage of four interleaved planes, at the sizes where a column's planes wrap, end inside
+a group or share a tile edge: operators against one launch per plane and against plain numpy (-m gpu)."""
+import numpy as np
+import pytest
+
+from fluid_simulator_amd import capi, scenes
+
+pytestmark = pytest.mark.gpu
+DT = scenes.DT
+
+
+def _labels(shape, x0, x1, seed):
+    """WATER in the rows x0 .. x1 - 1 with holes and solid cells, inside SOLID walls (open top)."""
+    rng = np.random.default_rng(seed)
+    lab = np.full(shape, capi.AIR, np.uint8)
+    lab[x0:x1] = capi.WATER
+    lab[rng.random(shape) < 0.08] = capi.AIR
+    lab[rng.random(shape) < 0.04] = capi.SOLID
+    lab[0], lab[-1], lab[:, 0], lab[:, :, 0], lab[:, :, -1] = (capi.SOLID,) * 5
+    lab[:, -1] = np.where(lab[:, -1] == capi.WATER, capi.AIR, lab[:, -1])
+    return lab
+
+
+# nx: nxp = nx + 1 rounded up to 4 takes every remainder, below and above the 64-lane rotation; nz: one lane,
+# a full z-tile (66), one lane in the next (67), three tiles; ny: rows that leave a tile's last rows empty
+@pytest.mark.parametrize("shape,x0,x1", [((4, 4, 4), 1, 3), ((5, 9, 66), 1, 4), ((6, 8, 67), 2, 5), ((7, 13, 12), 1, 6),
+                                         ((63, 7, 66), 0, 63), ((64, 8, 131), 60, 63), ((65, 14, 67), 1, 2),
+                                         ((66, 20, 65), 5, 61)])
+def test_solver_operators_at_group_edges(gpu, shape, x0, x1):
+    print(f"case: plane groups {shape}, water in x {x0} .. {x1 - 1}", flush=True)
+    nx, ny, nz = shape
+    grid = capi.Grid(nx, ny, nz, 1.0 / 32, 0.25 / 32)
+    lab = _labels(shape, x0, x1, sum(shape))
+    water = lab == capi.WATER
+    rng = np.random.default_rng(1)
+    vec = np.where(water, rng.standard_normal(shape), 0.0).astype(np.float32).astype(np.float64)
+    got = {}
+    for mode in (1, 0):
+        sim = capi.Simulation(grid, scenes.params())
+        sim.set_option(capi.OPT_SWEEP_MODE, mode)
+        sim.set_grid(capi.FIELD_LABEL, lab.reshape(-1))
+        got[mode] = [sim.solver_apply(capi.OP_FACTOR_MIC0, DT), sim.solver_apply(capi.OP_APPLY_MIC0, DT, vec),
+                     sim.solver_apply(capi.OP_APPLY_A, DT, vec)]
+        sim.close()
+    for a, b in zip(got[0], got[1]):
+        assert np.array_equal(a, b)
+    assert np.count_nonzero(got[0][0]) == np.count_nonzero(water)
+    pad = np.pad(lab, 1, constant_values=capi.SOLID)
+    vpad = np.pad(vec, 1)
+    count, near, size = np.zeros(shape), np.zeros(shape), np.zeros(shape)
+    for a in range(3):
+        for s in (-1, 1):
+            at = tuple(slice(1 + (s if k == a else 0), shape[k] + 1 + (s if k == a else 0)) for k in range(3))
+            count += pad[at] != capi.SOLID
+            near += np.where(pad[at] == capi.WATER, vpad[at], 0.0)
+            size += np.where(pad[at] == capi.WATER, np.abs(vpad[at]), 0.0)
+    scale = DT / (1.0 * grid.cell_d ** 2)
+    want = np.where(water, scale * (count * vec - near), 0.0).reshape(-1)
+    # seven FP32 products (scale rounded as well) and six sums, each within half an ulp of the terms' total
+    bound = (9 * 2.0 ** -24 * scale * (count * np.abs(vec) + size)).reshape(-1)
+    assert np.all(np.abs(got[0][2] - want) <= np.where(water.reshape(-1), bound, 0.0))
+
+
+@pytest.mark.parametrize("shape", [(5, 6, 7), (30, 17, 66), (67, 9, 70)])
+def test_solve_fields_at_group_edges(gpu, shape):
+    """Right-hand side, pressure and projected faces come back in flat order: the divergence left on the faces is
+    the residual, and the right-hand side is the divergence before."""
+    print(f"case: pressure solve on {shape}", flush=True)
+    nx, ny, nz = shape
+    grid = capi.Grid(nx, ny, nz, 1.0 / 32, 0.25 / 32)
+    lab = _labels(shape, 1, max(3, nx - 2), sum(shape))
+    water = lab == capi.WATER
+    rng = np.random.default_rng(2)
+    faces = [rng.standard_normal(shape).astype(np.float32) for _ in range(3)]
+    sim = capi.Simulation(grid, scenes.params(tol=1e-9))
+    sim.set_grid(capi.FIELD_LABEL, lab.reshape(-1))
+    for f, v in zip((capi.FIELD_U2, capi.FIELD_V2, capi.FIELD_W2), faces):
+        sim.set_grid(f, v.reshape(-1))
+
+    def rhs(f):
+        d = np.zeros(shape)
+        for a in range(3):
+            v = f[a].astype(np.float64)
+            d += v - np.roll(v, 1, axis=a)
+        return np.where(water, -d / grid.cell_d, 0.0)
+
+    b = rhs(faces)
+    sim.run_stage(capi.STAGE_SOLVE, DT)
+    st = sim.stats()
+    got_b = sim.get_grid(capi.FIELD_RHS).reshape(shape)
+    # b is rounded to FP32 once
+    assert np.all(np.abs(got_b - b) <= 2.0 ** -24 * np.abs(b) + 1e-30)
+    p = sim.get_grid(capi.FIELD_PRESSURE).reshape(shape)
+    assert not p[~water].any() and np.isfinite(p).all()
+    assert st.num_fluid_cells == np.count_nonzero(water) and st.residual_rel_l2 <= 1e-9 and not st.solve_nan
+    after = [sim.get_grid(f).reshape(shape) for f in (capi.FIELD_U2, capi.FIELD_V2, capi.FIELD_W2)]
+    sim.close()
+    # the faces are rounded to FP32 (at most twice, from either side): 12 half ulps of the largest face a cell
+    largest = max(np.abs(v).max() for v in after + faces)
+    left = rhs(after)
+    assert np.abs(left).max() <= 12 * 2.0 ** -24 * largest / grid.cell_d + 1e-9 * np.linalg.norm(b)
