@@ -101,9 +101,9 @@ __device__ inline double get_dev(const double* p) {
                                                         __HIP_MEMORY_SCOPE_AGENT));
 }
 
-template <int AUX>
+template <int AUX, int NT = kBlock>
 __device__ void block_finish(double sum, double aux, const Reduce& R) {
-    __shared__ double lds_s[kBlock], lds_m[kBlock];
+    __shared__ double lds_s[NT], lds_m[NT];
     __shared__ int last;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     sum = wave_sum(sum);
@@ -117,7 +117,7 @@ __device__ void block_finish(double sum, double aux, const Reduce& R) {
     const unsigned nparts = gridDim.x;
     if (threadIdx.x == 0) {
         double s = 0, m = 0;
-        for (int w = 0; w < kBlock / 64; w++) {
+        for (int w = 0; w < NT / 64; w++) {
             s += lds_s[w];
             m = AUX == AUX_SUM ? m + lds_m[w] : fmax(m, lds_m[w]);
         }
@@ -128,12 +128,12 @@ __device__ void block_finish(double sum, double aux, const Reduce& R) {
     }
     __syncthreads();
     if (!last) return;
-    // all loads first (at most kMaxParts / kBlock per thread), then the sums in order
-    constexpr int kPer = kMaxParts / kBlock;
+    // all loads first (at most kMaxParts / NT per thread), then the sums in order
+    constexpr int kPer = kMaxParts / NT;
     double vs[kPer], vm[kPer];
 #pragma unroll
     for (int k = 0; k < kPer; k++) {
-        const unsigned i = threadIdx.x + k * kBlock;
+        const unsigned i = threadIdx.x + k * NT;
         vs[k] = i < nparts ? get_dev(&R.partials[i]) : 0.0;
         vm[k] = AUX != AUX_NONE && i < nparts ? get_dev(&R.partials[nparts + i]) : 0.0;
     }
@@ -146,7 +146,7 @@ __device__ void block_finish(double sum, double aux, const Reduce& R) {
     lds_s[threadIdx.x] = s;
     lds_m[threadIdx.x] = m;
     __syncthreads();
-    for (int off = kBlock / 2; off > 0; off >>= 1) {
+    for (int off = NT / 2; off > 0; off >>= 1) {
         if ((int)threadIdx.x < off) {
             lds_s[threadIdx.x] += lds_s[threadIdx.x + off];
             lds_m[threadIdx.x] = AUX == AUX_SUM ? lds_m[threadIdx.x] + lds_m[threadIdx.x + off]
@@ -510,16 +510,19 @@ __global__ void __launch_bounds__(kBlock) k_spmv(SolveArgs S, const uint16_t* __
 // (grid stride) and issues all their loads before using any, so several
 // memory round trips are in flight.
 constexpr int kUnits = 4;
-// 1024 measured fastest at 256^3 (the dot: 38 us per launch with 2048 blocks, 29 us with 1024;
-// 512 is slower again)
+// Large blocks: every block takes a ticket from one counter at its end, and
+// the tickets are handed out one after the other.  256 blocks of 1024 threads
+// against 1024 of 256: dot 21 us (27) at 256^3 and 9.7 (13.7) at 128^3, r
+// update beside the x update 52 (53) and 13.6 (16.5); 128 and 512 blocks are
+// slower at 256^3 (24.5 / 20.9 and 65 / 58).
+constexpr int kStream = 1024;   // threads per block
 #ifndef FSIM_STREAM_BLOCKS
-#define FSIM_STREAM_BLOCKS 1024
+#define FSIM_STREAM_BLOCKS 256
 #endif
-static_assert(FSIM_STREAM_BLOCKS % 8 == 0 && FSIM_STREAM_BLOCKS <= (int)kMaxParts, "stream grid within the reduction");
-// blocks of the flagged-chunk kernels (at most kMaxParts, a multiple of 8)
+static_assert(FSIM_STREAM_BLOCKS <= (int)kMaxParts, "stream grid within the reduction");
 static unsigned stream_blocks(int64_t n) {
-    const unsigned need = (unsigned)((n / kChunk + kUnits * 4 - 1) / (kUnits * 4));
-    return std::max(8u, std::min<unsigned>((need + 7) / 8 * 8, FSIM_STREAM_BLOCKS));
+    const unsigned need = (unsigned)((n / kChunk + kUnits * (kStream / 64) - 1) / (kUnits * (kStream / 64)));
+    return std::max(1u, std::min<unsigned>(need, FSIM_STREAM_BLOCKS));
 }
 
 template <int NV, class Load, class Use>
@@ -554,7 +557,7 @@ __device__ inline void for_flagged_chunks(int64_t n, const uint32_t* __restrict_
 }
 
 // r -= alpha q, with ||r||^2 and max|r|
-__global__ void __launch_bounds__(kBlock) k_update_r(int64_t n, const uint32_t* __restrict__ flags,
+__global__ void __launch_bounds__(kStream) k_update_r(int64_t n, const uint32_t* __restrict__ flags,
                                                      const float* __restrict__ q, float* __restrict__ r, Reduce red) {
     double ss = 0.0, mx = 0.0;
     const float malpha = (float)(-red.sc->alpha);
@@ -576,11 +579,11 @@ __global__ void __launch_bounds__(kBlock) k_update_r(int64_t n, const uint32_t* 
             cell(v[0].w, v[1].w);
             *reinterpret_cast<float4*>(r + i) = v[1];
         });
-    block_finish<AUX_MAX>(ss, mx, red);
+    block_finish<AUX_MAX, kStream>(ss, mx, red);
 }
 
 // a . b (FP64 products of the FP32 values)
-__global__ void __launch_bounds__(kBlock) k_dot(int64_t n, const uint32_t* __restrict__ flags,
+__global__ void __launch_bounds__(kStream) k_dot(int64_t n, const uint32_t* __restrict__ flags,
                                                 const float* __restrict__ a, const float* __restrict__ b, Reduce red) {
     double d = 0.0;
     for_flagged_chunks<2>(
@@ -595,7 +598,7 @@ __global__ void __launch_bounds__(kBlock) k_dot(int64_t n, const uint32_t* __res
             d += (double)v[0].z * (double)v[1].z;
             d += (double)v[0].w * (double)v[1].w;
         });
-    block_finish<AUX_NONE>(d, 0.0, red);
+    block_finish<AUX_NONE, kStream>(d, 0.0, red);
 }
 
 // x += alpha s (FP64) for WATER cells, of the last direction step (STEPS 1) or
@@ -864,7 +867,7 @@ static int true_residual(fsim_ctx* ctx, const SolveArgs& S, bool replace) {
 static int dot_with(fsim_ctx* ctx, const float* a, const float* b, int op) {
     FSIM_PROF(ctx, KID_DOT);
     const int64_t n = ctx->g.ncr;
-    hipLaunchKernelGGL(k_dot, dim3(stream_blocks(n)), dim3(kBlock), 0, ctx->stream, n, ctx->chunk_flags, a, b,
+    hipLaunchKernelGGL(k_dot, dim3(stream_blocks(n)), dim3(kStream), 0, ctx->stream, n, ctx->chunk_flags, a, b,
                        reduce_to(ctx, op));
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;
@@ -996,7 +999,7 @@ static int pcg_run(fsim_ctx* ctx, const SolveArgs& S, double bnorm, bool flexibl
         }
         {
             FSIM_PROF(ctx, KID_UPDATE);
-            hipLaunchKernelGGL(k_update_r, dim3(stream_blocks(n)), dim3(kBlock), 0, ctx->stream, n, ctx->chunk_flags, ctx->q,
+            hipLaunchKernelGGL(k_update_r, dim3(stream_blocks(n)), dim3(kStream), 0, ctx->stream, n, ctx->chunk_flags, ctx->q,
                                ctx->r, reduce_to_host(ctx, FIN_RES));
         }
         FSIM_HIP(ctx, hipGetLastError());
