@@ -23,7 +23,7 @@
 #include <cstring>
 #include <type_traits>
 
-#include "fsim_internal.hpp"
+#include "fsim_march.hpp"
 
 namespace fsim {
 
@@ -437,68 +437,57 @@ constexpr int SPMV_PLAIN = 0, SPMV_COPY = 1, SPMV_XPAY = 2;
 // no block reads a value another block has already replaced.  A lane owns the
 // four cells of one column of a plane group and stores them whole, zero off
 // WATER (q and s are zeroed before a solve, so the columns without WATER that
-// it leaves out hold zeros as well).  Per 64 x 4 cells it issues 10 16-byte and 8
-// 4-byte vector loads where one cell per lane took 56 4-byte ones; 75 us at
-// 256^3 (80 us before), bound by memory.
-static_assert(kBlock == 64 * kRowWaves, "a wave per row of an item");
+// it leaves out hold zeros as well).  Bound by memory: at 256^3 65 us against
+// 53 that its 18 bytes per cell take at the rate of a large copy; 74 where
+// every lane gathered its neighbours (10 loads of 16 bytes and 8 of 4 per
+// lane, of which 6 and 0 are left), 17 against 31 at 128^3.
 template <int MODE>
-__global__ void __launch_bounds__(kBlock) k_spmv(SolveArgs S, const uint16_t* __restrict__ nbinfo,
-                                                 const float* __restrict__ z, const float* __restrict__ s,
-                                                 float* __restrict__ s_new, float* __restrict__ q, Reduce red) {
+__global__ void __launch_bounds__(64 * kMarchWaves) k_spmv(SolveArgs S, March m, const uint16_t* __restrict__ nbinfo,
+                                                           const float* __restrict__ z, const float* __restrict__ s,
+                                                           float* __restrict__ s_new, float* __restrict__ q, Reduce red) {
     double d = 0.0;
     const float ms = -S.scale_f;
     const float beta = MODE == SPMV_XPAY ? (float)red.sc->beta : 0.f;
-    auto dir = [&](int64_t j) {
-        if constexpr (MODE == SPMV_PLAIN) return s[j];
-        else if constexpr (MODE == SPMV_COPY) return z[j];
-        else return s[j] * beta + z[j];
+    struct Raw {
+        f32x4 s, z;
     };
-    auto dir4 = [&](int64_t j) {
-        if constexpr (MODE == SPMV_PLAIN) return *reinterpret_cast<const f32x4*>(s + j);
-        else if constexpr (MODE == SPMV_COPY) return *reinterpret_cast<const f32x4*>(z + j);
-        else return *reinterpret_cast<const f32x4*>(s + j) * beta + *reinterpret_cast<const f32x4*>(z + j);
-    };
-    const RowItems it = row_items(S.ny, S.nz, S.nxp);
-    const int ng = S.nxp / WF_G;
-    // the nbinfo words of the next item are loaded while this item's gathers are in flight
-    auto load_info = [&](int k) {
-        int g, y, z;
-        if (k >= it.end || !item_column(it, k, S.ny, S.nz, g, y, z)) return u16x4{0, 0, 0, 0};
-        return *reinterpret_cast<const u16x4*>(nbinfo + pidx(g * WF_G, y, z, S.ny, S.nz));
-    };
-    u16x4 info_next = load_info(it.first);
-    for (int k = it.first; k < it.end; k += it.step) {
-        const u16x4 info = info_next;
-        info_next = load_info(k + it.step);
-        if (((info[0] | info[1] | info[2] | info[3]) & NB_FLUID) == 0) continue;   // no WATER in the lane's cells
-        int g, y, zc;
-        item_column(it, k, S.ny, S.nz, g, y, zc);
-        // all gathers first, then the sums with the reference's term order, by mask
-        const ColumnNeighbours n = column_neighbours(S.ny, S.nz, ng, g, y, zc);
-        const f32x4 own = dir4(n.own), yp = dir4(n.yp), ym = dir4(n.ym), zp = dir4(n.zp), zm = dir4(n.zm);
-        const float xp3 = dir(n.xp3), xm0 = dir(n.xm0), zp3 = dir(n.zp3), zm0 = dir(n.zm0);
-        f32x4 out, snew;
+    march(
+        m, S.ny, S.nz, S.nxp, nbinfo,
+        [&](int64_t j) {
+            Raw v;
+            if constexpr (MODE != SPMV_COPY) v.s = *reinterpret_cast<const f32x4*>(s + j);
+            if constexpr (MODE != SPMV_PLAIN) v.z = *reinterpret_cast<const f32x4*>(z + j);
+            return v;
+        },
+        [&](const Raw& v) {
+            if constexpr (MODE == SPMV_PLAIN) return v.s;
+            else if constexpr (MODE == SPMV_COPY) return v.z;
+            else return v.s * beta + v.z;
+        },
+        [&](int64_t j, const MarchCells& n) {
+            f32x4 out, snew;
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-            const uint32_t f = info[c];
-            const int cnt = (f >> NB_NONSOLID_SHIFT) & 7;
-            const float si = own[c];
-            float val = (S.scale_f * (float)cnt) * si;
-            val = (f & NB_PX) ? val + ms * (c < 3 ? own[(c + 1) & 3] : xp3) : val;
-            val = (f & NB_PY) ? val + ms * yp[c] : val;
-            val = (f & NB_PZ) ? val + ms * (c < 3 ? zp[(c + 1) & 3] : zp3) : val;
-            val = (f & NB_MX) ? val + ms * (c > 0 ? own[(c + 3) & 3] : xm0) : val;
-            val = (f & NB_MY) ? val + ms * ym[c] : val;
-            val = (f & NB_MZ) ? val + ms * (c > 0 ? zm[(c + 3) & 3] : zm0) : val;
-            const bool fl = (f & NB_FLUID) != 0;
-            out[c] = fl ? val : 0.f;
-            snew[c] = fl ? si : 0.f;
-            d += (double)snew[c] * (double)out[c];
-        }
-        *reinterpret_cast<f32x4*>(q + n.own) = out;
-        if (MODE != SPMV_PLAIN) *reinterpret_cast<f32x4*>(s_new + n.own) = snew;
-    }
-    block_finish<AUX_NONE>(d, 0.0, red);
+            for (int c = 0; c < 4; c++) {
+                // the sums with the reference's term order, by mask
+                const uint32_t f = n.info[c];
+                const int cnt = (f >> NB_NONSOLID_SHIFT) & 7;
+                const float si = n.own[c];
+                float val = (S.scale_f * (float)cnt) * si;
+                val = (f & NB_PX) ? val + ms * n.xp[c] : val;
+                val = (f & NB_PY) ? val + ms * n.yp[c] : val;
+                val = (f & NB_PZ) ? val + ms * n.zp[c] : val;
+                val = (f & NB_MX) ? val + ms * n.xm[c] : val;
+                val = (f & NB_MY) ? val + ms * n.ym[c] : val;
+                val = (f & NB_MZ) ? val + ms * n.zm[c] : val;
+                const bool fl = (f & NB_FLUID) != 0;
+                out[c] = fl ? val : 0.f;
+                snew[c] = fl ? si : 0.f;
+                d += (double)snew[c] * (double)out[c];
+            }
+            *reinterpret_cast<f32x4*>(q + j) = out;
+            if (MODE != SPMV_PLAIN) *reinterpret_cast<f32x4*>(s_new + j) = snew;
+        });
+    block_finish<AUX_NONE, 64 * kMarchWaves>(d, 0.0, red);
 }
 
 // Streaming kernels without per-cell masks: the solver vectors r, q and z
@@ -745,15 +734,10 @@ static int check_wave_err(fsim_ctx* ctx) {
 // per CU keep HBM busy), a multiple of 8 for the XCD-aware row split, and
 // the last block sums the partials in one pass.
 static unsigned red_blocks(int64_t n) { return std::min<unsigned>((nblocks(n) + 7) / 8 * 8, kMaxParts); }
-// 2048 and 1024 measure alike at 256^3, 512 is slower
-#ifndef FSIM_SPMV_BLOCKS
-#define FSIM_SPMV_BLOCKS 2048
-#endif
-static_assert(FSIM_SPMV_BLOCKS % 8 == 0 && FSIM_SPMV_BLOCKS <= (int)kMaxParts, "SpMV grid within the reduction");
-// blocks of the column kernels: one per item, up to FSIM_SPMV_BLOCKS
-static unsigned spmv_blocks(const SolveArgs& S) {
+// blocks of the column kernels: one per item
+static unsigned column_blocks(const SolveArgs& S) {
     const unsigned items = (unsigned)row_item_count(S.ny, S.nz, S.nxp);
-    return std::max(8u, std::min<unsigned>((items + 7) / 8 * 8, FSIM_SPMV_BLOCKS));
+    return std::max(8u, std::min<unsigned>((items + 7) / 8 * 8, kMaxParts));
 }
 
 static Reduce reduce_to(fsim_ctx* ctx, int op) { return Reduce{ctx->partials, ctx->red_count, ctx->scal, op}; }
@@ -858,7 +842,7 @@ static int mic_apply(fsim_ctx* ctx, const SolveArgs& S, const float* r, float* q
 
 static int true_residual(fsim_ctx* ctx, const SolveArgs& S, bool replace) {
     FSIM_PROF(ctx, KID_TRUE_RES);
-    hipLaunchKernelGGL(k_true_residual, dim3(spmv_blocks(S)), dim3(kBlock), 0, ctx->stream, S, ctx->nbinfo, ctx->b, ctx->x,
+    hipLaunchKernelGGL(k_true_residual, dim3(column_blocks(S)), dim3(kBlock), 0, ctx->stream, S, ctx->nbinfo, ctx->b, ctx->x,
                        ctx->r, replace ? 1 : 0, reduce_to(ctx, FIN_TRUE));
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;
@@ -879,13 +863,14 @@ static int dot_zr(fsim_ctx* ctx, int op) { return dot_with(ctx, ctx->z, ctx->r, 
 static int direction_step(fsim_ctx* ctx, const SolveArgs& S, bool copy) {
     {
         FSIM_PROF(ctx, KID_SPMV);
-        const dim3 grid(spmv_blocks(S)), block(kBlock);
+        const March m = march_of(S.ny, S.nz, S.nxp);
+        const dim3 grid(march_blocks(m)), block(64 * kMarchWaves);
         const Reduce red = reduce_to(ctx, FIN_ALPHA);
         if (copy)
-            hipLaunchKernelGGL(k_spmv<SPMV_COPY>, grid, block, 0, ctx->stream, S, ctx->nbinfo, ctx->z, ctx->s, ctx->s2,
+            hipLaunchKernelGGL(k_spmv<SPMV_COPY>, grid, block, 0, ctx->stream, S, m, ctx->nbinfo, ctx->z, ctx->s, ctx->s2,
                                ctx->q, red);
         else
-            hipLaunchKernelGGL(k_spmv<SPMV_XPAY>, grid, block, 0, ctx->stream, S, ctx->nbinfo, ctx->z, ctx->s, ctx->s2,
+            hipLaunchKernelGGL(k_spmv<SPMV_XPAY>, grid, block, 0, ctx->stream, S, m, ctx->nbinfo, ctx->z, ctx->s, ctx->s2,
                                ctx->q, red);
     }
     FSIM_HIP(ctx, hipGetLastError());
@@ -1311,8 +1296,9 @@ int solver_apply(fsim_ctx* ctx, int op, double dt, const double* in, double* out
     FSIM_HIP(ctx, hipMemcpyAsync(ctx->r, hin.data(), sizeof(float) * n, hipMemcpyHostToDevice, ctx->stream));
     if (op == FSIM_OP_APPLY_A) {
         FSIM_TRY(fill_f32(ctx, ctx->q, 0.0f, n));   // the SpMV skips columns without WATER
-        hipLaunchKernelGGL(k_spmv<SPMV_PLAIN>, dim3(spmv_blocks(S)), dim3(kBlock), 0, ctx->stream, S, ctx->nbinfo, nullptr,
-                           ctx->r, nullptr, ctx->q, reduce_to(ctx, FIN_NONE));
+        const March m = march_of(S.ny, S.nz, S.nxp);
+        hipLaunchKernelGGL(k_spmv<SPMV_PLAIN>, dim3(march_blocks(m)), dim3(64 * kMarchWaves), 0, ctx->stream, S, m,
+                           ctx->nbinfo, nullptr, ctx->r, nullptr, ctx->q, reduce_to(ctx, FIN_NONE));
         FSIM_HIP(ctx, hipGetLastError());
         FSIM_HIP(ctx, hipMemcpyAsync(hout.data(), ctx->q, sizeof(float) * n, hipMemcpyDeviceToHost, ctx->stream));
     } else if (op == FSIM_OP_APPLY_MIC0) {

@@ -21,6 +21,25 @@ def _labels(shape, x0, x1, seed):
     return lab
 
 
+def _a_times(grid, lab, vec):
+    """A vec in FP64 and the error bound of the FP32 product, zero off WATER, flat."""
+    shape = lab.shape
+    pad = np.pad(lab, 1, constant_values=capi.SOLID)
+    vpad = np.pad(vec, 1)
+    count, near, size = np.zeros(shape), np.zeros(shape), np.zeros(shape)
+    for a in range(3):
+        for s in (-1, 1):
+            at = tuple(slice(1 + (s if k == a else 0), shape[k] + 1 + (s if k == a else 0)) for k in range(3))
+            count += pad[at] != capi.SOLID
+            near += np.where(pad[at] == capi.WATER, vpad[at], 0.0)
+            size += np.where(pad[at] == capi.WATER, np.abs(vpad[at]), 0.0)
+    scale = DT / (1.0 * grid.cell_d ** 2)
+    # seven FP32 products (scale rounded as well) and six sums, each within half an ulp of the terms' total
+    bound = 9 * 2.0 ** -24 * scale * (count * np.abs(vec) + size)
+    water = lab == capi.WATER
+    return np.where(water, scale * (count * vec - near), 0.0).reshape(-1), np.where(water, bound, 0.0).reshape(-1)
+
+
 # nx: nxp = nx + 1 rounded up to 4 takes every remainder, below and above the 64-lane rotation; nz: one lane,
 # a full z-tile (66), one lane in the next (67), three tiles; ny: rows that leave a tile's last rows empty
 @pytest.mark.parametrize("shape,x0,x1", [((4, 4, 4), 1, 3), ((5, 9, 66), 1, 4), ((6, 8, 67), 2, 5), ((7, 13, 12), 1, 6),
@@ -45,20 +64,23 @@ def test_solver_operators_at_group_edges(gpu, shape, x0, x1):
     for a, b in zip(got[0], got[1]):
         assert np.array_equal(a, b)
     assert np.count_nonzero(got[0][0]) == np.count_nonzero(water)
-    pad = np.pad(lab, 1, constant_values=capi.SOLID)
-    vpad = np.pad(vec, 1)
-    count, near, size = np.zeros(shape), np.zeros(shape), np.zeros(shape)
-    for a in range(3):
-        for s in (-1, 1):
-            at = tuple(slice(1 + (s if k == a else 0), shape[k] + 1 + (s if k == a else 0)) for k in range(3))
-            count += pad[at] != capi.SOLID
-            near += np.where(pad[at] == capi.WATER, vpad[at], 0.0)
-            size += np.where(pad[at] == capi.WATER, np.abs(vpad[at]), 0.0)
-    scale = DT / (1.0 * grid.cell_d ** 2)
-    want = np.where(water, scale * (count * vec - near), 0.0).reshape(-1)
-    # seven FP32 products (scale rounded as well) and six sums, each within half an ulp of the terms' total
-    bound = (9 * 2.0 ** -24 * scale * (count * np.abs(vec) + size)).reshape(-1)
-    assert np.all(np.abs(got[0][2] - want) <= np.where(water.reshape(-1), bound, 0.0))
+    want, bound = _a_times(grid, lab, vec)
+    assert np.all(np.abs(got[0][2] - want) <= bound)
+
+
+# runs of more than one plane group (3 of 36, the last one short), and more items than blocks
+@pytest.mark.parametrize("shape", [(140, 66, 200), (4, 2000, 560)])
+def test_matrix_product_in_runs(gpu, shape):
+    print(f"case: A v on {shape}", flush=True)
+    grid = capi.Grid(*shape, 1.0 / 32, 0.25 / 32)
+    lab = _labels(shape, 1, shape[0] - 1, sum(shape))
+    vec = np.where(lab == capi.WATER, np.random.default_rng(3).standard_normal(shape, np.float32), 0.0)
+    sim = capi.Simulation(grid, scenes.params())
+    sim.set_grid(capi.FIELD_LABEL, lab.reshape(-1))
+    got = sim.solver_apply(capi.OP_APPLY_A, DT, vec)
+    sim.close()
+    want, bound = _a_times(grid, lab, vec)
+    assert np.all(np.abs(got - want) <= bound)
 
 
 @pytest.mark.parametrize("shape", [(5, 6, 7), (30, 17, 66), (67, 9, 70)])
