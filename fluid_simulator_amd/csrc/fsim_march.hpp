@@ -30,11 +30,11 @@ static_assert(kMarchBlocks <= (int)kMaxParts, "march grid within the reduction")
 // Workgroups are dispatched round-robin over the 8 XCDs (blockIdx mod 8): each
 // XCD takes kMarchRun consecutive items (rows next to each other share its L2)
 // in turn, so that a fluid that fills one side of the grid loads them alike.
-struct March {
+struct MarchPlan {
     int ntile, nrow, len, items;
 };
-static inline March march_of(int ny, int nz, int nxp) {
-    March m;
+static inline MarchPlan march_of(int ny, int nz, int nxp) {
+    MarchPlan m;
     m.ntile = (nz - 2 + WF_TZ - 1) / WF_TZ;
     m.nrow = (ny - 2 + kMarchRows * kMarchWaves - 1) / (kMarchRows * kMarchWaves);
     const int ng = nxp / WF_G;
@@ -43,7 +43,7 @@ static inline March march_of(int ny, int nz, int nxp) {
     m.items = m.ntile * m.nrow * ((ng + m.len - 1) / m.len);
     return m;
 }
-static inline unsigned march_blocks(const March& m) {
+static inline unsigned march_blocks(const MarchPlan& m) {
     const int unit = 8 * kMarchRun;
     return (unsigned)std::min<int64_t>((m.items + unit - 1) / unit * unit, kMaxParts);
 }
@@ -71,7 +71,7 @@ struct MarchCells {
 // WATER; body(int64_t j, const MarchCells&): called for the lanes with WATER.
 // Columns without WATER read index 0, a border cell, whose values are zero.
 template <class Load, class Value, class Body>
-__device__ inline void march(const March& m, int ny, int nz, int nxp, const uint16_t* __restrict__ nbinfo, Load&& load,
+__device__ inline void march(const MarchPlan& m, int ny, int nz, int nxp, const uint16_t* __restrict__ nbinfo, Load&& load,
                              Value&& value, Body&& body) {
     constexpr int R = kMarchRows;
     using Raw = decltype(load((int64_t)0));

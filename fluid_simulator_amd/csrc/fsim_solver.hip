@@ -442,7 +442,7 @@ constexpr int SPMV_PLAIN = 0, SPMV_COPY = 1, SPMV_XPAY = 2;
 // every lane gathered its neighbours (10 loads of 16 bytes and 8 of 4 per
 // lane, of which 6 and 0 are left), 17 against 31 at 128^3.
 template <int MODE>
-__global__ void __launch_bounds__(64 * kMarchWaves) k_spmv(SolveArgs S, March m, const uint16_t* __restrict__ nbinfo,
+__global__ void __launch_bounds__(64 * kMarchWaves) k_spmv(SolveArgs S, MarchPlan m, const uint16_t* __restrict__ nbinfo,
                                                            const float* __restrict__ z, const float* __restrict__ s,
                                                            float* __restrict__ s_new, float* __restrict__ q, Reduce red) {
     double d = 0.0;
@@ -863,7 +863,7 @@ static int dot_zr(fsim_ctx* ctx, int op) { return dot_with(ctx, ctx->z, ctx->r, 
 static int direction_step(fsim_ctx* ctx, const SolveArgs& S, bool copy) {
     {
         FSIM_PROF(ctx, KID_SPMV);
-        const March m = march_of(S.ny, S.nz, S.nxp);
+        const MarchPlan m = march_of(S.ny, S.nz, S.nxp);
         const dim3 grid(march_blocks(m)), block(64 * kMarchWaves);
         const Reduce red = reduce_to(ctx, FIN_ALPHA);
         if (copy)
@@ -1296,7 +1296,7 @@ int solver_apply(fsim_ctx* ctx, int op, double dt, const double* in, double* out
     FSIM_HIP(ctx, hipMemcpyAsync(ctx->r, hin.data(), sizeof(float) * n, hipMemcpyHostToDevice, ctx->stream));
     if (op == FSIM_OP_APPLY_A) {
         FSIM_TRY(fill_f32(ctx, ctx->q, 0.0f, n));   // the SpMV skips columns without WATER
-        const March m = march_of(S.ny, S.nz, S.nxp);
+        const MarchPlan m = march_of(S.ny, S.nz, S.nxp);
         hipLaunchKernelGGL(k_spmv<SPMV_PLAIN>, dim3(march_blocks(m)), dim3(64 * kMarchWaves), 0, ctx->stream, S, m,
                            ctx->nbinfo, nullptr, ctx->r, nullptr, ctx->q, reduce_to(ctx, FIN_NONE));
         FSIM_HIP(ctx, hipGetLastError());

@@ -238,9 +238,16 @@ __device__ inline int z_groups(const March& me) {
 struct Counters {
     int in, zin, out, zout;
 };
+// Factor: the terms that depend on a cell's info word alone, so that a step has no loop or branch
+struct FactorTable {
+    f64x2 diag[8];   // by the number of non-SOLID neighbours: their sum of scales, and what replaces a small e
+    double up[4];    // by the two NB_UP bits of an axis: the sum of the -neighbour's other two A entries
+};
+struct NoTable {};
 template <int KIND>
 struct WaveLds {
     static constexpr int NP = Kind<KIND>::NP;
+    std::conditional_t<KIND == 0, FactorTable, NoTable> tab;
     // ring 0: the -y edge; ring w + 1: the last row of compute wave w
     alignas(16) uint32_t ring[WF_NW][kRing][NP][WF_TZ][4];
     // -z edge: lane 0's upstream value of every row; the other lanes read zeros from beside it
@@ -412,6 +419,10 @@ __device__ void send_wave(const WaveArgs& A, WaveLds<KIND>& S, const Tile& T) {
 // ---- compute waves -------------------------------------------------------------
 // Factor (KIND 0, FP64):   e = diag - sum_a (A_a p_a)^2 - tau sum_a A_a (o1 + o2) p_a^2,
 //                          guarded by sigma, p = 1/sqrt(e)  (calculatePreconditioner); passes p on
+//                          No branch or loop in a step: diag and o1 + o2 come from a table by the info
+//                          word, a neighbour that is not WATER carries 0.  450 us at 256^3 and 188 at
+//                          128^3 (1055 and 420 with a loop over the neighbours per cell), of which the
+//                          square root and the division are the larger part
 // forward sweep (KIND 1):  q = (r - sum_{-a fluid} A_a q_a p_a) * p; passes m = A_a q p on
 // backward sweep (KIND 2): z = (q - p * sum_{+a fluid} A_a z_a) * p; passes m = A_a z on
 // with A_a = -scale, products and sums in the reference's order (x, y, z).
@@ -576,28 +587,19 @@ __device__ __forceinline__ void compute_wave(const WaveArgs& A, WaveLds<KIND>& S
                 if constexpr (KIND == 0) {
                     const V vz = Group<V>::shr1(zp[r].get(j), prev[r]);
                     const uint32_t info = (nq[d][r][e >> 1] >> (16 * (e & 1))) & 0xffffu;
-                    double v = 0;
-                    if (info & NB_FLUID) {
-                        const double tau = 0.97, sigma = 0.25;
-                        const double upv[3] = {prev[r], above, vz};
-                        double eneg = 0, eneg_tau = 0;
+                    const double upv[3] = {prev[r], above, vz};
+                    double eneg = 0, eneg_tau = 0;
 #pragma unroll
-                        for (int ax = 0; ax < 3; ax++) {
-                            if (!(info & (NB_MX << ax))) continue;
-                            const double pj = upv[ax];
-                            const double ap = -scale * pj;
-                            const double o1 = (info & (1u << (NB_UP_SHIFT + 2 * ax))) ? -scale : 0.0;
-                            const double o2 = (info & (1u << (NB_UP_SHIFT + 2 * ax + 1))) ? -scale : 0.0;
-                            eneg += ap * ap;
-                            eneg_tau += ap * (o1 + o2) * pj;
-                        }
-                        const int cnt6 = (info >> NB_NONSOLID_SHIFT) & 7;
-                        double diag = 0;
-                        for (int k = 0; k < cnt6; k++) diag += scale;
-                        double ee = diag - eneg - eneg_tau * tau;
-                        if (ee < sigma * diag) ee = diag < 1e-6 ? 1.0 : diag;
-                        v = 1.0 / sqrt(ee);
+                    for (int ax = 0; ax < 3; ax++) {
+                        const double ap = -scale * upv[ax];
+                        eneg += ap * ap;
+                        eneg_tau += ap * S.tab.up[(info >> (NB_UP_SHIFT + 2 * ax)) & 3] * upv[ax];
                     }
+                    const f64x2 dg = S.tab.diag[(info >> NB_NONSOLID_SHIFT) & 7];
+                    double ee = dg[0] - eneg - eneg_tau * 0.97;
+                    ee = ee < 0.25 * dg[0] ? dg[1] : ee;
+                    double v = 1.0 / sqrt(ee);
+                    v = (info & NB_FLUID) ? v : 0.0;
                     res[r][e] = (float)v;
                     prev[r] = v;
                 } else {
@@ -650,12 +652,13 @@ __device__ __forceinline__ void compute_wave(const WaveArgs& A, WaveLds<KIND>& S
             constexpr int r = decltype(rc)::value;
             __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, res[r]), rC, lo[d][r], go[d], 0);
             if constexpr (KIND == 0) {
-                // FP64: 32 bytes per column and group, beyond 32-bit offsets on the largest grids
-                if (lo[d][r] < kOob) {
-                    f64x2* p64 = reinterpret_cast<f64x2*>(reinterpret_cast<char*>(A.P64) + 2 * ((int64_t)go[d] + lo[d][r]));
-                    p64[0] = f64x2{mine[r].get(0), mine[r].get(1)};
-                    p64[1] = f64x2{mine[r].get(2), mine[r].get(3)};
-                }
+                // FP64: 32 bytes per column and group, beyond 32-bit offsets on the largest grids: a
+                // resource per group
+                const __amdgpu_buffer_rsrc_t rD =
+                    rsrc(reinterpret_cast<char*>(A.P64) + 2 * (int64_t)go[d], 2 * (int64_t)gstride);
+                const uint32_t o = lo[d][r] < kOob ? 2 * lo[d][r] : kOob;
+                __builtin_amdgcn_raw_buffer_store_b128(mine[r].q[0], rD, o, 0, 0);
+                __builtin_amdgcn_raw_buffer_store_b128(mine[r].q[1], rD, o, 16, 0);
             }
         });
         fetch(std::integral_constant<int, (d + kPrefetch) % kRing>{}, g + kPrefetch);
@@ -723,6 +726,14 @@ __global__ void __launch_bounds__(WF_THREADS) k_wave(WaveArgs A) {
         c.zout = kAll;
         if (T.zdn) c.zout = kRingZ + max(0, z_shift<KD::FWD>(T.m, march_of<KD::FWD>(A, T.K + 1, xa, xb)) / WF_G);
         S.cnt[threadIdx.x] = c;
+    }
+    if constexpr (KIND == 0) {
+        if (threadIdx.x < 8) {
+            double d = 0;
+            for (unsigned k = 0; k < threadIdx.x; k++) d += A.scale;
+            S.tab.diag[threadIdx.x] = f64x2{d, d < 1e-6 ? 1.0 : d};
+        }
+        if (threadIdx.x < 4) S.tab.up[threadIdx.x] = ((threadIdx.x & 1) ? -A.scale : 0.0) + ((threadIdx.x & 2) ? -A.scale : 0.0);
     }
     __syncthreads();
     const int wave = threadIdx.x / 64;
