@@ -119,7 +119,6 @@ static void free_all(fsim_ctx* ctx) {
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (ctx->scal_host) (void)hipHostFree(ctx->scal_host);
-    if (ctx->res_ev) (void)hipEventDestroy(ctx->res_ev);
     if (ctx->dir_ev) (void)hipEventDestroy(ctx->dir_ev);
     if (ctx->x_ev) (void)hipEventDestroy(ctx->x_ev);
     for (auto& e : ctx->ev)
@@ -201,10 +200,10 @@ int fsim_create(const fsim_grid_desc* grid, const fsim_params* params, fsim_ctx*
     if ((rc = dalloc(ctx, &ctx->partials, 2 * kMaxParts))) return fail(rc);   // 2 per block of a reduction
     if (hipHostMalloc(reinterpret_cast<void**>(&ctx->scal_host), sizeof(SolveScalars), hipHostMallocDefault) != hipSuccess)
         return fail(FSIM_ERR_OOM);
+    *ctx->scal_host = SolveScalars{};   // seq 0: nothing has arrived
     for (auto& e : ctx->ev)
         if (hipEventCreate(&e) != hipSuccess) return fail(FSIM_ERR_HIP);
-    if (hipEventCreateWithFlags(&ctx->res_ev, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&ctx->dir_ev, hipEventDisableTiming) != hipSuccess ||
+    if (hipEventCreateWithFlags(&ctx->dir_ev, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&ctx->x_ev, hipEventDisableTiming) != hipSuccess)
         return fail(FSIM_ERR_HIP);
     // initial grid state: zero faces, AIR labels (MacGrid ctor, macGrid.cpp:9-17)

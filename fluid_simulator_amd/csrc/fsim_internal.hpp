@@ -250,7 +250,7 @@ struct SolveScalars {
     double zq;                       // z.q (flexible PCG)
     double nfluid;                   // number of WATER cells of the solve
     int nan_flag;
-    int pad;
+    unsigned seq;                    // host copy: number of the reduction that wrote it
 };
 
 // Kernel groups timed with HIP events when profiling is on.
@@ -321,7 +321,8 @@ struct fsim_ctx {
     double* sor64 = nullptr;          // BasicMacGrid SOR: FP64 faces u, v, w (allocated on first use)
     double* partials = nullptr;       // block partial sums (FP64)
     unsigned* red_count = nullptr;    // blocks finished in the running reduction (0 between launches)
-    hipEvent_t res_ev = nullptr;      // PCG: the iteration's scalars are on the host
+    unsigned scal_seq = 0;                 // last reduction that writes scal_host
+    bool x_pending = false;           // an x update on xstream that the main stream has not joined
     hipEvent_t dir_ev = nullptr;      // PCG: the direction step (s, alpha) is done
     hipEvent_t x_ev = nullptr;        // PCG: the x update on xstream is done
     int last_mic_iterations = 0;      // MIC(0)-PCG iterations of the last solve that used it

@@ -19,6 +19,8 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
+#include <chrono>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -58,6 +60,7 @@ struct Reduce {
     SolveScalars* sc;
     int op;             // FinOp
     SolveScalars* host = nullptr;   // pinned host copy written by the finishing block, or null
+    unsigned seq = 0;               // what the host waits for in it (host->seq)
 };
 
 __device__ inline void apply_fin(int op, double s, double m, SolveScalars* sc) {
@@ -159,16 +162,16 @@ __device__ void block_finish(double sum, double aux, const Reduce& R) {
         __hip_atomic_store(R.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (R.host) {
             // the words the host tests after the r update (rr, rmax, nan_flag) straight into pinned
-            // host memory with system-scope stores; the kernel's end and the event after it order
-            // them before the host's read
-            auto put_host = [](void* dst, const void* src) {
-                __hip_atomic_store(reinterpret_cast<uint64_t*>(dst), *reinterpret_cast<const uint64_t*>(src),
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            // host memory with system-scope stores, the word with seq, which the host polls, when the
+            // others have been acknowledged
+            auto put_host = [](void* dst, uint64_t v) {
+                __hip_atomic_store(reinterpret_cast<uint64_t*>(dst), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             };
-            put_host(&R.host->rr, &R.sc->rr);
-            put_host(&R.host->rmax, &R.sc->rmax);
-            static_assert(offsetof(SolveScalars, pad) == offsetof(SolveScalars, nan_flag) + 4, "one 8-byte word");
-            put_host(&R.host->nan_flag, &R.sc->nan_flag);
+            put_host(&R.host->rr, __builtin_bit_cast(uint64_t, R.sc->rr));
+            put_host(&R.host->rmax, __builtin_bit_cast(uint64_t, R.sc->rmax));
+            __builtin_amdgcn_s_waitcnt(0);
+            static_assert(offsetof(SolveScalars, seq) == offsetof(SolveScalars, nan_flag) + 4, "one 8-byte word");
+            put_host(&R.host->nan_flag, (uint32_t)R.sc->nan_flag | (uint64_t)R.seq << 32);
         }
     }
 }
@@ -545,9 +548,53 @@ __device__ inline void for_flagged_chunks(int64_t n, const uint32_t* __restrict_
     }
 }
 
-// r -= alpha q, with ||r||^2 and max|r|
+// x += alpha s (FP64) for WATER cells, of the last direction step (STEPS 1) or
+// of the last two in their order (STEPS 2: s_prev and the alpha before).  A NaN
+// alpha leaves x as it is: the reference breaks before multAdd
+// (bridsonSolverGrid.cpp:270-272) and applies the last pressure.
+struct UpdateX {
+    const uint16_t* nbinfo;
+    const float *s_prev, *s;
+    double* x;
+};
+template <int STEPS>
+__device__ inline void update_x_chunks(int64_t n, const uint32_t* __restrict__ flags, const UpdateX& A,
+                                       const SolveScalars* __restrict__ sc) {
+    const int lane = threadIdx.x & 63;
+    const int nchunks = (int)((n + kChunk - 1) / kChunk);
+    const int nwaves = (int)(gridDim.x * (blockDim.x / 64));
+    const double alpha_prev = sc->alpha_prev, alpha = sc->alpha;
+    const bool last = !(sc->nan_flag & 1);
+    for (int u = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6))); u < nchunks;
+         u += nwaves) {
+        const int64_t i = (int64_t)u * kChunk + 4 * lane;
+        if (flags[u] == 0u || i >= n) continue;
+        const u16x4 nb = *reinterpret_cast<const u16x4*>(A.nbinfo + i);
+        f64x4 v = *reinterpret_cast<const f64x4*>(A.x + i);
+        f32x4 a = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (STEPS == 2) a = *reinterpret_cast<const f32x4*>(A.s_prev + i);
+        const f32x4 b = *reinterpret_cast<const f32x4*>(A.s + i);
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            if (!(nb[c] & NB_FLUID)) continue;
+            if constexpr (STEPS == 2) v[c] += (double)a[c] * alpha_prev;
+            if (last) v[c] += (double)b[c] * alpha;
+        }
+        *reinterpret_cast<f64x4*>(A.x + i) = v;
+    }
+}
+template <int STEPS>
+__global__ void __launch_bounds__(kBlock) k_update_x(int64_t n, const uint32_t* __restrict__ flags, UpdateX A,
+                                                     const SolveScalars* __restrict__ sc) {
+    update_x_chunks<STEPS>(n, flags, A, sc);
+}
+
+// r -= alpha q, with ||r||^2 and max|r|; with X also the x update of the last
+// two steps, behind the block's part of the reduction.
+template <bool X>
 __global__ void __launch_bounds__(kStream) k_update_r(int64_t n, const uint32_t* __restrict__ flags,
-                                                     const float* __restrict__ q, float* __restrict__ r, Reduce red) {
+                                                     const float* __restrict__ q, float* __restrict__ r, UpdateX ux,
+                                                     Reduce red) {
     double ss = 0.0, mx = 0.0;
     const float malpha = (float)(-red.sc->alpha);
     auto cell = [&](float qv, float& rv) {
@@ -569,6 +616,7 @@ __global__ void __launch_bounds__(kStream) k_update_r(int64_t n, const uint32_t*
             *reinterpret_cast<float4*>(r + i) = v[1];
         });
     block_finish<AUX_MAX, kStream>(ss, mx, red);
+    if constexpr (X) update_x_chunks<2>(n, flags, ux, red.sc);
 }
 
 // a . b (FP64 products of the FP32 values)
@@ -588,38 +636,6 @@ __global__ void __launch_bounds__(kStream) k_dot(int64_t n, const uint32_t* __re
             d += (double)v[0].w * (double)v[1].w;
         });
     block_finish<AUX_NONE, kStream>(d, 0.0, red);
-}
-
-// x += alpha s (FP64) for WATER cells, of the last direction step (STEPS 1) or
-// of the last two in their order (STEPS 2: s_prev and the alpha before).  A NaN
-// alpha leaves x as it is: the reference breaks before multAdd
-// (bridsonSolverGrid.cpp:270-272) and applies the last pressure.
-template <int STEPS>
-__global__ void __launch_bounds__(kBlock) k_update_x(int64_t n, const uint32_t* __restrict__ flags,
-                                                     const uint16_t* __restrict__ nbinfo, const float* __restrict__ s_prev, const float* __restrict__ s,
-                                                     double* __restrict__ x, const SolveScalars* __restrict__ sc) {
-    const int lane = threadIdx.x & 63;
-    const int nchunks = (int)((n + kChunk - 1) / kChunk);
-    const int nwaves = (int)(gridDim.x * (blockDim.x / 64));
-    const double alpha_prev = sc->alpha_prev, alpha = sc->alpha;
-    const bool last = !(sc->nan_flag & 1);
-    for (int u = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6))); u < nchunks;
-         u += nwaves) {
-        const int64_t i = (int64_t)u * kChunk + 4 * lane;
-        if (flags[u] == 0u || i >= n) continue;
-        const u16x4 nb = *reinterpret_cast<const u16x4*>(nbinfo + i);
-        f64x4 v = *reinterpret_cast<const f64x4*>(x + i);
-        f32x4 a = {0.f, 0.f, 0.f, 0.f};
-        if constexpr (STEPS == 2) a = *reinterpret_cast<const f32x4*>(s_prev + i);
-        const f32x4 b = *reinterpret_cast<const f32x4*>(s + i);
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            if (!(nb[c] & NB_FLUID)) continue;
-            if constexpr (STEPS == 2) v[c] += (double)a[c] * alpha_prev;
-            if (last) v[c] += (double)b[c] * alpha;
-        }
-        *reinterpret_cast<f64x4*>(x + i) = v;
-    }
 }
 
 // FP64 true residual t = b - A x; optionally r = (float)t.
@@ -741,9 +757,9 @@ static unsigned column_blocks(const SolveArgs& S) {
 }
 
 static Reduce reduce_to(fsim_ctx* ctx, int op) { return Reduce{ctx->partials, ctx->red_count, ctx->scal, op}; }
-// the same, with the finished scalars also written to the pinned host copy (read after an event)
+// the same, with the finished scalars also written to the pinned host copy (wait_scalars)
 static Reduce reduce_to_host(fsim_ctx* ctx, int op) {
-    return Reduce{ctx->partials, ctx->red_count, ctx->scal, op, ctx->scal_host};
+    return Reduce{ctx->partials, ctx->red_count, ctx->scal, op, ctx->scal_host, ++ctx->scal_seq};
 }
 
 static int read_scalars(fsim_ctx* ctx) {
@@ -883,34 +899,60 @@ static int direction_step(fsim_ctx* ctx, const SolveArgs& S, bool copy) {
 // replaces alpha and the older of the two s buffers, so the main stream waits
 // for it (join_x) before the next direction step and before anything else
 // reads x.
+// Up to kInlineX values, and before the V-cycle, the r update's blocks do it
+// instead: the events of the second stream cost more than the x update's
+// memory traffic.  A step takes 1.71 ms inline, 1.77 beside at 32^3, 7.93 and
+// 8.07 at 96^3, 11.15 and 11.33 at 128^3, 72.4 and 71.4 at 256^3, where the
+// sweeps leave the bandwidth idle; with the V-cycle 12.06 and 12.78 at 128^3,
+// 42.2 and 43.0 at 256^3.
+constexpr int64_t kInlineX = 1 << 22;
 #ifndef FSIM_X_BLOCKS
 #define FSIM_X_BLOCKS 2048
 #endif
+static UpdateX update_x_args(fsim_ctx* ctx) { return UpdateX{ctx->nbinfo, ctx->s2, ctx->s, ctx->x}; }
 static int update_x_beside(fsim_ctx* ctx, int steps) {
     FSIM_HIP(ctx, hipEventRecord(ctx->dir_ev, ctx->stream));
     FSIM_HIP(ctx, hipStreamWaitEvent(ctx->xstream, ctx->dir_ev, 0));
     const int64_t n = ctx->g.ncr;
     const dim3 grid(std::max(1u, std::min(nblocks(n / 4), (unsigned)FSIM_X_BLOCKS))), block(kBlock);
     if (steps == 2)
-        hipLaunchKernelGGL(k_update_x<2>, grid, block, 0, ctx->xstream, n, ctx->chunk_flags, ctx->nbinfo, ctx->s2, ctx->s,
-                           ctx->x, ctx->scal);
+        hipLaunchKernelGGL(k_update_x<2>, grid, block, 0, ctx->xstream, n, ctx->chunk_flags, update_x_args(ctx), ctx->scal);
     else
-        hipLaunchKernelGGL(k_update_x<1>, grid, block, 0, ctx->xstream, n, ctx->chunk_flags, ctx->nbinfo, ctx->s2, ctx->s,
-                           ctx->x, ctx->scal);
+        hipLaunchKernelGGL(k_update_x<1>, grid, block, 0, ctx->xstream, n, ctx->chunk_flags, update_x_args(ctx), ctx->scal);
     FSIM_HIP(ctx, hipGetLastError());
     FSIM_HIP(ctx, hipEventRecord(ctx->x_ev, ctx->xstream));
+    ctx->x_pending = true;
     return FSIM_OK;
 }
 static int join_x(fsim_ctx* ctx) {
-    FSIM_HIP(ctx, hipStreamWaitEvent(ctx->stream, ctx->x_ev, 0));
+    if (ctx->x_pending) FSIM_HIP(ctx, hipStreamWaitEvent(ctx->stream, ctx->x_ev, 0));
+    ctx->x_pending = false;
     return FSIM_OK;
 }
 // joins the x stream on every exit of a solve, error returns included, so that no later work on the
 // main stream (the next solve clears x) runs beside a pending x update
 struct JoinXOnExit {
     fsim_ctx* ctx;
-    ~JoinXOnExit() { (void)hipStreamWaitEvent(ctx->stream, ctx->x_ev, 0); }
+    ~JoinXOnExit() { (void)join_x(ctx); }
 };
+
+// Waits until the finishing block of the last reduce_to_host reduction has
+// written its scalars: polls the pinned word, since an event after the kernel
+// is one more packet that the kernels behind it wait for (5 us an iteration).
+// A queue that takes longer than the polls is waited for as a whole, which
+// also reports a failed kernel.
+static int wait_scalars(fsim_ctx* ctx, SolveScalars* h) {
+    const volatile unsigned* seq = &ctx->scal_host->seq;
+    const auto t0 = std::chrono::steady_clock::now();
+    while (*seq != ctx->scal_seq) {
+        if (std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(100)) continue;
+        FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        if (*seq != ctx->scal_seq) return set_err(ctx, FSIM_ERR_HIP, "the solver's scalars did not arrive");
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    *h = *ctx->scal_host;
+    return FSIM_OK;
+}
 
 static bool stop_met(const fsim_ctx* ctx, double ss, double mx, double bnorm) {
     if (ctx->prm.stop_rule == FSIM_STOP_REL_L2) return std::sqrt(ss) <= ctx->prm.residual_tolerance * bnorm;
@@ -951,8 +993,9 @@ struct PcgResult {
 // One host round trip per iteration: the iteration's scalars are copied after
 // the r update, and the next preconditioner application and its dots run
 // while the host waits for them.  If the solve stops or restarts, those
-// results are discarded.  x += alpha s runs on the second stream beside the
-// preconditioner and is joined before the next direction step.
+// results are discarded.  x += alpha s runs with the r update, or on the
+// second stream beside it and the preconditioner, and is joined before the
+// next direction step.
 static int pcg_run(fsim_ctx* ctx, const SolveArgs& S, double bnorm, bool flexible, int max_it, PcgResult* res) {
     const JoinXOnExit join_on_exit{ctx};
     const int64_t n = S.ncr;
@@ -970,6 +1013,7 @@ static int pcg_run(fsim_ctx* ctx, const SolveArgs& S, double bnorm, bool flexibl
     double last_true = bnorm;
     bool copy = true;
     int it = 0;
+    const bool x_inline = flexible || n <= kInlineX;
     int behind = 0;   // direction steps that x does not hold yet (0 or 1 between iterations)
     res->converged = false;
     res->nan = false;
@@ -978,22 +1022,25 @@ static int pcg_run(fsim_ctx* ctx, const SolveArgs& S, double bnorm, bool flexibl
         FSIM_TRY(direction_step(ctx, S, copy));
         // x takes two steps at a time: it is read and written half as often (both s buffers still hold
         // their step)
-        if (++behind == 2) {
-            FSIM_TRY(update_x_beside(ctx, 2));
-            behind = 0;
-        }
+        const bool two = ++behind == 2;
+        if (two) behind = 0;
+        if (two && !x_inline) FSIM_TRY(update_x_beside(ctx, 2));
         {
             FSIM_PROF(ctx, KID_UPDATE);
-            hipLaunchKernelGGL(k_update_r, dim3(stream_blocks(n)), dim3(kStream), 0, ctx->stream, n, ctx->chunk_flags, ctx->q,
-                               ctx->r, reduce_to_host(ctx, FIN_RES));
+            const dim3 grid(stream_blocks(n)), block(kStream);
+            const Reduce red = reduce_to_host(ctx, FIN_RES);
+            if (two && x_inline)
+                hipLaunchKernelGGL(k_update_r<true>, grid, block, 0, ctx->stream, n, ctx->chunk_flags, ctx->q, ctx->r,
+                                   update_x_args(ctx), red);
+            else
+                hipLaunchKernelGGL(k_update_r<false>, grid, block, 0, ctx->stream, n, ctx->chunk_flags, ctx->q, ctx->r,
+                                   UpdateX{}, red);
         }
         FSIM_HIP(ctx, hipGetLastError());
-        // the r update's finishing block wrote rr, rmax and nan_flag into scal_host; the event orders the read
-        FSIM_HIP(ctx, hipEventRecord(ctx->res_ev, ctx->stream));
         FSIM_TRY(precondition(ctx, S, flexible));
         FSIM_TRY(next_beta(ctx, flexible));
-        FSIM_HIP(ctx, hipEventSynchronize(ctx->res_ev));
-        const SolveScalars h = *ctx->scal_host;
+        SolveScalars h;
+        FSIM_TRY(wait_scalars(ctx, &h));
         // the previous iteration's old-sigma test, then this iteration's alpha test
         if (h.nan_flag & 2) {
             it--;
