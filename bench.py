@@ -36,8 +36,8 @@ HBM_PEAK_GBS = 8000.0   # MI355X HBM3E
 # each array counted once per launch, no cache credit).  Units: f = WATER
 # cells, c = all cells, p = particles.
 ALGO_BYTES = {
-    "sweep_fwd": ("f", 13.0),      # R r 4, R P 4, R label 1, W q 4
-    "sweep_bwd": ("f", 13.0),      # R q 4, R P 4, R label 1, W z 4
+    "sweep_fwd": ("f", 21.0),      # R r 4, R q 4, R P 4, R label 1, W t 4, W r 4
+    "sweep_bwd": ("f", 25.0),      # R t 4, R P 4, R label 1, W z 4; every other time R x 8, R s 8, W x 8
     "mic_factor": ("f", 5.0),      # R label 1, W P 4
     "spmv": ("f", 17.0),           # direction step: R label 1, R z 4, R s 4, W s' 4, W q 4
     "update": ("f", 13.0),         # R label 1, R q 4, R/W r 8

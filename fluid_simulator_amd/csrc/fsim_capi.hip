@@ -114,17 +114,14 @@ static void free_all(fsim_ctx* ctx) {
     void* ptrs[] = {ctx->P.base, ctx->Palt.base, ctx->key, ctx->rank, ctx->perm, ctx->removed, ctx->u, ctx->v, ctx->w,
                     ctx->u2, ctx->v2, ctx->w2, ctx->label, ctx->valid, ctx->density, ctx->cell_count, ctx->cell_start,
                     ctx->scan_tmp, ctx->nbinfo, ctx->b, ctx->r, ctx->z, ctx->s, ctx->q, ctx->P32, ctx->P64,
-                    ctx->x, ctx->partials, ctx->scal, ctx->obs_dev, ctx->ybnd, ctx->zbnd, ctx->s2, ctx->red_count,
+                    ctx->x, ctx->partials, ctx->scal, ctx->obs_dev, ctx->ybnd, ctx->zbnd, ctx->s2, ctx->t, ctx->r_next, ctx->red_count,
                     ctx->wave_ticket, ctx->wave_err, ctx->sor64, ctx->colw};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (ctx->scal_host) (void)hipHostFree(ctx->scal_host);
-    if (ctx->dir_ev) (void)hipEventDestroy(ctx->dir_ev);
-    if (ctx->x_ev) (void)hipEventDestroy(ctx->x_ev);
     for (auto& e : ctx->ev)
         if (e) (void)hipEventDestroy(e);
     for (auto& e : ctx->prof_pool) (void)hipEventDestroy(e);
-    if (ctx->xstream) (void)hipStreamDestroy(ctx->xstream);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
 }
 
@@ -162,8 +159,7 @@ int fsim_create(const fsim_grid_desc* grid, const fsim_params* params, fsim_ctx*
         delete ctx;
         return rc;
     };
-    if (hipGetDevice(&ctx->device) != hipSuccess || hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipStreamCreateWithFlags(&ctx->xstream, hipStreamNonBlocking) != hipSuccess)
+    if (hipGetDevice(&ctx->device) != hipSuccess || hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess)
         return fail(FSIM_ERR_HIP);
     GridDims& g = ctx->g;
     g.nx = grid->nx;
@@ -190,7 +186,8 @@ int fsim_create(const fsim_grid_desc* grid, const fsim_params* params, fsim_ctx*
         (rc = dalloc(ctx, &ctx->density, nc)) || (rc = dalloc(ctx, &ctx->cell_count, nc + 1)) ||
         (rc = dalloc(ctx, &ctx->cell_start, nc + 2)) || (rc = dalloc(ctx, &ctx->nbinfo, ncr)) ||
         (rc = dalloc(ctx, &ctx->b, ncr)) || (rc = dalloc(ctx, &ctx->r, ncr)) || (rc = dalloc(ctx, &ctx->z, ncr)) ||
-        (rc = dalloc(ctx, &ctx->s, ncr)) || (rc = dalloc(ctx, &ctx->s2, ncr)) || (rc = dalloc(ctx, &ctx->q, ncr)) ||
+        (rc = dalloc(ctx, &ctx->s, ncr)) || (rc = dalloc(ctx, &ctx->s2, ncr)) ||
+        (rc = dalloc(ctx, &ctx->t, ncr)) || (rc = dalloc(ctx, &ctx->r_next, ncr)) || (rc = dalloc(ctx, &ctx->q, ncr)) ||
         (rc = dalloc(ctx, &ctx->red_count, 1)) ||
         (rc = dalloc(ctx, &ctx->P32, ncr)) || (rc = dalloc(ctx, &ctx->P64, ncr)) || (rc = dalloc(ctx, &ctx->x, ncr)) ||
         (rc = dalloc(ctx, &ctx->scal, 1)) || (rc = dalloc(ctx, &ctx->obs_dev, kMaxObstacles)))
@@ -203,14 +200,11 @@ int fsim_create(const fsim_grid_desc* grid, const fsim_params* params, fsim_ctx*
     *ctx->scal_host = SolveScalars{};   // seq 0: nothing has arrived
     for (auto& e : ctx->ev)
         if (hipEventCreate(&e) != hipSuccess) return fail(FSIM_ERR_HIP);
-    if (hipEventCreateWithFlags(&ctx->dir_ev, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&ctx->x_ev, hipEventDisableTiming) != hipSuccess)
-        return fail(FSIM_ERR_HIP);
     // initial grid state: zero faces, AIR labels (MacGrid ctor, macGrid.cpp:9-17)
     float* f32s[] = {ctx->u, ctx->v, ctx->w, ctx->u2, ctx->v2, ctx->w2, ctx->density};
     for (float* p : f32s)
         if (fill_f32(ctx, p, 0.0f, nc)) return fail(FSIM_ERR_HIP);
-    float* solver[] = {ctx->b, ctx->r, ctx->z, ctx->s, ctx->s2, ctx->q, ctx->P32};
+    float* solver[] = {ctx->b, ctx->r, ctx->z, ctx->s, ctx->s2, ctx->t, ctx->r_next, ctx->q, ctx->P32};
     for (float* p : solver)
         if (fill_f32(ctx, p, 0.0f, ncr)) return fail(FSIM_ERR_HIP);
     if (fill_u8(ctx, ctx->label, FSIM_AIR, nc) || fill_f64(ctx, ctx->x, 0.0, ncr) || fill_f64(ctx, ctx->P64, 0.0, ncr) ||

@@ -282,7 +282,6 @@ constexpr int kMgCoarseMaxSide = 16;   // the network's level: the first whose l
 struct fsim_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
-    hipStream_t xstream = nullptr;    // PCG: x += alpha s beside the r update and the preconditioner
     fsim::GridDims g{};
     fsim_params prm{};
     std::string err;
@@ -315,6 +314,8 @@ struct fsim_ctx {
     // pressure solve
     float *b = nullptr, *r = nullptr, *z = nullptr, *s = nullptr, *q = nullptr;
     float* s2 = nullptr;              // second search-direction buffer (swapped with s)
+    float* t = nullptr;               // forward sweep's result
+    float* r_next = nullptr;          // MIC(0)-PCG: second residual buffer
     float* P32 = nullptr;
     double* P64 = nullptr;
     double* x = nullptr;
@@ -322,9 +323,6 @@ struct fsim_ctx {
     double* partials = nullptr;       // block partial sums (FP64)
     unsigned* red_count = nullptr;    // blocks finished in the running reduction (0 between launches)
     unsigned scal_seq = 0;                 // last reduction that writes scal_host
-    bool x_pending = false;           // an x update on xstream that the main stream has not joined
-    hipEvent_t dir_ev = nullptr;      // PCG: the direction step (s, alpha) is done
-    hipEvent_t x_ev = nullptr;        // PCG: the x update on xstream is done
     int last_mic_iterations = 0;      // MIC(0)-PCG iterations of the last solve that used it
     int learned_since_mic = 0;        // learned solves since that MIC(0) solve
     int learned_refresh = 50;         // learned solves between MIC(0) solves that renew the count (0: never)
@@ -436,8 +434,10 @@ int fill_i32(fsim_ctx* ctx, int32_t* p, int32_t v, int64_t n);
 
 // ---- pressure solve (fsim_solver.hip) -------------------------------------
 int stage_solve(fsim_ctx* ctx, double dt);
-// kind 0 = MIC(0) factor, 1 = forward sweep, 2 = backward sweep
-int wave_launch(fsim_ctx* ctx, int kind, const float* in, float* out, double scale);
+// WAVE_FWD_UPDATE: the forward sweep of in - alpha side->q; side: null or what further blocks do (fsim_reduce.hpp)
+enum WaveKind { WAVE_FACTOR = 0, WAVE_FWD = 1, WAVE_BWD = 2, WAVE_FWD_UPDATE = 3 };
+struct SideWork;
+int wave_launch(fsim_ctx* ctx, WaveKind kind, const float* in, float* out, double scale, const SideWork* side);
 int wave_init(fsim_ctx* ctx);
 int solver_apply(fsim_ctx* ctx, int op, double dt, const double* in, double* out);
 

@@ -26,157 +26,9 @@
 #include <type_traits>
 
 #include "fsim_march.hpp"
+#include "fsim_reduce.hpp"
 
 namespace fsim {
-
-// ---- block reductions (FP64, fixed order) ------------------------------------
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v += __shfl_down(v, d, 64);
-    return v;
-}
-__device__ inline double wave_max(double v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v = fmax(v, __shfl_down(v, d, 64));
-    return v;
-}
-// ---- in-kernel finish of a reduction -------------------------------------------------
-// Each block reduces its values to one partial (plus an aux value: max or sum)
-// and stores it with device-scope stores; once they are acknowledged the block
-// takes a ticket from a device-scope counter.  The block with the last ticket
-// sums all partials in a fixed order (thread t: partials t, t + kBlock, ...,
-// then a pairwise tree), applies the reduction's scalar update and resets the
-// counter.  The sum's order does not depend on which block is last, so the
-// result is deterministic, and no separate finalize launch is needed.
-constexpr int AUX_NONE = 0, AUX_MAX = 1, AUX_SUM = 2;
-enum FinOp {
-    FIN_NONE = -1, FIN_BB = 0, FIN_SIGMA0 = 1, FIN_ALPHA = 2, FIN_RES = 3, FIN_BETA = 4, FIN_TRUE = 5, FIN_ZQ = 6,
-    FIN_FBETA = 7
-};
-
-struct Reduce {
-    double* partials;   // 2 x gridDim.x
-    unsigned* count;    // zero between launches
-    SolveScalars* sc;
-    int op;             // FinOp
-    SolveScalars* host = nullptr;   // pinned host copy written by the finishing block, or null
-    unsigned seq = 0;               // what the host waits for in it (host->seq)
-};
-
-__device__ inline void apply_fin(int op, double s, double m, SolveScalars* sc) {
-    switch (op) {
-    case FIN_BB: sc->bb = s; sc->nfluid = m; break;
-    case FIN_SIGMA0: sc->zr = s; break;
-    case FIN_ALPHA: {   // sigma is the last z.r (initial, restart or beta step)
-        sc->sigma = sc->zr;
-        sc->sq = s;
-        const double alpha = sc->sigma / s;
-        sc->alpha_prev = sc->alpha;
-        sc->alpha = alpha;
-        if (alpha != alpha) sc->nan_flag |= 1;
-        break;
-    }
-    case FIN_RES: sc->rr = s; sc->rmax = m; break;
-    case FIN_BETA: {
-        if (sc->sigma != sc->sigma) sc->nan_flag |= 2;   // the reference tests the old sigma (:285-286)
-        sc->zr = s;
-        sc->beta = s / sc->sigma;
-        break;
-    }
-    case FIN_TRUE: sc->tr_ss = s; sc->tr_max = m; break;
-    case FIN_ZQ: sc->zq = s; break;
-    case FIN_FBETA: {   // flexible PCG: beta = z'.(r' - r) / z.r = -alpha z'.q / z.r
-        if (sc->sigma != sc->sigma) sc->nan_flag |= 2;
-        sc->zr = s;
-        sc->beta = -sc->alpha * sc->zq / sc->sigma;
-        break;
-    }
-    default: break;
-    }
-}
-
-__device__ inline void put_dev(double* p, double v) {
-    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline double get_dev(const double* p) {
-    return __builtin_bit_cast(double, __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED,
-                                                        __HIP_MEMORY_SCOPE_AGENT));
-}
-
-template <int AUX, int NT = kBlock>
-__device__ void block_finish(double sum, double aux, const Reduce& R) {
-    __shared__ double lds_s[NT], lds_m[NT];
-    __shared__ int last;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    sum = wave_sum(sum);
-    if (AUX == AUX_MAX) aux = wave_max(aux);
-    if (AUX == AUX_SUM) aux = wave_sum(aux);
-    if (lane == 0) {
-        lds_s[wave] = sum;
-        lds_m[wave] = aux;
-    }
-    __syncthreads();
-    const unsigned nparts = gridDim.x;
-    if (threadIdx.x == 0) {
-        double s = 0, m = 0;
-        for (int w = 0; w < NT / 64; w++) {
-            s += lds_s[w];
-            m = AUX == AUX_SUM ? m + lds_m[w] : fmax(m, lds_m[w]);
-        }
-        put_dev(&R.partials[blockIdx.x], s);
-        if (AUX != AUX_NONE) put_dev(&R.partials[nparts + blockIdx.x], m);
-        __builtin_amdgcn_s_waitcnt(0);   // the partials are acknowledged before the ticket
-        last = __hip_atomic_fetch_add(R.count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nparts - 1;
-    }
-    __syncthreads();
-    if (!last) return;
-    // all loads first (at most kMaxParts / NT per thread), then the sums in order
-    constexpr int kPer = kMaxParts / NT;
-    double vs[kPer], vm[kPer];
-#pragma unroll
-    for (int k = 0; k < kPer; k++) {
-        const unsigned i = threadIdx.x + k * NT;
-        vs[k] = i < nparts ? get_dev(&R.partials[i]) : 0.0;
-        vm[k] = AUX != AUX_NONE && i < nparts ? get_dev(&R.partials[nparts + i]) : 0.0;
-    }
-    double s = 0, m = 0;
-#pragma unroll
-    for (int k = 0; k < kPer; k++) {
-        s += vs[k];
-        m = AUX == AUX_SUM ? m + vm[k] : fmax(m, vm[k]);
-    }
-    lds_s[threadIdx.x] = s;
-    lds_m[threadIdx.x] = m;
-    __syncthreads();
-    for (int off = NT / 2; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) {
-            lds_s[threadIdx.x] += lds_s[threadIdx.x + off];
-            lds_m[threadIdx.x] = AUX == AUX_SUM ? lds_m[threadIdx.x] + lds_m[threadIdx.x + off]
-                                                : fmax(lds_m[threadIdx.x], lds_m[threadIdx.x + off]);
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        apply_fin(R.op, lds_s[0], lds_m[0], R.sc);
-        __hip_atomic_store(R.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (R.host) {
-            // the words the host tests after the r update (rr, rmax, nan_flag) straight into pinned
-            // host memory with system-scope stores, the word with seq, which the host polls, when the
-            // others have been acknowledged
-            auto put_host = [](void* dst, uint64_t v) {
-                __hip_atomic_store(reinterpret_cast<uint64_t*>(dst), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            };
-            put_host(&R.host->rr, __builtin_bit_cast(uint64_t, R.sc->rr));
-            put_host(&R.host->rmax, __builtin_bit_cast(uint64_t, R.sc->rmax));
-            __builtin_amdgcn_s_waitcnt(0);
-            static_assert(offsetof(SolveScalars, seq) == offsetof(SolveScalars, nan_flag) + 4, "one 8-byte word");
-            put_host(&R.host->nan_flag, (uint32_t)R.sc->nan_flag | (uint64_t)R.seq << 32);
-        }
-    }
-}
-
-constexpr int kChunk = 256;   // values of a solver vector per chunk flag (the streaming kernels)
 
 // ---- RHS and neighbour masks (calculateRHS :79-89, calculateAMatrix :40-77) ------
 struct RhsArgs {
@@ -493,15 +345,6 @@ __global__ void __launch_bounds__(64 * kMarchWaves) k_spmv(SolveArgs S, MarchPla
     block_finish<AUX_NONE, 64 * kMarchWaves>(d, 0.0, red);
 }
 
-// Streaming kernels without per-cell masks: the solver vectors r, q and z
-// are exactly zero off WATER (zeroed at the start of a solve, written with
-// zeros there), so the extra terms are exact zeros.  The vectors are cut
-// into chunks of 256 values (16 bytes per lane); a chunk without WATER is
-// skipped.  Its flag is one 32-bit word (built with nbinfo for every solve),
-// so a wave reads it with a scalar load; a wave takes kUnits chunks per trip
-// (grid stride) and issues all their loads before using any, so several
-// memory round trips are in flight.
-constexpr int kUnits = 4;
 // Large blocks: every block takes a ticket from one counter at its end, and
 // the tickets are handed out one after the other.  256 blocks of 1024 threads
 // against 1024 of 256: dot 21 us (27) at 256^3 and 9.7 (13.7) at 128^3, r
@@ -517,106 +360,24 @@ static unsigned stream_blocks(int64_t n) {
     return std::max(1u, std::min<unsigned>(need, FSIM_STREAM_BLOCKS));
 }
 
-template <int NV, class Load, class Use>
-__device__ inline void for_flagged_chunks(int64_t n, const uint32_t* __restrict__ flags, Load&& load, Use&& use) {
-    const int lane = threadIdx.x & 63;
-    const int nchunks = (int)((n + kChunk - 1) / kChunk);
-    const int nwaves = (int)(gridDim.x * (blockDim.x / 64));
-    const int w0 = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6)));
-    for (int u0 = w0; u0 < nchunks; u0 += kUnits * nwaves) {
-        uint32_t f[kUnits];
-#pragma unroll
-        for (int k = 0; k < kUnits; k++) {
-            const int u = u0 + k * nwaves;
-            f[k] = u < nchunks ? flags[u] : 0u;
-        }
-        // loads without branches (a skipped lane reads cell 0 and uses nothing), so that all
-        // kUnits x NV loads are issued before the first wait
-        float4 v[kUnits][NV];
-        bool on[kUnits];
-        int64_t at[kUnits];
-#pragma unroll
-        for (int k = 0; k < kUnits; k++) {
-            const int64_t i = (int64_t)(u0 + k * nwaves) * kChunk + 4 * lane;
-            on[k] = f[k] != 0u && i < n;
-            at[k] = on[k] ? i : 0;
-            load(at[k], v[k]);
-        }
-#pragma unroll
-        for (int k = 0; k < kUnits; k++)
-            if (on[k]) use(at[k], v[k]);
-    }
-}
-
-// x += alpha s (FP64) for WATER cells, of the last direction step (STEPS 1) or
-// of the last two in their order (STEPS 2: s_prev and the alpha before).  A NaN
-// alpha leaves x as it is: the reference breaks before multAdd
-// (bridsonSolverGrid.cpp:270-272) and applies the last pressure.
-struct UpdateX {
-    const uint16_t* nbinfo;
-    const float *s_prev, *s;
-    double* x;
-};
-template <int STEPS>
-__device__ inline void update_x_chunks(int64_t n, const uint32_t* __restrict__ flags, const UpdateX& A,
-                                       const SolveScalars* __restrict__ sc) {
-    const int lane = threadIdx.x & 63;
-    const int nchunks = (int)((n + kChunk - 1) / kChunk);
-    const int nwaves = (int)(gridDim.x * (blockDim.x / 64));
-    const double alpha_prev = sc->alpha_prev, alpha = sc->alpha;
-    const bool last = !(sc->nan_flag & 1);
-    for (int u = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6))); u < nchunks;
-         u += nwaves) {
-        const int64_t i = (int64_t)u * kChunk + 4 * lane;
-        if (flags[u] == 0u || i >= n) continue;
-        const u16x4 nb = *reinterpret_cast<const u16x4*>(A.nbinfo + i);
-        f64x4 v = *reinterpret_cast<const f64x4*>(A.x + i);
-        f32x4 a = {0.f, 0.f, 0.f, 0.f};
-        if constexpr (STEPS == 2) a = *reinterpret_cast<const f32x4*>(A.s_prev + i);
-        const f32x4 b = *reinterpret_cast<const f32x4*>(A.s + i);
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-            if (!(nb[c] & NB_FLUID)) continue;
-            if constexpr (STEPS == 2) v[c] += (double)a[c] * alpha_prev;
-            if (last) v[c] += (double)b[c] * alpha;
-        }
-        *reinterpret_cast<f64x4*>(A.x + i) = v;
-    }
-}
 template <int STEPS>
 __global__ void __launch_bounds__(kBlock) k_update_x(int64_t n, const uint32_t* __restrict__ flags, UpdateX A,
                                                      const SolveScalars* __restrict__ sc) {
-    update_x_chunks<STEPS>(n, flags, A, sc);
+    update_x_chunks<STEPS>(whole_grid(), n, flags, A, sc);
 }
 
-// r -= alpha q, with ||r||^2 and max|r|; with X also the x update of the last
+// r_next = r - alpha q (r_next may be r); with X also the x update of the last
 // two steps, behind the block's part of the reduction.
-template <bool X>
-__global__ void __launch_bounds__(kStream) k_update_r(int64_t n, const uint32_t* __restrict__ flags,
-                                                     const float* __restrict__ q, float* __restrict__ r, UpdateX ux,
-                                                     Reduce red) {
-    double ss = 0.0, mx = 0.0;
-    const float malpha = (float)(-red.sc->alpha);
-    auto cell = [&](float qv, float& rv) {
-        rv = rv + qv * malpha;
-        ss += (double)rv * (double)rv;
-        mx = fmax(mx, fabs((double)rv));
-    };
-    for_flagged_chunks<2>(
-        n, flags,
-        [&](int64_t i, float4(&v)[2]) {
-            v[0] = *reinterpret_cast<const float4*>(q + i);
-            v[1] = *reinterpret_cast<const float4*>(r + i);
-        },
-        [&](int64_t i, float4(&v)[2]) {
-            cell(v[0].x, v[1].x);
-            cell(v[0].y, v[1].y);
-            cell(v[0].z, v[1].z);
-            cell(v[0].w, v[1].w);
-            *reinterpret_cast<float4*>(r + i) = v[1];
-        });
-    block_finish<AUX_MAX, kStream>(ss, mx, red);
-    if constexpr (X) update_x_chunks<2>(n, flags, ux, red.sc);
+template <int NT, bool X>
+__global__ void __launch_bounds__(NT) k_update_r(int64_t n, const uint32_t* __restrict__ flags, const float* q,
+                                                 const float* r, float* r_next, UpdateX ux, Reduce red) {
+    update_r<NT>(whole_grid(), n, flags, q, r, r_next, red);
+    if constexpr (X) update_x_chunks<2>(whole_grid(), n, flags, ux, red.sc);
+}
+
+template <int NT>
+__global__ void __launch_bounds__(NT) k_dot_self(int64_t n, const uint32_t* __restrict__ flags, const float* t, Reduce red) {
+    dot_self<NT>(whole_grid(), n, flags, t, red);
 }
 
 // a . b (FP64 products of the FP32 values)
@@ -624,7 +385,7 @@ __global__ void __launch_bounds__(kStream) k_dot(int64_t n, const uint32_t* __re
                                                 const float* __restrict__ a, const float* __restrict__ b, Reduce red) {
     double d = 0.0;
     for_flagged_chunks<2>(
-        n, flags,
+        whole_grid(), n, flags,
         [&](int64_t i, float4(&v)[2]) {
             v[0] = *reinterpret_cast<const float4*>(a + i);
             v[1] = *reinterpret_cast<const float4*>(b + i);
@@ -705,9 +466,25 @@ __global__ void __launch_bounds__(kBlock) k_apply_pressure(SolveArgs S, const ui
     }
 }
 
-__global__ void k_copy_f32(int64_t n, const float* __restrict__ a, float* __restrict__ b) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) b[i] = a[i];
+// Start of a solve: r = b, x = 0 and the other vectors 0 (n: a multiple of 4).
+constexpr int kZeroed = 6;
+struct SolveStart {
+    int64_t n;
+    const float* b;
+    float* r;
+    double* x;
+    float* zero[kZeroed];   // null: none
+};
+__global__ void __launch_bounds__(kBlock) k_solve_start(SolveStart A) {
+    const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+    const int64_t step = (int64_t)gridDim.x * kBlock * 4;
+    for (int64_t i = ((int64_t)blockIdx.x * kBlock + threadIdx.x) * 4; i < A.n; i += step) {
+        *reinterpret_cast<f32x4*>(A.r + i) = *reinterpret_cast<const f32x4*>(A.b + i);
+        *reinterpret_cast<f64x4*>(A.x + i) = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < kZeroed; k++)
+            if (A.zero[k]) *reinterpret_cast<f32x4*>(A.zero[k] + i) = none;
+    }
 }
 
 // ---- host driver --------------------------------------------------------------------
@@ -819,7 +596,7 @@ static int mic_factor(fsim_ctx* ctx, const SolveArgs& S) {
     FSIM_PROF(ctx, KID_MIC_FACTOR);
     FSIM_TRY(fill_f64(ctx, ctx->P64, 0.0, S.ncr));
     FSIM_TRY(fill_f32(ctx, ctx->P32, 0.0f, S.ncr));
-    if (ctx->sweep_mode == 0) return wave_launch(ctx, 0, nullptr, nullptr, S.scale);
+    if (ctx->sweep_mode == 0) return wave_launch(ctx, WAVE_FACTOR, nullptr, nullptr, S.scale, nullptr);
     PlaneArgs A{S, ctx->nbinfo, 0};
     const int nt = nplane_threads(S);
     const int lmax = (S.nx - 2) + (S.ny - 2) + (S.nz - 2);
@@ -831,35 +608,65 @@ static int mic_factor(fsim_ctx* ctx, const SolveArgs& S) {
     return FSIM_OK;
 }
 
-// z = M^-1 r (q is scratch; the backward sweep may run in place, q == z)
-static int mic_apply(fsim_ctx* ctx, const SolveArgs& S, const float* r, float* q, float* z) {
+// Blocks of WF_THREADS threads beside a sweep's tiles, on the compute units
+// that the tiles leave free.  At 256^3, where they have 300 MB to move, a solve
+// takes 66.8 ms with 128 blocks, 63.9 with 256 and 62.6 with 512; 128^3 does
+// not tell them apart.
+#ifndef FSIM_SIDE_BLOCKS
+#define FSIM_SIDE_BLOCKS 512
+#endif
+static_assert(FSIM_SIDE_BLOCKS <= (int)kMaxParts, "side blocks within the reduction");
+static unsigned side_blocks(int64_t n) {
+    const unsigned need = (unsigned)((n / kChunk + kUnits * (WF_THREADS / 64) - 1) / (kUnits * (WF_THREADS / 64)));
+    return std::max(1u, std::min<unsigned>(need, FSIM_SIDE_BLOCKS));
+}
+
+// t = L^-1 r and z = L^-T t, M = L L^T.
+// fwd: r -= alpha q on the way (side work of the forward sweep, the new r goes
+// to fwd->r_next); bwd: t . t and x (side work of the backward sweep).  Null:
+// none.  One launch per plane does the side work in launches of their own,
+// with the same blocks and so the same bits.
+static int mic_apply(fsim_ctx* ctx, const SolveArgs& S, const float* r, float* t, float* z, const SideWork* fwd = nullptr,
+                     const SideWork* bwd = nullptr) {
     if (ctx->sweep_mode == 0) {
         {
             FSIM_PROF(ctx, KID_SWEEP_FWD);
-            FSIM_TRY(wave_launch(ctx, 1, r, q, S.scale));
+            FSIM_TRY(wave_launch(ctx, fwd ? WAVE_FWD_UPDATE : WAVE_FWD, r, t, S.scale, fwd));
         }
         FSIM_PROF(ctx, KID_SWEEP_BWD);
-        return wave_launch(ctx, 2, q, z, S.scale);
+        return wave_launch(ctx, WAVE_BWD, t, z, S.scale, bwd);
+    }
+    if (fwd) {
+        hipLaunchKernelGGL((k_update_r<WF_THREADS, false>), dim3(fwd->blocks), dim3(WF_THREADS), 0, ctx->stream, fwd->n,
+                           fwd->flags, fwd->q, fwd->r, fwd->r_next, UpdateX{}, fwd->red);
+        r = fwd->r_next;
     }
     PlaneArgs A{S, ctx->nbinfo, 0};
     const int nt = nplane_threads(S);
     const int lmax = (S.nx - 2) + (S.ny - 2) + (S.nz - 2);
     for (int L = 3; L <= lmax; L++) {
         A.level = L;
-        hipLaunchKernelGGL(k_fwd_plane, dim3(nblocks(nt)), dim3(kBlock), 0, ctx->stream, A, r, q, ctx->P32);
+        hipLaunchKernelGGL(k_fwd_plane, dim3(nblocks(nt)), dim3(kBlock), 0, ctx->stream, A, r, t, ctx->P32);
+    }
+    if (bwd) {
+        hipLaunchKernelGGL(k_dot_self<WF_THREADS>, dim3(bwd->blocks), dim3(WF_THREADS), 0, ctx->stream, bwd->n, bwd->flags,
+                           bwd->t, bwd->red);
+        if (bwd->x_steps == 2)
+            hipLaunchKernelGGL(k_update_x<2>, dim3(bwd->blocks), dim3(kBlock), 0, ctx->stream, bwd->n, bwd->flags, bwd->x,
+                               ctx->scal);
     }
     for (int L = lmax; L >= 3; L--) {
         A.level = L;
-        hipLaunchKernelGGL(k_bwd_plane, dim3(nblocks(nt)), dim3(kBlock), 0, ctx->stream, A, q, z, ctx->P32);
+        hipLaunchKernelGGL(k_bwd_plane, dim3(nblocks(nt)), dim3(kBlock), 0, ctx->stream, A, t, z, ctx->P32);
     }
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;
 }
 
-static int true_residual(fsim_ctx* ctx, const SolveArgs& S, bool replace) {
+static int true_residual(fsim_ctx* ctx, const SolveArgs& S, float* r, bool replace) {
     FSIM_PROF(ctx, KID_TRUE_RES);
     hipLaunchKernelGGL(k_true_residual, dim3(column_blocks(S)), dim3(kBlock), 0, ctx->stream, S, ctx->nbinfo, ctx->b, ctx->x,
-                       ctx->r, replace ? 1 : 0, reduce_to(ctx, FIN_TRUE));
+                       r, replace ? 1 : 0, reduce_to(ctx, FIN_TRUE));
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;
 }
@@ -872,7 +679,6 @@ static int dot_with(fsim_ctx* ctx, const float* a, const float* b, int op) {
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;
 }
-static int dot_zr(fsim_ctx* ctx, int op) { return dot_with(ctx, ctx->z, ctx->r, op); }
 
 // New search direction s (z, or z + beta s) into the second buffer, q = A s,
 // s.q -> alpha.
@@ -894,47 +700,18 @@ static int direction_step(fsim_ctx* ctx, const SolveArgs& S, bool copy) {
     return FSIM_OK;
 }
 
-// x += alpha s of the last `steps` (1 or 2) direction steps, on the second
-// stream beside what the main stream runs next.  The next direction step
-// replaces alpha and the older of the two s buffers, so the main stream waits
-// for it (join_x) before the next direction step and before anything else
-// reads x.
-// Up to kInlineX values, and before the V-cycle, the r update's blocks do it
-// instead: the events of the second stream cost more than the x update's
-// memory traffic.  A step takes 1.71 ms inline, 1.77 beside at 32^3, 7.93 and
-// 8.07 at 96^3, 11.15 and 11.33 at 128^3, 72.4 and 71.4 at 256^3, where the
-// sweeps leave the bandwidth idle; with the V-cycle 12.06 and 12.78 at 128^3,
-// 42.2 and 43.0 at 256^3.
-constexpr int64_t kInlineX = 1 << 22;
-#ifndef FSIM_X_BLOCKS
-#define FSIM_X_BLOCKS 2048
-#endif
+// x takes two direction steps at a time: it is read and written half as often
+// (both s buffers still hold their step).  What is left when the loop ends is
+// one step.
 static UpdateX update_x_args(fsim_ctx* ctx) { return UpdateX{ctx->nbinfo, ctx->s2, ctx->s, ctx->x}; }
-static int update_x_beside(fsim_ctx* ctx, int steps) {
-    FSIM_HIP(ctx, hipEventRecord(ctx->dir_ev, ctx->stream));
-    FSIM_HIP(ctx, hipStreamWaitEvent(ctx->xstream, ctx->dir_ev, 0));
+static int update_x_last(fsim_ctx* ctx) {
+    FSIM_PROF(ctx, KID_UPDATE);
     const int64_t n = ctx->g.ncr;
-    const dim3 grid(std::max(1u, std::min(nblocks(n / 4), (unsigned)FSIM_X_BLOCKS))), block(kBlock);
-    if (steps == 2)
-        hipLaunchKernelGGL(k_update_x<2>, grid, block, 0, ctx->xstream, n, ctx->chunk_flags, update_x_args(ctx), ctx->scal);
-    else
-        hipLaunchKernelGGL(k_update_x<1>, grid, block, 0, ctx->xstream, n, ctx->chunk_flags, update_x_args(ctx), ctx->scal);
+    hipLaunchKernelGGL(k_update_x<1>, dim3(std::max(1u, std::min(nblocks(n / 4), kMaxParts))), dim3(kBlock), 0, ctx->stream, n,
+                       ctx->chunk_flags, update_x_args(ctx), ctx->scal);
     FSIM_HIP(ctx, hipGetLastError());
-    FSIM_HIP(ctx, hipEventRecord(ctx->x_ev, ctx->xstream));
-    ctx->x_pending = true;
     return FSIM_OK;
 }
-static int join_x(fsim_ctx* ctx) {
-    if (ctx->x_pending) FSIM_HIP(ctx, hipStreamWaitEvent(ctx->stream, ctx->x_ev, 0));
-    ctx->x_pending = false;
-    return FSIM_OK;
-}
-// joins the x stream on every exit of a solve, error returns included, so that no later work on the
-// main stream (the next solve clears x) runs beside a pending x update
-struct JoinXOnExit {
-    fsim_ctx* ctx;
-    ~JoinXOnExit() { (void)join_x(ctx); }
-};
 
 // Waits until the finishing block of the last reduce_to_host reduction has
 // written its scalars: polls the pinned word, since an event after the kernel
@@ -959,21 +736,72 @@ static bool stop_met(const fsim_ctx* ctx, double ss, double mx, double bnorm) {
     return mx < ctx->prm.residual_tolerance;
 }
 
-// z = M^-1 r with the solve's preconditioner: the MIC(0) sweeps, or the
-// learned multigrid V-cycle (fsim_mg.hip), whose coarsest level the network
-// solves.
-static int precondition(fsim_ctx* ctx, const SolveArgs& S, bool flexible) {
-    if (!flexible) return mic_apply(ctx, S, ctx->r, ctx->z, ctx->z);
-    return mg_apply(ctx, ctx->r, ctx->z, S.scale);
+// One iteration's update and preconditioner application, after the direction
+// step: r -= alpha q with its norms (which the host waits for), z = M^-1 r,
+// beta, and x if two steps are due.
+//
+// MIC(0): the r update and its norms run beside the forward sweep, which
+// computes the new r for itself, and sigma and the x update beside the backward
+// sweep: the sweeps are chains of waits that leave most of the chip idle.
+// sigma = z.r = r^T L^-T L^-1 r = t.t with t = L^-1 r, the forward sweep's
+// result, which is there before the backward sweep starts.  Summed in FP64,
+// it is off by the FP32 rounding inside the sweeps, 1e-9 to 6e-8 of its value
+// (z.r: 1e-9 to 2e-8; 8 to 26 cells a side, random and smooth r), where the
+// rounding of alpha and beta to FP32 may take 6e-8.  r has two buffers, since
+// the tiles read the old one.
+// An iteration, against launches of their own for the r update, the dot
+// product and the x update (the last on a second stream at 256^3): 32^3 62 ->
+// 49 us, 2D 128^2 100 -> 86, 128^3 132 -> 114, 256^3 395 -> 378.
+static int update_mic(fsim_ctx* ctx, const SolveArgs& S, float** r, float** r_next, bool x_due) {
+    SideWork fwd, bwd;
+    fwd.blocks = bwd.blocks = side_blocks(S.ncr);
+    fwd.n = bwd.n = S.ncr;
+    fwd.flags = bwd.flags = ctx->chunk_flags;
+    fwd.q = ctx->q;
+    fwd.r = *r;
+    fwd.r_next = *r_next;
+    fwd.red = reduce_to_host(ctx, FIN_RES);
+    bwd.t = ctx->t;
+    bwd.x = update_x_args(ctx);
+    bwd.x_steps = x_due ? 2 : 0;
+    bwd.red = reduce_to(ctx, FIN_BETA);
+    FSIM_TRY(mic_apply(ctx, S, *r, ctx->t, ctx->z, &fwd, &bwd));
+    std::swap(*r, *r_next);
+    return FSIM_OK;
 }
-
-// After a new z: z.r (and, flexible, z.q first), giving beta.  Plain PCG:
-// beta = z'.r' / z.r (Fletcher-Reeves form of the reference).  Flexible PCG
-// (the preconditioner is not a fixed linear map): beta = z'.(r' - r) / z.r
+// The learned multigrid V-cycle (fsim_mg.hip), whose coarsest level the network
+// solves, is not a fixed symmetric map: flexible PCG, beta = z'.(r' - r) / z.r
 // = -alpha z'.q / z.r, since r' - r = -alpha q.
-static int next_beta(fsim_ctx* ctx, bool flexible) {
-    if (flexible) FSIM_TRY(dot_with(ctx, ctx->z, ctx->q, FIN_ZQ));
-    return dot_zr(ctx, flexible ? FIN_FBETA : FIN_BETA);
+static int update_flexible(fsim_ctx* ctx, const SolveArgs& S, bool x_due) {
+    {
+        FSIM_PROF(ctx, KID_UPDATE);
+        const dim3 grid(stream_blocks(S.ncr)), block(kStream);
+        const Reduce red = reduce_to_host(ctx, FIN_RES);
+        if (x_due)
+            hipLaunchKernelGGL((k_update_r<kStream, true>), grid, block, 0, ctx->stream, S.ncr, ctx->chunk_flags, ctx->q, ctx->r,
+                               ctx->r, update_x_args(ctx), red);
+        else
+            hipLaunchKernelGGL((k_update_r<kStream, false>), grid, block, 0, ctx->stream, S.ncr, ctx->chunk_flags, ctx->q,
+                               ctx->r, ctx->r, UpdateX{}, red);
+        FSIM_HIP(ctx, hipGetLastError());
+    }
+    FSIM_TRY(mg_apply(ctx, ctx->r, ctx->z, S.scale));
+    FSIM_TRY(dot_with(ctx, ctx->z, ctx->q, FIN_ZQ));
+    return dot_with(ctx, ctx->z, ctx->r, FIN_FBETA);
+}
+// z = M^-1 r and sigma, at the start and after a restart
+static int precondition(fsim_ctx* ctx, const SolveArgs& S, const float* r, bool flexible) {
+    if (flexible) {
+        FSIM_TRY(mg_apply(ctx, ctx->r, ctx->z, S.scale));
+        return dot_with(ctx, ctx->z, ctx->r, FIN_SIGMA0);
+    }
+    SideWork bwd;
+    bwd.blocks = side_blocks(S.ncr);
+    bwd.n = S.ncr;
+    bwd.flags = ctx->chunk_flags;
+    bwd.t = ctx->t;
+    bwd.red = reduce_to(ctx, FIN_SIGMA0);
+    return mic_apply(ctx, S, r, ctx->t, ctx->z, nullptr, &bwd);
 }
 
 struct PcgResult {
@@ -990,55 +818,36 @@ struct PcgResult {
 // the direction instead, with beta from the replaced residual, was measured:
 // 185 iterations against 145 at the 256^3 double dam break, 1e-6.)
 //
-// One host round trip per iteration: the iteration's scalars are copied after
-// the r update, and the next preconditioner application and its dots run
-// while the host waits for them.  If the solve stops or restarts, those
-// results are discarded.  x += alpha s runs with the r update, or on the
-// second stream beside it and the preconditioner, and is joined before the
-// next direction step.
+// One host round trip per iteration: the r update's finishing block writes the
+// scalars for the host, and the preconditioner application and beta run while
+// the host waits for them.  If the solve stops or restarts, those results are
+// discarded.
 static int pcg_run(fsim_ctx* ctx, const SolveArgs& S, double bnorm, bool flexible, int max_it, PcgResult* res) {
-    const JoinXOnExit join_on_exit{ctx};
     const int64_t n = S.ncr;
     fsim_step_stats& st = ctx->stats;
-    FSIM_TRY(fill_f64(ctx, ctx->x, 0.0, n));
-    hipLaunchKernelGGL(k_copy_f32, dim3(nblocks(n)), dim3(kBlock), 0, ctx->stream, n, ctx->b, ctx->r);
-    FSIM_TRY(fill_f32(ctx, ctx->q, 0.0f, n));
-    FSIM_TRY(fill_f32(ctx, ctx->z, 0.0f, n));
-    FSIM_TRY(fill_f32(ctx, ctx->s, 0.0f, n));
-    FSIM_TRY(fill_f32(ctx, ctx->s2, 0.0f, n));
-    FSIM_TRY(precondition(ctx, S, flexible));
-    FSIM_TRY(dot_zr(ctx, FIN_SIGMA0));
+    float *r = ctx->r, *r_next = ctx->r_next;   // flexible: r stays where the V-cycle's graph reads it
+    {
+        // t and r_next as well: the sweeps leave out the tiles without WATER, and the cells there are summed
+        const SolveStart A{n, ctx->b, r, ctx->x,
+                           {ctx->q, ctx->z, ctx->s, ctx->s2, flexible ? nullptr : ctx->t, flexible ? nullptr : r_next}};
+        hipLaunchKernelGGL(k_solve_start, dim3(std::min(nblocks(n / 4), kMaxParts)), dim3(kBlock), 0, ctx->stream, A);
+        FSIM_HIP(ctx, hipGetLastError());
+    }
+    FSIM_TRY(precondition(ctx, S, r, flexible));
     const int max_reliable = 64;
     const double kDelta = ctx->reliable_drop > 0 ? std::pow(10.0, -ctx->reliable_drop) : 0.0;
     double last_true = bnorm;
     bool copy = true;
     int it = 0;
-    const bool x_inline = flexible || n <= kInlineX;
     int behind = 0;   // direction steps that x does not hold yet (0 or 1 between iterations)
     res->converged = false;
     res->nan = false;
     for (; it < max_it; it++) {
-        FSIM_TRY(join_x(ctx));
         FSIM_TRY(direction_step(ctx, S, copy));
-        // x takes two steps at a time: it is read and written half as often (both s buffers still hold
-        // their step)
         const bool two = ++behind == 2;
         if (two) behind = 0;
-        if (two && !x_inline) FSIM_TRY(update_x_beside(ctx, 2));
-        {
-            FSIM_PROF(ctx, KID_UPDATE);
-            const dim3 grid(stream_blocks(n)), block(kStream);
-            const Reduce red = reduce_to_host(ctx, FIN_RES);
-            if (two && x_inline)
-                hipLaunchKernelGGL(k_update_r<true>, grid, block, 0, ctx->stream, n, ctx->chunk_flags, ctx->q, ctx->r,
-                                   update_x_args(ctx), red);
-            else
-                hipLaunchKernelGGL(k_update_r<false>, grid, block, 0, ctx->stream, n, ctx->chunk_flags, ctx->q, ctx->r,
-                                   UpdateX{}, red);
-        }
-        FSIM_HIP(ctx, hipGetLastError());
-        FSIM_TRY(precondition(ctx, S, flexible));
-        FSIM_TRY(next_beta(ctx, flexible));
+        if (flexible) FSIM_TRY(update_flexible(ctx, S, two));
+        else FSIM_TRY(update_mic(ctx, S, &r, &r_next, two));
         SolveScalars h;
         FSIM_TRY(wait_scalars(ctx, &h));
         // the previous iteration's old-sigma test, then this iteration's alpha test
@@ -1053,11 +862,10 @@ static int pcg_run(fsim_ctx* ctx, const SolveArgs& S, double bnorm, bool flexibl
         }
         bool restart = false;
         if (stop_met(ctx, h.rr, h.rmax, bnorm) || std::sqrt(h.rr) < kDelta * last_true) {
-            if (behind) FSIM_TRY(update_x_beside(ctx, 1));
+            if (behind) FSIM_TRY(update_x_last(ctx));
             behind = 0;
-            FSIM_TRY(join_x(ctx));
             const bool replace = st.reliable_updates < max_reliable;
-            FSIM_TRY(true_residual(ctx, S, replace));
+            FSIM_TRY(true_residual(ctx, S, r, replace));
             FSIM_TRY(read_scalars(ctx));
             if (stop_met(ctx, ctx->scal_host->tr_ss, ctx->scal_host->tr_max, bnorm)) {
                 res->converged = true;
@@ -1071,14 +879,10 @@ static int pcg_run(fsim_ctx* ctx, const SolveArgs& S, double bnorm, bool flexibl
                 restart = true;
             }
         }
-        if (restart) {
-            FSIM_TRY(precondition(ctx, S, flexible));
-            FSIM_TRY(dot_zr(ctx, FIN_SIGMA0));
-        }
+        if (restart) FSIM_TRY(precondition(ctx, S, r, flexible));
         copy = restart;
     }
-    if (behind) FSIM_TRY(update_x_beside(ctx, 1));
-    FSIM_TRY(join_x(ctx));
+    if (behind) FSIM_TRY(update_x_last(ctx));
     res->iterations = it;
     return FSIM_OK;
 }
@@ -1226,7 +1030,7 @@ int stage_solve(fsim_ctx* ctx, double dt) {
     st.num_fluid_cells = (int64_t)ctx->scal_host->nfluid;
     if (bb < 1e-7) {   // early exit without pressure (bridsonSolverGrid.cpp:254-258)
         st.early_exit = 1;
-        FSIM_TRY(true_residual(ctx, S, false));
+        FSIM_TRY(true_residual(ctx, S, ctx->r, false));
         FSIM_TRY(read_scalars(ctx));
         st.residual_abs_inf = ctx->scal_host->tr_max;
         st.residual_rel_l2 = 1.0;
@@ -1273,7 +1077,7 @@ int stage_solve(fsim_ctx* ctx, double dt) {
                            ctx->u2, ctx->v2, ctx->w2, sc);
     }
     FSIM_HIP(ctx, hipGetLastError());
-    FSIM_TRY(true_residual(ctx, S, false));
+    FSIM_TRY(true_residual(ctx, S, ctx->r, false));
     FSIM_TRY(read_scalars(ctx));
     st.residual_abs_inf = ctx->scal_host->tr_max;
     st.residual_rel_l2 = bnorm > 0 ? std::sqrt(ctx->scal_host->tr_ss) / bnorm : 0.0;
@@ -1350,8 +1154,9 @@ int solver_apply(fsim_ctx* ctx, int op, double dt, const double* in, double* out
         FSIM_HIP(ctx, hipMemcpyAsync(hout.data(), ctx->q, sizeof(float) * n, hipMemcpyDeviceToHost, ctx->stream));
     } else if (op == FSIM_OP_APPLY_MIC0) {
         FSIM_TRY(mic_factor(ctx, S));
+        FSIM_TRY(fill_f32(ctx, ctx->t, 0.0f, n));
         FSIM_TRY(fill_f32(ctx, ctx->z, 0.0f, n));
-        FSIM_TRY(mic_apply(ctx, S, ctx->r, ctx->z, ctx->z));
+        FSIM_TRY(mic_apply(ctx, S, ctx->r, ctx->t, ctx->z));
         FSIM_TRY(check_wave_err(ctx));
         FSIM_HIP(ctx, hipMemcpyAsync(hout.data(), ctx->z, sizeof(float) * n, hipMemcpyDeviceToHost, ctx->stream));
     } else if (op == FSIM_OP_APPLY_MG) {

@@ -62,6 +62,14 @@
 // waves' prefetch stream (kPrefetch groups ahead, each prefetch slot in fixed
 // registers).
 //
+// Side work.  At most a tile per compute unit runs, and the tiles wait most of
+// the time: blocks behind the tiles' do the iteration's streaming passes
+// (SideWork) beside them.  The forward sweep of an iteration computes r - alpha
+// q itself while they store it: a third load a row, 46 instead of 43 us at
+// 128^3, 164 instead of 132 at 256^3, where the tiles are bound by their memory
+// accesses (a separate pass takes 13 and 35).  The backward sweep with t . t
+// takes 44 (44) and 129 (126), with the x update as well 44 and 160.
+//
 // Every wait is bounded: past kSpinLimit polls, or as soon as any wave in the
 // grid has given up, a wave raises the error flag and carries on, so the
 // grid always drains.  Workgroups take tiles from a ticket counter in
@@ -71,7 +79,7 @@
 
 #include <type_traits>
 
-#include "fsim_internal.hpp"
+#include "fsim_reduce.hpp"
 
 namespace fsim {
 
@@ -92,9 +100,9 @@ constexpr int kDeviceScope = 16;              // sc1 of a buffer access: past th
 constexpr int kVolatile = (int)0x80000000;    // a buffer load that is neither merged nor moved
 
 template <int KIND>
-struct Kind {   // 1 = forward sweep, 2 = backward sweep (FP32)
+struct Kind {   // WaveKind: the sweeps (FP32)
     using T = float;
-    static constexpr bool FWD = KIND == 1;
+    static constexpr bool FWD = KIND == WAVE_FWD || KIND == WAVE_FWD_UPDATE;
     static constexpr int NP = 1;     // 32-bit words per value
 };
 template <>
@@ -433,12 +441,13 @@ __device__ void send_wave(const WaveArgs& A, WaveLds<KIND>& S, const Tile& T) {
 // LAST: the tile's last wave, whose last row is the +y edge: it stores the packets itself, which
 // spares the edge a round trip through LDS and another wave.
 template <int KIND, bool LAST>
-__device__ __forceinline__ void compute_wave(const WaveArgs& A, WaveLds<KIND>& S, const Tile& T) {
+__device__ __forceinline__ void compute_wave(const WaveArgs& A, const SideWork& W, WaveLds<KIND>& S, const Tile& T) {
 #pragma clang fp contract(off)
     using KD = Kind<KIND>;
     using V = typename KD::T;
     constexpr bool FWD = KD::FWD;
     constexpr int NP = KD::NP, R = WF_R;
+    constexpr bool UPD = KIND == WAVE_FWD_UPDATE;
     const int w = LAST ? WF_NW - 1 : __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const int tz = threadIdx.x % 64;
     const uint32_t cells = (uint32_t)(A.ny * A.nz);   // of one plane
@@ -446,23 +455,26 @@ __device__ __forceinline__ void compute_wave(const WaveArgs& A, WaveLds<KIND>& S
     // byte offsets are counted for the float vectors: 16 per (y, z) column and group
     const uint32_t gstride = cells * 16u, total = gstride * ngroups;
     // buffer resources.  sweeps: rA P32, rB in, rC out; factor: rA nbinfo (offsets halved), rC P32
-    __amdgpu_buffer_rsrc_t rA, rB, rC;
+    __amdgpu_buffer_rsrc_t rA, rB, rC, rQ;
     if constexpr (KIND == 0) {
         rA = rsrc(A.nbinfo, (int64_t)total / 2);
         rC = rsrc(A.P32, (int64_t)total);
-        rB = rA;
+        rB = rQ = rA;
     } else {
         // ranges one and two words longer than the arrays (never addressed): distinct descriptor
         // words keep the compiler from rebuilding one descriptor from another at every access
         rA = rsrc(A.P32, (int64_t)total + 8);
         rB = rsrc(A.in, (int64_t)total);
         rC = rsrc(A.out, (int64_t)total + 4);
+        rQ = UPD ? rsrc(W.q, (int64_t)total + 12) : rA;
         // opaque to the compiler from here on, so that it keeps each descriptor whole in
         // four SGPRs instead of sharing equal words and reassembling them at every access
         asm volatile("" : "+s"(rA), "+s"(rB), "+s"(rC));
+        if constexpr (UPD) asm volatile("" : "+s"(rQ));
     }
     const float ms = A.ms;
     const double scale = A.scale;
+    const float malpha = UPD ? (float)(-W.red.sc->alpha) : 0.f;
     const int z = z_of<FWD>(A, T.K, tz);
     const int rho = FWD ? tz : WF_TZ - 1 - tz;   // rot(z)
     uint32_t off[R];                             // the lane's byte offset per row, kOob off the grid
@@ -498,7 +510,7 @@ __device__ __forceinline__ void compute_wave(const WaveArgs& A, WaveLds<KIND>& S
     uint32_t op = __builtin_amdgcn_readfirstlane((uint32_t)T.m.g0 % ngroups * gstride);   // prefetched group's offset
     // inputs of the next kPrefetch groups, with the offsets they were loaded from: the result of a
     // group goes to the same place of another vector.  factor: nbinfo; sweeps: P32 and the input vector
-    f32x4 pq[kRing][R], iq[kRing][R];
+    f32x4 pq[kRing][R], iq[kRing][R], uq[kRing][R];
     u32x2 nq[kRing][R];
     uint32_t lo[kRing][R], go[kRing];
     auto fetch = [&](auto dc, int g) {
@@ -514,6 +526,7 @@ __device__ __forceinline__ void compute_wave(const WaveArgs& A, WaveLds<KIND>& S
             } else {
                 pq[d][r] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rA, o, op, 0));
                 iq[d][r] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rB, o, op, 0));
+                if constexpr (UPD) uq[d][r] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rQ, o, op, 0));
             }
         });
         advance(op);
@@ -604,6 +617,8 @@ __device__ __forceinline__ void compute_wave(const WaveArgs& A, WaveLds<KIND>& S
                     prev[r] = v;
                 } else {
                     const float p = pq[d][r][e];
+                    float in = iq[d][r][e];
+                    if constexpr (UPD) in = __builtin_fmaf(uq[d][r][e], malpha, in);
                     // -z: the packet's value on lane 0 (+0 on the others), lane tz - 1's on the others (+0 on
                     // lane 0): their sum is the one that counts
                     const float vz = zp[r].get(j) + Group<V>::shr1(prev[r]);
@@ -611,10 +626,10 @@ __device__ __forceinline__ void compute_wave(const WaveArgs& A, WaveLds<KIND>& S
                     acc += vz;
                     float outv, v;
                     if (FWD) {
-                        outv = (iq[d][r][e] - acc) * p;
+                        outv = (in - acc) * p;
                         v = outv * p;
                     } else {
-                        outv = (iq[d][r][e] - acc * p) * p;
+                        outv = (in - acc * p) * p;
                         v = outv;
                     }
                     res[r][e] = outv;
@@ -680,9 +695,20 @@ __device__ __forceinline__ void compute_wave(const WaveArgs& A, WaveLds<KIND>& S
 }
 
 template <int KIND>
-__global__ void __launch_bounds__(WF_THREADS) k_wave(WaveArgs A) {
+__global__ void __launch_bounds__(WF_THREADS) k_wave(WaveArgs A, SideWork W) {
     using KD = Kind<KIND>;
     constexpr int NP = KD::NP;
+    const unsigned tiles = gridDim.x - W.blocks;
+    if (KIND >= WAVE_BWD && blockIdx.x >= tiles) {
+        const Part part{blockIdx.x - tiles, W.blocks};
+        if constexpr (KIND == WAVE_FWD_UPDATE) {
+            update_r<WF_THREADS>(part, W.n, W.flags, W.q, W.r, W.r_next, W.red);
+        } else {
+            dot_self<WF_THREADS>(part, W.n, W.flags, W.t, W.red);
+            if (W.x_steps == 2) update_x_chunks<2>(part, W.n, W.flags, W.x, W.red.sc);
+        }
+        return;
+    }
     __shared__ WaveLds<KIND> S;
     const int tile = take_tile(A);
     if (tile < 0) return;
@@ -737,27 +763,34 @@ __global__ void __launch_bounds__(WF_THREADS) k_wave(WaveArgs A) {
     }
     __syncthreads();
     const int wave = threadIdx.x / 64;
-    if (wave < WF_NW - 1) compute_wave<KIND, false>(A, S, T);
-    else if (wave == WF_NW - 1) compute_wave<KIND, true>(A, S, T);
+    if (wave < WF_NW - 1) compute_wave<KIND, false>(A, W, S, T);
+    else if (wave == WF_NW - 1) compute_wave<KIND, true>(A, W, S, T);
     else if (wave == WF_NW) recv_wave<KIND, true>(A, S, T);
     else if (wave == WF_NW + 1) recv_wave<KIND, false>(A, S, T);
     else send_wave<KIND>(A, S, T);
 }
 
-int wave_launch(fsim_ctx* ctx, int kind, const float* in, float* out, double scale) {
+int wave_launch(fsim_ctx* ctx, WaveKind kind, const float* in, float* out, double scale, const SideWork* side) {
     WaveArgs A = ctx->wave;
     A.in = in;
     A.out = out;
     A.scale = scale;
     A.ms = -(float)scale;
     const unsigned ntiles = (unsigned)(A.TJ * A.TK);
-    A.ticket = ctx->wave_ticket + kind;
-    A.ticket_base = ctx->wave_ticket_base[kind];
-    ctx->wave_ticket_base[kind] += ntiles;
+    const int counter = kind == WAVE_FWD_UPDATE ? WAVE_FWD : kind;
+    A.ticket = ctx->wave_ticket + counter;
+    A.ticket_base = ctx->wave_ticket_base[counter];
+    ctx->wave_ticket_base[counter] += ntiles;
     A.send_delay = ctx->wave_send_delay;
-    if (kind == 0) hipLaunchKernelGGL(k_wave<0>, dim3(ntiles), dim3(WF_THREADS), 0, ctx->stream, A);
-    else if (kind == 1) hipLaunchKernelGGL(k_wave<1>, dim3(ntiles), dim3(WF_THREADS), 0, ctx->stream, A);
-    else hipLaunchKernelGGL(k_wave<2>, dim3(ntiles), dim3(WF_THREADS), 0, ctx->stream, A);
+    // the blocks beside the tiles come last: the tiles, which wait for each other, start first
+    const SideWork W = side ? *side : SideWork{};
+    const dim3 grid(ntiles + W.blocks), block(WF_THREADS);
+    switch (kind) {
+    case WAVE_FACTOR: hipLaunchKernelGGL(k_wave<WAVE_FACTOR>, grid, block, 0, ctx->stream, A, W); break;
+    case WAVE_FWD: hipLaunchKernelGGL(k_wave<WAVE_FWD>, grid, block, 0, ctx->stream, A, W); break;
+    case WAVE_BWD: hipLaunchKernelGGL(k_wave<WAVE_BWD>, grid, block, 0, ctx->stream, A, W); break;
+    case WAVE_FWD_UPDATE: hipLaunchKernelGGL(k_wave<WAVE_FWD_UPDATE>, grid, block, 0, ctx->stream, A, W); break;
+    }
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;
 }

@@ -122,3 +122,36 @@ def test_solve_fields_at_group_edges(gpu, shape):
     largest = max(np.abs(v).max() for v in after + faces)
     left = rhs(after)
     assert np.abs(left).max() <= 12 * 2.0 ** -24 * largest / grid.cell_d + 1e-9 * np.linalg.norm(b)
+
+
+# one block beside the tiles, several, and more chunks of values than these blocks take in one trip
+@pytest.mark.parametrize("shape", [(5, 6, 7), (30, 17, 66), (67, 40, 70), (40, 260, 300)])
+def test_solve_beside_the_sweeps(gpu, shape):
+    """The residual, its norms, sigma and the pressure updated by the blocks beside the sweeps' tiles: the same bits
+    as with kernels of their own around one launch per plane, over solves that stop, restart and run out."""
+    print(f"case: side work of the sweeps on {shape}", flush=True)
+    grid = capi.Grid(*shape, 1.0 / 32, 0.25 / 32)
+    lab = _labels(shape, 1, max(3, shape[0] - 2), sum(shape))
+    rng = np.random.default_rng(4)
+    faces = [rng.standard_normal(shape).astype(np.float32) for _ in range(3)]
+    got = {}
+    for mode in (1, 0):
+        sim = capi.Simulation(grid, scenes.params(tol=1e-6))
+        sim.set_option(capi.OPT_SWEEP_MODE, mode)
+        sim.set_grid(capi.FIELD_LABEL, lab.reshape(-1))
+        got[mode] = []
+        for most in (500, 4, 3):
+            prm = scenes.params(tol=1e-6)
+            prm.max_iterations = most
+            sim.set_params(prm)
+            for f, v in zip((capi.FIELD_U2, capi.FIELD_V2, capi.FIELD_W2), faces):
+                sim.set_grid(f, v.reshape(-1))
+            sim.run_stage(capi.STAGE_SOLVE, DT)
+            st = sim.stats()
+            got[mode].append((st.pcg_iterations, st.reliable_updates, st.residual_rel_l2, sim.get_grid(capi.FIELD_PRESSURE)))
+        sim.close()
+    for a, b in zip(got[0], got[1]):
+        assert a[:3] == b[:3]
+        assert np.array_equal(a[3], b[3])
+    # 500 iterations suffice; the others run out, with x one step behind on the odd one
+    assert got[0][0][2] <= 1e-6 and got[0][1][0] <= 4 and got[0][2][0] <= 3
