@@ -111,6 +111,7 @@ static void free_all(fsim_ctx* ctx) {
     learned_free(ctx);
     mg_free(ctx);
     gfx_free(ctx);
+    readback_free(ctx);
     void* ptrs[] = {ctx->P.base, ctx->Palt.base, ctx->key, ctx->rank, ctx->perm, ctx->removed, ctx->u, ctx->v, ctx->w,
                     ctx->u2, ctx->v2, ctx->w2, ctx->label, ctx->valid, ctx->density, ctx->cell_count, ctx->cell_start,
                     ctx->scan_tmp, ctx->nbinfo, ctx->b, ctx->r, ctx->z, ctx->s, ctx->q, ctx->P32, ctx->P64,
@@ -154,6 +155,7 @@ int fsim_create(const fsim_grid_desc* grid, const fsim_params* params, fsim_ctx*
     if (hipGetDeviceCount(&ndev) != hipSuccess || ndev <= 0) return FSIM_ERR_NO_DEVICE;
     fsim_ctx* ctx = new (std::nothrow) fsim_ctx();
     if (!ctx) return FSIM_ERR_OOM;
+    readback_init(ctx);
     auto fail = [&](int rc) {
         free_all(ctx);
         delete ctx;
@@ -300,29 +302,7 @@ int fsim_get_particles(fsim_ctx* ctx, int64_t capacity, float* pos, float* vel, 
     if (!pos && !vel && !c) return FSIM_OK;
     if (capacity < n) return set_err(ctx, FSIM_ERR_INVALID, "capacity smaller than the particle count");
     FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    std::vector<int32_t> ids((size_t)n);
-    std::vector<float> plane((size_t)n);
-    if (n) FSIM_HIP(ctx, hipMemcpy(ids.data(), ctx->P.pid, sizeof(int32_t) * n, hipMemcpyDeviceToHost));
-    for (int64_t i = 0; i < n; i++)
-        if (ids[i] < 0 || ids[i] >= n) return set_err(ctx, FSIM_ERR_INVALID, "corrupt particle ids");
-    auto get = [&](const float* src, float* dst, int stride, int off) -> int {
-        if (!n) return FSIM_OK;
-        FSIM_HIP(ctx, hipMemcpy(plane.data(), src, sizeof(float) * n, hipMemcpyDeviceToHost));
-        for (int64_t i = 0; i < n; i++) dst[(int64_t)stride * ids[i] + off] = plane[i];
-        return FSIM_OK;
-    };
-    for (int a = 0; a < 3; a++) {
-        if (pos) FSIM_TRY(get(ctx->P.pos[a], pos, 3, a));
-        if (vel) FSIM_TRY(get(ctx->P.vel[a], vel, 3, a));
-    }
-    if (c) {
-        if (ctx->c_valid) {
-            for (int k = 0; k < 9; k++) FSIM_TRY(get(ctx->P.c[k], c, 9, k));
-        } else {
-            std::memset(c, 0, sizeof(float) * 9 * n);
-        }
-    }
-    return FSIM_OK;
+    return particles_out(ctx, pos, vel, c);
 }
 
 int fsim_set_obstacles(fsim_ctx* ctx, int n, const fsim_obstacle* obs) {
@@ -469,8 +449,7 @@ int fsim_get_grid(fsim_ctx* ctx, int field, void* dst, size_t bytes) {
     FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
     const bool rotated = field == FSIM_FIELD_PRESSURE || field == FSIM_FIELD_RHS || field == FSIM_FIELD_PRECON;
     if (!rotated) {
-        FSIM_HIP(ctx, hipMemcpy(dst, src, need, hipMemcpyDeviceToHost));
-        return FSIM_OK;
+        return read_back(ctx, dst, src, need);
     }
     // solver vectors are stored in the rotated layout: gather into flat order
     const size_t elem = need / nc;

@@ -115,11 +115,12 @@ static GfxArgs gfx_args(fsim_ctx* ctx, fsim_gfx_particle* dev_out) {
     return A;
 }
 
-static int gfx_run(fsim_ctx* ctx, fsim_gfx_particle* staging, fsim_gfx_particle* host_out) {
+static int gfx_run(fsim_ctx* ctx, fsim_gfx_particle* staging, fsim_gfx_particle* host_out, bool alloc) {
     const int64_t n = ctx->P.n;
     if (n == 0) return FSIM_OK;
     hipLaunchKernelGGL(k_gfx_snapshot, dim3(nblocks(n)), dim3(kBlock), 0, ctx->stream, gfx_args(ctx, staging));
     FSIM_HIP(ctx, hipGetLastError());
+    if (alloc) return read_back(ctx, host_out, staging, sizeof(fsim_gfx_particle) * (size_t)n);
     FSIM_HIP(ctx, hipMemcpyAsync(host_out, staging, sizeof(fsim_gfx_particle) * (size_t)n, hipMemcpyDeviceToHost,
                                  ctx->stream));
     FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -139,7 +140,7 @@ int gfx_snapshot(fsim_ctx* ctx, fsim_gfx_particle* host_out) {
         ctx->gfx_staging = buf;
         ctx->gfx_cap = cap;
     }
-    return gfx_run(ctx, ctx->gfx_staging, host_out);
+    return gfx_run(ctx, ctx->gfx_staging, host_out, true);
 }
 
 // The same kernel and copy with the staging in this GPU's scratch array:
@@ -155,7 +156,7 @@ int gfx_snapshot_noalloc(fsim_ctx* ctx, fsim_gfx_particle* host_out) {
         p = g_scratch[ctx->device];
     }
     if (!p) return set_err(ctx, FSIM_ERR_INVALID, "scratch address of this device was not resolved");
-    return gfx_run(ctx, static_cast<fsim_gfx_particle*>(p), host_out);
+    return gfx_run(ctx, static_cast<fsim_gfx_particle*>(p), host_out, false);
 }
 
 void gfx_free(fsim_ctx* ctx) {

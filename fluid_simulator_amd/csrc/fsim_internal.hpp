@@ -27,6 +27,7 @@ namespace fsim {
 
 constexpr int kMaxObstacles = 64;
 constexpr int kBlock = 256;
+constexpr int kReadSlots = 12;         // pinned slots of read_back
 constexpr unsigned kMaxParts = 2048;   // reduction grids have at most this many blocks
 
 // nbinfo bit layout
@@ -355,6 +356,9 @@ struct fsim_ctx {
     fsim_gfx_particle* gfx_staging = nullptr;
     int64_t gfx_cap = 0;
 
+    hipEvent_t rb_ev[fsim::kReadSlots] = {};   // read_back: a pinned slot is filled
+    bool rb_counted = false;
+
     // obstacles
     std::vector<fsim_obstacle> obs;
     fsim_obstacle* obs_dev = nullptr;
@@ -447,6 +451,14 @@ int gfx_snapshot_noalloc(fsim_ctx* ctx, fsim_gfx_particle* host_out);
 int scratch_init(fsim_ctx* ctx);
 int64_t scratch_particles();
 void gfx_free(fsim_ctx* ctx);
+
+// ---- results to host memory (fsim_readback.hip) ------------------------------
+// dst = src after the stream's work so far; returns when dst is complete
+int read_back(fsim_ctx* ctx, void* dst, const void* src, size_t bytes);
+// positions, velocities and C in the reference's particle order; each may be null
+int particles_out(fsim_ctx* ctx, float* pos, float* vel, float* c);
+void readback_init(fsim_ctx* ctx);
+void readback_free(fsim_ctx* ctx);
 
 // ---- multigrid of the learned preconditioner (fsim_mg.hip) ------------------
 int mg_levels_for(int nx, int ny, int nz);
