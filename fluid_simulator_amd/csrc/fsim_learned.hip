@@ -96,7 +96,12 @@ struct ConvArgs {
     int64_t part_cap;     // floats in part
 };
 
-template <int CIN, int CU, int NT, int MT, bool OUT_F32>
+// AHEAD: K chunks whose operands are loaded before the first one's product.  A
+// chunk's loads take about a microsecond (weights and activations come from
+// the L2), and a wave of a small level has nobody beside it to hide that.
+// us at 16^3, with four voxel tiles a wave and two chunks ahead before: 8 -> 16
+// 11.8 -> 6.1, 16 -> 32 19.1 -> 11.4, 48 -> 16 7.9 -> 5.8, 192 -> 64 7.6 -> 6.2.
+template <int CIN, int CU, int NT, int MT, int AHEAD, bool OUT_F32>
 __global__ void __launch_bounds__(256) k_conv3(ConvArgs a) {
     constexpr int KTOT = 27 * CIN;
     constexpr int NCH = (KTOT + 31) / 32;
@@ -131,31 +136,43 @@ __global__ void __launch_bounds__(256) k_conv3(ConvArgs a) {
     // split K: block z sums the K chunks of its slice (one slice: all of them)
     const int cps = (NCH + (int)gridDim.z - 1) / (int)gridDim.z;
     const int c_lo = (int)blockIdx.z * cps, c_hi = min(NCH, c_lo + cps);
-#pragma unroll 2
-    for (int c = c_lo; c < c_hi; c++) {
-        const int k0 = 32 * c + 8 * kq;
-        const bool kin = (KTOT % 32 == 0) || k0 < KTOT;
-        const int t = k0 / CIN, ci = k0 - t * CIN;
-        const int dx = t / 9 - 1, dy = (t / 3) % 3 - 1, dz = t % 3 - 1;
-        const bool up = CU > 0 && ci < CU;
-        const int64_t toff = (((int64_t)dx * a.H + dy) * a.W + dz) * CS + (ci - CU);
-        bf16x8 av[MT], bv[NT];
+    for (int cb = c_lo; cb < c_hi; cb += AHEAD) {
+        bf16x8 av[AHEAD][MT], bv[AHEAD][NT];
 #pragma unroll
-        for (int m = 0; m < MT; m++) {
-            const int xx = xs[m] + dx, yy = ys[m] + dy, zz = zs[m] + dz;
-            const bool ok = kin && rin[m] && (unsigned)xx < (unsigned)a.D && (unsigned)yy < (unsigned)a.H &&
-                            (unsigned)zz < (unsigned)a.W;
-            const __bf16* src = xl[m] + toff;
-            if (up) src = a.xc + (((int64_t)(xx >> 1) * Hc + (yy >> 1)) * Wc + (zz >> 1)) * (CU > 0 ? CU : 1) + ci;
-            av[m] = ok ? *reinterpret_cast<const bf16x8*>(src) : zero;
+        for (int u = 0; u < AHEAD; u++) {
+            const int c = cb + u;
+            const int k0 = 32 * c + 8 * kq;
+            const bool kin = c < c_hi && ((KTOT % 32 == 0) || k0 < KTOT);
+            const int t = k0 / CIN, ci = k0 - t * CIN;
+            const int dx = t / 9 - 1, dy = (t / 3) % 3 - 1, dz = t % 3 - 1;
+            const bool up = CU > 0 && ci < CU;
+            const int64_t toff = (((int64_t)dx * a.H + dy) * a.W + dz) * CS + (ci - CU);
+#pragma unroll
+            for (int m = 0; m < MT; m++) {
+                const int xx = xs[m] + dx, yy = ys[m] + dy, zz = zs[m] + dz;
+                const bool ok = kin && rin[m] && (unsigned)xx < (unsigned)a.D && (unsigned)yy < (unsigned)a.H &&
+                                (unsigned)zz < (unsigned)a.W;
+                const __bf16* src = xl[m] + toff;
+                if (up) src = a.xc + (((int64_t)(xx >> 1) * Hc + (yy >> 1)) * Wc + (zz >> 1)) * (CU > 0 ? CU : 1) + ci;
+                // a lane without a value reads the weights' first ones, so that no load waits for a branch
+                const bf16x8 got = *reinterpret_cast<const bf16x8*>(ok ? src : a.w);
+                av[u][m] = ok ? got : zero;
+            }
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                const bf16x8 got = *reinterpret_cast<const bf16x8*>(kin ? wl + (int64_t)16 * j * KTOT + 32 * c : a.w);
+                bv[u][j] = kin ? got : zero;
+            }
         }
 #pragma unroll
-        for (int j = 0; j < NT; j++)
-            bv[j] = kin ? *reinterpret_cast<const bf16x8*>(wl + (int64_t)16 * j * KTOT + 32 * c) : zero;
+        for (int u = 0; u < AHEAD; u++) {
+            if (cb + u >= c_hi) break;
 #pragma unroll
-        for (int m = 0; m < MT; m++)
+            for (int m = 0; m < MT; m++)
 #pragma unroll
-            for (int j = 0; j < NT; j++) acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], bv[j], acc[m][j], 0, 0, 0);
+                for (int j = 0; j < NT; j++)
+                    acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[u][m], bv[u][j], acc[m][j], 0, 0, 0);
+        }
     }
     if (gridDim.z > 1) {   // raw partial sums; k_conv3_reduce adds the slices, bias and ReLU
         float* P = a.part + (int64_t)blockIdx.z * V * a.cout;
@@ -188,14 +205,30 @@ __global__ void __launch_bounds__(256) k_conv3(ConvArgs a) {
     }
 }
 
+// The sum of `count` values `stride` apart, in order, kSumAhead loads at a time: a
+// loop that adds each value as it comes takes a memory latency per value (54
+// slices 17 us, in batches 5).
+constexpr int kSumAhead = 16;
+__device__ inline float sum_in_order(const float* p, int64_t stride, int count) {
+    float s = 0.f;
+    for (int k = 0; k < count; k += kSumAhead) {
+        float v[kSumAhead];
+#pragma unroll
+        for (int j = 0; j < kSumAhead; j++) v[j] = p[(int64_t)min(k + j, count - 1) * stride];
+#pragma unroll
+        for (int j = 0; j < kSumAhead; j++)
+            if (k + j < count) s += v[j];
+    }
+    return s;
+}
+
 // Sum of the split-K slices in slice order, then bias and ReLU (deterministic).
 template <bool OUT_F32>
 __global__ void __launch_bounds__(256) k_conv3_reduce(ConvArgs a, int slices) {
     const int64_t n = (int64_t)a.D * a.H * a.W * a.cout;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    float s = 0.f;
-    for (int k = 0; k < slices; k++) s += a.part[k * n + i];
+    const float s = sum_in_order(a.part + i, n, slices);
     float o = s + (a.bias ? a.bias[i % a.cout] : 0.f);
     if (a.relu) o = fmaxf(o, 0.f);
     if (OUT_F32) static_cast<float*>(a.y)[i] = o;
@@ -210,6 +243,7 @@ __global__ void __launch_bounds__(256) k_conv3_reduce(ConvArgs a, int slices) {
 // split: the reduction's launch costs more than their short K loop (measured
 // at 16^3: 8 -> 16, 7 chunks, 10.0 us unsplit, 7.6 + 7.3 us split).
 constexpr int64_t kSplitWaves = 1024;
+constexpr int64_t kSmallWaves = 4096;   // 4 waves a SIMD
 constexpr int kSplitMinChunks = 24;
 constexpr int64_t kConvPartFloats = int64_t(4) << 20;   // 16 MB of split-K partial sums per context
 template <int CIN, int CU, int COUT, int NT, int MT, bool OUT_F32>
@@ -226,8 +260,14 @@ static void conv3_launch(hipStream_t st, const ConvArgs& a) {
         const int64_t cps = (NCH + slices - 1) / slices;   // every slice gets at least one chunk
         slices = (NCH + cps - 1) / cps;
     }
-    hipLaunchKernelGGL((k_conv3<CIN, CU, NT, MT, OUT_F32>),
-                       dim3((unsigned)((waves + 3) / 4), COUT / (16 * NT), (unsigned)slices), dim3(256), 0, st, a);
+    // Few waves even so: a voxel tile a wave (the sums are the same), with more chunks of loads ahead than
+    // the registers of a large level's waves would hold.
+    if (all * slices * MT <= kSmallWaves)
+        hipLaunchKernelGGL((k_conv3<CIN, CU, NT, 1, NT <= 2 ? 7 : 4, OUT_F32>),
+                           dim3((unsigned)(((V + 15) / 16 + 3) / 4), COUT / (16 * NT), (unsigned)slices), dim3(256), 0, st, a);
+    else
+        hipLaunchKernelGGL((k_conv3<CIN, CU, NT, MT, 2, OUT_F32>),
+                           dim3((unsigned)((waves + 3) / 4), COUT / (16 * NT), (unsigned)slices), dim3(256), 0, st, a);
     if (slices > 1)
         hipLaunchKernelGGL((k_conv3_reduce<OUT_F32>), dim3((unsigned)((V * COUT + 255) / 256)), dim3(256), 0, st, a,
                            (int)slices);
@@ -678,18 +718,15 @@ __global__ void __launch_bounds__(256) k_conv3_wgrad(const __bf16* __restrict__ 
 __global__ void k_sum_parts(const float* __restrict__ parts, int nparts, int64_t n, float* __restrict__ out) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    float s = 0.f;
-    for (int p = 0; p < nparts; p++) s += parts[(int64_t)p * n + i];
-    out[i] = s;
+    out[i] = sum_in_order(parts + i, n, nparts);
 }
 
 // bias gradient: db[c] = sum_v g[v][c] (one block per channel, fixed order)
 __global__ void __launch_bounds__(256) k_bias_grad(const float* __restrict__ g, int64_t V, int C, float* __restrict__ db) {
     __shared__ float red[256];
     const int c = blockIdx.x;
-    float s = 0.f;
-    for (int64_t v = threadIdx.x; v < V; v += blockDim.x) s += g[v * C + c];
-    red[threadIdx.x] = s;
+    const int64_t mine = (int64_t)threadIdx.x < V ? (V - threadIdx.x + blockDim.x - 1) / blockDim.x : 0;
+    red[threadIdx.x] = mine > 0 ? sum_in_order(g + (int64_t)threadIdx.x * C + c, (int64_t)blockDim.x * C, (int)mine) : 0.f;
     __syncthreads();
     for (int off = 128; off > 0; off >>= 1) {
         if ((int)threadIdx.x < off) red[threadIdx.x] += red[threadIdx.x + off];

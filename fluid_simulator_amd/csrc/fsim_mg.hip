@@ -221,6 +221,35 @@ __global__ void __launch_bounds__(kBlock) k_mg_rbgs0(Mg0 A) {
     }
 }
 
+// The couplings and neighbour values of cell i in the order +x, -x, +y, -y, +z,
+// -z, all 12 loads issued together (a branch per coupling would wait for each
+// load in turn: a half-sweep 3.7 us at 64^3 and 7.8 at 128^3, so 3.1 and 5.0).
+// A coupling beyond the level's edge is 0, its x the cell's own.
+struct LevelTerms {
+    float o[6], x[6];
+};
+__device__ inline LevelTerms level_terms(const MgGrid& G, int x, int y, int z, int64_t i) {
+    const int64_t sx = (int64_t)G.ny * G.nz, sy = G.nz;
+    const int64_t mx = x > 0 ? i - sx : i, my = y > 0 ? i - sy : i, mz = z > 0 ? i - 1 : i;
+    LevelTerms t;
+    t.o[0] = G.ox[i];
+    t.o[1] = G.ox[mx];
+    t.o[2] = G.oy[i];
+    t.o[3] = G.oy[my];
+    t.o[4] = G.oz[i];
+    t.o[5] = G.oz[mz];
+    t.x[0] = G.x[x + 1 < G.nx ? i + sx : i];
+    t.x[1] = G.x[mx];
+    t.x[2] = G.x[y + 1 < G.ny ? i + sy : i];
+    t.x[3] = G.x[my];
+    t.x[4] = G.x[z + 1 < G.nz ? i + 1 : i];
+    t.x[5] = G.x[mz];
+    if (x == 0) t.o[1] = 0.f;
+    if (y == 0) t.o[3] = 0.f;
+    if (z == 0) t.o[5] = 0.f;
+    return t;
+}
+
 template <int PAR, bool FIRST>
 __global__ void __launch_bounds__(kMgBz * kMgBy) k_mg_rbgs(MgGrid G) {
     const int z = blockIdx.x * blockDim.x + threadIdx.x;
@@ -238,14 +267,9 @@ __global__ void __launch_bounds__(kMgBz * kMgBy) k_mg_rbgs(MgGrid G) {
     }
     float s = G.b[i];
     if (!FIRST) {
-        const int64_t sx = (int64_t)G.ny * G.nz, sy = G.nz;
-        float o;
-        if ((o = G.ox[i]) != 0.f) s += o * G.x[i + sx];
-        if (x > 0 && (o = G.ox[i - sx]) != 0.f) s += o * G.x[i - sx];
-        if ((o = G.oy[i]) != 0.f) s += o * G.x[i + sy];
-        if (y > 0 && (o = G.oy[i - sy]) != 0.f) s += o * G.x[i - sy];
-        if ((o = G.oz[i]) != 0.f) s += o * G.x[i + 1];
-        if (z > 0 && (o = G.oz[i - 1]) != 0.f) s += o * G.x[i - 1];
+        const LevelTerms t = level_terms(G, x, y, z, i);
+#pragma unroll
+        for (int j = 0; j < 6; j++) s = t.o[j] != 0.f ? s + t.o[j] * t.x[j] : s;
     }
     G.x[i] = s / d;
 }
@@ -321,34 +345,40 @@ __global__ void __launch_bounds__(256) k_mg_resid_restrict0(Mg0 A, MgGrid C) {
     }
 }
 
+// Levels >= 1: a thread per child, the eight of a coarse cell in consecutive
+// lanes, whose residuals the first sums in order.  A thread that took all
+// eight waited for 56 pairs of loads one after the other: 17.6 us from 64^3, so
+// 4.9; 21 us a level at 256^3, so 13.
 __global__ void __launch_bounds__(kBlock) k_mg_restrict(MgGrid F, MgGrid C) {
-    const int64_t I = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (I >= (int64_t)C.nx * C.ny * C.nz) return;
-    if (C.diag[I] == 0.f) {
-        C.b[I] = 0.f;
-        return;
-    }
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t n = (int64_t)C.nx * C.ny * C.nz;
+    const int64_t I = min(t >> 3, n - 1);   // every lane takes part in the exchange
+    const int k = (int)(t & 7);
     int X, Y, Z;
     unlin(I, C.ny, C.nz, X, Y, Z);
-    const int64_t sx = (int64_t)F.ny * F.nz, sy = F.nz;
-    float sum = 0.f;
-    for (int k = 0; k < 8; k++) {
-        const int x = 2 * X + (k >> 2), y = 2 * Y + ((k >> 1) & 1), z = 2 * Z + (k & 1);
-        if (x >= F.nx || y >= F.ny || z >= F.nz) continue;
+    const int x = 2 * X + (k >> 2), y = 2 * Y + ((k >> 1) & 1), z = 2 * Z + (k & 1);
+    bool on = x < F.nx && y < F.ny && z < F.nz;
+    float res = 0.f;
+    if (on) {
         const int64_t i = lin(F.nx, F.ny, F.nz, x, y, z);
-        const float d = F.diag[i];
-        if (d == 0.f) continue;
-        float ax = d * F.x[i];
-        float o;
-        if ((o = F.ox[i]) != 0.f) ax -= o * F.x[i + sx];
-        if (x > 0 && (o = F.ox[i - sx]) != 0.f) ax -= o * F.x[i - sx];
-        if ((o = F.oy[i]) != 0.f) ax -= o * F.x[i + sy];
-        if (y > 0 && (o = F.oy[i - sy]) != 0.f) ax -= o * F.x[i - sy];
-        if ((o = F.oz[i]) != 0.f) ax -= o * F.x[i + 1];
-        if (z > 0 && (o = F.oz[i - 1]) != 0.f) ax -= o * F.x[i - 1];
-        sum += F.b[i] - ax;
+        const float d = F.diag[i], own = F.x[i], b = F.b[i];
+        const LevelTerms v = level_terms(F, x, y, z, i);
+        on = d != 0.f;
+        float ax = d * own;
+#pragma unroll
+        for (int j = 0; j < 6; j++) ax = v.o[j] != 0.f ? ax - v.o[j] * v.x[j] : ax;
+        res = b - ax;
     }
-    C.b[I] = sum;
+    float sum = 0.f;
+    const uint64_t take = __ballot(on);
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        const int from = (lane & ~7) + c;
+        const float r = __shfl(res, from, 64);
+        if ((take >> from) & 1) sum += r;
+    }
+    if (k == 0 && (t >> 3) < n) C.b[I] = C.diag[I] == 0.f ? 0.f : sum;
 }
 
 // ---- prolongation: x_i += 1.6 x_{l+1}[parent(i)] on the level's unknowns ----------------
@@ -571,7 +601,7 @@ static int vcycle(fsim_ctx* ctx, const float* r, float* z, double scale) {
     }
     for (int l = 1; l < c; l++) {
         smooth(ctx, M->lv[l], kMgPreSweeps, true);
-        hipLaunchKernelGGL(k_mg_restrict, dim3(nblocks(M->lv[l + 1].nc)), dim3(kBlock), 0, ctx->stream,
+        hipLaunchKernelGGL(k_mg_restrict, dim3(nblocks(8 * M->lv[l + 1].nc)), dim3(kBlock), 0, ctx->stream,
                            grid_of(M->lv[l]), grid_of(M->lv[l + 1]));
     }
     FSIM_TRY(coarse_solve(ctx, A, c));
