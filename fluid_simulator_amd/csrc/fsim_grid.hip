@@ -294,30 +294,40 @@ __global__ void __launch_bounds__(kBlock) k_p2g_gather(P2GArgs A) {
 // (x, y) neighbourhood holds it.  Rows are staged in (x, y) order, so every
 // cell adds the rows of its neighbourhood in k_p2g_gather's (dx, dy) order,
 // and each row's particles in sorted order, with the same arithmetic: the
-// sums are bit-identical.  It serves APIC; PIC and FLIP take k_p2g_tile_w.
-#ifndef FSIM_P2G_TX
-#define FSIM_P2G_TX 2
-#endif
-#ifndef FSIM_P2G_TY
-#define FSIM_P2G_TY 4
-#endif
-constexpr int P2G_TX = FSIM_P2G_TX, P2G_TY = FSIM_P2G_TY, P2G_TZ = 64;
-constexpr int P2G_TILE_CAP = 1024;   // particles per staged chunk (a row segment is 66 cells)
-template <int APIC, int TX, int TY, int TWOD>
+// sums are bit-identical.  k_p2g_tile serves APIC, k_p2g_tile_w PIC and FLIP.
+//
+// Slots.  The lanes of a wave read particles 8 apart, where every cell holds
+// 8: an unused slot behind every 8 spreads them over the LDS banks.  Without
+// it PIC/FLIP takes 4.3 ms at 256^3 (2.7 with it), APIC 0.96 ms at 128^3
+// (0.42).  A chunk holds the 66 cells of a row at 8 particles each, so that a
+// full row is one chunk: with 512 a second one of 16 particles follows (5.1
+// ms for 4.3).
+//
+// Tiles: 4 x 2 rows; 2 x 2 below 1024 blocks and 1 x 2 below 256, since a block
+// takes its rows one after the other (us: 61x45x77 118 -> 107, 32^3 92 -> 62 ->
+// 52; 4 x 2 against 2 x 2 at 96^3 140 / 151, at 256^3 2.7 / 3.1 ms).
+constexpr int P2G_TZ = 64;
+constexpr int p2g_slots(int cap) { return cap + cap / 8; }
+__device__ inline int p2g_slot(int k) { return k + (k >> 3); }
+
+// APIC.  A particle is four 16-byte words, z position index and a word with
+// its offsets from the staged row (t_d - row + 3, held to 0 .. 6: further off
+// it reaches no cell of the tile) and its half-cell bits.
+template <int TX, int TY, int TWOD>
 __global__ void __launch_bounds__(P2G_TZ * TX * TY) k_p2g_tile(P2GArgs A) {
-    constexpr int CAP = P2G_TILE_CAP;
-    constexpr int NC = APIC ? 9 : 1;
+    constexpr int CAP = 560;   // particles per staged chunk (72 bytes of LDS each: three blocks a CU)
     constexpr int NT = P2G_TZ * TX * TY;
-    __shared__ float s_pos[3][CAP], s_vel[3][CAP];
-    __shared__ int s_t[3][CAP];
-    __shared__ uint8_t s_h[CAP];
-    __shared__ float s_c[NC][APIC ? CAP : 1];
+    __shared__ float4 s_a[p2g_slots(CAP)];   // position, velocity x
+    __shared__ float4 s_b[p2g_slots(CAP)];   // velocity y, z, C 0, 1
+    __shared__ float4 s_c[p2g_slots(CAP)];   // C 2 .. 5
+    __shared__ float4 s_d[p2g_slots(CAP)];   // C 6 .. 8
+    __shared__ int2 s_t[p2g_slots(CAP)];     // t_z; half-cell bits 0 .. 2, x offset 3 .. 5, y offset 6 .. 8
     const GridArgs& G = A.G;
     const int tid = threadIdx.x + P2G_TZ * threadIdx.y;
     const int zc0 = blockIdx.x * P2G_TZ;
-    const int ri = threadIdx.y / TY, rj = threadIdx.y % TY;   // this wave's cell row in the tile
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
     const int x0 = blockIdx.z * TX, y0 = blockIdx.y * TY;
-    const int x = x0 + ri, y = y0 + rj, z = zc0 + threadIdx.x;
+    const int x = x0 + wave / TY, y = y0 + wave % TY, z = zc0 + threadIdx.x;   // x, y: the wave's
     const bool valid = x < G.nx && y < G.ny && z < G.nz;
     const int xc = min(x, G.nx - 1), yc = min(y, G.ny - 1), zc = min(z, G.nz - 1);
     float fal[3], fce[3];
@@ -328,7 +338,6 @@ __global__ void __launch_bounds__(P2G_TZ * TX * TY) k_p2g_tile(P2GArgs A) {
         fal[0] = f[0][0], fal[1] = f[1][1], fal[2] = f[2][2];
         fce[0] = f[1][0], fce[1] = f[0][1], fce[2] = f[0][2];
     }
-    const int cc[3] = {xc, yc, zc};
     float swv[3] = {0.f, 0.f, 0.f}, sw[3] = {0.f, 0.f, 0.f};
     float dens = 0.f;
     for (int rx = x0 - 1; rx <= x0 + TX; rx++) {
@@ -347,67 +356,71 @@ __global__ void __launch_bounds__(P2G_TZ * TX * TY) k_p2g_tile(P2GArgs A) {
                 j0 = A.start[rb + (z > 0 ? z - 1 : z)];
                 j1 = A.start[rb + (z < G.nz - 1 ? z + 2 : z + 1)];
             }
+            const int ox = x - rx + 4, oy = y - ry + 4;   // ua = ox - offset
             for (int base = u0; base < u1; base += CAP) {
                 const int cnt = min(CAP, u1 - base);
                 __syncthreads();   // the previous chunk is consumed
-                for (int k = tid; k < cnt; k += NT) {
-                    const int j = base + k;
-                    uint8_t h = 0;
+                for (int kk = tid; kk < cnt; kk += NT) {
+                    const int j = base + kk, k = p2g_slot(kk);
+                    const float p[3] = {A.pos[0][j], A.pos[1][j], A.pos[2][j]};
+                    int t[3], info = 0;
 #pragma unroll
                     for (int d = 0; d < 3; d++) {
-                        const float pv = A.pos[d][j];
-                        const double v = (double)pv * cdinv_t<TWOD>(G, d);
-                        const int t = (int)v;
-                        s_pos[d][k] = pv;
-                        s_vel[d][k] = A.vel[d][j];
-                        s_t[d][k] = t;
-                        if ((int)(v - 0.5) == t) h |= (uint8_t)(1u << d);
+                        const double v = (double)p[d] * cdinv_t<TWOD>(G, d);
+                        t[d] = (int)v;
+                        if ((int)(v - 0.5) == t[d]) info |= 1 << d;
                     }
-                    s_h[k] = h;
-                    if (APIC) {
-#pragma unroll
-                        for (int m = 0; m < NC; m++) s_c[m][k] = A.c[m][j];
-                    }
+                    info |= min(max(t[0] - rx, -3), 3) + 3 << 3;
+                    info |= min(max(t[1] - ry, -3), 3) + 3 << 6;
+                    s_a[k] = make_float4(p[0], p[1], p[2], A.vel[0][j]);
+                    s_b[k] = make_float4(A.vel[1][j], A.vel[2][j], A.c[0][j], A.c[1][j]);
+                    s_c[k] = make_float4(A.c[2][j], A.c[3][j], A.c[4][j], A.c[5][j]);
+                    s_d[k] = make_float4(A.c[6][j], A.c[7][j], A.c[8][j], 0.f);
+                    s_t[k] = make_int2(t[2], info);
                 }
                 __syncthreads();
                 const int e = min(j1, base + cnt);
-#pragma unroll 4
+#pragma unroll 1
                 for (int j = max(j0, base); j < e; j++) {
-                    const int k = j - base;
-                    const float p[3] = {s_pos[0][k], s_pos[1][k], s_pos[2][k]};
-                    const uint32_t h = s_h[k];
-                    int ua[3], uc[3];
+                    const int k = p2g_slot(j - base);
+                    const float4 qa = s_a[k], qb = s_b[k], qc = s_c[k], qd = s_d[k];
+                    const int2 ti = s_t[k];
+                    const float p[3] = {qa.x, qa.y, qa.z}, vel[3] = {qa.w, qb.x, qb.y};
+                    const float c[9] = {qb.z, qb.w, qc.x, qc.y, qc.z, qc.w, qd.x, qd.y, qd.z};
+                    // face_base: b_a = t_a - 1, b_d = (int)(p_d/dx - 0.5) = t_d - 1 + h_d (d != a); the face of
+                    // this cell is in the stencil when cell - b is 0 or 1 on every axis
+                    const int ua[3] = {ox - ((ti.y >> 3) & 7), oy - ((ti.y >> 6) & 7), zc - ti.x + 1};
+                    bool ia[3], ic[3];
                     float tal[3], tce[3];
 #pragma unroll
                     for (int d = 0; d < 3; d++) {
-                        ua[d] = cc[d] - s_t[d][k] + 1;
-                        uc[d] = ua[d] - (int)((h >> d) & 1u);
+                        ia[d] = (unsigned)ua[d] <= 1u;
+                        ic[d] = (unsigned)(ua[d] - ((ti.y >> d) & 1)) <= 1u;
                         tal[d] = 1.0f - fabsf((p[d] - fal[d]) * invf_t<TWOD>(G, d));
                         tce[d] = 1.0f - fabsf((p[d] - fce[d]) * invf_t<TWOD>(G, d));
                     }
-                    if ((unsigned)uc[0] <= 1u && (unsigned)uc[1] <= 1u && (unsigned)uc[2] <= 1u)
-                        dens += tce[0] * tce[1] * tce[2];
+                    // getCellsAround (macGrid.cpp:188-202): base (int)(p/dx - 0.5) on every axis.  A term
+                    // outside the stencil is formed and dropped: no branches
+                    const float dn = dens + tce[0] * tce[1] * tce[2];
+                    dens = ic[0] && ic[1] && ic[2] ? dn : dens;
 #pragma unroll
                     for (int a = 0; a < 3; a++) {
                         bool in = true;
                         float tw[3];
 #pragma unroll
                         for (int d = 0; d < 3; d++) {
-                            const int u = d == a ? ua[d] : uc[d];
-                            in = in && (unsigned)u <= 1u;
+                            in = in && (d == a ? ia[d] : ic[d]);
                             tw[d] = d == a ? tal[d] : tce[d];
                         }
-                        if (!in) continue;
                         const float w = tw[0] * tw[1] * tw[2];
-                        float va = s_vel[a][k];
-                        if (APIC) {
-                            const float f0 = a == 0 ? fal[0] : fce[0], f1 = a == 1 ? fal[1] : fce[1],
-                                        f2 = a == 2 ? fal[2] : fce[2];
-                            const float d0 = f0 - p[0], d1 = f1 - p[1], d2 = f2 - p[2];
-                            va = va + (s_c[3 * a][k] * d0 + s_c[3 * a + 1][k] * d1 + s_c[3 * a + 2][k] * d2);
-                        }
-                        swv[a] += va * w;
-                        sw[a] += w;
+                        // (v_a + c[a] . (face - p)) * w, simulator.cpp:326-328
+                        const float f0 = a == 0 ? fal[0] : fce[0], f1 = a == 1 ? fal[1] : fce[1],
+                                    f2 = a == 2 ? fal[2] : fce[2];
+                        const float d0 = f0 - p[0], d1 = f1 - p[1], d2 = f2 - p[2];
+                        const float va = vel[a] + (c[3 * a] * d0 + c[3 * a + 1] * d1 + c[3 * a + 2] * d2);
+                        const float nv = swv[a] + va * w, nw = sw[a] + w;
+                        swv[a] = in ? nv : swv[a];
+                        sw[a] = in ? nw : sw[a];
                     }
                 }
             }
@@ -433,27 +446,25 @@ __global__ void __launch_bounds__(P2G_TZ * TX * TY) k_p2g_tile(P2GArgs A) {
 // reads the pair for its own offset.  The walk computes only the z weights,
 // and p2g_terms sums without branches.  Same rows, same particle order, same
 // weights and terms as the row gather: the sums are bit-identical.
-// The walk is latency-bound, so occupancy decides: 36 KB of LDS per block
-// allows 8 waves per SIMD, and the register budget is held to that (60
-// VGPRs with the walk not unrolled).  Measured at 256^3 (FLIP double dam
-// break): 3.75 ms, against 4.1 ms at 69 VGPRs, 4.6-4.8 ms unrolled by 2 and
-// 5.6 ms unrolled by 4 (94 VGPRs); 4 x 4 tiles took 4.9 ms.
-constexpr int P2G_W_CAP = 512;   // particles per staged chunk (72 bytes of LDS each)
+// Occupancy decides as well: 40 KB of LDS per block allows 8 waves per SIMD,
+// and the register budget is held to that (the walk is not unrolled).
+constexpr int P2G_W_CAP = 533;   // particles per staged chunk (68 bytes of LDS each: four blocks of 600 slots a CU)
 template <int TX, int TY, int TWOD>
 __global__ void __launch_bounds__(P2G_TZ * TX * TY) __attribute__((amdgpu_waves_per_eu(8)))
 k_p2g_tile_w(P2GArgs A) {
     constexpr int CAP = P2G_W_CAP;
     constexpr int NT = P2G_TZ * TX * TY;
-    __shared__ float4 s_pv[CAP];      // z position, velocity x, y, z
-    __shared__ int2 s_zz[CAP];        // t_z - 1, t_z - 1 + h_z (face_base along z of the two face kinds)
-    __shared__ float2 s_wx[3][CAP];   // [x - row + 1]: (al_x, ce_x)
-    __shared__ float2 s_wy[3][CAP];   // [y - row + 1]: (al_y, ce_y)
+    constexpr int SL = p2g_slots(CAP);
+    __shared__ float4 s_pv[SL];      // z position, velocity x, y, z
+    __shared__ int s_zh[SL];         // 2 (t_z - 1) + h_z: face_base along z is t_z - 1 and t_z - 1 + h_z
+    __shared__ float2 s_wx[3][SL];   // [x - row + 1]: (al_x, ce_x)
+    __shared__ float2 s_wy[3][SL];   // [y - row + 1]: (al_y, ce_y)
     const GridArgs& G = A.G;
     const int tid = threadIdx.x + P2G_TZ * threadIdx.y;
     const int zc0 = blockIdx.x * P2G_TZ;
-    const int ri = threadIdx.y / TY, rj = threadIdx.y % TY;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.y);
     const int x0 = blockIdx.z * TX, y0 = blockIdx.y * TY;
-    const int x = x0 + ri, y = y0 + rj, z = zc0 + threadIdx.x;
+    const int x = x0 + wave / TY, y = y0 + wave % TY, z = zc0 + threadIdx.x;   // x, y: the wave's
     const bool valid = x < G.nx && y < G.ny && z < G.nz;
     const int zc = min(z, G.nz - 1);
     float fz[3][3];
@@ -477,12 +488,13 @@ k_p2g_tile_w(P2GArgs A) {
                 j0 = A.start[rb + (z > 0 ? z - 1 : z)];
                 j1 = A.start[rb + (z < G.nz - 1 ? z + 2 : z + 1)];
             }
-            const int ex = near ? x - rx + 1 : 0, ey = near ? y - ry + 1 : 0;   // wave-uniform
+            // wave-uniform (a wave that is not near walks no particle)
+            const int ex = min(max(x - rx + 1, 0), 2), ey = min(max(y - ry + 1, 0), 2);
             for (int base = u0; base < u1; base += CAP) {
                 const int cnt = min(CAP, u1 - base);
                 __syncthreads();   // the previous chunk is consumed
-                for (int k = tid; k < cnt; k += NT) {
-                    const int j = base + k;
+                for (int kk = tid; kk < cnt; kk += NT) {
+                    const int j = base + kk, k = p2g_slot(kk);
                     const float p[3] = {A.pos[0][j], A.pos[1][j], A.pos[2][j]};
                     int t[3], h[3];
 #pragma unroll
@@ -504,18 +516,18 @@ k_p2g_tile_w(P2GArgs A) {
                             (d == 0 ? s_wx : s_wy)[e][k] = make_float2(al, ce);
                         }
                     }
-                    s_zz[k] = make_int2(t[2] - 1, t[2] - 1 + h[2]);
+                    s_zh[k] = 2 * (t[2] - 1) + h[2];
                     s_pv[k] = make_float4(p[2], A.vel[0][j], A.vel[1][j], A.vel[2][j]);
                 }
                 __syncthreads();
                 const int e = min(j1, base + cnt);
 #pragma unroll 1
                 for (int j = max(j0, base); j < e; j++) {
-                    const int k = j - base;
+                    const int k = p2g_slot(j - base);
                     const float4 pv = s_pv[k];
-                    const int2 zz = s_zz[k];
+                    const int zh = s_zh[k];
                     const float2 wx = s_wx[ex][k], wy = s_wy[ey][k];
-                    const int ua = zc - zz.x, uc = zc - zz.y;
+                    const int ua = zc - (zh >> 1), uc = ua - (zh & 1);
                     const float alz = (unsigned)ua <= 1u ? 1.0f - fabsf((pv.x - falz) * invz) : 0.f;
                     const float cez = (unsigned)uc <= 1u ? 1.0f - fabsf((pv.x - fcez) * invz) : 0.f;
                     p2g_terms(wx.x, wx.y, wy.x, wy.y, alz, cez, pv.y, pv.z, pv.w, swv, sw, dens);
@@ -532,6 +544,25 @@ k_p2g_tile_w(P2GArgs A) {
     }
     A.label[i] = (A.fuse_mark && A.count[i] > 0) ? (uint8_t)FSIM_WATER : (uint8_t)FSIM_AIR;
     A.density[i] = dens;
+}
+
+template <int TX, int TY, int TWOD>
+static void p2g_tiles(fsim_ctx* ctx, const P2GArgs& A, bool apic) {
+    const GridDims& d = ctx->g;
+    const dim3 g((unsigned)((d.nz + P2G_TZ - 1) / P2G_TZ), (unsigned)((d.ny + TY - 1) / TY), (unsigned)((d.nx + TX - 1) / TX));
+    const dim3 b(P2G_TZ, TX * TY);
+    if (apic) hipLaunchKernelGGL((k_p2g_tile<TX, TY, TWOD>), g, b, 0, ctx->stream, A);
+    else hipLaunchKernelGGL((k_p2g_tile_w<TX, TY, TWOD>), g, b, 0, ctx->stream, A);
+}
+
+// tiles by the number of 4 x 2 blocks ("Tiles" above)
+template <int TWOD>
+static void p2g_sized(fsim_ctx* ctx, const P2GArgs& A, bool apic) {
+    const GridDims& d = ctx->g;
+    const int64_t blocks = (int64_t)((d.nz + P2G_TZ - 1) / P2G_TZ) * ((d.ny + 1) / 2) * ((d.nx + 3) / 4);
+    if (blocks >= 1024) p2g_tiles<4, 2, TWOD>(ctx, A, apic);
+    else if (blocks >= 256) p2g_tiles<2, 2, TWOD>(ctx, A, apic);
+    else p2g_tiles<1, 2, TWOD>(ctx, A, apic);
 }
 
 static int p2g(fsim_ctx* ctx, int fuse_mark) {
@@ -566,16 +597,8 @@ static int p2g(fsim_ctx* ctx, int fuse_mark) {
             else hipLaunchKernelGGL((k_p2g_gather<0, 0>), g, b, 0, ctx->stream, A);
         }
     } else {
-        const dim3 g((unsigned)((ctx->g.nz + P2G_TZ - 1) / P2G_TZ), (unsigned)((ctx->g.ny + P2G_TY - 1) / P2G_TY),
-                     (unsigned)((ctx->g.nx + P2G_TX - 1) / P2G_TX));
-        const dim3 b(P2G_TZ, P2G_TX * P2G_TY);
-        if (ctx->g.two_d) {
-            if (A.apic) hipLaunchKernelGGL((k_p2g_tile<1, P2G_TX, P2G_TY, 1>), g, b, 0, ctx->stream, A);
-            else hipLaunchKernelGGL((k_p2g_tile_w<P2G_TX, P2G_TY, 1>), g, b, 0, ctx->stream, A);
-        } else {
-            if (A.apic) hipLaunchKernelGGL((k_p2g_tile<1, P2G_TX, P2G_TY, 0>), g, b, 0, ctx->stream, A);
-            else hipLaunchKernelGGL((k_p2g_tile_w<P2G_TX, P2G_TY, 0>), g, b, 0, ctx->stream, A);
-        }
+        if (ctx->g.two_d) p2g_sized<1>(ctx, A, A.apic != 0);
+        else p2g_sized<0>(ctx, A, A.apic != 0);
     }
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;
