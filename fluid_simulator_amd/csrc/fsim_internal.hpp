@@ -250,6 +250,7 @@ struct SolveScalars {
     double zr;                       // z.r
     double zq;                       // z.q (flexible PCG)
     double nfluid;                   // number of WATER cells of the solve
+    int64_t wave_err;                // host copy: the wavefront kernels' error flag
     int nan_flag;
     unsigned seq;                    // host copy: number of the reduction that wrote it
 };

@@ -38,6 +38,7 @@ struct Reduce {
     int op;             // FinOp
     SolveScalars* host = nullptr;   // pinned host copy written by the finishing block, or null
     unsigned seq = 0;               // what the host waits for in it (host->seq)
+    const int* wave_err = nullptr;  // the wavefront kernels' error flag, copied along
 };
 
 __device__ inline void apply_fin(int op, double s, double m, SolveScalars* sc) {
@@ -148,14 +149,19 @@ __device__ void block_finish(double sum, double aux, const Reduce& R, const Part
         apply_fin(R.op, lds_s[0], lds_m[0], R.sc);
         __hip_atomic_store(R.count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (R.host) {
-            // the words the host tests after the r update (rr, rmax, nan_flag) straight into pinned
-            // host memory with system-scope stores, the word with seq, which the host polls, when the
-            // others have been acknowledged
+            // the words the host tests after the reduction straight into pinned host memory with
+            // system-scope stores, the word with seq, which the host polls, when the others have been
+            // acknowledged
             auto put_host = [](void* dst, uint64_t v) {
                 __hip_atomic_store(reinterpret_cast<uint64_t*>(dst), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             };
-            put_host(&R.host->rr, __builtin_bit_cast(uint64_t, R.sc->rr));
-            put_host(&R.host->rmax, __builtin_bit_cast(uint64_t, R.sc->rmax));
+            double* const to = R.op == FIN_BB ? &R.host->bb : R.op == FIN_TRUE ? &R.host->tr_ss : &R.host->rr;
+            double* const to2 = R.op == FIN_BB ? &R.host->nfluid : R.op == FIN_TRUE ? &R.host->tr_max : &R.host->rmax;
+            put_host(to, __builtin_bit_cast(uint64_t, lds_s[0]));
+            put_host(to2, __builtin_bit_cast(uint64_t, lds_m[0]));
+            if (R.wave_err)
+                put_host(&R.host->wave_err,
+                         (uint64_t)(uint32_t)__hip_atomic_load(R.wave_err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
             __builtin_amdgcn_s_waitcnt(0);
             static_assert(offsetof(SolveScalars, seq) == offsetof(SolveScalars, nan_flag) + 4, "one 8-byte word");
             put_host(&R.host->nan_flag, (uint32_t)R.sc->nan_flag | (uint64_t)R.seq << 32);

@@ -510,17 +510,21 @@ static int clear_packets(fsim_ctx* ctx) {
 
 // A wavefront kernel whose boundary poll ran out of spins sets wave_err; its
 // results are then invalid and the call fails.
-static int check_wave_err(fsim_ctx* ctx) {
-    if (ctx->sweep_mode != 0) return FSIM_OK;
-    int err = 0;
-    FSIM_HIP(ctx, hipMemcpyAsync(&err, ctx->wave_err, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+static int wave_failed(fsim_ctx* ctx, int err) {
     if (err) {
         FSIM_HIP(ctx, hipMemsetAsync(ctx->wave_err, 0, sizeof(int), ctx->stream));
         FSIM_TRY(clear_packets(ctx));   // what the launch sent and nobody received
         return set_err(ctx, FSIM_ERR_TIMEOUT, "wavefront sweep boundary wait timed out");
     }
     return FSIM_OK;
+}
+
+static int check_wave_err(fsim_ctx* ctx) {
+    if (ctx->sweep_mode != 0) return FSIM_OK;
+    int err = 0;
+    FSIM_HIP(ctx, hipMemcpyAsync(&err, ctx->wave_err, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+    FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return wave_failed(ctx, err);
 }
 
 // Reduction grids: at most kMaxParts blocks (grid-stride; 8 blocks of 4 waves
@@ -539,9 +543,21 @@ static Reduce reduce_to_host(fsim_ctx* ctx, int op) {
     return Reduce{ctx->partials, ctx->red_count, ctx->scal, op, ctx->scal_host, ++ctx->scal_seq};
 }
 
-static int read_scalars(fsim_ctx* ctx) {
-    FSIM_HIP(ctx, hipMemcpyAsync(ctx->scal_host, ctx->scal, sizeof(SolveScalars), hipMemcpyDeviceToHost, ctx->stream));
-    FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+// Waits until the finishing block of the last reduce_to_host reduction has
+// written its scalars: polls the pinned word, since an event after the kernel
+// is one more packet that the kernels behind it wait for (5 us an iteration),
+// and a copy another, with the stream's synchronisation behind it (20 to 40 us).
+// A queue that takes longer than the polls is waited for as a whole, which
+// also reports a failed kernel.
+static int wait_scalars(fsim_ctx* ctx) {
+    const volatile unsigned* seq = &ctx->scal_host->seq;
+    const auto t0 = std::chrono::steady_clock::now();
+    while (*seq != ctx->scal_seq) {
+        if (std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(100)) continue;
+        FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        if (*seq != ctx->scal_seq) return set_err(ctx, FSIM_ERR_HIP, "the solver's scalars did not arrive");
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
     return FSIM_OK;
 }
 
@@ -571,7 +587,7 @@ static int build_nbinfo(fsim_ctx* ctx, const SolveArgs& S, bool with_rhs) {
     A.avg_p = ctx->prm.average_pressure;
     A.pk = ctx->prm.pressure_k;
     A.pressure_enabled = ctx->prm.pressure_enabled;
-    A.red = reduce_to(ctx, FIN_BB);
+    A.red = with_rhs ? reduce_to_host(ctx, FIN_BB) : reduce_to(ctx, FIN_BB);
     FSIM_TRY(fill_u8(ctx, ctx->colw, 0, colw_bytes(S)));   // and xrange and the chunk flags behind it
     hipLaunchKernelGGL(k_nbinfo_rhs, dim3(red_blocks(S.nc)), dim3(kBlock), 0, ctx->stream, A, with_rhs ? 1 : 0);
     // wide windows leave fewer lanes idle, narrow ones give small grids more and shorter blocks
@@ -665,8 +681,10 @@ static int mic_apply(fsim_ctx* ctx, const SolveArgs& S, const float* r, float* t
 
 static int true_residual(fsim_ctx* ctx, const SolveArgs& S, float* r, bool replace) {
     FSIM_PROF(ctx, KID_TRUE_RES);
+    Reduce red = reduce_to_host(ctx, FIN_TRUE);
+    red.wave_err = ctx->wave_err;
     hipLaunchKernelGGL(k_true_residual, dim3(column_blocks(S)), dim3(kBlock), 0, ctx->stream, S, ctx->nbinfo, ctx->b, ctx->x,
-                       r, replace ? 1 : 0, reduce_to(ctx, FIN_TRUE));
+                       r, replace ? 1 : 0, red);
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;
 }
@@ -710,24 +728,6 @@ static int update_x_last(fsim_ctx* ctx) {
     hipLaunchKernelGGL(k_update_x<1>, dim3(std::max(1u, std::min(nblocks(n / 4), kMaxParts))), dim3(kBlock), 0, ctx->stream, n,
                        ctx->chunk_flags, update_x_args(ctx), ctx->scal);
     FSIM_HIP(ctx, hipGetLastError());
-    return FSIM_OK;
-}
-
-// Waits until the finishing block of the last reduce_to_host reduction has
-// written its scalars: polls the pinned word, since an event after the kernel
-// is one more packet that the kernels behind it wait for (5 us an iteration).
-// A queue that takes longer than the polls is waited for as a whole, which
-// also reports a failed kernel.
-static int wait_scalars(fsim_ctx* ctx, SolveScalars* h) {
-    const volatile unsigned* seq = &ctx->scal_host->seq;
-    const auto t0 = std::chrono::steady_clock::now();
-    while (*seq != ctx->scal_seq) {
-        if (std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(100)) continue;
-        FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        if (*seq != ctx->scal_seq) return set_err(ctx, FSIM_ERR_HIP, "the solver's scalars did not arrive");
-    }
-    std::atomic_thread_fence(std::memory_order_acquire);
-    *h = *ctx->scal_host;
     return FSIM_OK;
 }
 
@@ -848,8 +848,8 @@ static int pcg_run(fsim_ctx* ctx, const SolveArgs& S, double bnorm, bool flexibl
         if (two) behind = 0;
         if (flexible) FSIM_TRY(update_flexible(ctx, S, two));
         else FSIM_TRY(update_mic(ctx, S, &r, &r_next, two));
-        SolveScalars h;
-        FSIM_TRY(wait_scalars(ctx, &h));
+        FSIM_TRY(wait_scalars(ctx));
+        const SolveScalars h = *ctx->scal_host;
         // the previous iteration's old-sigma test, then this iteration's alpha test
         if (h.nan_flag & 2) {
             it--;
@@ -866,7 +866,7 @@ static int pcg_run(fsim_ctx* ctx, const SolveArgs& S, double bnorm, bool flexibl
             behind = 0;
             const bool replace = st.reliable_updates < max_reliable;
             FSIM_TRY(true_residual(ctx, S, r, replace));
-            FSIM_TRY(read_scalars(ctx));
+            FSIM_TRY(wait_scalars(ctx));
             if (stop_met(ctx, ctx->scal_host->tr_ss, ctx->scal_host->tr_max, bnorm)) {
                 res->converged = true;
                 break;
@@ -961,7 +961,7 @@ static int stage_basic_sor(fsim_ctx* ctx, const SolveArgs& S) {
     FSIM_HIP(ctx, hipMemsetAsync(ctx->scal, 0, sizeof(SolveScalars), ctx->stream));
     FSIM_TRY(fill_f64(ctx, ctx->x, 0.0, S.ncr));   // no pressure field
     FSIM_TRY(build_nbinfo(ctx, S, true));
-    FSIM_TRY(read_scalars(ctx));
+    FSIM_TRY(wait_scalars(ctx));
     const double b0 = std::sqrt(ctx->scal_host->bb);
     st.b_norm_l2 = b0;
     st.num_fluid_cells = (int64_t)ctx->scal_host->nfluid;
@@ -994,7 +994,7 @@ static int stage_basic_sor(fsim_ctx* ctx, const SolveArgs& S) {
     // the right-hand side left on the projected faces (FSIM_FIELD_RHS reads it)
     FSIM_HIP(ctx, hipMemsetAsync(ctx->scal, 0, sizeof(SolveScalars), ctx->stream));
     FSIM_TRY(build_nbinfo(ctx, S, true));
-    FSIM_TRY(read_scalars(ctx));
+    FSIM_TRY(wait_scalars(ctx));
     st.residual_rel_l2 = b0 > 0 ? std::sqrt(ctx->scal_host->bb) / b0 : 0.0;
     st.residual_abs_inf = 0.0;
     st.pcg_iterations = iters;   // BasicMacGrid returns its iteration count (basicMacGrid.cpp:10)
@@ -1021,17 +1021,17 @@ int stage_solve(fsim_ctx* ctx, double dt) {
         return set_err(ctx, FSIM_ERR_INVALID, "learned preconditioner selected but it has no parameters "
                                               "(fsim_learned_init or fsim_learned_set_params)");
     FSIM_HIP(ctx, hipMemsetAsync(ctx->scal, 0, sizeof(SolveScalars), ctx->stream));
-    FSIM_TRY(fill_f64(ctx, ctx->x, 0.0, nc));
     FSIM_TRY(build_nbinfo(ctx, S, true));
-    FSIM_TRY(read_scalars(ctx));
+    FSIM_TRY(wait_scalars(ctx));
     const double bb = ctx->scal_host->bb;
     const double bnorm = std::sqrt(bb);
     st.b_norm_l2 = bnorm;
     st.num_fluid_cells = (int64_t)ctx->scal_host->nfluid;
     if (bb < 1e-7) {   // early exit without pressure (bridsonSolverGrid.cpp:254-258)
         st.early_exit = 1;
+        FSIM_TRY(fill_f64(ctx, ctx->x, 0.0, S.ncr));
         FSIM_TRY(true_residual(ctx, S, ctx->r, false));
-        FSIM_TRY(read_scalars(ctx));
+        FSIM_TRY(wait_scalars(ctx));
         st.residual_abs_inf = ctx->scal_host->tr_max;
         st.residual_rel_l2 = 1.0;
         return FSIM_OK;
@@ -1078,14 +1078,13 @@ int stage_solve(fsim_ctx* ctx, double dt) {
     }
     FSIM_HIP(ctx, hipGetLastError());
     FSIM_TRY(true_residual(ctx, S, ctx->r, false));
-    FSIM_TRY(read_scalars(ctx));
+    FSIM_TRY(wait_scalars(ctx));
     st.residual_abs_inf = ctx->scal_host->tr_max;
     st.residual_rel_l2 = bnorm > 0 ? std::sqrt(ctx->scal_host->tr_ss) / bnorm : 0.0;
     // a NaN alpha or sigma ended the solve: like the reference, the last
     // finite pressure has been applied and the step goes on
     st.solve_nan = res.nan ? 1 : 0;
-    FSIM_TRY(check_wave_err(ctx));
-    return FSIM_OK;
+    return ctx->sweep_mode == 0 ? wave_failed(ctx, (int)ctx->scal_host->wave_err) : FSIM_OK;
 }
 
 int wave_init(fsim_ctx* ctx) {
