@@ -770,12 +770,189 @@ __global__ void __launch_bounds__(WF_THREADS) k_wave(WaveArgs A, SideWork W) {
     else send_wave<KIND>(A, S, T);
 }
 
+// ---- 2D grids ----------------------------------------------------------------------
+// One column of cells along z leaves 63 lanes of a compute wave idle, and the
+// chain passes from wave to wave every two rows: 29 us a sweep of 128 x 128.
+// Here a wave takes 64 rows, a row per lane, and lane l works on x = step - l:
+// its -x value is its own of the step before and its -y value lane l - 1's of
+// the step before (DPP wave shift), so a sweep is a chain of nx + ny steps,
+// 15 us.  One workgroup does it; a wave's last row goes to the next one over
+// LDS.
+// A lane moves four steps of its row with one 16-byte access, but the lanes
+// reach the ends of their groups at different steps: lane l is l mod 4 elements
+// behind its group, and a group of four steps takes its operands from two
+// consecutive storage groups, shifted by selects, and puts its results
+// together in the same way.  The operations on a cell and their order are those
+// of compute_wave: the same bits.
+constexpr int k2dAhead = 8;    // groups of steps loaded ahead, and the unroll of their loop
+constexpr int k2dLag = 17;     // groups of steps from a wave's first to its last row, + 1
+constexpr int k2dPad = 64;     // elements before an edge row's first
+__host__ __device__ inline int groups_2d(int ng) { return (ng + k2dLag + k2dAhead - 1) / k2dAhead * k2dAhead; }
+__host__ __device__ inline int edge_2d(int ng) { return WF_G * groups_2d(ng) + k2dPad; }
+static int waves_2d(int ny) { return (ny - 2 + WF_TZ - 1) / WF_TZ; }
+static size_t lds_2d(int ny, int nxp) { return sizeof(float) * (size_t)(waves_2d(ny) - 1) * edge_2d(nxp / WF_G); }
+constexpr size_t kLds2d = size_t(40) << 10;   // what the side blocks' reductions leave of 64 KB
+static bool fits_2d(const WaveArgs& A) {
+    return A.nz == 3 && waves_2d(A.ny) <= WF_THREADS / WF_TZ && lds_2d(A.ny, A.nxp) <= kLds2d;
+}
+
+// t[j] = seq[4 + j - c] and back, seq the elements of lo and hi, c = 2 c2 + c1
+__device__ inline f32x4 behind(f32x4 lo, f32x4 hi, bool c1, bool c2) {
+    const float seq[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    float t[8];
+#pragma unroll
+    for (int k = 2; k < 8; k++) t[k] = c1 ? seq[k - 1] : seq[k];
+    f32x4 out;
+#pragma unroll
+    for (int j = 0; j < 4; j++) out[j] = c2 ? t[2 + j] : t[4 + j];
+    return out;
+}
+__device__ inline f32x4 ahead(f32x4 lo, f32x4 hi, bool c1, bool c2) {   // seq[j + c]
+    const float seq[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+    float t[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) t[k] = c1 ? seq[k + 1] : seq[k];
+    f32x4 out;
+#pragma unroll
+    for (int j = 0; j < 4; j++) out[j] = c2 ? t[j + 2] : t[j];
+    return out;
+}
+
+template <int KIND>
+__global__ void __launch_bounds__(WF_THREADS) k_wave_2d(WaveArgs A, SideWork W) {
+#pragma clang fp contract(off)
+    constexpr bool FWD = Kind<KIND>::FWD, UPD = KIND == WAVE_FWD_UPDATE;
+    if (blockIdx.x > 0) {
+        const Part part{blockIdx.x - 1, W.blocks};
+        if constexpr (UPD) {
+            update_r<WF_THREADS>(part, W.n, W.flags, W.q, W.r, W.r_next, W.red);
+        } else if constexpr (!FWD) {
+            dot_self<WF_THREADS>(part, W.n, W.flags, W.t, W.red);
+            if (W.x_steps == 2) update_x_chunks<2>(part, W.n, W.flags, W.x, W.red.sc);
+        }
+        return;
+    }
+    extern __shared__ __align__(16) uint32_t edges[];   // row w: what wave w hands to wave w + 1
+    __shared__ int done[WF_THREADS / WF_TZ];            // groups of steps that wave w has finished
+    const int xa = __builtin_amdgcn_readfirstlane(A.xrange[0]), xb = __builtin_amdgcn_readfirstlane(A.xrange[1]);
+    if (xb < xa) return;   // no WATER
+    const int g0 = xa / WF_G, g1 = xb / WF_G, ng = g1 - g0 + 1;
+    const int steps = groups_2d(ng), elen = edge_2d(ng);
+    const int nwaves = (A.ny - 2 + WF_TZ - 1) / WF_TZ;
+    for (int i = threadIdx.x; i < (nwaves - 1) * elen; i += WF_THREADS) edges[i] = 0;
+    if (threadIdx.x < WF_THREADS / WF_TZ) done[threadIdx.x] = 0;
+    __syncthreads();
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WF_TZ), lane = threadIdx.x % WF_TZ;
+    if (w >= nwaves) return;
+    const uint32_t gstride = (uint32_t)A.ny * 3u * 16u, total = gstride * (uint32_t)(A.nxp / WF_G);
+    const __amdgpu_buffer_rsrc_t rP = rsrc(A.P32, (int64_t)total), rI = rsrc(A.in, (int64_t)total),
+                                 rO = rsrc(A.out, (int64_t)total), rQ = rsrc(UPD ? W.q : A.in, (int64_t)total);
+    const float ms = A.ms;
+    const float malpha = UPD ? (float)(-W.red.sc->alpha) : 0.f;
+    const int row = WF_TZ * w + lane, q = lane / WF_G;
+    const bool in_grid = row < A.ny - 2, c1 = (lane & 1) != 0, c2 = (lane & 2) != 0;
+    const uint32_t column = (uint32_t)((FWD ? 1 + row : A.ny - 2 - row) * 3 + 1) * 16u;
+    // byte offset of the lane's k-th group in the order of the march, beyond the arrays if it has none
+    auto at = [&](int k) {
+        return in_grid && (unsigned)k < (unsigned)ng ? (uint32_t)(FWD ? g0 + k : g1 - k) * gstride + column : kOob;
+    };
+    auto marched = [](f32x4 v) { return FWD ? v : f32x4{v[3], v[2], v[1], v[0]}; };
+    f32x4 pv[k2dAhead], iv[k2dAhead], uv[k2dAhead];
+    auto fetch = [&](auto dc, int g) {
+        constexpr int d = decltype(dc)::value;
+        const uint32_t o = at(g - q);
+        pv[d] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rP, o, 0, 0));
+        iv[d] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rI, o, 0, 0));
+        if constexpr (UPD) uv[d] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rQ, o, 0, 0));
+    };
+    unroll<k2dAhead>([&](auto dc) { fetch(dc, decltype(dc)::value); });
+    // the row above the wave's first: elements 4 g .. 4 g + 3 once wave w - 1 has done g + k2dLag groups
+    const uint32_t* const above = edges + (w - 1) * elen + k2dPad;
+    uint32_t* const below = edges + w * elen + k2dPad;
+    u32x4 edge = {0, 0, 0, 0};
+    auto wait_edge = [&](int g) {
+        if (w == 0) return;
+        const int need = min(g + k2dLag, steps);
+        int spins = 0;
+        for (;;) {
+            const int have = lget(&done[w - 1]);
+            edge = lget4(above + WF_G * min(g, steps - 1));
+            if (__builtin_amdgcn_readfirstlane(have) >= need) return;
+            if ((++spins & 1023) == 0 && (spins >= kSpinLimit || gave_up(A.err))) {
+                if (lane == 0) atomicOr(A.err, 1);
+                return;   // carry on with whatever is there
+            }
+        }
+    };
+    wait_edge(0);
+    const f32x4 none = {0.f, 0.f, 0.f, 0.f};
+    f32x4 plo = none, ilo = none, rlo = none;   // the group of steps before: operands and results
+    float m = 0.f;                              // what the lane passed on at the step before
+    for (int g8 = 0; g8 < steps; g8 += k2dAhead) {
+        unroll<k2dAhead>([&](auto dc) {
+            constexpr int d = decltype(dc)::value;
+            const int g = g8 + d;
+            const f32x4 phi = marched(pv[d]);
+            f32x4 ihi = marched(iv[d]);
+            if constexpr (UPD) {
+                const f32x4 u = marched(uv[d]);
+#pragma unroll
+                for (int j = 0; j < 4; j++) ihi[j] = __builtin_fmaf(u[j], malpha, ihi[j]);
+            }
+            fetch(dc, g + k2dAhead);
+            const f32x4 p = behind(plo, phi, c1, c2), in = behind(ilo, ihi, c1, c2);
+            plo = phi;
+            ilo = ihi;
+            f32x4 res;
+            float pass[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                // +-y: lane l - 1's value of the step before, the upstream wave's on lane 0
+                const float up = __builtin_bit_cast(
+                    float, __builtin_amdgcn_update_dpp((int)edge[j], __builtin_bit_cast(int, m), 0x138, 0xf, 0xf, false));
+                const float acc = m + up;
+                float outv, v;
+                if (FWD) {
+                    outv = (in[j] - acc) * p[j];
+                    v = outv * p[j];
+                } else {
+                    outv = (in[j] - acc * p[j]) * p[j];
+                    v = outv;
+                }
+                m = __builtin_fmaf(ms, v, 0.f);
+                res[j] = outv;
+                pass[j] = m;
+            }
+            if (w + 1 < nwaves && lane == WF_TZ - 1) {
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    *(lds_u32*)(below + WF_G * (g - 15) + j - 3) = __builtin_bit_cast(uint32_t, pass[j]);
+                lput(&done[w], g + 1);
+            }
+            const f32x4 whole = marched(ahead(rlo, res, c1, c2));
+            rlo = res;
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, whole), rO, at(g - q - 1), 0, 0);
+            wait_edge(g + 1);
+        });
+    }
+}
+
 int wave_launch(fsim_ctx* ctx, WaveKind kind, const float* in, float* out, double scale, const SideWork* side) {
     WaveArgs A = ctx->wave;
     A.in = in;
     A.out = out;
     A.scale = scale;
     A.ms = -(float)scale;
+    if (kind != WAVE_FACTOR && fits_2d(A)) {
+        const SideWork W = side ? *side : SideWork{};
+        const dim3 grid(1 + W.blocks), block(WF_THREADS);
+        const size_t lds = lds_2d(A.ny, A.nxp);
+        if (kind == WAVE_FWD) hipLaunchKernelGGL(k_wave_2d<WAVE_FWD>, grid, block, lds, ctx->stream, A, W);
+        else if (kind == WAVE_BWD) hipLaunchKernelGGL(k_wave_2d<WAVE_BWD>, grid, block, lds, ctx->stream, A, W);
+        else hipLaunchKernelGGL(k_wave_2d<WAVE_FWD_UPDATE>, grid, block, lds, ctx->stream, A, W);
+        FSIM_HIP(ctx, hipGetLastError());
+        return FSIM_OK;
+    }
     const unsigned ntiles = (unsigned)(A.TJ * A.TK);
     const int counter = kind == WAVE_FWD_UPDATE ? WAVE_FWD : kind;
     A.ticket = ctx->wave_ticket + counter;
