@@ -583,18 +583,17 @@ __global__ void k_net_output_op(const float* __restrict__ out, const float* __re
 }
 
 // ---- backward pieces (training) ----------------------------------------------------------
-// g = dy * (y > 0), as FP32 and BF16 (the BF16 copy feeds the MFMA data-gradient convolution)
-__global__ void k_relu_bwd(const float* __restrict__ dy, const __bf16* __restrict__ y, float* __restrict__ g,
-                           __bf16* __restrict__ g16, int64_t n) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float v = (float)y[i] > 0.f ? dy[i] : 0.f;
+// Every layer's output gradient g = dy * (y > 0) is kept as FP32 and BF16 (the
+// BF16 copy feeds the MFMA data-gradient convolution).  The levels of a sample
+// are small, so a pass costs its launch: dy is formed where g is.
+__device__ inline void put_relu_grad(float dy, __bf16 y, float* g, __bf16* g16, int64_t i) {
+    const float v = (float)y > 0.f ? dy : 0.f;
     g[i] = v;
     g16[i] = (__bf16)v;
 }
 
-// encoder gradient: g = (dskip + dpool[parent] / 8) * (y > 0)
-__global__ void k_pool_bwd_relu(const float* __restrict__ dskip, const float* __restrict__ dpool,
+// encoder gradient: dy = the skip's slice of dcat + dpool[parent] / 8
+__global__ void k_pool_bwd_relu(const float* __restrict__ dcat, int Cu, const float* __restrict__ dpool,
                                 const __bf16* __restrict__ y, float* __restrict__ g, __bf16* __restrict__ g16, Dims fine,
                                 int C) {
     const int64_t n = fine.V() * C;
@@ -604,15 +603,14 @@ __global__ void k_pool_bwd_relu(const float* __restrict__ dskip, const float* __
     const int64_t v = i / C;
     const int z = (int)(v % fine.W), yy = (int)((v / fine.W) % fine.H), x = (int)(v / ((int64_t)fine.W * fine.H));
     const int64_t pv = ((int64_t)(x / 2) * (fine.H / 2) + yy / 2) * (fine.W / 2) + z / 2;
-    float d = dpool ? dpool[pv * C + c] * 0.125f : 0.f;
-    if (dskip) d += dskip[i];
-    const float o = (float)y[i] > 0.f ? d : 0.f;
-    g[i] = o;
-    g16[i] = (__bf16)o;
+    float d = dpool[pv * C + c] * 0.125f;
+    d += dcat[v * (Cu + C) + Cu + c];
+    put_relu_grad(d, y[i], g, g16, i);
 }
 
-// gradient of cat(up(coarse), skip): dcoarse = sum over the 8 children, dskip = slice
-__global__ void k_upcat_bwd_up(const float* __restrict__ dcat, float* __restrict__ dcoarse, Dims fine, int Cu, int Cs) {
+// gradient of the coarse part of cat(up(coarse), skip): dy = sum over the 8 children
+__global__ void k_up_bwd_relu(const float* __restrict__ dcat, const __bf16* __restrict__ y, float* __restrict__ g,
+                              __bf16* __restrict__ g16, Dims fine, int Cu, int Cs) {
     const Dims cs{fine.D / 2, fine.H / 2, fine.W / 2};
     const int C = Cu + Cs;
     const int64_t n = cs.V() * Cu;
@@ -620,39 +618,41 @@ __global__ void k_upcat_bwd_up(const float* __restrict__ dcat, float* __restrict
     if (i >= n) return;
     const int c = (int)(i % Cu);
     const int64_t v = i / Cu;
-    const int z = (int)(v % cs.W), y = (int)((v / cs.W) % cs.H), x = (int)(v / ((int64_t)cs.W * cs.H));
+    const int z = (int)(v % cs.W), yy = (int)((v / cs.W) % cs.H), x = (int)(v / ((int64_t)cs.W * cs.H));
+    float t[8];
+#pragma unroll
+    for (int d = 0; d < 8; d++)
+        t[d] = dcat[(((int64_t)(2 * x + (d >> 2)) * fine.H + 2 * yy + ((d >> 1) & 1)) * fine.W + 2 * z + (d & 1)) * C + c];
     float s = 0.f;
-    for (int d = 0; d < 8; d++) {
-        const int64_t fv = ((int64_t)(2 * x + (d >> 2)) * fine.H + 2 * y + ((d >> 1) & 1)) * fine.W + 2 * z + (d & 1);
-        s += dcat[fv * C + c];
-    }
-    dcoarse[i] = s;
-}
-__global__ void k_upcat_bwd_skip(const float* __restrict__ dcat, float* __restrict__ dskip, Dims fine, int Cu, int Cs) {
-    const int64_t n = fine.V() * Cs;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const int c = (int)(i % Cs);
-    const int64_t v = i / Cs;
-    dskip[i] = dcat[v * (Cu + Cs) + Cu + c];
+#pragma unroll
+    for (int d = 0; d < 8; d++) s += t[d];
+    put_relu_grad(s, y[i], g, g16, i);
 }
 
-// data-gradient weights: Wb[ci][t' * Cout + co] = W[co][(26 - t') * Cin + ci]
-__global__ void k_flip_weights(const __bf16* __restrict__ w, __bf16* __restrict__ wb, int cin, int cout) {
-    const int64_t n = (int64_t)cout * 27 * cin;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+// data-gradient weights: Wb[ci][t' * Cout + co] = W[co][(26 - t') * Cin + ci], of layers 1 .. 6
+struct FlipArgs {
+    const __bf16* w;
+    __bf16* wb;
+    int64_t from[kNetLayers], to[kNetLayers + 1];   // offsets of a layer's weights in w and wb; wb's end
+};
+__global__ void k_flip_weights(FlipArgs A) {
+    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= A.to[kNetLayers]) return;
+    int l = 1;
+    while (i >= A.to[l + 1]) l++;
+    const int cin = kLayers[l].cin, cout = kLayers[l].cout;
+    i -= A.to[l];
     const int co = (int)(i % cout);
     const int64_t r = i / cout;
     const int tp = (int)(r % 27), ci = (int)(r / 27);
-    wb[i] = w[(int64_t)co * 27 * cin + (int64_t)(26 - tp) * cin + ci];
+    A.wb[A.to[l] + i] = A.w[A.from[l] + (int64_t)co * 27 * cin + (int64_t)(26 - tp) * cin + ci];
 }
 
 // Weight gradient of one 3x3x3 convolution on MFMA: dW[co][t][ci] = sum_v g[v][co] x[v + off(t)][ci],
 // one GEMM per tap with M = Cout, N = Cin, K = voxels.  Block (voxel slice, tap t): its 4 waves take
 // the slice's 32-voxel chunks in turn, each accumulating every 16 x 16 (co, ci) tile with
 // v_mfma_f32_16x16x32_bf16; a wave's partial goes to partials[slice * 4 + wave][co][t][ci] and the
-// partials are summed in that order (k_sum_parts).  A (16 co x 32 v): lane l holds co = 16 mi + l % 16
+// partials are summed in that order (k_wgrad_sums).  A (16 co x 32 v): lane l holds co = 16 mi + l % 16
 // at voxels v0 + 8 (l / 16) .. + 7; B (32 v x 16 ci): ci = 16 ni + l % 16 at the same voxels,
 // shifted by the tap (zero outside the grid; Cin = 8 is padded to one 16-wide tile).  Operands are
 // the layer's BF16 output gradient and its BF16 input activations, sums in FP32.
@@ -715,16 +715,18 @@ __global__ void __launch_bounds__(256) k_conv3_wgrad(const __bf16* __restrict__ 
 }
 
 // sum of nparts partial vectors of length n, in partial order
-__global__ void k_sum_parts(const float* __restrict__ parts, int nparts, int64_t n, float* __restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    out[i] = sum_in_order(parts + i, n, nparts);
-}
-
-// bias gradient: db[c] = sum_v g[v][c] (one block per channel, fixed order)
-__global__ void __launch_bounds__(256) k_bias_grad(const float* __restrict__ g, int64_t V, int C, float* __restrict__ db) {
+// and the bias gradient db[c] = sum_v g[v][c], a block per channel behind the weights' blocks, in a fixed order
+__global__ void __launch_bounds__(256) k_wgrad_sums(const float* __restrict__ parts, int nparts, int64_t n,
+                                                    float* __restrict__ out, const float* __restrict__ g, int64_t V, int C,
+                                                    float* __restrict__ db) {
+    const unsigned wblocks = (unsigned)((n + 255) / 256);
+    if (blockIdx.x < wblocks) {
+        const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+        if (i < n) out[i] = sum_in_order(parts + i, n, nparts);
+        return;
+    }
     __shared__ float red[256];
-    const int c = blockIdx.x;
+    const int c = (int)(blockIdx.x - wblocks);
     const int64_t mine = (int64_t)threadIdx.x < V ? (V - threadIdx.x + blockDim.x - 1) / blockDim.x : 0;
     red[threadIdx.x] = mine > 0 ? sum_in_order(g + (int64_t)threadIdx.x * C + c, (int64_t)blockDim.x * C, (int)mine) : 0.f;
     __syncthreads();
@@ -735,12 +737,12 @@ __global__ void __launch_bounds__(256) k_bias_grad(const float* __restrict__ g, 
     if (threadIdx.x == 0) db[c] = red[0];
 }
 
-// output layer backward: dd0[v][c] = dout[v] * w[c];  dw[c] = sum_v dout[v] d0[v][c];  db = sum dout
-__global__ void k_conv1_bwd_data(const float* __restrict__ dout, const float* __restrict__ w, float* __restrict__ dd0,
-                                 int64_t V) {
+// output layer backward: dy of d0 = dout[v] * w[c];  dw[c] = sum_v dout[v] d0[v][c];  db = sum dout
+__global__ void k_conv1_bwd_relu(const float* __restrict__ dout, const float* __restrict__ w, const __bf16* __restrict__ y,
+                                 float* __restrict__ g, __bf16* __restrict__ g16, int64_t V) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= V * kOutIn) return;
-    dd0[i] = dout[i / kOutIn] * (float)(__bf16)w[i % kOutIn];
+    put_relu_grad(dout[i / kOutIn] * (float)(__bf16)w[i % kOutIn], y[i], g, g16, i);
 }
 __global__ void __launch_bounds__(256) k_conv1_bwd_weight(const float* __restrict__ dout, const __bf16* __restrict__ d0,
                                                           int64_t V, float* __restrict__ dw) {
@@ -860,14 +862,15 @@ struct LearnedNet {
     int64_t part_cap = 0;
     // training (per size)
     bool train_ready = false;
-    float *in_b = nullptr, *in_op = nullptr, *target = nullptr, *dout = nullptr, *dd0 = nullptr;
+    float *in_b = nullptr, *in_op = nullptr, *target = nullptr, *dout = nullptr;
+    int64_t unknowns = 0;             // of the uploaded sample
     uint8_t* fluid = nullptr;
     float* aop = nullptr;             // the sample's operator in network layout (energy loss)
     float* eres = nullptr;            // energy loss: out - target on the unknowns
     double energy_t = 0.0;            // energy loss: t^T A t of the uploaded sample
     float* g32[kNetLayers] = {};
     __bf16* g16[kNetLayers] = {};
-    float *dcat[3] = {}, *dcoarse[3] = {}, *dskip[3] = {}, *dpool[3] = {};
+    float *dcat[3] = {}, *dpool[3] = {};
     std::vector<void*> pallocs, allocs;   // parameter-sized, per-size
 };
 
@@ -938,6 +941,17 @@ static int learned_alloc(fsim_ctx* ctx, int nx, int ny, int nz) {
     return FSIM_OK;
 }
 
+static FlipArgs flip_args(const LearnedNet* N) {
+    FlipArgs A{};
+    A.w = N->w16;
+    A.wb = N->wflip;
+    for (int l = 1; l < kNetLayers; l++) {
+        A.from[l] = N->woff[l];
+        A.to[l + 1] = A.to[l] + conv_weights(l);
+    }
+    return A;
+}
+
 // training buffers for samples on the context's own grid
 static int learned_alloc_train(fsim_ctx* ctx) {
     FSIM_TRY(learned_alloc(ctx, ctx->g.nx, ctx->g.ny, ctx->g.nz));
@@ -947,7 +961,7 @@ static int learned_alloc_train(fsim_ctx* ctx) {
         std::vector<void*>& P = N->pallocs;
         if ((rc = nalloc(ctx, P, &N->adam_m, N->nparams)) || (rc = nalloc(ctx, P, &N->adam_v, N->nparams)) ||
             (rc = nalloc(ctx, P, &N->grad, N->nparams)) || (rc = nalloc(ctx, P, &N->grad_acc, N->nparams)) ||
-            (rc = nalloc(ctx, P, &N->loss_parts, 1024)) || (rc = nalloc(ctx, P, &N->wflip, 64 * 27 * 192)))
+            (rc = nalloc(ctx, P, &N->loss_parts, 1024)) || (rc = nalloc(ctx, P, &N->wflip, flip_args(N).to[kNetLayers])))
             return rc;
         N->wparts_cap = 64LL * 64 * 27 * 192;
         if ((rc = nalloc(ctx, P, &N->wparts, N->wparts_cap))) return rc;
@@ -962,7 +976,7 @@ static int learned_alloc_train(fsim_ctx* ctx) {
     std::vector<void*>& A = N->allocs;
     if ((rc = nalloc(ctx, A, &N->in_b, ctx->g.nc)) || (rc = nalloc(ctx, A, &N->in_op, 4 * ctx->g.nc)) ||
         (rc = nalloc(ctx, A, &N->target, V0)) || (rc = nalloc(ctx, A, &N->fluid, V0)) ||
-        (rc = nalloc(ctx, A, &N->dout, V0)) || (rc = nalloc(ctx, A, &N->dd0, V0 * 16)) ||
+        (rc = nalloc(ctx, A, &N->dout, V0)) ||
         (rc = nalloc(ctx, A, &N->cat[2], V2 * 192)) || (rc = nalloc(ctx, A, &N->cat[1], V1 * 96)) ||
         (rc = nalloc(ctx, A, &N->cat[0], V0 * 48)) || (rc = nalloc(ctx, A, &N->aop, 4 * V0)) ||
         (rc = nalloc(ctx, A, &N->eres, V0)))
@@ -971,12 +985,10 @@ static int learned_alloc_train(fsim_ctx* ctx) {
         const int64_t n = Vl[kLayers[l].level] * kLayers[l].cout;
         if ((rc = nalloc(ctx, A, &N->g32[l], n)) || (rc = nalloc(ctx, A, &N->g16[l], n))) return rc;
     }
-    // concat data gradients at levels 2, 1, 0 and their splits
+    // concat data gradients at levels 2, 1, 0
     const int cu[3] = {32, 64, 128}, cs[3] = {16, 32, 64};   // index = level
     for (int l = 0; l < 3; l++) {
-        if ((rc = nalloc(ctx, A, &N->dcat[l], Vl[l] * (cu[l] + cs[l]))) ||
-            (rc = nalloc(ctx, A, &N->dcoarse[l], Vl[l + 1] * cu[l])) || (rc = nalloc(ctx, A, &N->dskip[l], Vl[l] * cs[l])))
-            return rc;
+        if ((rc = nalloc(ctx, A, &N->dcat[l], Vl[l] * (cu[l] + cs[l])))) return rc;
     }
     // data gradients of the pooled inputs: dpool[l] at level l + 1 with the channels of e[l]
     const int pc[3] = {16, 32, 64};
@@ -1172,22 +1184,25 @@ static int upload_sample(fsim_ctx* ctx, const float* b, const float* op, const d
     if (p) {
         const Dims d = N->lv[0];
         const int64_t V = d.V();
-        std::vector<float> t((size_t)V, 0.f), a((size_t)(4 * V), 0.f);
+        const bool energy = ctx->learned_loss == 1;   // which alone reads the operator
+        std::vector<float> t((size_t)V, 0.f), a(energy ? (size_t)(4 * V) : 0, 0.f);
         std::vector<uint8_t> f((size_t)V, 0);
         const float inv = s > 0.f ? 1.f / s : 0.f;
+        int64_t unknowns = 0;
         for (int x = 0; x < nx; x++)
             for (int y = 0; y < ny; y++)
                 for (int z = 0; z < nz; z++) {
                     const int64_t i = ((int64_t)x * ny + y) * nz + z, v = ((int64_t)x * d.H + y) * d.W + z;
                     if (!(op[i] > 0.f)) continue;
                     f[(size_t)v] = 1;
+                    unknowns++;
                     t[(size_t)v] = (float)p[i] * inv;
-                    for (int k = 0; k < 4; k++) a[(size_t)(k * V + v)] = op[k * nc + i];
+                    for (int k = 0; energy && k < 4; k++) a[(size_t)(k * V + v)] = op[k * nc + i];
                 }
         // t^T A t in FP64 over the unknowns
         double et = 0.0;
         const int64_t sx = (int64_t)d.H * d.W, sy = d.W;
-        for (int x = 0; x < nx; x++)
+        for (int x = 0; energy && x < nx; x++)
             for (int y = 0; y < ny; y++)
                 for (int z = 0; z < nz; z++) {
                     const int64_t v = ((int64_t)x * d.H + y) * d.W + z;
@@ -1202,9 +1217,11 @@ static int upload_sample(fsim_ctx* ctx, const float* b, const float* op, const d
                     et += (double)t[(size_t)v] * at;
                 }
         N->energy_t = et;
+        N->unknowns = unknowns;
         FSIM_HIP(ctx, hipMemcpyAsync(N->target, t.data(), sizeof(float) * t.size(), hipMemcpyHostToDevice, ctx->stream));
         FSIM_HIP(ctx, hipMemcpyAsync(N->fluid, f.data(), f.size(), hipMemcpyHostToDevice, ctx->stream));
-        FSIM_HIP(ctx, hipMemcpyAsync(N->aop, a.data(), sizeof(float) * a.size(), hipMemcpyHostToDevice, ctx->stream));
+        if (energy)
+            FSIM_HIP(ctx, hipMemcpyAsync(N->aop, a.data(), sizeof(float) * a.size(), hipMemcpyHostToDevice, ctx->stream));
         // the host vectors go out of scope: wait for the copies
         FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
     }
@@ -1257,21 +1274,18 @@ static int wgrad(fsim_ctx* ctx, int l, const float* g32, const __bf16* g16, cons
     default: ok = false;
     }
     if (!ok) return set_err(ctx, FSIM_ERR_INVALID, "learned network: no weight-gradient kernel for this layer");
-    hipLaunchKernelGGL(k_sum_parts, dim3(gb(n)), dim3(256), 0, ctx->stream, N->wparts, nblk * kWgWaves, n,
-                       N->grad + N->woff[l]);
-    hipLaunchKernelGGL(k_bias_grad, dim3(cout), dim3(256), 0, ctx->stream, g32, V, cout, N->grad + N->boff[l]);
+    hipLaunchKernelGGL(k_wgrad_sums, dim3(gb(n) + (unsigned)cout), dim3(256), 0, ctx->stream, N->wparts, nblk * kWgWaves, n,
+                       N->grad + N->woff[l], g32, V, cout, N->grad + N->boff[l]);
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;
 }
 
-// data gradient of layer l's input: dx = conv3(g16, flipped weights)
+// data gradient of layer l's input: dx = conv3(g16, flipped weights of k_flip_weights)
 static int dgrad(fsim_ctx* ctx, int l, const __bf16* g16, float* dx) {
     LearnedNet* N = ctx->learned;
     const Dims d = N->lv[kLayers[l].level];
     const int cin = kLayers[l].cin, cout = kLayers[l].cout;
-    hipLaunchKernelGGL(k_flip_weights, dim3(gb((int64_t)cout * 27 * cin)), dim3(256), 0, ctx->stream, N->w16 + N->woff[l],
-                       N->wflip, cin, cout);
-    ConvArgs a{g16, N->wflip, nullptr, dx, d.D, d.H, d.W, cout, cin, 0, nullptr, 0, 0, N->part, N->part_cap};
+    ConvArgs a{g16, N->wflip + flip_args(N).to[l], nullptr, dx, d.D, d.H, d.W, cout, cin, 0, nullptr, 0, 0, N->part, N->part_cap};
     if (!launch_conv3<true>(ctx->stream, a))
         return set_err(ctx, FSIM_ERR_INVALID, "learned network: convolution shape without a kernel");
     FSIM_HIP(ctx, hipGetLastError());
@@ -1284,13 +1298,7 @@ static int net_backward(fsim_ctx* ctx, double* loss) {
     hipStream_t st = ctx->stream;
     const Dims* L = N->lv;
     const int64_t V0 = L[0].V();
-    int64_t nfl = 0;
-    {
-        std::vector<uint8_t> f((size_t)V0);
-        FSIM_HIP(ctx, hipMemcpyAsync(f.data(), N->fluid, f.size(), hipMemcpyDeviceToHost, st));
-        FSIM_HIP(ctx, hipStreamSynchronize(st));
-        for (uint8_t c : f) nfl += c;
-    }
+    const int64_t nfl = N->unknowns;
     const float inv_n = nfl > 0 ? 1.f / (float)nfl : 0.f;
     const int nlb = 256;
     if (ctx->learned_loss == 1) {
@@ -1301,35 +1309,29 @@ static int net_backward(fsim_ctx* ctx, double* loss) {
         hipLaunchKernelGGL(k_mse, dim3(nlb), dim3(256), 0, st, N->out, N->target, N->fluid, V0, inv_n, N->dout,
                            N->loss_parts);
     }
+    const FlipArgs flip = flip_args(N);
+    hipLaunchKernelGGL(k_flip_weights, dim3(gb(flip.to[kNetLayers])), dim3(256), 0, st, flip);
     // output layer
-    hipLaunchKernelGGL(k_conv1_bwd_data, dim3(gb(V0 * kOutIn)), dim3(256), 0, st, N->dout, N->w32 + N->out_w, N->dd0, V0);
+    hipLaunchKernelGGL(k_conv1_bwd_relu, dim3(gb(V0 * kOutIn)), dim3(256), 0, st, N->dout, N->w32 + N->out_w, N->dd[0],
+                       N->g32[6], N->g16[6], V0);
     hipLaunchKernelGGL(k_conv1_bwd_weight, dim3(kOutIn + 1), dim3(256), 0, st, N->dout, N->dd[0], V0, N->grad + N->out_w);
-    // decoder: layer 6 (level 0), 5 (level 1), 4 (level 2)
-    const float* dy = N->dd0;
+    // decoder: layer 6 (level 0), 5 (level 1), 4 (level 2); each leaves the output gradient of the layer
+    // before it, whose output is its coarse input (d1, d2, e3)
     for (int l = 6; l >= 4; l--) {
         const int lev = kLayers[l].level;
-        const int64_t n = L[lev].V() * kLayers[l].cout;
-        hipLaunchKernelGGL(k_relu_bwd, dim3(gb(n)), dim3(256), 0, st, dy, N->dd[lev], N->g32[l], N->g16[l], n);
         FSIM_TRY(wgrad(ctx, l, N->g32[l], N->g16[l], N->cat[lev]));
         FSIM_TRY(dgrad(ctx, l, N->g16[l], N->dcat[lev]));
         const int Cs = kLayers[l].cin / 3, Cu = kLayers[l].cin - Cs;
-        hipLaunchKernelGGL(k_upcat_bwd_up, dim3(gb(L[lev + 1].V() * Cu)), dim3(256), 0, st, N->dcat[lev], N->dcoarse[lev],
-                           L[lev], Cu, Cs);
-        hipLaunchKernelGGL(k_upcat_bwd_skip, dim3(gb(L[lev].V() * Cs)), dim3(256), 0, st, N->dcat[lev], N->dskip[lev],
-                           L[lev], Cu, Cs);
-        dy = N->dcoarse[lev];   // gradient of the coarse decoder output (d1, d2) or of e3
+        hipLaunchKernelGGL(k_up_bwd_relu, dim3(gb(L[lev + 1].V() * Cu)), dim3(256), 0, st, N->dcat[lev],
+                           l == 4 ? N->e[3] : N->dd[lev + 1], N->g32[l - 1], N->g16[l - 1], L[lev], Cu, Cs);
     }
-    // bottleneck, layer 3 at level 3: its output e3's gradient is dcoarse[2]
-    {
-        const int64_t n = L[3].V() * 128;
-        hipLaunchKernelGGL(k_relu_bwd, dim3(gb(n)), dim3(256), 0, st, N->dcoarse[2], N->e[3], N->g32[3], N->g16[3], n);
-        FSIM_TRY(wgrad(ctx, 3, N->g32[3], N->g16[3], N->pl[2]));
-        FSIM_TRY(dgrad(ctx, 3, N->g16[3], N->dpool[2]));
-    }
+    // bottleneck, layer 3 at level 3
+    FSIM_TRY(wgrad(ctx, 3, N->g32[3], N->g16[3], N->pl[2]));
+    FSIM_TRY(dgrad(ctx, 3, N->g16[3], N->dpool[2]));
     // encoder layers 2, 1, 0: gradient of e[l] = skip gradient + pooled-input gradient of layer l + 1
     for (int l = 2; l >= 0; l--) {
         const int C = kLayers[l].cout;
-        hipLaunchKernelGGL(k_pool_bwd_relu, dim3(gb(L[l].V() * C)), dim3(256), 0, st, N->dskip[l], N->dpool[l], N->e[l],
+        hipLaunchKernelGGL(k_pool_bwd_relu, dim3(gb(L[l].V() * C)), dim3(256), 0, st, N->dcat[l], 2 * C, N->dpool[l], N->e[l],
                            N->g32[l], N->g16[l], L[l], C);
         FSIM_TRY(wgrad(ctx, l, N->g32[l], N->g16[l], l == 0 ? N->x0 : N->pl[l - 1]));
         if (l > 0) FSIM_TRY(dgrad(ctx, l, N->g16[l], N->dpool[l - 1]));
@@ -1352,9 +1354,7 @@ int learned_grad_host(fsim_ctx* ctx, const float* b, const float* op, const doub
     FSIM_TRY(upload_sample(ctx, b, op, p, &s));
     FSIM_TRY(net_forward(ctx, true));
     FSIM_TRY(net_backward(ctx, loss));
-    FSIM_HIP(ctx, hipMemcpyAsync(grad, N->grad, sizeof(float) * N->nparams, hipMemcpyDeviceToHost, ctx->stream));
-    FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return FSIM_OK;
+    return read_back(ctx, grad, N->grad, sizeof(float) * N->nparams);
 }
 
 __global__ void k_axpy_f(float* __restrict__ y, const float* __restrict__ x, int64_t n) {
