@@ -314,6 +314,7 @@ struct fsim_ctx {
     uint32_t* chunk_flags = nullptr;  // solver-vector chunks (256 values) holding a WATER cell, per solve
 
     // pressure solve
+    float* vectors = nullptr;         // the allocation of the FP32 vectors below
     float *b = nullptr, *r = nullptr, *z = nullptr, *s = nullptr, *q = nullptr;
     float* s2 = nullptr;              // second search-direction buffer (swapped with s)
     float* t = nullptr;               // forward sweep's result
