@@ -248,7 +248,6 @@ struct SolveScalars {
     double rr, rmax, bb;             // recursive residual ||r||^2, max|r|, ||b||^2
     double tr_ss, tr_max;            // true residual ||b-Ax||^2, max|b-Ax|
     double zr;                       // z.r
-    double zq;                       // z.q (flexible PCG)
     double nfluid;                   // number of WATER cells of the solve
     int64_t wave_err;                // host copy: the wavefront kernels' error flag
     int nan_flag;

@@ -27,8 +27,7 @@ __device__ inline double wave_max(double v) {
 // result is deterministic, and no separate finalize launch is needed.
 constexpr int AUX_NONE = 0, AUX_MAX = 1, AUX_SUM = 2;
 enum FinOp {
-    FIN_NONE = -1, FIN_BB = 0, FIN_SIGMA0 = 1, FIN_ALPHA = 2, FIN_RES = 3, FIN_BETA = 4, FIN_TRUE = 5, FIN_ZQ = 6,
-    FIN_FBETA = 7
+    FIN_NONE = -1, FIN_BB = 0, FIN_SIGMA0 = 1, FIN_ALPHA = 2, FIN_RES = 3, FIN_BETA = 4, FIN_TRUE = 5, FIN_FBETA = 6
 };
 
 struct Reduce {
@@ -62,11 +61,10 @@ __device__ inline void apply_fin(int op, double s, double m, SolveScalars* sc) {
         break;
     }
     case FIN_TRUE: sc->tr_ss = s; sc->tr_max = m; break;
-    case FIN_ZQ: sc->zq = s; break;
-    case FIN_FBETA: {   // flexible PCG: beta = z'.(r' - r) / z.r = -alpha z'.q / z.r
+    case FIN_FBETA: {   // s = z'.r', m = z'.q.  Flexible PCG: beta = z'.(r' - r) / z.r = -alpha z'.q / z.r
         if (sc->sigma != sc->sigma) sc->nan_flag |= 2;
         sc->zr = s;
-        sc->beta = -sc->alpha * sc->zq / sc->sigma;
+        sc->beta = -sc->alpha * m / sc->sigma;
         break;
     }
     default: break;

@@ -403,6 +403,32 @@ __global__ void __launch_bounds__(kStream) k_dot(int64_t n, const uint32_t* __re
     block_finish<AUX_NONE, kStream>(d, 0.0, red);
 }
 
+// z . r and z . q: z is read once, and one launch and its tickets are saved
+// (128^3: 2 x 7.5 -> 9.3 us, 256^3: 2 x 18.5 -> 27.5)
+__global__ void __launch_bounds__(kStream) k_dot_zr_zq(int64_t n, const uint32_t* __restrict__ flags,
+                                                      const float* __restrict__ z, const float* __restrict__ r,
+                                                      const float* __restrict__ q, Reduce red) {
+    double zr = 0.0, zq = 0.0;
+    for_flagged_chunks<3>(
+        whole_grid(), n, flags,
+        [&](int64_t i, float4(&v)[3]) {
+            v[0] = *reinterpret_cast<const float4*>(z + i);
+            v[1] = *reinterpret_cast<const float4*>(r + i);
+            v[2] = *reinterpret_cast<const float4*>(q + i);
+        },
+        [&](int64_t, float4(&v)[3]) {
+            zr += (double)v[0].x * (double)v[1].x;
+            zr += (double)v[0].y * (double)v[1].y;
+            zr += (double)v[0].z * (double)v[1].z;
+            zr += (double)v[0].w * (double)v[1].w;
+            zq += (double)v[0].x * (double)v[2].x;
+            zq += (double)v[0].y * (double)v[2].y;
+            zq += (double)v[0].z * (double)v[2].z;
+            zq += (double)v[0].w * (double)v[2].w;
+        });
+    block_finish<AUX_SUM, kStream>(zr, zq, red);
+}
+
 // FP64 true residual t = b - A x; optionally r = (float)t.
 __global__ void __launch_bounds__(kBlock) k_true_residual(SolveArgs S, const uint16_t* __restrict__ nbinfo,
                                                           const float* __restrict__ b, const double* __restrict__ x,
@@ -790,8 +816,11 @@ static int update_flexible(fsim_ctx* ctx, const SolveArgs& S, bool x_due) {
         FSIM_HIP(ctx, hipGetLastError());
     }
     FSIM_TRY(mg_apply(ctx, ctx->r, ctx->z, S.scale));
-    FSIM_TRY(dot_with(ctx, ctx->z, ctx->q, FIN_ZQ));
-    return dot_with(ctx, ctx->z, ctx->r, FIN_FBETA);
+    FSIM_PROF(ctx, KID_DOT);
+    hipLaunchKernelGGL(k_dot_zr_zq, dim3(stream_blocks(S.ncr)), dim3(kStream), 0, ctx->stream, S.ncr, ctx->chunk_flags, ctx->z,
+                       ctx->r, ctx->q, reduce_to(ctx, FIN_FBETA));
+    FSIM_HIP(ctx, hipGetLastError());
+    return FSIM_OK;
 }
 // z = M^-1 r and sigma, at the start and after a restart
 static int precondition(fsim_ctx* ctx, const SolveArgs& S, const float* r, bool flexible) {
