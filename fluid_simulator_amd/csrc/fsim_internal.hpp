@@ -27,7 +27,6 @@ namespace fsim {
 
 constexpr int kMaxObstacles = 64;
 constexpr int kBlock = 256;
-constexpr int kReadSlots = 12;         // pinned slots of read_back
 constexpr unsigned kMaxParts = 2048;   // reduction grids have at most this many blocks
 
 // nbinfo bit layout
@@ -357,7 +356,6 @@ struct fsim_ctx {
     fsim_gfx_particle* gfx_staging = nullptr;
     int64_t gfx_cap = 0;
 
-    hipEvent_t rb_ev[fsim::kReadSlots] = {};   // read_back: a pinned slot is filled
     bool rb_counted = false;
 
     // obstacles

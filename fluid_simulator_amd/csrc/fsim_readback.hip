@@ -16,6 +16,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstdint>
 #include <cstring>
 #include <exception>
@@ -28,14 +29,16 @@
 namespace fsim {
 
 constexpr size_t kSlotBytes = size_t(2) << 20;
+constexpr int kReadSlots = 12;                // pinned slots
 constexpr int kMaxThreads = 8;               // 67 MB of new pages: 1.2 ms by 8 threads, 1.0 by 16, 5.1 by one
 // Below it hipMemcpy, which copies pages that exist (small arrays come from a
 // program's heap) in 0.1 ms.
 constexpr size_t kDirectBytes = size_t(1) << 20;
-// A piece costs 10 to 20 us beside its bytes, but the threads need several
-// each: 1 MB pieces take 0.40 / 0.63 / 1.33 / 2.46 ms for 8 / 15 / 34 / 67 MB of
-// existing pages, 2 MB pieces 0.48 / 0.77 / 1.08 / 1.91 (hipMemcpy 0.49 / 0.86 /
-// 1.95 / 3.91; new pages 0.5 / 0.7 / 1.5 / 2.3 against 1.1 / 2.0 / 3.7 / 6.7).
+// The threads need several pieces each, and a piece costs its launch.  ms for
+// existing pages of 4 / 8 / 15 / 34 / 67 MB: 0.19 / 0.32 / 0.52 / 0.95 / 1.7
+// (with hipMemcpyAsync and an event per piece 0.25 / 0.41 / 0.67 / 1.1 / 2.0,
+// hipMemcpy 0.25 / 0.49 / 0.86 / 1.95 / 3.91); new pages 0.4 / 0.45 / 0.66 / 1.4
+// / 2.1 (hipMemcpy 0.7 / 1.1 / 2.0 / 3.7 / 6.7).
 static size_t piece_of(size_t bytes) {
     return bytes >= size_t(24) << 20 ? kSlotBytes : bytes >= size_t(4) << 20 ? kSlotBytes / 2 : kSlotBytes / 4;
 }
@@ -87,8 +90,6 @@ void readback_init(fsim_ctx* ctx) {
     g_contexts++;
 }
 void readback_free(fsim_ctx* ctx) {
-    for (auto& e : ctx->rb_ev)
-        if (e) (void)hipEventDestroy(e);
     if (!ctx->rb_counted) return;
     char* unused = nullptr;
     {
@@ -107,7 +108,7 @@ struct PinnedSlots {
         }
         if (p) return;
         // portable: the next borrower may be a context of another GPU
-        if (hipHostMalloc(reinterpret_cast<void**>(&p), kSlotBytes * kReadSlots, hipHostMallocPortable) != hipSuccess) {
+        if (hipHostMalloc(reinterpret_cast<void**>(&p), kSlotBytes * kReadSlots + sizeof(unsigned) * kReadSlots, hipHostMallocPortable) != hipSuccess) {
             (void)hipGetLastError();
             p = nullptr;
         }
@@ -123,25 +124,55 @@ struct PinnedSlots {
     PinnedSlots& operator=(const PinnedSlots&) = delete;
 };
 
-static bool make_events(fsim_ctx* ctx) {
-    for (auto& e : ctx->rb_ev) {
-        if (e || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess) continue;
-        (void)hipGetLastError();
-        e = nullptr;
-        return false;
+// A piece into its pinned slot, by a kernel: the next piece's follows without an
+// event between them (which cost 20 us a piece), and the last block to finish
+// stores the piece's number + 1 in the slot's flag, behind the data.  The flags
+// are in pinned memory as well.
+constexpr int kPieceBlocks = 64;
+struct Piece {
+    const char* src;
+    char* slot;
+    unsigned bytes;
+    unsigned* finished;   // blocks done (0 between launches)
+    unsigned* flag;
+    unsigned value;
+};
+__global__ void __launch_bounds__(256) k_piece(Piece P) {
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    const unsigned words = P.bytes / 16, step = gridDim.x * 256;
+    // 16 bytes at a time where the source allows it (the slots are aligned), 4 otherwise
+    if ((reinterpret_cast<uintptr_t>(P.src) & 15) == 0) {
+        const u32x4* const from = reinterpret_cast<const u32x4*>(P.src);
+        u32x4* const to = reinterpret_cast<u32x4*>(P.slot);
+        for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < words; i += step) to[i] = from[i];
+        for (unsigned i = words * 16 + blockIdx.x * 256 + threadIdx.x; i < P.bytes; i += step) P.slot[i] = P.src[i];
+    } else if ((reinterpret_cast<uintptr_t>(P.src) & 3) == 0) {
+        for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < P.bytes / 4; i += step)
+            reinterpret_cast<unsigned*>(P.slot)[i] = reinterpret_cast<const unsigned*>(P.src)[i];
+        for (unsigned i = P.bytes / 4 * 4 + blockIdx.x * 256 + threadIdx.x; i < P.bytes; i += step) P.slot[i] = P.src[i];
+    } else {
+        for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < P.bytes; i += step) P.slot[i] = P.src[i];
     }
-    return true;
+    __threadfence_system();
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (__hip_atomic_fetch_add(P.finished, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1) {
+            __hip_atomic_store(P.finished, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __threadfence_system();
+            __hip_atomic_store(P.flag, P.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    }
 }
 
-// One copy: the calling thread has the device fill the slots in order and says
-// how many pieces have arrived; thread t copies the pieces t, t + threads, ...
+// One copy: the calling thread has the device fill the slots in order; thread t
+// copies the pieces t, t + threads, ... as their flags arrive.
 struct Copy {
     char* dst;
     const char* src;
     size_t bytes, piece, skew;   // pieces end at multiples of `piece` in the destination's addresses
     int pieces, threads;
     char* pin;
-    std::atomic<int> arrived{0};
+    unsigned* flags;                     // of the slots, pinned
     std::atomic<bool> stop{false};
     std::atomic<int> left[kReadSlots];   // last piece copied out of the slot, + 1
 
@@ -154,32 +185,52 @@ struct Copy {
     }
     void work(int t) {
         for (int k = t; k < pieces; k += threads) {
-            while (arrived.load(std::memory_order_acquire) <= k) {
+            while (!arrived(k)) {
                 if (stop.load(std::memory_order_relaxed)) return;
                 std::this_thread::yield();
             }
             copy_out(k);
         }
     }
+    bool arrived(int k) const { return __atomic_load_n(&flags[k % kReadSlots], __ATOMIC_ACQUIRE) == (unsigned)k + 1; }
     bool slot_free(int k) const {
         return k < kReadSlots || left[k % kReadSlots].load(std::memory_order_acquire) == k - kReadSlots + 1;
     }
 };
 
+// Waits for `there`; a device that takes long is waited for as a whole, which also reports its failure.
+template <class F>
+static int wait_until(fsim_ctx* ctx, F&& there) {
+    auto t0 = std::chrono::steady_clock::now();
+    while (!there()) {
+        std::this_thread::yield();
+        if (std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(100)) continue;
+        FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        t0 = std::chrono::steady_clock::now();
+    }
+    return FSIM_OK;
+}
+
 static int run_copy(fsim_ctx* ctx, Copy& C, bool alone) {
+    auto ask = [&](int k) -> int {
+        const Piece P{C.src + C.from(k), C.slot(k), (unsigned)(C.upto(k) - C.from(k)), ctx->red_count,
+                      &C.flags[k % kReadSlots], (unsigned)k + 1};
+        hipLaunchKernelGGL(k_piece, dim3(kPieceBlocks), dim3(256), 0, ctx->stream, P);
+        FSIM_HIP(ctx, hipGetLastError());
+        return FSIM_OK;
+    };
     int asked = 0;
     for (int k = 0; k < C.pieces; k++) {
-        while (asked < C.pieces && asked < k + kReadSlots && (C.slot_free(asked) || asked == k)) {
-            while (!C.slot_free(asked)) std::this_thread::yield();   // asked == k: nothing else to wait for
-            FSIM_HIP(ctx, hipMemcpyAsync(C.slot(asked), C.src + C.from(asked), C.upto(asked) - C.from(asked),
-                                         hipMemcpyDeviceToHost, ctx->stream));
-            FSIM_HIP(ctx, hipEventRecord(ctx->rb_ev[asked % kReadSlots], ctx->stream));
-            asked++;
+        if (alone) {
+            for (; asked < std::min(C.pieces, k + kReadSlots); asked++) FSIM_TRY(ask(asked));
+            FSIM_TRY(wait_until(ctx, [&] { return C.arrived(k); }));
+            C.copy_out(k);
+        } else {
+            FSIM_TRY(wait_until(ctx, [&] { return C.slot_free(k); }));
+            FSIM_TRY(ask(k));
         }
-        FSIM_HIP(ctx, hipEventSynchronize(ctx->rb_ev[k % kReadSlots]));
-        if (alone) C.copy_out(k);
-        else C.arrived.store(k + 1, std::memory_order_release);
     }
+    FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
     return FSIM_OK;
 }
 
@@ -192,7 +243,7 @@ static int direct_copy(fsim_ctx* ctx, void* dst, const void* src, size_t bytes) 
 int read_back(fsim_ctx* ctx, void* dst, const void* src, size_t bytes) {
     if (bytes < kDirectBytes) return direct_copy(ctx, dst, src, bytes);
     const PinnedSlots pinned;
-    if (!pinned.p || !make_events(ctx)) return direct_copy(ctx, dst, src, bytes);
+    if (!pinned.p) return direct_copy(ctx, dst, src, bytes);
     Copy C;
     C.dst = static_cast<char*>(dst);
     C.src = static_cast<const char*>(src);
@@ -202,6 +253,8 @@ int read_back(fsim_ctx* ctx, void* dst, const void* src, size_t bytes) {
     C.pieces = (int)((bytes + C.skew + C.piece - 1) / C.piece);
     C.threads = (int)std::min<size_t>({(size_t)kMaxThreads, (size_t)std::max(1, usable_cpus() - 1), bytes / kSlotBytes + 1});
     C.pin = pinned.p;
+    C.flags = reinterpret_cast<unsigned*>(pinned.p + kSlotBytes * kReadSlots);
+    for (int k = 0; k < kReadSlots; k++) __atomic_store_n(&C.flags[k], 0u, __ATOMIC_RELEASE);
     for (auto& v : C.left) v.store(0, std::memory_order_relaxed);
     std::thread team[kMaxThreads];
     int started = 0;
