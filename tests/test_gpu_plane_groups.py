@@ -83,7 +83,7 @@ def test_matrix_product_in_runs(gpu, shape):
     assert np.all(np.abs(got - want) <= bound)
 
 
-# the last: more than 2^22 values, where x is updated on the second stream
+# the last: more than 2^22 values
 @pytest.mark.parametrize("shape", [(5, 6, 7), (30, 17, 66), (67, 9, 70), (6, 900, 900)])
 def test_solve_fields_at_group_edges(gpu, shape):
     """Right-hand side, pressure and projected faces come back in flat order: the divergence left on the faces is
