@@ -223,7 +223,7 @@ struct WaveArgs {
     unsigned long long* ticket;
     unsigned long long ticket_base;
     int* err;
-    const uint8_t* colw;          // [y * nz + z]: 1 if the (y, z) column holds a WATER cell
+    const uint8_t* tilew;         // [2][TJ * TK]: 1 if the tile holds a WATER cell, forward and backward tiles
     const int* xrange;            // {least x, greatest x} of the WATER cells
     int send_delay;               // test option: s_sleep(127) periods of the sending waves per group
 };

@@ -132,7 +132,8 @@ template <int W>
 __global__ void __launch_bounds__(kBlock) k_rotate(SolveArgs S, const uint16_t* __restrict__ info_flat,
                                                    const float* __restrict__ b_flat, uint16_t* __restrict__ nbinfo,
                                                    float* __restrict__ b, uint32_t* __restrict__ flags,
-                                                   const uint8_t* __restrict__ xw, int* __restrict__ xrange) {
+                                                   const uint8_t* __restrict__ colw, const uint8_t* __restrict__ xw,
+                                                   int* __restrict__ xrange, uint8_t* __restrict__ tilew) {
     __shared__ uint16_t info_lds[W][WF_TZ];
     __shared__ float b_lds[W][WF_TZ];
     constexpr int nwaves = kBlock / 64, kRows = (W + WF_TZ - 1 + nwaves - 1) / nwaves;   // rows per wave
@@ -165,6 +166,21 @@ __global__ void __launch_bounds__(kBlock) k_rotate(SolveArgs S, const uint16_t* 
                 (&info_lds[0][0])[slot[j]] = n[j];
                 (&b_lds[0][0])[slot[j]] = v[j];
             }
+    }
+    // which wavefront tiles hold WATER: a wave per tile and direction (fewer than this kernel's blocks)
+    const int tk = (S.nz - 2 + WF_TZ - 1) / WF_TZ, tiles = (S.ny - 2 + WF_TY - 1) / WF_TY * tk;
+    if (k < 2 * tiles && wave == 1) {
+        const bool fwd = k < tiles;
+        const int J = (fwd ? k : k - tiles) / tk, K = (fwd ? k : k - tiles) % tk;
+        const int z = 1 + (fwd ? K : tk - 1 - K) * WF_TZ + lane;
+        bool any = false;
+#pragma unroll
+        for (int ty = 0; ty < WF_TY; ty++) {
+            const int row = J * WF_TY + ty;
+            if (row < S.ny - 2 && z <= S.nz - 2) any = any || colw[(fwd ? 1 + row : S.ny - 2 - row) * S.nz + z] != 0;
+        }
+        const bool water = __any(any);
+        if (lane == 0) tilew[k] = water ? 1 : 0;
     }
     if (k == 0 && wave == 0) {   // the x range with WATER, for the wavefront kernels
         int xlo = S.nx, xhi = -1;
@@ -592,10 +608,11 @@ static int wait_scalars(fsim_ctx* ctx) {
 }
 
 // colw: one byte per (y, z) column; behind it, each from a multiple of 4 bytes,
-// the two words of xrange, a byte per x row, and the chunk flags, cleared with it
+// the two words of xrange, a byte per x row, the chunk flags and the tiles' flags, cleared with it
 static int64_t colw_columns(int ny, int nz) { return ((int64_t)ny * nz + 3) / 4 * 4; }
 static int64_t colw_bytes(const SolveArgs& S) {
-    return colw_columns(S.ny, S.nz) + 8 + (S.nx + 3) / 4 * 4 + 4 * (S.ncr / kChunk + 1);
+    const int64_t tiles = (int64_t)((S.ny - 2 + WF_TY - 1) / WF_TY) * ((S.nz - 2 + WF_TZ - 1) / WF_TZ);
+    return colw_columns(S.ny, S.nz) + 8 + (S.nx + 3) / 4 * 4 + 4 * (S.ncr / kChunk + 1) + 2 * tiles;
 }
 static int* xrange_of(uint8_t* colw, int ny, int nz) { return reinterpret_cast<int*>(colw + colw_columns(ny, nz)); }
 
@@ -628,10 +645,12 @@ static int build_nbinfo(fsim_ctx* ctx, const SolveArgs& S, bool with_rhs) {
     int* xrange = xrange_of(ctx->colw, S.ny, S.nz);
     if (items(64) >= 2 * 256)
         hipLaunchKernelGGL(k_rotate<64>, dim3(items(64)), dim3(kBlock), 0, ctx->stream, S, A.info_flat, b_flat, ctx->nbinfo,
-                           ctx->b, ctx->chunk_flags, A.xw, xrange);
+                           ctx->b, ctx->chunk_flags, A.colw, A.xw, xrange,
+                           const_cast<uint8_t*>(ctx->wave.tilew));
     else
         hipLaunchKernelGGL(k_rotate<16>, dim3(items(16)), dim3(kBlock), 0, ctx->stream, S, A.info_flat, b_flat, ctx->nbinfo,
-                           ctx->b, ctx->chunk_flags, A.xw, xrange);
+                           ctx->b, ctx->chunk_flags, A.colw, A.xw, xrange,
+                           const_cast<uint8_t*>(ctx->wave.tilew));
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;
 }
@@ -1151,7 +1170,7 @@ int wave_init(fsim_ctx* ctx) {
     A.ybnd = ctx->ybnd;
     A.zbnd = ctx->zbnd;
     A.err = ctx->wave_err;
-    A.colw = ctx->colw;
+    A.tilew = reinterpret_cast<const uint8_t*>(ctx->chunk_flags + ctx->g.ncr / kChunk + 1);
     A.xrange = xrange_of(ctx->colw, A.ny, A.nz);
     return FSIM_OK;
 }
