@@ -516,7 +516,9 @@ k_p2g_tile_w(P2GArgs A) {
                             (d == 0 ? s_wx : s_wy)[e][k] = make_float2(al, ce);
                         }
                     }
-                    s_zh[k] = 2 * (t[2] - 1) + h[2];
+                    // held to -2 .. 2^29, beyond which no cell's stencil is reached: the doubled value stays in
+                    // 32 bits (a z far below the grid would come back as cell 0's)
+                    s_zh[k] = 2 * (min(max(t[2], -2), 1 << 29) - 1) + h[2];
                     s_pv[k] = make_float4(p[2], A.vel[0][j], A.vel[1][j], A.vel[2][j]);
                 }
                 __syncthreads();
