@@ -699,7 +699,7 @@ static int mic_apply(fsim_ctx* ctx, const SolveArgs& S, const float* r, float* t
             FSIM_TRY(wave_launch(ctx, fwd ? WAVE_FWD_UPDATE : WAVE_FWD, r, t, S.scale, fwd));
         }
         FSIM_PROF(ctx, KID_SWEEP_BWD);
-        return wave_launch(ctx, WAVE_BWD, t, z, S.scale, bwd);
+        return wave_launch(ctx, bwd ? WAVE_BWD : WAVE_BWD_ALONE, t, z, S.scale, bwd);
     }
     if (fwd) {
         hipLaunchKernelGGL((k_update_r<WF_THREADS, false>), dim3(fwd->blocks), dim3(WF_THREADS), 0, ctx->stream, fwd->n,

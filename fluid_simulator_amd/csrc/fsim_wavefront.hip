@@ -5,7 +5,8 @@
 // factor and the forward sweep, +x,+y,+z for the backward sweep), so the
 // serial lexicographic loop of the reference can run on i+j+k planes; every
 // cell performs the same operations in the same order as the serial loop, so
-// the result is bit-identical to it whatever the schedule.
+// the result is bit-identical to it whatever the schedule (values that are not
+// finite: on_water).
 //
 // Decomposition.  One workgroup owns a tile of WF_TY x 64 (y, z) columns and
 // marches along x, one rotated plane (ridx) per step: lane tz of every row
@@ -42,7 +43,8 @@
 // of the group is in the marched x range, or the lane is off the grid.  A
 // group never holds the first and the last cells of a column at once
 // (rot_planes), so the values around the range inside a group belong to cells
-// without WATER: their factor is 0 and so is every value derived from it.
+// without WATER: their factor is 0 and so is every value derived from it
+// (on_water).
 // Storing such zeros needs no mask.  The march covers the x range that holds
 // WATER (xrange), which the first pass over the labels found.
 //
@@ -103,6 +105,7 @@ template <int KIND>
 struct Kind {   // WaveKind: the sweeps (FP32)
     using T = float;
     static constexpr bool FWD = KIND == WAVE_FWD || KIND == WAVE_FWD_UPDATE;
+    static constexpr bool MASK = KIND == WAVE_FWD || KIND == WAVE_BWD_ALONE;   // on_water
     static constexpr int NP = 1;     // 32-bit words per value
 };
 template <>
@@ -416,6 +419,21 @@ __device__ void send_wave(const WaveArgs& A, WaveLds<KIND>& S, const Tile& T) {
     release(kAll);
 }
 
+// A sweep's value v of a cell whose factor is p (0 off WATER).  Off WATER it is
+// 0 by itself while every value is finite.  What is not finite (an input, or
+// the infinite factor of a WATER cell between SOLID ones) would pass through
+// AIR and SOLID cells to WATER that does not depend on it, which the sweeps
+// outside an iteration (WAVE_FWD, WAVE_BWD_ALONE) keep from it by a select.  In
+// an iteration it makes s.q and alpha NaN and the solve ends with the pressure
+// of before, wherever else it has been; there the select, a comparison and a
+// move on the chain of every cell, costs a frame 32^3 1.17 -> 1.26 ms, 128^3
+// APIC 12.3 -> 12.9, 256^3 148 -> 151.
+template <int KIND>
+__device__ inline float on_water(float v, float p) {
+    if constexpr (Kind<KIND>::MASK) return p != 0.f ? v : 0.f;
+    else return v;
+}
+
 // ---- compute waves -------------------------------------------------------------
 // Factor (KIND 0, FP64):   e = diag - sum_a (A_a p_a)^2 - tau sum_a A_a (o1 + o2) p_a^2,
 //                          guarded by sigma, p = 1/sqrt(e)  (calculatePreconditioner); passes p on
@@ -618,10 +636,10 @@ __device__ __forceinline__ void compute_wave(const WaveArgs& A, const SideWork& 
                     acc += vz;
                     float outv, v;
                     if (FWD) {
-                        outv = (in - acc) * p;
+                        outv = on_water<KIND>((in - acc) * p, p);
                         v = outv * p;
                     } else {
-                        outv = (in - acc * p) * p;
+                        outv = on_water<KIND>((in - acc * p) * p, p);
                         v = outv;
                     }
                     res[r][e] = outv;
@@ -901,10 +919,10 @@ __global__ void __launch_bounds__(WF_THREADS) k_wave_2d(WaveArgs A, SideWork W) 
                 const float acc = m + up;
                 float outv, v;
                 if (FWD) {
-                    outv = (in[j] - acc) * p[j];
+                    outv = on_water<KIND>((in[j] - acc) * p[j], p[j]);
                     v = outv * p[j];
                 } else {
-                    outv = (in[j] - acc * p[j]) * p[j];
+                    outv = on_water<KIND>((in[j] - acc * p[j]) * p[j], p[j]);
                     v = outv;
                 }
                 m = __builtin_fmaf(ms, v, 0.f);
@@ -937,12 +955,13 @@ int wave_launch(fsim_ctx* ctx, WaveKind kind, const float* in, float* out, doubl
         const size_t lds = lds_2d(A.ny, A.nxp);
         if (kind == WAVE_FWD) hipLaunchKernelGGL(k_wave_2d<WAVE_FWD>, grid, block, lds, ctx->stream, A, W);
         else if (kind == WAVE_BWD) hipLaunchKernelGGL(k_wave_2d<WAVE_BWD>, grid, block, lds, ctx->stream, A, W);
+        else if (kind == WAVE_BWD_ALONE) hipLaunchKernelGGL(k_wave_2d<WAVE_BWD_ALONE>, grid, block, lds, ctx->stream, A, W);
         else hipLaunchKernelGGL(k_wave_2d<WAVE_FWD_UPDATE>, grid, block, lds, ctx->stream, A, W);
         FSIM_HIP(ctx, hipGetLastError());
         return FSIM_OK;
     }
     const unsigned ntiles = (unsigned)(A.TJ * A.TK);
-    const int counter = kind == WAVE_FWD_UPDATE ? WAVE_FWD : kind;
+    const int counter = kind == WAVE_FWD_UPDATE ? WAVE_FWD : kind == WAVE_BWD_ALONE ? WAVE_BWD : kind;
     A.ticket = ctx->wave_ticket + counter;
     A.ticket_base = ctx->wave_ticket_base[counter];
     ctx->wave_ticket_base[counter] += ntiles;
@@ -954,6 +973,7 @@ int wave_launch(fsim_ctx* ctx, WaveKind kind, const float* in, float* out, doubl
     case WAVE_FACTOR: hipLaunchKernelGGL(k_wave<WAVE_FACTOR>, grid, block, 0, ctx->stream, A, W); break;
     case WAVE_FWD: hipLaunchKernelGGL(k_wave<WAVE_FWD>, grid, block, 0, ctx->stream, A, W); break;
     case WAVE_BWD: hipLaunchKernelGGL(k_wave<WAVE_BWD>, grid, block, 0, ctx->stream, A, W); break;
+    case WAVE_BWD_ALONE: hipLaunchKernelGGL(k_wave<WAVE_BWD_ALONE>, grid, block, 0, ctx->stream, A, W); break;
     case WAVE_FWD_UPDATE: hipLaunchKernelGGL(k_wave<WAVE_FWD_UPDATE>, grid, block, 0, ctx->stream, A, W); break;
     }
     FSIM_HIP(ctx, hipGetLastError());
