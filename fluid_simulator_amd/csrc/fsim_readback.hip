@@ -107,8 +107,11 @@ struct PinnedSlots {
             std::swap(p, g_idle);
         }
         if (p) return;
-        // portable: the next borrower may be a context of another GPU
-        if (hipHostMalloc(reinterpret_cast<void**>(&p), kSlotBytes * kReadSlots + sizeof(unsigned) * kReadSlots, hipHostMallocPortable) != hipSuccess) {
+        // portable: the next borrower may be a context of another GPU.  coherent: the host takes flags and data
+        // while later kernels run, and any flag but this one would leave that to HIP_HOST_COHERENT (off by
+        // default), with the data promised only once the stream has been synchronised
+        if (hipHostMalloc(reinterpret_cast<void**>(&p), kSlotBytes * kReadSlots + sizeof(unsigned) * kReadSlots,
+                          hipHostMallocPortable | hipHostMallocCoherent) != hipSuccess) {
             (void)hipGetLastError();
             p = nullptr;
         }
