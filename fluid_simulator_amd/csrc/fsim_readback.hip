@@ -201,14 +201,21 @@ struct Copy {
     }
 };
 
-// Waits for `there`; a device that takes long is waited for as a whole, which also reports its failure.
+// The stream's work is done: a piece whose flag is not there now never arrives.
+static int expect_arrived(fsim_ctx* ctx, const Copy& C, int k) {
+    return C.arrived(k) ? FSIM_OK : set_err(ctx, FSIM_ERR_HIP, "a piece of the copy to host memory did not arrive");
+}
+
+// Waits for `there`, which follows once piece k has arrived.  A device that
+// takes long is waited for as a whole, which also reports its failure.
 template <class F>
-static int wait_until(fsim_ctx* ctx, F&& there) {
+static int wait_until(fsim_ctx* ctx, const Copy& C, int k, F&& there) {
     auto t0 = std::chrono::steady_clock::now();
     while (!there()) {
         std::this_thread::yield();
         if (std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(100)) continue;
         FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        FSIM_TRY(expect_arrived(ctx, C, k));
         t0 = std::chrono::steady_clock::now();
     }
     return FSIM_OK;
@@ -226,14 +233,16 @@ static int run_copy(fsim_ctx* ctx, Copy& C, bool alone) {
     for (int k = 0; k < C.pieces; k++) {
         if (alone) {
             for (; asked < std::min(C.pieces, k + kReadSlots); asked++) FSIM_TRY(ask(asked));
-            FSIM_TRY(wait_until(ctx, [&] { return C.arrived(k); }));
+            FSIM_TRY(wait_until(ctx, C, k, [&] { return C.arrived(k); }));
             C.copy_out(k);
         } else {
-            FSIM_TRY(wait_until(ctx, [&] { return C.slot_free(k); }));
+            FSIM_TRY(wait_until(ctx, C, k - kReadSlots, [&] { return C.slot_free(k); }));
             FSIM_TRY(ask(k));
         }
     }
     FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    // the threads wait for the last pieces' flags (the others' have been copied out)
+    for (int k = std::max(0, C.pieces - kReadSlots); k < C.pieces; k++) FSIM_TRY(expect_arrived(ctx, C, k));
     return FSIM_OK;
 }
 

@@ -92,6 +92,12 @@ int main(int argc, char** argv) {
         copy(&ctx, size_t(67) << 20);
         std::printf("flags coherent %d portable %d noncoherent %d\n", (g_flags & hipHostMallocCoherent) != 0,
                     (g_flags & hipHostMallocPortable) != 0, (g_flags & hipHostMallocNonCoherent) != 0);
+    } else if (what == "lost") {
+        g_lost = argc > 3 ? std::atoi(argv[3]) : 0;
+        copy(&ctx, size_t(67) << 20);
+        std::printf("said: %s\n", ctx.err.c_str());
+        g_lost = -1;
+        copy(&ctx, size_t(67) << 20);
     } else {
         return 2;
     }

@@ -34,3 +34,15 @@ def test_pinned_memory_is_coherent(program, threads):
     assert lines[0].split("mallocs")[0].strip() == f"copy {67 << 20} status 0 whole 1"
     assert lines[1] == "flags coherent 1 portable 1 noncoherent 0"
     assert lines[2] == "end mallocs 1 frees 1"
+
+
+# of 34 pieces through 12 slots: the first, the last of the first round, one whose slot is not needed again, the last
+@pytest.mark.parametrize("piece", [0, 11, 12, 25, 33])
+@pytest.mark.parametrize("threads", ["team", "alone"])
+def test_a_piece_that_never_arrives_ends_the_copy(program, threads, piece):
+    """A stream that has finished without a piece's flag is an error, and not a wait without end."""
+    lines = _run(program, "lost", threads, str(piece))
+    assert lines[0].split()[3] == "2" and "arrive" in lines[1]
+    # and the next copy is whole again
+    assert lines[2].split()[3:6] == ["0", "whole", "1"]
+    assert lines[3] == "end mallocs 1 frees 1"
