@@ -23,6 +23,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <thread>
 #include <type_traits>
 
 #include "fsim_march.hpp"
@@ -593,12 +594,16 @@ static Reduce reduce_to_host(fsim_ctx* ctx, int op) {
 // written its scalars: polls the pinned word, since an event after the kernel
 // is one more packet that the kernels behind it wait for (5 us an iteration),
 // and a copy another, with the stream's synchronisation behind it (20 to 40 us).
+// After kScalarPolls, some 20 us, it gives up the processor between polls:
+// with more contexts than cores the others' threads would wait for it.
 // A queue that takes longer than the polls is waited for as a whole, which
 // also reports a failed kernel.
+constexpr int kScalarPolls = 256;
 static int wait_scalars(fsim_ctx* ctx) {
     const volatile unsigned* seq = &ctx->scal_host->seq;
     const auto t0 = std::chrono::steady_clock::now();
-    while (*seq != ctx->scal_seq) {
+    for (int polls = 0; *seq != ctx->scal_seq; polls++) {
+        if (polls >= kScalarPolls) std::this_thread::yield();
         if (std::chrono::steady_clock::now() - t0 < std::chrono::milliseconds(100)) continue;
         FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
         if (*seq != ctx->scal_seq) return set_err(ctx, FSIM_ERR_HIP, "the solver's scalars did not arrive");
