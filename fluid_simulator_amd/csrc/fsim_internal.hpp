@@ -96,7 +96,6 @@ __host__ __device__ inline int64_t ridx(int x, int y, int z, int nxp, int ny, in
 struct SolveArgs {
     int nx, ny, nz;
     int nxp;            // planes of the rotated layout
-    int off63;          // 63 mod nxp: the plane shift of a z step across a 64-wide z-tile edge
     int64_t nc;         // cells (flat fields)
     int64_t ncr;        // values of a solver vector: nxp * ny * nz
     float scale_f;      // dt / (rho dx^2)
@@ -107,27 +106,6 @@ struct SolveArgs {
 __device__ inline int64_t sidx(const SolveArgs& S, int x, int y, int z) { return ((int64_t)x * S.ny + y) * S.nz + z; }
 // index of the solver vectors, nbinfo and the factor (rotated layout)
 __device__ inline int64_t rsidx(const SolveArgs& S, int x, int y, int z) { return ridx(x, y, z, S.nxp, S.ny, S.nz); }
-// Rotated indices of the six neighbours of the interior cell at plane p, row
-// y, column z: +-y stay in the plane; +-x are the next/previous plane; +-z
-// move one column and one plane, except across a 64-wide z-tile edge where
-// rot(z) wraps 63 <-> 0 and the plane moves by 63.
-struct RNeighbours {
-    int64_t px, mx, py, my, pz, mz;
-};
-__device__ inline RNeighbours rneighbours(const SolveArgs& S, int p, int y, int z) {
-    const int rz = rot_of(z);
-    const int pn = p + 1 == S.nxp ? 0 : p + 1;
-    const int pp = p == 0 ? S.nxp - 1 : p - 1;
-    const int o = S.off63;
-    RNeighbours n;
-    n.px = pidx(pn, y, z, S.ny, S.nz);
-    n.mx = pidx(pp, y, z, S.ny, S.nz);
-    n.py = pidx(p, y + 1, z, S.ny, S.nz);
-    n.my = pidx(p, y - 1, z, S.ny, S.nz);
-    n.pz = pidx(rz == WF_TZ - 1 ? (p >= o ? p - o : p - o + S.nxp) : pn, y, z + 1, S.ny, S.nz);
-    n.mz = pidx(rz == 0 ? (p + o >= S.nxp ? p + o - S.nxp : p + o) : pp, y, z - 1, S.ny, S.nz);
-    return n;
-}
 // Indices around the four cells that one lane owns: planes 4g .. 4g + 3 of
 // column (y, z).  +-y are the same planes of the next rows; the +-x
 // neighbours of three of the four are the lane's own, the fourth's are element

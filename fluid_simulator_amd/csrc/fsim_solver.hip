@@ -446,7 +446,14 @@ __global__ void __launch_bounds__(kStream) k_dot_zr_zq(int64_t n, const uint32_t
     block_finish<AUX_SUM, kStream>(zr, zq, red);
 }
 
-// FP64 true residual t = b - A x; optionally r = (float)t.
+// FP64 true residual t = b - A x; optionally r = (float)t (0 off WATER, as r is).
+// A lane owns the four cells of a column of a plane group and reads whole
+// columns (ColumnNeighbours): 32 bytes of x where a gather cell by cell takes
+// 8 bytes from every 32.  At most kResidualBlocks blocks, each of which takes a
+// ticket of the reduction.  us a launch, 64^3 / 128^3 / 192^3 / 256^3: cell by
+// cell with 2048 blocks 12.7 / 36 / 54 / 113, columns with 2048 11.8 / 35 / 44 /
+// 77, 1024 12.1 / 24 / 35 / 71, 512 12 / 22 / 41 / 90.  256^3 needs 14 bytes a
+// cell, 48 us at the rate of a large copy.
 __global__ void __launch_bounds__(kBlock) k_true_residual(SolveArgs S, const uint16_t* __restrict__ nbinfo,
                                                           const float* __restrict__ b, const double* __restrict__ x,
                                                           float* __restrict__ r, int replace, Reduce red) {
@@ -456,33 +463,36 @@ __global__ void __launch_bounds__(kBlock) k_true_residual(SolveArgs S, const uin
     for (int k = it.first; k < it.end; k += it.step) {
         int g, y, zc;
         if (!item_column(it, k, S.ny, S.nz, g, y, zc)) continue;
-        const u16x4 info = *reinterpret_cast<const u16x4*>(nbinfo + pidx(g * WF_G, y, zc, S.ny, S.nz));
+        const ColumnNeighbours n = column_neighbours(S.ny, S.nz, S.nxp / WF_G, g, y, zc);
+        const u16x4 info = *reinterpret_cast<const u16x4*>(nbinfo + n.own);
+        if (((info[0] | info[1] | info[2] | info[3]) & NB_FLUID) == 0) continue;
+        // all loads first, then the reference's terms in order, each kept by its flag
+        const f64x4 own = *reinterpret_cast<const f64x4*>(x + n.own), yp = *reinterpret_cast<const f64x4*>(x + n.yp),
+                    ym = *reinterpret_cast<const f64x4*>(x + n.ym), zp = *reinterpret_cast<const f64x4*>(x + n.zp),
+                    zm = *reinterpret_cast<const f64x4*>(x + n.zm);
+        const double xp3 = x[n.xp3], xm0 = x[n.xm0], zp3 = x[n.zp3], zm0 = x[n.zm0];
+        const f32x4 bv = *reinterpret_cast<const f32x4*>(b + n.own);
+        f32x4 out = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int c = 0; c < 4; c++) {
-            if (!(info[c] & NB_FLUID)) continue;
-            const int p = g * WF_G + c;
-            const int64_t i = pidx(p, y, zc, S.ny, S.nz);
-            const RNeighbours n = rneighbours(S, p, y, zc);
-            // all 7 loads first (a WATER cell is interior: every neighbour index is in range), then the
-            // reference's terms in order, each kept by its flag
-            const double xi = x[i], xpx = x[n.px], xpy = x[n.py], xpz = x[n.pz], xmx = x[n.mx], xmy = x[n.my],
-                         xmz = x[n.mz];
             const uint16_t f = info[c];
+            if (!(f & NB_FLUID)) continue;
             const int cnt = (f >> NB_NONSOLID_SHIFT) & 7;
             double diag = 0;
             for (int j = 0; j < cnt; j++) diag += S.scale;
-            double val = diag * xi;
-            val = (f & NB_PX) ? val + -S.scale * xpx : val;
-            val = (f & NB_PY) ? val + -S.scale * xpy : val;
-            val = (f & NB_PZ) ? val + -S.scale * xpz : val;
-            val = (f & NB_MX) ? val + -S.scale * xmx : val;
-            val = (f & NB_MY) ? val + -S.scale * xmy : val;
-            val = (f & NB_MZ) ? val + -S.scale * xmz : val;
-            const double t = (double)b[i] - val;
+            double val = diag * own[c];
+            val = (f & NB_PX) ? val + -S.scale * (c < 3 ? own[(c + 1) & 3] : xp3) : val;
+            val = (f & NB_PY) ? val + -S.scale * yp[c] : val;
+            val = (f & NB_PZ) ? val + -S.scale * (c < 3 ? zp[(c + 1) & 3] : zp3) : val;
+            val = (f & NB_MX) ? val + -S.scale * (c > 0 ? own[(c + 3) & 3] : xm0) : val;
+            val = (f & NB_MY) ? val + -S.scale * ym[c] : val;
+            val = (f & NB_MZ) ? val + -S.scale * (c > 0 ? zm[(c + 3) & 3] : zm0) : val;
+            const double t = (double)bv[c] - val;
             ss += t * t;
             mx = fmax(mx, fabs(t));
-            if (replace) r[i] = (float)t;
+            out[c] = (float)t;
         }
+        if (replace) *reinterpret_cast<f32x4*>(r + n.own) = out;
     }
     block_finish<AUX_MAX>(ss, mx, red);
 }
@@ -543,7 +553,6 @@ static SolveArgs solve_args(const fsim_ctx* ctx, double dt) {
     S.nc = ctx->g.nc;
     S.nxp = ctx->g.nxp;
     S.ncr = ctx->g.ncr;
-    S.off63 = (WF_TZ - 1) % S.nxp;
     S.scale = dt / (ctx->prm.fluid_density * ctx->g.cd * ctx->g.cd);
     S.scale_f = (float)S.scale;
     return S;
@@ -578,10 +587,12 @@ static int check_wave_err(fsim_ctx* ctx) {
 // per CU keep HBM busy), a multiple of 8 for the XCD-aware row split, and
 // the last block sums the partials in one pass.
 static unsigned red_blocks(int64_t n) { return std::min<unsigned>((nblocks(n) + 7) / 8 * 8, kMaxParts); }
-// blocks of the column kernels: one per item
-static unsigned column_blocks(const SolveArgs& S) {
+// blocks of the true residual: one per item up to kResidualBlocks (its comment)
+constexpr unsigned kResidualBlocks = 1024;
+static_assert(kResidualBlocks % 8 == 0 && kResidualBlocks <= kMaxParts, "true residual's grid within the reduction");
+static unsigned residual_blocks(const SolveArgs& S) {
     const unsigned items = (unsigned)row_item_count(S.ny, S.nz, S.nxp);
-    return std::max(8u, std::min<unsigned>((items + 7) / 8 * 8, kMaxParts));
+    return std::max(8u, std::min<unsigned>((items + 7) / 8 * 8, kResidualBlocks));
 }
 
 static Reduce reduce_to(fsim_ctx* ctx, int op) { return Reduce{ctx->partials, ctx->red_count, ctx->scal, op}; }
@@ -737,7 +748,7 @@ static int true_residual(fsim_ctx* ctx, const SolveArgs& S, float* r, bool repla
     FSIM_PROF(ctx, KID_TRUE_RES);
     Reduce red = reduce_to_host(ctx, FIN_TRUE);
     red.wave_err = ctx->wave_err;
-    hipLaunchKernelGGL(k_true_residual, dim3(column_blocks(S)), dim3(kBlock), 0, ctx->stream, S, ctx->nbinfo, ctx->b, ctx->x,
+    hipLaunchKernelGGL(k_true_residual, dim3(residual_blocks(S)), dim3(kBlock), 0, ctx->stream, S, ctx->nbinfo, ctx->b, ctx->x,
                        r, replace ? 1 : 0, red);
     FSIM_HIP(ctx, hipGetLastError());
     return FSIM_OK;
