@@ -36,11 +36,11 @@ HBM_PEAK_GBS = 8000.0   # MI355X HBM3E
 # each array counted once per launch, no cache credit).  Units: f = WATER
 # cells, c = all cells, p = particles.
 ALGO_BYTES = {
-    "sweep_fwd": ("f", 21.0),      # R r 4, R q 4, R P 4, R label 1, W t 4, W r 4
-    "sweep_bwd": ("f", 25.0),      # R t 4, R P 4, R label 1, W z 4; every other time R x 8, R s 8, W x 8
+    "sweep_fwd": ("f", 20.0),      # R r 4, R q 4, R P 4, W t 4, W r 4
+    "sweep_bwd": ("f", 24.5),      # R t 4, R P 4, W z 4; every other time R x 8, R s 8, R label 1, W x 8
     "mic_factor": ("f", 5.0),      # R label 1, W P 4
     "spmv": ("f", 17.0),           # direction step: R label 1, R z 4, R s 4, W s' 4, W q 4
-    "update": ("f", 13.0),         # R label 1, R q 4, R/W r 8
+    "update": ("f", 12.0),         # R q 4, R/W r 8
     "dot": ("f", 8.0),             # R z 4, R r 4
     "p2g": ("p+c", (24.0, 12.0)),  # R particle pos+vel 24 B/p, W u,v,w 12 B/cell
     "g2p": ("p+c", (36.0, 24.0)),  # R pos,vel W vel 36 B/p, R u,v,w,u2,v2,w2 24 B/cell
