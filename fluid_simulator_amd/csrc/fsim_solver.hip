@@ -372,13 +372,11 @@ __global__ void __launch_bounds__(64 * kMarchWaves) k_spmv(SolveArgs S, MarchPla
 // update beside the x update 52 (53) and 13.6 (16.5); 128 and 512 blocks are
 // slower at 256^3 (24.5 / 20.9 and 65 / 58).
 constexpr int kStream = 1024;   // threads per block
-#ifndef FSIM_STREAM_BLOCKS
-#define FSIM_STREAM_BLOCKS 256
-#endif
-static_assert(FSIM_STREAM_BLOCKS <= (int)kMaxParts, "stream grid within the reduction");
+constexpr unsigned kStreamBlocks = 256;
+static_assert(kStreamBlocks <= kMaxParts, "stream grid within the reduction");
 static unsigned stream_blocks(int64_t n) {
     const unsigned need = (unsigned)((n / kChunk + kUnits * (kStream / 64) - 1) / (kUnits * (kStream / 64)));
-    return std::max(1u, std::min<unsigned>(need, FSIM_STREAM_BLOCKS));
+    return std::max(1u, std::min<unsigned>(need, kStreamBlocks));
 }
 
 template <int STEPS>
@@ -653,7 +651,9 @@ static int build_nbinfo(fsim_ctx* ctx, const SolveArgs& S, bool with_rhs) {
     A.red = with_rhs ? reduce_to_host(ctx, FIN_BB) : reduce_to(ctx, FIN_BB);
     FSIM_TRY(fill_u8(ctx, ctx->colw, 0, colw_bytes(S)));   // and xrange and the chunk flags behind it
     hipLaunchKernelGGL(k_nbinfo_rhs, dim3(red_blocks(S.nc)), dim3(kBlock), 0, ctx->stream, A, with_rhs ? 1 : 0);
-    // wide windows leave fewer lanes idle, narrow ones give small grids more and shorter blocks
+    // wide windows leave fewer lanes idle, narrow ones give small grids more and shorter blocks (this stage in us
+    // with windows of 16 / 64: 32^3 22 / 25, 64^3 34.5 / 36, 96^3 53 / 53, 128^3 60 / 56, 192^3 130 / 115, 256^3
+    // 267 / 235): wide ones from two blocks a compute unit on (wide windows make 376 blocks at 96^3, 756 at 128^3)
     auto items = [&](int w) {
         return (unsigned)((S.nxp + w - 1) / w * (S.ny - 2) * ((S.nz - 2 + WF_TZ - 1) / WF_TZ));
     };
@@ -691,15 +691,14 @@ static int mic_factor(fsim_ctx* ctx, const SolveArgs& S) {
 
 // Blocks of WF_THREADS threads beside a sweep's tiles, on the compute units
 // that the tiles leave free.  At 256^3, where they have 300 MB to move, a solve
-// takes 66.8 ms with 128 blocks, 63.9 with 256 and 62.6 with 512; 128^3 does
-// not tell them apart.
-#ifndef FSIM_SIDE_BLOCKS
-#define FSIM_SIDE_BLOCKS 512
-#endif
-static_assert(FSIM_SIDE_BLOCKS <= (int)kMaxParts, "side blocks within the reduction");
+// takes 66.8 ms with 128 blocks, 63.9 with 256 and 62.6 with 512.  Frames of
+// 32^3 to 203x67x131 do not tell 256 from 512 (128^3 12.2 to 12.6 ms with
+// either).
+constexpr unsigned kSideBlocks = 512;
+static_assert(kSideBlocks <= kMaxParts, "side blocks within the reduction");
 static unsigned side_blocks(int64_t n) {
     const unsigned need = (unsigned)((n / kChunk + kUnits * (WF_THREADS / 64) - 1) / (kUnits * (WF_THREADS / 64)));
-    return std::max(1u, std::min<unsigned>(need, FSIM_SIDE_BLOCKS));
+    return std::max(1u, std::min<unsigned>(need, kSideBlocks));
 }
 
 // t = L^-1 r and z = L^-T t, M = L L^T.

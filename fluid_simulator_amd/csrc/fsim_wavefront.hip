@@ -30,10 +30,14 @@
 // step measured 0.30 us a step, 209 and 202 us a sweep at 256^3 (water in 0.6
 // of the height) and 98 us at 128^3; groups take 0.07 us a step, 132 and 126
 // us at 256^3 and 46 us at 128^3, the same bits.  At 256^3 the tiles' memory
-// traffic counts: a compute unit moves 24 KB per group of an 8-row tile, and
-// without the result's stores the sweep takes 113 us.  Three compute waves of
-// two rows measured best (2 x 4: 142 us forward, 2 x 8: 190 us, 1 x 4: 164 us,
-// 4 x 2: 154 us); storing waves that take the results over LDS, so that the
+// traffic counts: a compute unit moves 18 KB per group of a 6-row tile (24 in
+// the forward sweep of an iteration), and without the result's stores the
+// sweep takes 113 us.  Three compute waves of two rows measured best (2 x 4:
+// 142 us forward, 2 x 8: 190 us, 1 x 4: 164 us, 4 x 2: 154 us), and at no size
+// clearly worse than another number of waves (frames in ms with 2 / 3 / 4 / 5
+// waves: 32^3 1.29 / 1.21 / 1.23 / 1.18, 70x52x91 5.9 / 5.6 / 6.0 / 6.2, 96^3
+// 9.0 / 8.8 / 8.7 / 8.9, 128^3 13.1 / 12.5 / 12.6 / 12.9, 203x67x131 20.8 /
+// 21.3 / 23.1 / 25.3, 256^3 147 / 144 / 149 / 168); storing waves that take the results over LDS, so that the
 // in-order memory counter does not hold loads behind stores, did not pay
 // (166 us), nor did stores past the caches.
 //
@@ -88,10 +92,7 @@ namespace fsim {
 constexpr int kSpinLimit = 1 << 21;
 constexpr int kBusyPolls = 64;   // polls before a waiting wave starts to sleep
 constexpr int kRing = 8;         // ring slots (groups) between waves, and the unroll of the group loop
-#ifndef FSIM_WF_PREFETCH
-#define FSIM_WF_PREFETCH 6
-#endif
-constexpr int kPrefetch = FSIM_WF_PREFETCH;   // groups of per-cell inputs loaded ahead
+constexpr int kPrefetch = 6;     // groups of per-cell inputs loaded ahead (7: no change)
 static_assert(kPrefetch >= 1 && kPrefetch <= kRing, "a prefetch slot per unrolled group");
 constexpr int kRingZ = 32;   // +z out-ring slots (groups): the z edge runs 16 groups behind its tile
 constexpr int kAll = 0x3fffffff;              // counter value "everything": no upstream, or no consumer
