@@ -13,6 +13,7 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <memory>
 #include <new>
 #include <vector>
 
@@ -129,6 +130,18 @@ static void free_all(fsim_ctx* ctx) {
         if (e) (void)hipEventDestroy(e);
     for (auto& e : ctx->prof_pool) (void)hipEventDestroy(e);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
+}
+
+// solver vectors are stored in the rotated layout: gathered into flat order on the host
+template <class T>
+static int get_rotated(fsim_ctx* ctx, const void* src, void* dst) {
+    const GridDims& g = ctx->g;
+    const std::unique_ptr<T[]> tmp(new (std::nothrow) T[(size_t)g.ncr]);
+    if (!tmp) return set_err(ctx, FSIM_ERR_OOM, "host buffer allocation failed");
+    FSIM_TRY(read_back(ctx, tmp.get(), src, sizeof(T) * (size_t)g.ncr));
+    char* const out = static_cast<char*>(dst);
+    for_rotated(g.nx, g.ny, g.nz, g.nxp, [&](int64_t i, int64_t r) { std::memcpy(out + i * sizeof(T), &tmp[r], sizeof(T)); });
+    return FSIM_OK;
 }
 
 extern "C" {
@@ -457,19 +470,7 @@ int fsim_get_grid(fsim_ctx* ctx, int field, void* dst, size_t bytes) {
     if (!rotated) {
         return read_back(ctx, dst, src, need);
     }
-    // solver vectors are stored in the rotated layout: gather into flat order
-    const size_t elem = need / nc;
-    std::vector<unsigned char> tmp(elem * ctx->g.ncr);
-    FSIM_HIP(ctx, hipMemcpy(tmp.data(), src, tmp.size(), hipMemcpyDeviceToHost));
-    unsigned char* out = static_cast<unsigned char*>(dst);
-    const GridDims& g = ctx->g;
-    for (int x = 0; x < g.nx; x++)
-        for (int y = 0; y < g.ny; y++)
-            for (int z = 0; z < g.nz; z++) {
-                const int64_t i = ((int64_t)x * g.ny + y) * g.nz + z;
-                std::memcpy(out + i * elem, tmp.data() + ridx(x, y, z, g.nxp, g.ny, g.nz) * elem, elem);
-            }
-    return FSIM_OK;
+    return need == 8 * (size_t)nc ? get_rotated<double>(ctx, src, dst) : get_rotated<float>(ctx, src, dst);
 }
 
 int fsim_set_grid(fsim_ctx* ctx, int field, const void* src, size_t bytes) {

@@ -86,6 +86,18 @@ __host__ __device__ inline int64_t ridx(int x, int y, int z, int nxp, int ny, in
     return pidx(rot_plane(x, z, nxp), y, z, ny, nz);
 }
 
+// f(flat index, index in the rotated layout) of every cell, in flat order, on the host.  The planes' places come from a
+// table: the index arithmetic of ridx for every cell made reading a small field 15 % slower than with one plane a row.
+template <class F>
+inline void for_rotated(int nx, int ny, int nz, int nxp, F&& f) {
+    std::vector<int64_t> place((size_t)nx + WF_TZ - 1);   // of plane p, unwrapped
+    for (size_t p = 0; p < place.size(); p++) place[p] = pidx((int)(p % nxp), 0, 0, ny, nz);
+    int64_t i = 0;
+    for (int x = 0; x < nx; x++)
+        for (int y = 0; y < ny; y++)
+            for (int z = 0; z < nz; z++, i++) f(i, place[x + rot_of(z)] + ((int64_t)y * nz + z) * WF_G);
+}
+
 // Dimensions and scale of a pressure solve; stencil neighbours in the rotated layout.
 struct SolveArgs {
     int nx, ny, nz;

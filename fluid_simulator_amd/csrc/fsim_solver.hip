@@ -23,6 +23,8 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <memory>
+#include <new>
 #include <thread>
 #include <type_traits>
 
@@ -1192,24 +1194,26 @@ int wave_init(fsim_ctx* ctx) {
 
 int solver_apply(fsim_ctx* ctx, int op, double dt, const double* in, double* out) {
     const SolveArgs S = solve_args(ctx, dt);
-    const int64_t nc = S.nc, n = S.ncr;
+    const int64_t n = S.ncr;
     FSIM_TRY(build_nbinfo(ctx, S, false));
     // host vectors are in flat order, device solver vectors in the rotated one
-    std::vector<int64_t> rmap(nc);
-    for (int x = 0; x < S.nx; x++)
-        for (int y = 0; y < S.ny; y++)
-            for (int z = 0; z < S.nz; z++) rmap[((int64_t)x * S.ny + y) * S.nz + z] = ridx(x, y, z, S.nxp, S.ny, S.nz);
-    std::vector<float> hin(n), hout(n);   // padding values 0
+    auto each = [&](auto&& f) { for_rotated(S.nx, S.ny, S.nz, S.nxp, f); };
+    // a host buffer without a first pass over its pages
+    auto result = [&](auto* src) {
+        using T = std::remove_cv_t<std::remove_pointer_t<decltype(src)>>;
+        const std::unique_ptr<T[]> h(new (std::nothrow) T[(size_t)n]);
+        if (!h) return set_err(ctx, FSIM_ERR_OOM, "host buffer allocation failed");
+        FSIM_TRY(read_back(ctx, h.get(), src, sizeof(T) * (size_t)n));
+        each([&](int64_t i, int64_t r) { out[i] = h[r]; });
+        return (int)FSIM_OK;
+    };
     if (op == FSIM_OP_FACTOR_MIC0) {
         FSIM_TRY(mic_factor(ctx, S));
         FSIM_TRY(check_wave_err(ctx));
-        std::vector<double> hp(n);
-        FSIM_HIP(ctx, hipMemcpyAsync(hp.data(), ctx->P64, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
-        FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        for (int64_t i = 0; i < nc; i++) out[i] = hp[rmap[i]];
-        return FSIM_OK;
+        return result(ctx->P64);
     }
-    for (int64_t i = 0; i < nc; i++) hin[rmap[i]] = (float)in[i];
+    std::vector<float> hin(n);   // padding values 0
+    each([&](int64_t i, int64_t r) { hin[r] = (float)in[i]; });
     FSIM_HIP(ctx, hipMemcpyAsync(ctx->r, hin.data(), sizeof(float) * n, hipMemcpyHostToDevice, ctx->stream));
     if (op == FSIM_OP_APPLY_A) {
         FSIM_TRY(fill_f32(ctx, ctx->q, 0.0f, n));   // the SpMV skips columns without WATER
@@ -1217,27 +1221,25 @@ int solver_apply(fsim_ctx* ctx, int op, double dt, const double* in, double* out
         hipLaunchKernelGGL(k_spmv<SPMV_PLAIN>, dim3(march_blocks(m)), dim3(64 * kMarchWaves), 0, ctx->stream, S, m,
                            ctx->nbinfo, nullptr, ctx->r, nullptr, ctx->q, reduce_to(ctx, FIN_NONE));
         FSIM_HIP(ctx, hipGetLastError());
-        FSIM_HIP(ctx, hipMemcpyAsync(hout.data(), ctx->q, sizeof(float) * n, hipMemcpyDeviceToHost, ctx->stream));
-    } else if (op == FSIM_OP_APPLY_MIC0) {
+        return result(ctx->q);
+    }
+    if (op == FSIM_OP_APPLY_MIC0) {
         FSIM_TRY(mic_factor(ctx, S));
         FSIM_TRY(fill_f32(ctx, ctx->t, 0.0f, n));
         FSIM_TRY(fill_f32(ctx, ctx->z, 0.0f, n));
         FSIM_TRY(mic_apply(ctx, S, ctx->r, ctx->t, ctx->z));
         FSIM_TRY(check_wave_err(ctx));
-        FSIM_HIP(ctx, hipMemcpyAsync(hout.data(), ctx->z, sizeof(float) * n, hipMemcpyDeviceToHost, ctx->stream));
-    } else if (op == FSIM_OP_APPLY_MG) {
+        return result(ctx->z);
+    }
+    if (op == FSIM_OP_APPLY_MG) {
         if (ctx->mg_coarse == FSIM_MG_COARSE_NETWORK && !learned_ready(ctx))
             return set_err(ctx, FSIM_ERR_INVALID, "the multigrid's coarse network has no parameters");
         FSIM_TRY(mg_setup(ctx));
         FSIM_TRY(fill_f32(ctx, ctx->z, 0.0f, n));
         FSIM_TRY(mg_apply(ctx, ctx->r, ctx->z, S.scale));
-        FSIM_HIP(ctx, hipMemcpyAsync(hout.data(), ctx->z, sizeof(float) * n, hipMemcpyDeviceToHost, ctx->stream));
-    } else {
-        return set_err(ctx, FSIM_ERR_INVALID, "unknown solver op");
+        return result(ctx->z);
     }
-    FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    for (int64_t i = 0; i < nc; i++) out[i] = hout[rmap[i]];
-    return FSIM_OK;
+    return set_err(ctx, FSIM_ERR_INVALID, "unknown solver op");
 }
 
 }  // namespace fsim
