@@ -32,7 +32,10 @@ constexpr size_t kSlotBytes = size_t(2) << 20;
 constexpr int kReadSlots = 12;                // pinned slots
 constexpr int kMaxThreads = 8;               // 67 MB of new pages: 1.2 ms by 8 threads, 1.0 by 16, 5.1 by one
 // Below it hipMemcpy, which copies pages that exist (small arrays come from a
-// program's heap) in 0.1 ms.
+// program's heap) in 0.1 ms.  us by hipMemcpy, and by hipMemcpyAsync with the
+// stream's synchronisation: 4 KB 15 and 23, 16 KB 19 and 27, 64 KB 36 and 36,
+// 128 KB 15 and 23, 160 KB 17 and 73, 512 KB 31 and 31.  Where the two take
+// turns, each is slower than by itself (128 KB 62).
 constexpr size_t kDirectBytes = size_t(1) << 20;
 // The threads need several pieces each, and a piece costs its launch.  ms for
 // existing pages of 4 / 8 / 15 / 34 / 67 MB: 0.19 / 0.32 / 0.52 / 0.95 / 1.7
@@ -247,8 +250,8 @@ static int run_copy(fsim_ctx* ctx, Copy& C, bool alone) {
 }
 
 static int direct_copy(fsim_ctx* ctx, void* dst, const void* src, size_t bytes) {
-    FSIM_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
     FSIM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    FSIM_HIP(ctx, hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost));
     return FSIM_OK;
 }
 

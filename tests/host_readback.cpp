@@ -7,7 +7,7 @@
 #include <string>
 #include <vector>
 
-static int g_mallocs = 0, g_frees = 0, g_copies = 0, g_launches = 0, g_lost = -1;
+static int g_mallocs = 0, g_frees = 0, g_copies = 0, g_plain = 0, g_launches = 0, g_lost = -1;
 static unsigned g_flags = 0;
 
 extern "C" {
@@ -24,6 +24,11 @@ hipError_t hipHostFree(void* p) {
 }
 hipError_t hipMemcpyAsync(void* dst, const void* src, size_t bytes, hipMemcpyKind, hipStream_t) {
     g_copies++;
+    std::memcpy(dst, src, bytes);
+    return hipSuccess;
+}
+hipError_t hipMemcpy(void* dst, const void* src, size_t bytes, hipMemcpyKind) {
+    g_plain++;
     std::memcpy(dst, src, bytes);
     return hipSuccess;
 }
@@ -98,6 +103,12 @@ int main(int argc, char** argv) {
         std::printf("said: %s\n", ctx.err.c_str());
         g_lost = -1;
         copy(&ctx, size_t(67) << 20);
+    } else if (what == "direct") {
+        for (int k = 2; k < argc; k++) {
+            g_copies = g_plain = 0;
+            copy(&ctx, (size_t)std::atoll(argv[k]));
+            std::printf("plain %d on the stream %d\n", g_plain, g_copies);
+        }
     } else {
         return 2;
     }

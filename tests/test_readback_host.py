@@ -46,3 +46,11 @@ def test_a_piece_that_never_arrives_ends_the_copy(program, threads, piece):
     # and the next copy is whole again
     assert lines[2].split()[3:6] == ["0", "whole", "1"]
     assert lines[3] == "end mallocs 1 frees 1"
+
+
+def test_small_results_take_the_runtimes_plain_copy(program):
+    """A copy on the stream and its synchronisation cost a result of a few KB half as much again."""
+    sizes = [1, 4096, 100_000, (1 << 20) - 1]
+    lines = _run(program, "direct", *map(str, sizes))
+    assert all(v.split()[3:6] == ["0", "whole", "1"] for v in lines[0:-1:2])
+    assert lines[1:-1:2] == ["plain 1 on the stream 0"] * len(sizes)
