@@ -283,8 +283,9 @@ __global__ void __launch_bounds__(kMgBz * kMgBy) k_mg_rbgs(MgGrid G) {
 // plane groups, each wave contiguous memory, puts it into LDS, and sums every
 // coarse cell's 8 children there in a fixed order.
 // The residual follows the last pre-smoothing half-sweep, which solved the
-// cells of colour 0 exactly: their residual is 0 (up to rounding) and only the
-// cells of colour 1 are computed.
+// cells of colour 0 exactly: their residual is the rounding of that division,
+// which evaluating it in FP32 would not resolve.  It is taken as 0, for every
+// width of the grid, and only the cells of colour 1 are computed.
 constexpr int kRtC = 32;   // coarse cells per block along x and along z (a 64 x 2 x 64 fine box)
 __global__ void __launch_bounds__(256) k_mg_resid_restrict0(Mg0 A, MgGrid C) {
     // fine box [yy][x - fx0][z - fz0]; a row of 64 words: the lanes of a wave store into a different

@@ -811,10 +811,12 @@ static bool stop_met(const fsim_ctx* ctx, double ss, double mx, double bnorm) {
 // sweep: the sweeps are chains of waits that leave most of the chip idle.
 // sigma = z.r = r^T L^-T L^-1 r = t.t with t = L^-1 r, the forward sweep's
 // result, which is there before the backward sweep starts.  Summed in FP64,
-// it is off by the FP32 rounding inside the sweeps, 1e-9 to 6e-8 of its value
-// (z.r: 1e-9 to 2e-8; 8 to 26 cells a side, random and smooth r), where the
-// rounding of alpha and beta to FP32 may take 6e-8.  r has two buffers, since
-// the tiles read the old one.
+// it is off by the FP32 rounding inside the sweeps, where the rounding of alpha
+// and beta to FP32 may take 6e-8 (mean error against 64 bits of t.t and z.r,
+// random and smooth r: 8^3 3.5e-8 / 6.3e-8 and 1.6e-8 / 1.6e-8, 24^3 3.4e-9 /
+// 5.5e-9 and 1.5e-9 / 3.5e-9, 64^3 9e-10 / 2.1e-9 and 6e-10 / 1.5e-9, 128^3
+// 2.6e-10 / 1.4e-9 and 1.7e-10 / 1.4e-9, 2D 128^2 3.9e-9 / 5.3e-9 and 2.4e-9 /
+// 5.1e-9).  r has two buffers, since the tiles read the old one.
 // An iteration, against launches of their own for the r update, the dot
 // product and the x update (the last on a second stream at 256^3): 32^3 62 ->
 // 49 us, 2D 128^2 100 -> 86, 128^3 132 -> 114, 256^3 395 -> 378.

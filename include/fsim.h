@@ -253,6 +253,12 @@ int fsim_run_stage(fsim_ctx* ctx, int stage, double dt);
 int fsim_get_stats(const fsim_ctx* ctx, fsim_step_stats* out);
 
 /* ---- grid access ---------------------------------------------------------- */
+/* Results of 1 MiB or more (here, of fsim_get_particles, fsim_gfx_snapshot and
+ * fsim_learned_grad*) are copied out through pinned memory, 24 MB that the
+ * contexts of a process share.  The first such call makes it and the last
+ * context's fsim_destroy releases it, which takes 0.1 to 1 ms together; a
+ * call that finds it in use by another thread makes one of its own.  Up to 8
+ * threads copy, for the length of the call. */
 int fsim_get_grid(fsim_ctx* ctx, int field, void* dst, size_t bytes);
 int fsim_set_grid(fsim_ctx* ctx, int field, const void* src, size_t bytes);
 int fsim_solver_apply(fsim_ctx* ctx, int op, double dt, const double* in, double* out);
@@ -263,7 +269,7 @@ int fsim_solver_apply(fsim_ctx* ctx, int op, double dt, const double* in, double
  * getParticleGfxData returns (:40-43): out[i] is particle i of the reference's
  * particle order, {pos, glm::length(v), sum over getCellsAround's 8 cells of
  * trilinearInterpoll(pos, cell centre) * avgPNum}.  Computed on the device
- * from the current state (call it between steps), one device-to-host copy. */
+ * from the current state (call it between steps) and copied out once. */
 int fsim_gfx_snapshot(fsim_ctx* ctx, int64_t capacity, fsim_gfx_particle* out, int64_t* n_out);
 /* No counterpart in the reference: fsim_gfx_snapshot for callers that cannot
  * allocate device memory (a render loop under HIP graph capture, a serving
@@ -325,8 +331,11 @@ typedef enum fsim_option {
     FSIM_OPT_P2G_KERNEL = 10,
     /* test option: the sending waves of the wavefront kernels pause about
      * value x 3.4 us after each group of four steps they send (0 .. 64,
-     * default 0), so the compute waves run into the out-ring limit and wait
-     * for them.  The results are the same bits; only the time changes. */
+     * default 0).  Where a tile has a neighbour along z and a march of more
+     * than 32 to 47 groups (about 130 cells along x on a full z-tile of 64), the
+     * compute waves run into the out-ring limit and wait for them; on smaller
+     * grids only the neighbour waits.  The results are the same bits; only
+     * the time changes. */
     FSIM_OPT_WAVE_SEND_DELAY = 11
 } fsim_option;
 int fsim_set_option(fsim_ctx* ctx, int option, int value);
