@@ -24,7 +24,8 @@ constexpr int kMarchRows = 2;      // rows of a wave
 constexpr int kMarchWaves = 4;     // waves of a block: consecutive row blocks
 constexpr int kMarchBlocks = 512;  // blocks that the runs are cut for
 constexpr int kMarchRun = 16;      // consecutive items of one XCD
-static_assert(kMarchBlocks <= (int)kMaxParts, "march grid within the reduction");
+constexpr unsigned kBesideMarch = 256;   // blocks that a kernel may run beside the march in the same reduction
+static_assert(kMarchBlocks + kBesideMarch <= kMaxParts, "march grid within the reduction");
 
 // Items are ordered row blocks first, then z-tiles, then runs of groups.
 // Workgroups are dispatched round-robin over the 8 XCDs (blockIdx mod 8): each
@@ -45,7 +46,7 @@ static inline MarchPlan march_of(int ny, int nz, int nxp) {
 }
 static inline unsigned march_blocks(const MarchPlan& m) {
     const int unit = 8 * kMarchRun;
-    return (unsigned)std::min<int64_t>((m.items + unit - 1) / unit * unit, kMaxParts);
+    return (unsigned)std::min<int64_t>((m.items + unit - 1) / unit * unit, (kMaxParts - kBesideMarch) / unit * unit);
 }
 
 __device__ inline float lane_next(float v, float last) {   // lane i + 1's value; lane 63: last
@@ -68,11 +69,11 @@ struct MarchCells {
 
 // Raw load(int64_t j): the vectors at index j (a multiple of 4), without
 // branches; f32x4 value(const Raw&): what the stencil is applied to, 0 off
-// WATER; body(int64_t j, const MarchCells&): called for the lanes with WATER.
+// WATER; blocks: the grid's first ones, that march (a multiple of 8 kMarchRun); body(int64_t j, const MarchCells&): called for the lanes with WATER.
 // Columns without WATER read index 0, a border cell, whose values are zero.
 template <class Load, class Value, class Body>
-__device__ inline void march(const MarchPlan& m, int ny, int nz, int nxp, const uint16_t* __restrict__ nbinfo, Load&& load,
-                             Value&& value, Body&& body) {
+__device__ inline void march(const MarchPlan& m, unsigned blocks, int ny, int nz, int nxp,
+                             const uint16_t* __restrict__ nbinfo, Load&& load, Value&& value, Body&& body) {
     constexpr int R = kMarchRows;
     using Raw = decltype(load((int64_t)0));
     const int lane = threadIdx.x & 63;
@@ -81,7 +82,7 @@ __device__ inline void march(const MarchPlan& m, int ny, int nz, int nxp, const 
     const int64_t gs = (int64_t)ny * nz * WF_G, rs = (int64_t)nz * WF_G;
     const int far = ng > 16 ? 16 : 16 % ng;
     auto any = [](u16x4 f) { return ((f[0] | f[1] | f[2] | f[3]) & NB_FLUID) != 0; };
-    for (int b = blockIdx.x;; b += gridDim.x) {
+    for (int b = blockIdx.x;; b += blocks) {
         const int j = b >> 3;
         const int item = (j / kMarchRun * 8 + (b & 7)) * kMarchRun + j % kMarchRun;
         if (j / kMarchRun * 8 * kMarchRun >= m.items) break;

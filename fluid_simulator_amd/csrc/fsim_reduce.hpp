@@ -27,7 +27,8 @@ __device__ inline double wave_max(double v) {
 // result is deterministic, and no separate finalize launch is needed.
 constexpr int AUX_NONE = 0, AUX_MAX = 1, AUX_SUM = 2;
 enum FinOp {
-    FIN_NONE = -1, FIN_BB = 0, FIN_SIGMA0 = 1, FIN_ALPHA = 2, FIN_RES = 3, FIN_BETA = 4, FIN_TRUE = 5, FIN_FBETA = 6
+    FIN_NONE = -1, FIN_BB = 0, FIN_SIGMA0 = 1, FIN_ALPHA = 2, FIN_RES = 3, FIN_BETA = 4, FIN_TRUE = 5, FIN_FBETA = 6,
+    FIN_ALPHA_ZR = 7
 };
 
 struct Reduce {
@@ -44,8 +45,9 @@ __device__ inline void apply_fin(int op, double s, double m, SolveScalars* sc) {
     switch (op) {
     case FIN_BB: sc->bb = s; sc->nfluid = m; break;
     case FIN_SIGMA0: sc->zr = s; break;
-    case FIN_ALPHA: {   // sigma is the last z.r (initial, restart or beta step)
-        sc->sigma = sc->zr;
+    case FIN_ALPHA:      // sigma is the last z.r (initial, restart or beta step)
+    case FIN_ALPHA_ZR: { // sigma = m, z.r summed beside s.q
+        sc->sigma = op == FIN_ALPHA ? sc->zr : m;
         sc->sq = s;
         const double alpha = sc->sigma / s;
         sc->alpha_prev = sc->alpha;
@@ -291,6 +293,25 @@ __device__ inline void update_r(const Part part, int64_t n, const uint32_t* __re
             *reinterpret_cast<float4*>(r_next + i) = v[1];
         });
     block_finish<AUX_MAX, NT>(ss, mx, red, part);
+}
+
+// a . b over this thread's part of the flagged chunks (FP64 products of the FP32 values)
+__device__ inline double dot_part(const Part part, int64_t n, const uint32_t* __restrict__ flags, const float* __restrict__ a,
+                                  const float* __restrict__ b) {
+    double d = 0.0;
+    for_flagged_chunks<2>(
+        part, n, flags,
+        [&](int64_t i, float4(&v)[2]) {
+            v[0] = *reinterpret_cast<const float4*>(a + i);
+            v[1] = *reinterpret_cast<const float4*>(b + i);
+        },
+        [&](int64_t, float4(&v)[2]) {
+            d += (double)v[0].x * (double)v[1].x;
+            d += (double)v[0].y * (double)v[1].y;
+            d += (double)v[0].z * (double)v[1].z;
+            d += (double)v[0].w * (double)v[1].w;
+        });
+    return d;
 }
 
 // t . t (FP64 products of the FP32 values)

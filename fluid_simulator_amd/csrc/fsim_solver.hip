@@ -309,6 +309,14 @@ __global__ void __launch_bounds__(kBlock) k_bwd_plane(PlaneArgs A, const float* 
 // ---- SpMV (applyAMatrix :165-198) with the s.q dot ---------------------------------
 constexpr int SPMV_PLAIN = 0, SPMV_COPY = 1, SPMV_XPAY = 2;
 
+// z.r beside the product, in blocks of its own, for alpha = z.r / s'.q
+struct SpmvDot {
+    unsigned blocks = 0;   // the grid's last ones; 0: none
+    int64_t n = 0;
+    const uint32_t* flags = nullptr;
+    const float* r = nullptr;
+};
+
 // SPMV_PLAIN: q = A s.  SPMV_COPY: s' = z, q = A s'.  SPMV_XPAY: s' = s * beta + z
 // (multSelfAndAdd :229-242), q = A s'.  The new search direction s' goes to a
 // second buffer and is recomputed for the neighbours from z and the old s, so
@@ -322,7 +330,13 @@ constexpr int SPMV_PLAIN = 0, SPMV_COPY = 1, SPMV_XPAY = 2;
 template <int MODE>
 __global__ void __launch_bounds__(64 * kMarchWaves) k_spmv(SolveArgs S, MarchPlan m, const uint16_t* __restrict__ nbinfo,
                                                            const float* __restrict__ z, const float* __restrict__ s,
-                                                           float* __restrict__ s_new, float* __restrict__ q, Reduce red) {
+                                                           float* __restrict__ s_new, float* __restrict__ q, Reduce red,
+                                                           SpmvDot dot) {
+    if (MODE != SPMV_PLAIN && blockIdx.x >= gridDim.x - dot.blocks) {
+        const double zr = dot_part(Part{blockIdx.x - (gridDim.x - dot.blocks), dot.blocks}, dot.n, dot.flags, z, dot.r);
+        block_finish<AUX_SUM, 64 * kMarchWaves>(0.0, zr, red);
+        return;
+    }
     double d = 0.0;
     const float ms = -S.scale_f;
     const float beta = MODE == SPMV_XPAY ? (float)red.sc->beta : 0.f;
@@ -330,7 +344,7 @@ __global__ void __launch_bounds__(64 * kMarchWaves) k_spmv(SolveArgs S, MarchPla
         f32x4 s, z;
     };
     march(
-        m, S.ny, S.nz, S.nxp, nbinfo,
+        m, gridDim.x - dot.blocks, S.ny, S.nz, S.nxp, nbinfo,
         [&](int64_t j) {
             Raw v;
             if constexpr (MODE != SPMV_COPY) v.s = *reinterpret_cast<const f32x4*>(s + j);
@@ -365,7 +379,8 @@ __global__ void __launch_bounds__(64 * kMarchWaves) k_spmv(SolveArgs S, MarchPla
             *reinterpret_cast<f32x4*>(q + j) = out;
             if (MODE != SPMV_PLAIN) *reinterpret_cast<f32x4*>(s_new + j) = snew;
         });
-    block_finish<AUX_NONE, 64 * kMarchWaves>(d, 0.0, red);
+    if constexpr (MODE == SPMV_PLAIN) block_finish<AUX_NONE, 64 * kMarchWaves>(d, 0.0, red);
+    else block_finish<AUX_SUM, 64 * kMarchWaves>(d, 0.0, red);
 }
 
 // Large blocks: every block takes a ticket from one counter at its end, and
@@ -404,20 +419,7 @@ __global__ void __launch_bounds__(NT) k_dot_self(int64_t n, const uint32_t* __re
 // a . b (FP64 products of the FP32 values)
 __global__ void __launch_bounds__(kStream) k_dot(int64_t n, const uint32_t* __restrict__ flags,
                                                 const float* __restrict__ a, const float* __restrict__ b, Reduce red) {
-    double d = 0.0;
-    for_flagged_chunks<2>(
-        whole_grid(), n, flags,
-        [&](int64_t i, float4(&v)[2]) {
-            v[0] = *reinterpret_cast<const float4*>(a + i);
-            v[1] = *reinterpret_cast<const float4*>(b + i);
-        },
-        [&](int64_t i, float4(&v)[2]) {
-            d += (double)v[0].x * (double)v[1].x;
-            d += (double)v[0].y * (double)v[1].y;
-            d += (double)v[0].z * (double)v[1].z;
-            d += (double)v[0].w * (double)v[1].w;
-        });
-    block_finish<AUX_NONE, kStream>(d, 0.0, red);
+    block_finish<AUX_NONE, kStream>(dot_part(whole_grid(), n, flags, a, b), 0.0, red);
 }
 
 // z . r and z . q: z is read once, and one launch and its tickets are saved
@@ -764,20 +766,32 @@ static int dot_with(fsim_ctx* ctx, const float* a, const float* b, int op) {
     return FSIM_OK;
 }
 
+// Blocks beside the product's for z.r, of two trips a wave up to their limit: each takes a ticket of the reduction, and
+// fewer end after the product.  us a launch of both with 1 / 2 / 4 / 8 trips: 64^3 11.6 / 10.9 / 11.1 / 14.4, 96^3 16.2 /
+// 15.2 / 15.5 / 19.5, 128^3 19.1 / 19.5 / 19.4 / 21.2; with a limit of 64 / 128 / 256 / 384 / 512 blocks: 256^3 143 / 91
+// / 71 / 75 / 73.  The product alone takes 10.3, 14.2, 17.9 and 63, a launch of its own for z.r 6 to 18.
+static unsigned dot_blocks(int64_t n) {
+    const unsigned per = 2 * kUnits * kMarchWaves;
+    const unsigned need = (unsigned)((n / kChunk + per - 1) / per);
+    return std::max(1u, std::min<unsigned>(need, kBesideMarch));
+}
+
 // New search direction s (z, or z + beta s) into the second buffer, q = A s,
 // s.q -> alpha.
-static int direction_step(fsim_ctx* ctx, const SolveArgs& S, bool copy) {
+static int direction_step(fsim_ctx* ctx, const SolveArgs& S, bool copy, const float* r) {
     {
         FSIM_PROF(ctx, KID_SPMV);
         const MarchPlan m = march_of(S.ny, S.nz, S.nxp);
-        const dim3 grid(march_blocks(m)), block(64 * kMarchWaves);
-        const Reduce red = reduce_to(ctx, FIN_ALPHA);
+        SpmvDot dot;
+        if (r) dot = SpmvDot{dot_blocks(S.ncr), S.ncr, ctx->chunk_flags, r};
+        const dim3 grid(march_blocks(m) + dot.blocks), block(64 * kMarchWaves);
+        const Reduce red = reduce_to(ctx, r ? FIN_ALPHA_ZR : FIN_ALPHA);
         if (copy)
             hipLaunchKernelGGL(k_spmv<SPMV_COPY>, grid, block, 0, ctx->stream, S, m, ctx->nbinfo, ctx->z, ctx->s, ctx->s2,
-                               ctx->q, red);
+                               ctx->q, red, dot);
         else
             hipLaunchKernelGGL(k_spmv<SPMV_XPAY>, grid, block, 0, ctx->stream, S, m, ctx->nbinfo, ctx->z, ctx->s, ctx->s2,
-                               ctx->q, red);
+                               ctx->q, red, dot);
     }
     FSIM_HIP(ctx, hipGetLastError());
     std::swap(ctx->s, ctx->s2);
@@ -807,19 +821,20 @@ static bool stop_met(const fsim_ctx* ctx, double ss, double mx, double bnorm) {
 // beta, and x if two steps are due.
 //
 // MIC(0): the r update and its norms run beside the forward sweep, which
-// computes the new r for itself, and sigma and the x update beside the backward
+// computes the new r for itself, and t.t and the x update beside the backward
 // sweep: the sweeps are chains of waits that leave most of the chip idle.
-// sigma = z.r = r^T L^-T L^-1 r = t.t with t = L^-1 r, the forward sweep's
-// result, which is there before the backward sweep starts.  Summed in FP64,
-// it is off by the FP32 rounding inside the sweeps, where the rounding of alpha
-// and beta to FP32 may take 6e-8 (mean error against 64 bits of t.t and z.r,
-// random and smooth r: 8^3 3.5e-8 / 6.3e-8 and 1.6e-8 / 1.6e-8, 24^3 3.4e-9 /
-// 5.5e-9 and 1.5e-9 / 3.5e-9, 64^3 9e-10 / 2.1e-9 and 6e-10 / 1.5e-9, 128^3
-// 2.6e-10 / 1.4e-9 and 1.7e-10 / 1.4e-9, 2D 128^2 3.9e-9 / 5.3e-9 and 2.4e-9 /
-// 5.1e-9).  r has two buffers, since the tiles read the old one.
+// z'.r' = r'^T L^-T L^-1 r' = t.t with t = L^-1 r', the forward sweep's result,
+// which is there before the backward sweep starts: beta = t.t / z.r, which the
+// product takes rounded to FP32 (6e-8; t.t is off by the FP32 rounding inside
+// the sweeps, mean error against 64 bits with random and smooth r' 24^3 3.4e-9 /
+// 5.5e-9, 64^3 9e-10 / 2.1e-9, 128^3 2.6e-10 / 1.4e-9, 2D 128^2 3.9e-9 / 5.3e-9).
+// alpha, which x takes in FP64, has z.r itself, of the z that is used: with
+// t.t there 4 steps of the 128^3 dam break took 333 iterations instead of 330,
+// 256^3 588 instead of 586.  r has two buffers, since the tiles read the old
+// one.
 // An iteration, against launches of their own for the r update, the dot
 // product and the x update (the last on a second stream at 256^3): 32^3 62 ->
-// 49 us, 2D 128^2 100 -> 86, 128^3 132 -> 114, 256^3 395 -> 378.
+// 49 us, 2D 128^2 100 -> 86, 128^3 132 -> 115, 256^3 395 -> 386.
 static int update_mic(fsim_ctx* ctx, const SolveArgs& S, float** r, float** r_next, bool x_due) {
     SideWork fwd, bwd;
     fwd.blocks = bwd.blocks = side_blocks(S.ncr);
@@ -866,13 +881,7 @@ static int precondition(fsim_ctx* ctx, const SolveArgs& S, const float* r, bool 
         FSIM_TRY(mg_apply(ctx, ctx->r, ctx->z, S.scale));
         return dot_with(ctx, ctx->z, ctx->r, FIN_SIGMA0);
     }
-    SideWork bwd;
-    bwd.blocks = side_blocks(S.ncr);
-    bwd.n = S.ncr;
-    bwd.flags = ctx->chunk_flags;
-    bwd.t = ctx->t;
-    bwd.red = reduce_to(ctx, FIN_SIGMA0);
-    return mic_apply(ctx, S, r, ctx->t, ctx->z, nullptr, &bwd);
+    return mic_apply(ctx, S, r, ctx->t, ctx->z);   // sigma comes with the matrix product
 }
 
 struct PcgResult {
@@ -914,7 +923,7 @@ static int pcg_run(fsim_ctx* ctx, const SolveArgs& S, double bnorm, bool flexibl
     res->converged = false;
     res->nan = false;
     for (; it < max_it; it++) {
-        FSIM_TRY(direction_step(ctx, S, copy));
+        FSIM_TRY(direction_step(ctx, S, copy, flexible ? nullptr : r));
         const bool two = ++behind == 2;
         if (two) behind = 0;
         if (flexible) FSIM_TRY(update_flexible(ctx, S, two));
@@ -1221,7 +1230,7 @@ int solver_apply(fsim_ctx* ctx, int op, double dt, const double* in, double* out
         FSIM_TRY(fill_f32(ctx, ctx->q, 0.0f, n));   // the SpMV skips columns without WATER
         const MarchPlan m = march_of(S.ny, S.nz, S.nxp);
         hipLaunchKernelGGL(k_spmv<SPMV_PLAIN>, dim3(march_blocks(m)), dim3(64 * kMarchWaves), 0, ctx->stream, S, m,
-                           ctx->nbinfo, nullptr, ctx->r, nullptr, ctx->q, reduce_to(ctx, FIN_NONE));
+                           ctx->nbinfo, nullptr, ctx->r, nullptr, ctx->q, reduce_to(ctx, FIN_NONE), SpmvDot{});
         FSIM_HIP(ctx, hipGetLastError());
         return result(ctx->q);
     }
