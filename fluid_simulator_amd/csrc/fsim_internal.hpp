@@ -422,8 +422,10 @@ int fill_i32(fsim_ctx* ctx, int32_t* p, int32_t v, int64_t n);
 // ---- pressure solve (fsim_solver.hip) -------------------------------------
 int stage_solve(fsim_ctx* ctx, double dt);
 // WAVE_FWD_UPDATE: the forward sweep of in - alpha side->q; side: null or what further blocks do (fsim_reduce.hpp)
-// WAVE_FWD and WAVE_BWD_ALONE: the sweeps outside an iteration, which hold the cells off WATER at 0 whatever the input
-enum WaveKind { WAVE_FACTOR = 0, WAVE_FWD = 1, WAVE_BWD = 2, WAVE_FWD_UPDATE = 3, WAVE_BWD_ALONE = 4 };
+// WAVE_FWD_ALONE and WAVE_BWD_ALONE: the sweeps outside a solve, which hold the cells off WATER at 0 whatever the input
+enum WaveKind {
+    WAVE_FACTOR = 0, WAVE_FWD = 1, WAVE_BWD = 2, WAVE_FWD_UPDATE = 3, WAVE_FWD_ALONE = 4, WAVE_BWD_ALONE = 5
+};
 struct SideWork;
 int wave_launch(fsim_ctx* ctx, WaveKind kind, const float* in, float* out, double scale, const SideWork* side);
 int wave_init(fsim_ctx* ctx);

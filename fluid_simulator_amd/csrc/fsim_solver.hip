@@ -708,17 +708,17 @@ static unsigned side_blocks(int64_t n) {
 // t = L^-1 r and z = L^-T t, M = L L^T.
 // fwd: r -= alpha q on the way (side work of the forward sweep, the new r goes
 // to fwd->r_next); bwd: t . t and x (side work of the backward sweep).  Null:
-// none.  One launch per plane does the side work in launches of their own,
-// with the same blocks and so the same bits.
+// none.  alone: outside a solve.  One launch per plane does the side work in
+// launches of their own, with the same blocks and so the same bits.
 static int mic_apply(fsim_ctx* ctx, const SolveArgs& S, const float* r, float* t, float* z, const SideWork* fwd = nullptr,
-                     const SideWork* bwd = nullptr) {
+                     const SideWork* bwd = nullptr, bool alone = false) {
     if (ctx->sweep_mode == 0) {
         {
             FSIM_PROF(ctx, KID_SWEEP_FWD);
-            FSIM_TRY(wave_launch(ctx, fwd ? WAVE_FWD_UPDATE : WAVE_FWD, r, t, S.scale, fwd));
+            FSIM_TRY(wave_launch(ctx, fwd ? WAVE_FWD_UPDATE : alone ? WAVE_FWD_ALONE : WAVE_FWD, r, t, S.scale, fwd));
         }
         FSIM_PROF(ctx, KID_SWEEP_BWD);
-        return wave_launch(ctx, bwd ? WAVE_BWD : WAVE_BWD_ALONE, t, z, S.scale, bwd);
+        return wave_launch(ctx, alone ? WAVE_BWD_ALONE : WAVE_BWD, t, z, S.scale, bwd);
     }
     if (fwd) {
         hipLaunchKernelGGL((k_update_r<WF_THREADS, false>), dim3(fwd->blocks), dim3(WF_THREADS), 0, ctx->stream, fwd->n,
@@ -1238,7 +1238,7 @@ int solver_apply(fsim_ctx* ctx, int op, double dt, const double* in, double* out
         FSIM_TRY(mic_factor(ctx, S));
         FSIM_TRY(fill_f32(ctx, ctx->t, 0.0f, n));
         FSIM_TRY(fill_f32(ctx, ctx->z, 0.0f, n));
-        FSIM_TRY(mic_apply(ctx, S, ctx->r, ctx->t, ctx->z));
+        FSIM_TRY(mic_apply(ctx, S, ctx->r, ctx->t, ctx->z, nullptr, nullptr, true));
         FSIM_TRY(check_wave_err(ctx));
         return result(ctx->z);
     }

@@ -105,8 +105,8 @@ constexpr int kVolatile = (int)0x80000000;    // a buffer load that is neither m
 template <int KIND>
 struct Kind {   // WaveKind: the sweeps (FP32)
     using T = float;
-    static constexpr bool FWD = KIND == WAVE_FWD || KIND == WAVE_FWD_UPDATE;
-    static constexpr bool MASK = KIND == WAVE_FWD || KIND == WAVE_BWD_ALONE;   // on_water
+    static constexpr bool FWD = KIND == WAVE_FWD || KIND == WAVE_FWD_UPDATE || KIND == WAVE_FWD_ALONE;
+    static constexpr bool MASK = KIND == WAVE_FWD_ALONE || KIND == WAVE_BWD_ALONE;   // on_water
     static constexpr int NP = 1;     // 32-bit words per value
 };
 template <>
@@ -424,9 +424,9 @@ __device__ void send_wave(const WaveArgs& A, WaveLds<KIND>& S, const Tile& T) {
 // 0 by itself while every value is finite.  What is not finite (an input, or
 // the infinite factor of a WATER cell between SOLID ones) would pass through
 // AIR and SOLID cells to WATER that does not depend on it, which the sweeps
-// outside an iteration (WAVE_FWD, WAVE_BWD_ALONE) keep from it by a select.  In
-// an iteration it makes s.q and alpha NaN and the solve ends with the pressure
-// of before, wherever else it has been; there the select, a comparison and a
+// outside a solve (WAVE_FWD_ALONE, WAVE_BWD_ALONE) keep from it by a select.  In
+// a solve it makes s.q and alpha NaN and the solve ends with the pressure of
+// before, wherever else it has been; there the select, a comparison and a
 // move on the chain of every cell, costs a frame 32^3 1.17 -> 1.26 ms, 128^3
 // APIC 12.3 -> 12.9, 256^3 148 -> 151.
 template <int KIND>
@@ -710,11 +710,11 @@ __global__ void __launch_bounds__(WF_THREADS) k_wave(WaveArgs A, SideWork W) {
     using KD = Kind<KIND>;
     constexpr int NP = KD::NP;
     const unsigned tiles = gridDim.x - W.blocks;
-    if (KIND >= WAVE_BWD && blockIdx.x >= tiles) {
+    if (blockIdx.x >= tiles) {
         const Part part{blockIdx.x - tiles, W.blocks};
         if constexpr (KIND == WAVE_FWD_UPDATE) {
             update_r<WF_THREADS>(part, W.n, W.flags, W.q, W.r, W.r_next, W.red);
-        } else {
+        } else if constexpr (KIND == WAVE_BWD) {
             dot_self<WF_THREADS>(part, W.n, W.flags, W.t, W.red);
             if (W.x_steps == 2) update_x_chunks<2>(part, W.n, W.flags, W.x, W.red.sc);
         }
@@ -833,7 +833,7 @@ __global__ void __launch_bounds__(WF_THREADS) k_wave_2d(WaveArgs A, SideWork W) 
         const Part part{blockIdx.x - 1, W.blocks};
         if constexpr (UPD) {
             update_r<WF_THREADS>(part, W.n, W.flags, W.q, W.r, W.r_next, W.red);
-        } else if constexpr (!FWD) {
+        } else if constexpr (KIND == WAVE_BWD) {
             dot_self<WF_THREADS>(part, W.n, W.flags, W.t, W.red);
             if (W.x_steps == 2) update_x_chunks<2>(part, W.n, W.flags, W.x, W.red.sc);
         }
@@ -956,13 +956,14 @@ int wave_launch(fsim_ctx* ctx, WaveKind kind, const float* in, float* out, doubl
         const size_t lds = lds_2d(A.ny, A.nxp);
         if (kind == WAVE_FWD) hipLaunchKernelGGL(k_wave_2d<WAVE_FWD>, grid, block, lds, ctx->stream, A, W);
         else if (kind == WAVE_BWD) hipLaunchKernelGGL(k_wave_2d<WAVE_BWD>, grid, block, lds, ctx->stream, A, W);
+        else if (kind == WAVE_FWD_ALONE) hipLaunchKernelGGL(k_wave_2d<WAVE_FWD_ALONE>, grid, block, lds, ctx->stream, A, W);
         else if (kind == WAVE_BWD_ALONE) hipLaunchKernelGGL(k_wave_2d<WAVE_BWD_ALONE>, grid, block, lds, ctx->stream, A, W);
         else hipLaunchKernelGGL(k_wave_2d<WAVE_FWD_UPDATE>, grid, block, lds, ctx->stream, A, W);
         FSIM_HIP(ctx, hipGetLastError());
         return FSIM_OK;
     }
     const unsigned ntiles = (unsigned)(A.TJ * A.TK);
-    const int counter = kind == WAVE_FWD_UPDATE ? WAVE_FWD : kind == WAVE_BWD_ALONE ? WAVE_BWD : kind;
+    const int counter = kind == WAVE_FACTOR ? 0 : kind == WAVE_BWD || kind == WAVE_BWD_ALONE ? 2 : 1;
     A.ticket = ctx->wave_ticket + counter;
     A.ticket_base = ctx->wave_ticket_base[counter];
     ctx->wave_ticket_base[counter] += ntiles;
@@ -974,6 +975,7 @@ int wave_launch(fsim_ctx* ctx, WaveKind kind, const float* in, float* out, doubl
     case WAVE_FACTOR: hipLaunchKernelGGL(k_wave<WAVE_FACTOR>, grid, block, 0, ctx->stream, A, W); break;
     case WAVE_FWD: hipLaunchKernelGGL(k_wave<WAVE_FWD>, grid, block, 0, ctx->stream, A, W); break;
     case WAVE_BWD: hipLaunchKernelGGL(k_wave<WAVE_BWD>, grid, block, 0, ctx->stream, A, W); break;
+    case WAVE_FWD_ALONE: hipLaunchKernelGGL(k_wave<WAVE_FWD_ALONE>, grid, block, 0, ctx->stream, A, W); break;
     case WAVE_BWD_ALONE: hipLaunchKernelGGL(k_wave<WAVE_BWD_ALONE>, grid, block, 0, ctx->stream, A, W); break;
     case WAVE_FWD_UPDATE: hipLaunchKernelGGL(k_wave<WAVE_FWD_UPDATE>, grid, block, 0, ctx->stream, A, W); break;
     }
