@@ -96,11 +96,12 @@ struct ConvArgs {
     int64_t part_cap;     // floats in part
 };
 
-// AHEAD: K chunks whose operands are loaded before the first one's product.  A
-// chunk's loads take about a microsecond (weights and activations come from
-// the L2), and a wave of a small level has nobody beside it to hide that.
-// us at 16^3, with four voxel tiles a wave and two chunks ahead before: 8 -> 16
-// 11.8 -> 6.1, 16 -> 32 19.1 -> 11.4, 48 -> 16 7.9 -> 5.8, 192 -> 64 7.6 -> 6.2.
+// AHEAD: K chunks whose operands are loaded, without branches, before the first
+// one's product; 0: each chunk's before its own, the compiler's unrolling by
+// two, and no load for a value outside the grid.  A chunk's loads take about a
+// microsecond (weights and activations come from the L2), and a wave of a small
+// level has nobody beside it to hide that; where the chip is full, loads that
+// nobody uses and operands that fewer tiles share cost more (conv3_launch).
 template <int CIN, int CU, int NT, int MT, int AHEAD, bool OUT_F32>
 __global__ void __launch_bounds__(256) k_conv3(ConvArgs a) {
     constexpr int KTOT = 27 * CIN;
@@ -136,17 +137,16 @@ __global__ void __launch_bounds__(256) k_conv3(ConvArgs a) {
     // split K: block z sums the K chunks of its slice (one slice: all of them)
     const int cps = (NCH + (int)gridDim.z - 1) / (int)gridDim.z;
     const int c_lo = (int)blockIdx.z * cps, c_hi = min(NCH, c_lo + cps);
-    for (int cb = c_lo; cb < c_hi; cb += AHEAD) {
-        bf16x8 av[AHEAD][MT], bv[AHEAD][NT];
-#pragma unroll
-        for (int u = 0; u < AHEAD; u++) {
-            const int c = cb + u;
+    if constexpr (AHEAD == 0) {
+#pragma unroll 2
+        for (int c = c_lo; c < c_hi; c++) {
             const int k0 = 32 * c + 8 * kq;
-            const bool kin = c < c_hi && ((KTOT % 32 == 0) || k0 < KTOT);
+            const bool kin = (KTOT % 32 == 0) || k0 < KTOT;
             const int t = k0 / CIN, ci = k0 - t * CIN;
             const int dx = t / 9 - 1, dy = (t / 3) % 3 - 1, dz = t % 3 - 1;
             const bool up = CU > 0 && ci < CU;
             const int64_t toff = (((int64_t)dx * a.H + dy) * a.W + dz) * CS + (ci - CU);
+            bf16x8 av[MT], bv[NT];
 #pragma unroll
             for (int m = 0; m < MT; m++) {
                 const int xx = xs[m] + dx, yy = ys[m] + dy, zz = zs[m] + dz;
@@ -154,24 +154,55 @@ __global__ void __launch_bounds__(256) k_conv3(ConvArgs a) {
                                 (unsigned)zz < (unsigned)a.W;
                 const __bf16* src = xl[m] + toff;
                 if (up) src = a.xc + (((int64_t)(xx >> 1) * Hc + (yy >> 1)) * Wc + (zz >> 1)) * (CU > 0 ? CU : 1) + ci;
-                // a lane without a value reads the weights' first ones, so that no load waits for a branch
-                const bf16x8 got = *reinterpret_cast<const bf16x8*>(ok ? src : a.w);
-                av[u][m] = ok ? got : zero;
+                av[m] = ok ? *reinterpret_cast<const bf16x8*>(src) : zero;
             }
 #pragma unroll
-            for (int j = 0; j < NT; j++) {
-                const bf16x8 got = *reinterpret_cast<const bf16x8*>(kin ? wl + (int64_t)16 * j * KTOT + 32 * c : a.w);
-                bv[u][j] = kin ? got : zero;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < AHEAD; u++) {
-            if (cb + u >= c_hi) break;
+            for (int j = 0; j < NT; j++)
+                bv[j] = kin ? *reinterpret_cast<const bf16x8*>(wl + (int64_t)16 * j * KTOT + 32 * c) : zero;
 #pragma unroll
             for (int m = 0; m < MT; m++)
 #pragma unroll
                 for (int j = 0; j < NT; j++)
-                    acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[u][m], bv[u][j], acc[m][j], 0, 0, 0);
+                    acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[m], bv[j], acc[m][j], 0, 0, 0);
+        }
+    } else {
+        for (int cb = c_lo; cb < c_hi; cb += AHEAD) {
+            bf16x8 av[AHEAD][MT], bv[AHEAD][NT];
+#pragma unroll
+            for (int u = 0; u < AHEAD; u++) {
+                const int c = cb + u;
+                const int k0 = 32 * c + 8 * kq;
+                const bool kin = c < c_hi && ((KTOT % 32 == 0) || k0 < KTOT);
+                const int t = k0 / CIN, ci = k0 - t * CIN;
+                const int dx = t / 9 - 1, dy = (t / 3) % 3 - 1, dz = t % 3 - 1;
+                const bool up = CU > 0 && ci < CU;
+                const int64_t toff = (((int64_t)dx * a.H + dy) * a.W + dz) * CS + (ci - CU);
+#pragma unroll
+                for (int m = 0; m < MT; m++) {
+                    const int xx = xs[m] + dx, yy = ys[m] + dy, zz = zs[m] + dz;
+                    const bool ok = kin && rin[m] && (unsigned)xx < (unsigned)a.D && (unsigned)yy < (unsigned)a.H &&
+                                    (unsigned)zz < (unsigned)a.W;
+                    const __bf16* src = xl[m] + toff;
+                    if (up) src = a.xc + (((int64_t)(xx >> 1) * Hc + (yy >> 1)) * Wc + (zz >> 1)) * (CU > 0 ? CU : 1) + ci;
+                    // a lane without a value reads the weights' first ones, so that no load waits for a branch
+                    const bf16x8 got = *reinterpret_cast<const bf16x8*>(ok ? src : a.w);
+                    av[u][m] = ok ? got : zero;
+                }
+#pragma unroll
+                for (int j = 0; j < NT; j++) {
+                    const bf16x8 got = *reinterpret_cast<const bf16x8*>(kin ? wl + (int64_t)16 * j * KTOT + 32 * c : a.w);
+                    bv[u][j] = kin ? got : zero;
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < AHEAD; u++) {
+                if (cb + u >= c_hi) break;
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+#pragma unroll
+                    for (int j = 0; j < NT; j++)
+                        acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[u][m], bv[u][j], acc[m][j], 0, 0, 0);
+            }
         }
     }
     if (gridDim.z > 1) {   // raw partial sums; k_conv3_reduce adds the slices, bias and ReLU
@@ -205,20 +236,24 @@ __global__ void __launch_bounds__(256) k_conv3(ConvArgs a) {
     }
 }
 
-// The sum of `count` values `stride` apart, in order, kSumAhead loads at a time: a
-// loop that adds each value as it comes takes a memory latency per value (54
-// slices 17 us, in batches 5).
-constexpr int kSumAhead = 16;
+// The sum of `count` values `stride` apart, in order, 16 loads at a time, and four
+// for a last eight or fewer: a loop that adds each value as it comes takes a
+// memory latency per value (54 slices 17 us, in batches 5), and loads beyond
+// the last value cost large levels (3 slices for 24^3 x 64 values 20 us by 16, 14 by 4).
+template <int N>
+__device__ inline void sum_batch(const float* p, int64_t stride, int k, int count, float& s) {
+    float v[N];
+#pragma unroll
+    for (int j = 0; j < N; j++) v[j] = p[(int64_t)min(k + j, count - 1) * stride];
+#pragma unroll
+    for (int j = 0; j < N; j++)
+        if (k + j < count) s += v[j];
+}
 __device__ inline float sum_in_order(const float* p, int64_t stride, int count) {
     float s = 0.f;
-    for (int k = 0; k < count; k += kSumAhead) {
-        float v[kSumAhead];
-#pragma unroll
-        for (int j = 0; j < kSumAhead; j++) v[j] = p[(int64_t)min(k + j, count - 1) * stride];
-#pragma unroll
-        for (int j = 0; j < kSumAhead; j++)
-            if (k + j < count) s += v[j];
-    }
+    int k = 0;
+    for (; count - k > 8; k += 16) sum_batch<16>(p, stride, k, count, s);
+    for (; k < count; k += 4) sum_batch<4>(p, stride, k, count, s);
     return s;
 }
 
@@ -243,7 +278,6 @@ __global__ void __launch_bounds__(256) k_conv3_reduce(ConvArgs a, int slices) {
 // split: the reduction's launch costs more than their short K loop (measured
 // at 16^3: 8 -> 16, 7 chunks, 10.0 us unsplit, 7.6 + 7.3 us split).
 constexpr int64_t kSplitWaves = 1024;
-constexpr int64_t kSmallWaves = 4096;   // 4 waves a SIMD
 constexpr int kSplitMinChunks = 24;
 constexpr int64_t kConvPartFloats = int64_t(4) << 20;   // 16 MB of split-K partial sums per context
 template <int CIN, int CU, int COUT, int NT, int MT, bool OUT_F32>
@@ -260,13 +294,18 @@ static void conv3_launch(hipStream_t st, const ConvArgs& a) {
         const int64_t cps = (NCH + slices - 1) / slices;   // every slice gets at least one chunk
         slices = (NCH + cps - 1) / cps;
     }
-    // Few waves even so: a voxel tile a wave (the sums are the same), with more chunks of loads ahead than
-    // the registers of a large level's waves would hold.
-    if (all * slices * MT <= kSmallWaves)
+    // Fewer than kSplitWaves waves even so, one a SIMD: a voxel tile a wave (the sums are the same), with more
+    // chunks of loads ahead than the registers of a large level's waves would hold.  us of a layer with MT voxel
+    // tiles a wave and so, by the waves of the former: 8 -> 16 at 16^3 (64 waves) 11.0 / 5.7 and 48^3 (1728) 13.7 /
+    // 13.3; 16 -> 32 in a 64^3 network (512) 18.9 / 10.8, 80^3 (1000) 19.1 / 14.8, 96^3 (1728) 20.6 / 23.2; 48 ->
+    // 16 at 16^3 (704) 8.4 / 6.2, 48^3 (1728) 41 / 50; 96 -> 32 in 16^3 (216) 7.3 / 4.8, 48^3 (1080) 21.8 / 23.4;
+    // 192 -> 64 in 24^3 (378) 7.5 / 6.2, 48^3 (1026) 14.1 / 15.1, 128^3 (1024) 124 / 188.
+    if (all * slices < kSplitWaves)
         hipLaunchKernelGGL((k_conv3<CIN, CU, NT, 1, NT <= 2 ? 7 : 4, OUT_F32>),
                            dim3((unsigned)(((V + 15) / 16 + 3) / 4), COUT / (16 * NT), (unsigned)slices), dim3(256), 0, st, a);
-    else
-        hipLaunchKernelGGL((k_conv3<CIN, CU, NT, MT, 2, OUT_F32>),
+    else   // two chunks ahead where two tiles share the operands (us at 128^3, 32 -> 64 and 192 -> 64: 25 -> 23, 141 ->
+           // 124); with four, and with one, it costs (16 -> 32 28.7 -> 41, 96 -> 32 150 -> 167, 64 -> 128 27.5 -> 30)
+        hipLaunchKernelGGL((k_conv3<CIN, CU, NT, MT, MT == 2 ? 2 : 0, OUT_F32>),
                            dim3((unsigned)((waves + 3) / 4), COUT / (16 * NT), (unsigned)slices), dim3(256), 0, st, a);
     if (slices > 1)
         hipLaunchKernelGGL((k_conv3_reduce<OUT_F32>), dim3((unsigned)((V * COUT + 255) / 256)), dim3(256), 0, st, a,
